@@ -375,7 +375,10 @@ static int alloc_context(tsph_ctx *c) {
   if ((e = dalloc(&c->scal, S_NSCAL + (size_t)kCostTables * (nct + 8))) ||
       (e = dalloc(&c->cell_count, nct + 1)) || (e = dalloc(&c->cell_start, nct + 2)) ||
       (e = dalloc(&c->cell_start_next, nct + 2)) ||
-      (e = dalloc(&c->cellof, cap)) || (e = dalloc(&c->hrank, cap)) || (e = dalloc(&c->hcell, cap)) ||
+      (e = dalloc(&c->cellof, cap)) ||
+      // (hcell and hrank also serve the download's bitmap over the positions)
+      (e = dalloc(&c->hrank, std::max<size_t>(cap, dl_words(c->seq_cap)))) ||
+      (e = dalloc(&c->hcell, std::max<size_t>(cap, dl_words(c->seq_cap)))) ||
       (e = dalloc(&c->perm, cap)) || (e = dalloc(&c->arrival, cap)) ||
       (e = dalloc(&c->arrival_seq, cap)) || (e = dalloc(&c->arrival_span, cap)) ||
       (e = dalloc(&c->seqstate, (size_t)c->seq_cap)) || (e = dalloc(&c->probe_out, 4)) ||
@@ -526,40 +529,40 @@ static int upload_impl(tsph_ctx *c, const tsph_particles *h, const uint32_t *seq
   TSPH_HIP(hipStreamSynchronize(c->stream));
   drop_graph(c);
   std::vector<uint8_t> t(n);
-  std::vector<uint32_t> seq(n);
-  std::vector<int32_t> idx(n);
   for (int i = 0; i < n; ++i) {
     if (h->type[i] < 0 || h->type[i] > 254) return fail(TSPH_EINVAL, "particle type out of range");
     t[i] = (uint8_t)h->type[i];
-    seq[i] = seq_in ? seq_in[i] : (uint32_t)i;
-    idx[i] = h->index ? h->index[i] : i;
   }
-  std::vector<double> zeros(2 * (size_t)n, 0.0);
   const size_t s1 = sizeof(double) * n, s2 = 2 * s1;
   Soa &d = c->cur;
+  // host fields over PCIe; the fields a caller leaves out are filled on the
+  // device (zeros, or what Add_particle sets: the old values equal to the new)
   auto cp = [&](void *dst, const void *src, size_t bytes) {
-    return hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice);
+    return hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c->stream);
   };
-  const double *v = h->v ? h->v : zeros.data();
-  const double *p = h->p ? h->p : zeros.data();
+  auto put = [&](void *dst, const void *src, const void *like, size_t bytes) {
+    if (src) return cp(dst, src, bytes);
+    if (like) return hipMemcpyAsync(dst, like, bytes, hipMemcpyDeviceToDevice, c->stream);
+    return hipMemsetAsync(dst, 0, bytes, c->stream);
+  };
   if (n > 0) {
     TSPH_HIP(cp(d.r, h->r, s2));
-    TSPH_HIP(cp(d.v, v, s2));
-    TSPH_HIP(cp(d.a, h->a ? h->a : zeros.data(), s2));
-    TSPH_HIP(cp(d.r_o, h->r_o ? h->r_o : h->r, s2));
-    TSPH_HIP(cp(d.v_o, h->v_o ? h->v_o : v, s2));
+    TSPH_HIP(put(d.v, h->v, nullptr, s2));
+    TSPH_HIP(put(d.a, h->a, nullptr, s2));
+    TSPH_HIP(put(d.r_o, h->r_o, d.r, s2));
+    TSPH_HIP(put(d.v_o, h->v_o, d.v, s2));
     TSPH_HIP(cp(d.rho, h->rho, s1));
-    TSPH_HIP(cp(d.drho, h->drho ? h->drho : zeros.data(), s1));
-    TSPH_HIP(cp(d.p, p, s1));
-    TSPH_HIP(cp(d.rho_o, h->rho_o ? h->rho_o : h->rho, s1));
+    TSPH_HIP(put(d.drho, h->drho, nullptr, s1));
+    TSPH_HIP(put(d.p, h->p, nullptr, s1));
+    TSPH_HIP(put(d.rho_o, h->rho_o, d.rho, s1));
     TSPH_HIP(cp(d.type, t.data(), n));
-    TSPH_HIP(cp(d.seq, seq.data(), 4 * (size_t)n));
-    TSPH_HIP(cp(d.index, idx.data(), 4 * (size_t)n));
+    if (seq_in) TSPH_HIP(cp(d.seq, seq_in, 4 * (size_t)n));
+    else if ((e = launch_iota(c, reinterpret_cast<int *>(d.seq), n))) return e;
+    if (h->index) TSPH_HIP(cp(d.index, h->index, 4 * (size_t)n));
+    else if ((e = launch_iota(c, d.index, n))) return e;
     if (cid) TSPH_HIP(cp(d.cid, cid, n));
-    if (h->gnr) TSPH_HIP(cp(d.gnr, h->gnr, s2));
-    else if (c->has_gnr) TSPH_HIP(cp(d.gnr, zeros.data(), s2));
-    if (h->n) TSPH_HIP(cp(d.n, h->n, s2));
-    else if (c->has_n) TSPH_HIP(cp(d.n, zeros.data(), s2));
+    if (h->gnr || c->has_gnr) TSPH_HIP(put(d.gnr, h->gnr, nullptr, s2));
+    if (h->n || c->has_n) TSPH_HIP(put(d.n, h->n, nullptr, s2));
   }
   if (d.rc) {  // compensation starts from zero
     TSPH_HIP(hipMemsetAsync(d.rc, 0, sizeof(double2) * (size_t)c->capacity, c->stream));
@@ -569,7 +572,7 @@ static int upload_impl(tsph_ctx *c, const tsph_particles *h, const uint32_t *seq
   sc[S_NP] = n;
   sc[S_MAXSEQ] = maxseq;
   c->seq_ub = maxseq;
-  TSPH_HIP(hipMemcpy(c->scal, sc, sizeof sc, hipMemcpyHostToDevice));
+  TSPH_HIP(cp(c->scal, sc, sizeof sc));
   TSPH_HIP(hipMemsetAsync(c->seqstate, 0, (size_t)c->seq_cap, c->stream));
   TSPH_HIP(hipStreamSynchronize(c->stream));
   c->n_ub = n;
@@ -604,24 +607,18 @@ int tsph_get_np(tsph_ctx *c, int *np) {
 
 namespace tsph {
 
-// order of the live slots in reference order (by seq), skipping removed ones;
-// icase >= 0 keeps the slots of that case of a batched context only
-static int live_order(tsph_ctx *c, int n, int icase, std::vector<int> &order,
-                      std::vector<uint32_t> &seq, std::vector<uint8_t> &type) {
+// order of the live slots in reference order (by seq), skipping removed ones
+static int live_order(tsph_ctx *c, int n, std::vector<int> &order, std::vector<uint32_t> &seq,
+                      std::vector<uint8_t> &type) {
   seq.resize(n);
   type.resize(n);
-  std::vector<uint8_t> cid;
   if (n > 0) {
     TSPH_HIP(hipMemcpy(seq.data(), c->cur.seq, 4 * (size_t)n, hipMemcpyDeviceToHost));
     TSPH_HIP(hipMemcpy(type.data(), c->cur.type, n, hipMemcpyDeviceToHost));
-    if (icase >= 0) {
-      cid.resize(n);
-      TSPH_HIP(hipMemcpy(cid.data(), c->cur.cid, n, hipMemcpyDeviceToHost));
-    }
   }
   order.clear();
   for (int i = 0; i < n; ++i)
-    if (type[i] != kRemoved && (icase < 0 || cid[i] == icase)) order.push_back(i);
+    if (type[i] != kRemoved) order.push_back(i);
   std::sort(order.begin(), order.end(), [&](int a, int b) { return seq[a] < seq[b]; });
   return 0;
 }
@@ -643,7 +640,7 @@ static int renumber_seq(tsph_ctx *c) {
   std::vector<int> order;
   std::vector<uint32_t> seq;
   std::vector<uint8_t> type;
-  if ((e = live_order(c, n, -1, order, seq, type))) return e;
+  if ((e = live_order(c, n, order, seq, type))) return e;
   std::vector<uint8_t> st((size_t)c->seq_cap), nst((size_t)c->seq_cap, 0);
   TSPH_HIP(hipMemcpy(st.data(), c->seqstate, (size_t)c->seq_cap, hipMemcpyDeviceToHost));
   std::vector<uint32_t> nseq((size_t)std::max(n, 1));
@@ -681,50 +678,43 @@ static int seq_room(tsph_ctx *c, int *passes) {
 }
 
 static int download_impl(tsph_ctx *c, tsph_particles *h, int icase) {
-  int n = 0, e = 0;
+  int n[2] = {0, 0}, e = 0;
   if ((e = ensure_olds(c))) return e;
+  const Soa &d = c->alt;  // the gathered fields
+  struct Field {
+    unsigned bit;
+    double *to;
+    const void *from;
+    int width;
+  } fields[] = {{DL_P, h->p, d.p, 1},          {DL_RHO, h->rho, d.rho, 1},
+                {DL_DRHO, h->drho, d.drho, 1}, {DL_RHO_O, h->rho_o, d.rho_o, 1},
+                {DL_R, h->r, d.r, 2},          {DL_V, h->v, d.v, 2},
+                {DL_A, h->a, d.a, 2},          {DL_R_O, h->r_o, d.r_o, 2},
+                {DL_V_O, h->v_o, d.v_o, 2},    {DL_GNR, h->gnr, d.gnr, 2},
+                {DL_N, h->n, d.n, 2}};
+  unsigned mask = (h->type ? DL_TYPE : 0u) | (h->index ? DL_INDEX : 0u);
+  for (const Field &f : fields)
+    if (f.to && f.from) mask |= f.bit;
+  if ((e = launch_download_gather(c, icase, mask))) return e;
+  TSPH_HIP(hipMemcpyAsync(&n[0], &c->scal[S_NP], sizeof(int), hipMemcpyDeviceToHost, c->stream));
+  TSPH_HIP(hipMemcpyAsync(&n[1], &c->scal[S_DLNP], sizeof(int), hipMemcpyDeviceToHost, c->stream));
   TSPH_HIP(hipStreamSynchronize(c->stream));
-  TSPH_HIP(hipMemcpy(&n, &c->scal[S_NP], sizeof(int), hipMemcpyDeviceToHost));
-  std::vector<int> order;
-  std::vector<uint32_t> seq;
-  std::vector<uint8_t> type;
-  if ((e = live_order(c, n, icase, order, seq, type))) return e;
-  const int m = (int)order.size();
+  const int m = n[0] > 0 ? n[1] : 0;
   h->np = m;
-  std::vector<double> b1(n), b2(2 * (size_t)n);
-  auto get1 = [&](double *dst, const double *src) -> int {
-    if (!dst) return 0;
-    TSPH_HIP(hipMemcpy(b1.data(), src, sizeof(double) * n, hipMemcpyDeviceToHost));
-    for (int k = 0; k < m; ++k) dst[k] = b1[order[k]];
-    return 0;
+  if (m == 0) return 0;
+  auto get = [&](void *to, const void *from, size_t bytes) {
+    return hipMemcpyAsync(to, from, bytes, hipMemcpyDeviceToHost, c->stream);
   };
-  auto get2 = [&](double *dst, const double2 *src) -> int {
-    if (!dst) return 0;
-    if (!src) {
-      std::fill(dst, dst + 2 * (size_t)m, 0.0);
-      return 0;
-    }
-    TSPH_HIP(hipMemcpy(b2.data(), src, 2 * sizeof(double) * n, hipMemcpyDeviceToHost));
-    for (int k = 0; k < m; ++k) {
-      dst[2 * k] = b2[2 * order[k]];
-      dst[2 * k + 1] = b2[2 * order[k] + 1];
-    }
-    return 0;
-  };
-  if (n == 0) return 0;
-  const Soa &d = c->cur;
-  if ((e = get1(h->p, d.p)) || (e = get1(h->rho, d.rho)) || (e = get1(h->drho, d.drho)) ||
-      (e = get1(h->rho_o, d.rho_o)) || (e = get2(h->r, d.r)) || (e = get2(h->v, d.v)) ||
-      (e = get2(h->a, d.a)) || (e = get2(h->r_o, d.r_o)) || (e = get2(h->v_o, d.v_o)) ||
-      (e = get2(h->gnr, d.gnr)) || (e = get2(h->n, d.n)))
-    return e;
-  if (h->type)
-    for (int k = 0; k < m; ++k) h->type[k] = type[order[k]];
-  if (h->index) {
-    std::vector<int32_t> idx(n);
-    TSPH_HIP(hipMemcpy(idx.data(), d.index, 4 * (size_t)n, hipMemcpyDeviceToHost));
-    for (int k = 0; k < m; ++k) h->index[k] = idx[order[k]];
+  for (const Field &f : fields) {
+    if (!f.to) continue;
+    if (f.from) TSPH_HIP(get(f.to, f.from, sizeof(double) * f.width * (size_t)m));
+    else std::fill(f.to, f.to + f.width * (size_t)m, 0.0);
   }
+  std::vector<uint8_t> type(h->type ? m : 0);
+  if (h->type) TSPH_HIP(get(type.data(), d.type, (size_t)m));
+  if (h->index) TSPH_HIP(get(h->index, d.index, 4 * (size_t)m));
+  TSPH_HIP(hipStreamSynchronize(c->stream));
+  for (size_t k = 0; k < type.size(); ++k) h->type[k] = type[k];
   return 0;
 }
 
@@ -758,7 +748,7 @@ int tsph_get_cell_lists(tsph_ctx *c, int32_t *start, int32_t *items) {
   std::vector<int> order;
   std::vector<uint32_t> seq;
   std::vector<uint8_t> type;
-  if ((e = live_order(c, n, -1, order, seq, type))) return e;
+  if ((e = live_order(c, n, order, seq, type))) return e;
   // reference index of slot = its rank in reference order
   std::vector<int> rank(n, -1);
   for (size_t k = 0; k < order.size(); ++k) rank[order[k]] = (int)k;
@@ -850,7 +840,7 @@ int tsph_ale_upload(tsph_ctx *c, const tsph_ale_fields *h) {
   std::vector<int> order;
   std::vector<uint32_t> seq;
   std::vector<uint8_t> type;
-  if ((e = live_order(c, n, -1, order, seq, type))) return e;
+  if ((e = live_order(c, n, order, seq, type))) return e;
   const int m = (int)order.size();
   if (h->np != m) return fail(TSPH_EINVAL, "ALE field count differs from the particle count");
   std::vector<double> b(2 * (size_t)n + 2, 0.0);
@@ -892,7 +882,7 @@ int tsph_ale_download(tsph_ctx *c, tsph_ale_fields *h) {
   std::vector<int> order;
   std::vector<uint32_t> seq;
   std::vector<uint8_t> type;
-  if ((e = live_order(c, n, -1, order, seq, type))) return e;
+  if ((e = live_order(c, n, order, seq, type))) return e;
   const int m = (int)order.size();
   std::vector<double> b(2 * (size_t)n + 2);
   auto get1 = [&](double *dst, const double *src) -> int {
@@ -1257,7 +1247,7 @@ int tsph_history_upload(tsph_ctx *c, const tsph_history *h) {
   std::vector<int> order;
   std::vector<uint32_t> seq;
   std::vector<uint8_t> type;
-  if ((e = live_order(c, n, -1, order, seq, type))) return e;
+  if ((e = live_order(c, n, order, seq, type))) return e;
   const int m = (int)order.size();
   if (h->np != m) return fail(TSPH_EINVAL, "history field count differs from the particle count");
   std::vector<double> b(2 * (size_t)n + 2, 0.0);
@@ -1285,7 +1275,7 @@ int tsph_history_download(tsph_ctx *c, tsph_history *h) {
   std::vector<int> order;
   std::vector<uint32_t> seq;
   std::vector<uint8_t> type;
-  if ((e = live_order(c, n, -1, order, seq, type))) return e;
+  if ((e = live_order(c, n, order, seq, type))) return e;
   const int m = (int)order.size();
   h->np = m;
   std::vector<double> b(2 * (size_t)n + 2);
@@ -1684,17 +1674,11 @@ int tsph_batch_upload(tsph_ctx *c, const tsph_particles *h) {
 int tsph_batch_get_np(tsph_ctx *c, int *np) {
   if (!c || !np) return fail(TSPH_EINVAL, "null argument");
   if (!c->cases) return fail(TSPH_ESTATE, "not a batched context");
-  int n = 0;
+  // counted in hrank, free between builds (one entry per particle slot, of which
+  // every case has at least one)
+  if (int e = launch_case_counts(c, c->hrank)) return e;
+  TSPH_HIP(hipMemcpyAsync(np, c->hrank, sizeof(int) * c->ncases, hipMemcpyDeviceToHost, c->stream));
   TSPH_HIP(hipStreamSynchronize(c->stream));
-  TSPH_HIP(hipMemcpy(&n, &c->scal[S_NP], sizeof(int), hipMemcpyDeviceToHost));
-  std::vector<uint8_t> type(n), cid(n);
-  if (n > 0) {
-    TSPH_HIP(hipMemcpy(type.data(), c->cur.type, n, hipMemcpyDeviceToHost));
-    TSPH_HIP(hipMemcpy(cid.data(), c->cur.cid, n, hipMemcpyDeviceToHost));
-  }
-  std::fill(np, np + c->ncases, 0);
-  for (int i = 0; i < n; ++i)
-    if (type[i] != kRemoved) np[cid[i]]++;
   return 0;
 }
 

@@ -52,7 +52,8 @@ inline CostEstimate cost_estimate(bool mixed) { return mixed ? kCostMixed : kCos
 // (the wall count alternates between S_NWALL and S_NWALL_B with the cell-offset
 // buffers: a build fills the other one, see cell_start_next); the per-tile
 // costs follow them (kCostTables (ncells_tot + 8) slots)
-enum { S_NP = 0, S_MAXSEQ = 1, S_NTILES = 2, S_NWALL = 3, S_BZCNT = 4, S_NWALL_B = 5, S_NSCAL = 32 };
+enum { S_NP = 0, S_MAXSEQ = 1, S_NTILES = 2, S_NWALL = 3, S_BZCNT = 4, S_NWALL_B = 5,
+       S_DLNP = 6, S_NSCAL = 32 };
 // device counter slots (uint64)
 enum {
   C_PAIRS = 0, C_CAND = 1, C_ACTIVE = 2, C_PASSES = 3, C_BADRHO = 4, C_OUTGRID = 5,
@@ -357,6 +358,22 @@ int run_water_elevation(tsph_ctx *c, double x, double y0, int inverse, double *o
 // soa: out holds rho[n], p[n], then v[2n] (n = ncx ncy); else 4 values per point
 int launch_interp_grid(tsph_ctx *c, double x0, double y0, double dh, int ncx, int ncy, double *out,
                        bool soa = false);
+// The live particles of one case (icase; -1: all) gathered from cur into the
+// same fields of alt, in reference order, for a download; alt holds nothing
+// between builds once the olds are in place (ensure_olds first).  fields: a
+// mask of DL_*.  Leaves the particle count in scal[S_DLNP].
+enum {
+  DL_R = 1, DL_V = 2, DL_A = 4, DL_R_O = 8, DL_V_O = 16, DL_GNR = 32, DL_N = 64, DL_P = 128,
+  DL_RHO = 256, DL_DRHO = 512, DL_RHO_O = 1024, DL_TYPE = 2048, DL_INDEX = 4096
+};
+int launch_download_gather(tsph_ctx *c, int icase, unsigned fields);
+// p[i] = i for i < n
+int launch_iota(tsph_ctx *c, int *p, int n);
+// live particles of every case of a batch into counts[ncases] (device memory)
+int launch_case_counts(tsph_ctx *c, int *counts);
+// words of the bitmap over reference positions that launch_download_gather
+// keeps in hcell (and its prefix in hrank)
+inline size_t dl_words(int seq_cap) { return ((size_t)seq_cap + 31) / 32; }
 // device address of the allocation-free interpolation grid's scratch on the
 // current device (looked up once per device)
 int grid_scratch_ptr(double **out);

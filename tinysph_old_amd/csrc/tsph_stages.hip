@@ -10,6 +10,8 @@
 #include <cmath>
 #include <vector>
 
+#include <algorithm>
+
 #include "tsph_internal.h"
 #include "tsph_physics.h"
 #include "tsph_walls.h"
@@ -259,7 +261,147 @@ __global__ void k_interp_grid(Soa d, const int *__restrict__ cell_start, Consts 
   }
 }
 
+// --------------------------------------------------------------------------
+// Download: the live particles in reference order.  A particle's place is the
+// number of live particles with a smaller reference position, so the order
+// needs no sort: a bitmap over the positions, its prefix popcounts, and a
+// gather into the other particle generation, whose fields then go to the host
+// as they are.  Bound by the copies over PCIe that follow (740k particles, r v
+// rho p: 36 MB, 0.7 ms at the link's rate; the four launches take 70 us); the
+// host sort and permuting copies this replaces took 40 ms.
+// --------------------------------------------------------------------------
+constexpr int kDlScan = 1024;  // threads of the one workgroup that scans the bitmap
+constexpr int kDlItems = 4;    // words per thread and round
+
+__global__ void k_dl_clear(const int *__restrict__ scal, uint32_t *__restrict__ bits) {
+  const int w = (scal[S_MAXSEQ] + 31) / 32;
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < w; i += gridDim.x * blockDim.x) bits[i] = 0;
+}
+
+__device__ __forceinline__ bool dl_live(const Soa &d, int i, int icase) {
+  return d.type[i] != kRemoved && (icase < 0 || d.cid[i] == icase);
+}
+
+__global__ void k_dl_mark(Soa d, const int *__restrict__ scal, int icase,
+                          uint32_t *__restrict__ bits) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= scal[S_NP] || !dl_live(d, i, icase)) return;
+  const uint32_t s = d.seq[i];
+  atomicOr(&bits[s >> 5], 1u << (s & 31));
+}
+
+// live positions before each word, and their total (scal[S_DLNP])
+__global__ __launch_bounds__(kDlScan) void k_dl_scan(int *__restrict__ scal,
+                                                     const uint32_t *__restrict__ bits,
+                                                     int *__restrict__ before) {
+  __shared__ int part[kDlScan / 64];
+  const int words = (scal[S_MAXSEQ] + 31) / 32;
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  int carry = 0;
+  for (int w0 = 0; w0 < words; w0 += kDlScan * kDlItems) {
+    const int w = w0 + threadIdx.x * kDlItems;
+    int n[kDlItems], sum = 0;
+#pragma unroll
+    for (int q = 0; q < kDlItems; ++q) {
+      n[q] = w + q < words ? __popc(bits[w + q]) : 0;
+      sum += n[q];
+    }
+    int x = sum;
+    for (int o = 1; o < 64; o <<= 1) {
+      const int y = __shfl_up(x, o, 64);
+      if (lane >= o) x += y;
+    }
+    if (lane == 63) part[wid] = x;
+    __syncthreads();
+    int at = carry + x - sum;
+    for (int u = 0; u < kDlScan / 64; ++u) {
+      const int v = part[u];
+      if (u < wid) at += v;
+      carry += v;
+    }
+#pragma unroll
+    for (int q = 0; q < kDlItems; ++q) {
+      if (w + q < words) before[w + q] = at;
+      at += n[q];
+    }
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) scal[S_DLNP] = carry;
+}
+
+__global__ void k_dl_gather(Soa d, Soa o, const int *__restrict__ scal, int icase, unsigned fields,
+                            const uint32_t *__restrict__ bits, const int *__restrict__ before) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= scal[S_NP] || !dl_live(d, i, icase)) return;
+  const uint32_t s = d.seq[i];
+  const int k = before[s >> 5] + __popc(bits[s >> 5] & ((1u << (s & 31)) - 1u));
+  if (fields & DL_R) o.r[k] = d.r[i];
+  if (fields & DL_V) o.v[k] = d.v[i];
+  if (fields & DL_A) o.a[k] = d.a[i];
+  if (fields & DL_R_O) o.r_o[k] = d.r_o[i];
+  if (fields & DL_V_O) o.v_o[k] = d.v_o[i];
+  if (fields & DL_GNR) o.gnr[k] = d.gnr[i];
+  if (fields & DL_N) o.n[k] = d.n[i];
+  if (fields & DL_P) o.p[k] = d.p[i];
+  if (fields & DL_RHO) o.rho[k] = d.rho[i];
+  if (fields & DL_DRHO) o.drho[k] = d.drho[i];
+  if (fields & DL_RHO_O) o.rho_o[k] = d.rho_o[i];
+  if (fields & DL_TYPE) o.type[k] = d.type[i];
+  if (fields & DL_INDEX) o.index[k] = d.index[i];
+}
+
+// live particles per case: a histogram in LDS per workgroup, then one atomic
+// per case that the workgroup saw
+__global__ __launch_bounds__(256) void k_case_counts(Soa d, const int *__restrict__ scal, int ncases,
+                                                     int *__restrict__ counts) {
+  __shared__ int h[256];
+  h[threadIdx.x] = 0;
+  __syncthreads();
+  const int n = scal[S_NP];
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
+    if (d.type[i] != kRemoved) atomicAdd(&h[d.cid[i]], 1);
+  __syncthreads();
+  if ((int)threadIdx.x < ncases && h[threadIdx.x]) atomicAdd(&counts[threadIdx.x], h[threadIdx.x]);
+}
+
+__global__ void k_iota(int *__restrict__ p, int n) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) p[i] = i;
+}
+
+__global__ void k_zero_ints(int *__restrict__ p, int n) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) p[i] = 0;
+}
+
 }  // namespace
+
+int launch_download_gather(tsph_ctx *c, int icase, unsigned fields) {
+  uint32_t *bits = reinterpret_cast<uint32_t *>(c->hcell);
+  const int g = grid_for(c->n_ub, 256);
+  const int wg = grid_for((int)std::min<size_t>(dl_words(c->seq_cap), 1 << 18), 256);
+  hipLaunchKernelGGL(k_dl_clear, dim3(wg), dim3(256), 0, c->stream, c->scal, bits);
+  hipLaunchKernelGGL(k_dl_mark, dim3(g), dim3(256), 0, c->stream, c->cur, c->scal, icase, bits);
+  hipLaunchKernelGGL(k_dl_scan, dim3(1), dim3(kDlScan), 0, c->stream, c->scal, bits, c->hrank);
+  hipLaunchKernelGGL(k_dl_gather, dim3(g), dim3(256), 0, c->stream, c->cur, c->alt, c->scal, icase,
+                     fields, bits, c->hrank);
+  TSPH_HIP(hipGetLastError());
+  return 0;
+}
+
+int launch_iota(tsph_ctx *c, int *p, int n) {
+  hipLaunchKernelGGL(k_iota, dim3(grid_for(n, 256)), dim3(256), 0, c->stream, p, n);
+  TSPH_HIP(hipGetLastError());
+  return 0;
+}
+
+int launch_case_counts(tsph_ctx *c, int *counts) {
+  hipLaunchKernelGGL(k_zero_ints, dim3(1), dim3(256), 0, c->stream, counts, c->ncases);
+  hipLaunchKernelGGL(k_case_counts, dim3(std::min(grid_for(c->n_ub, 1024), 4 * c->num_cu)), dim3(256), 0,
+                     c->stream, c->cur, c->scal, c->ncases, counts);
+  TSPH_HIP(hipGetLastError());
+  return 0;
+}
 
 int launch_eos(tsph_ctx *c) {
   Mixed mx = c->prm.precision == TSPH_PREC_MIXED ? c->mx : Mixed{};
