@@ -354,6 +354,9 @@ static int make_consts(const tsph_params *prm, Consts &k) {
   k.of = prm->h * 0.273;                           // src/SPH_find_pairs.h:13
   k.awen = (double)(float)(0.557 / (prm->h * prm->h));
   k.bwen = (double)(float)(-2.7852 / (prm->h * prm->h * prm->h));
+  k.ih = 1. / prm->h;
+  k.cb = prm->cs * prm->cs * prm->rho0 / 7.;
+  k.icb = 1. / k.cb;
   k.ncx = (int)((k.xm - k.x0 + k.of) / k.kh) + 1;  // src/SPH_find_pairs.h:19-20
   k.ncy = (int)((k.ym - k.y0 + k.of) / k.kh) + 1;
   const long long nc = (long long)k.ncx * k.ncy;

@@ -111,6 +111,7 @@ struct Consts {
   double x0, xm, y0, ym;
   double kh, of;
   double awen, bwen;  // float-rounded Wendland constants, src/SPH_kernel.h:56-57
+  double ih, cb, icb; // 1/h, cs^2 rho0 / 7, 1/cb
   int ncx, ncy, ncells;
   // batched ensembles: the case's first global cell id and its time step
   // (single cases: 0 and unused)

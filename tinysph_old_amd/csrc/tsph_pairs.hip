@@ -68,39 +68,43 @@ struct Acc64 {
 };
 
 
+// (airho, nirho = recip64 of the densities)
 template <int VAR>
 __device__ __forceinline__ void pair64(const Consts &k, Acc64 &s, double2 ar, double2 av, double arho,
-                                       double ap, double2 nr, double2 nv, double nrho, double np,
-                                       int nt, double2 nb, unsigned &npair) {
+                                       double airho, double ap, double2 nr, double2 nv, double nrho,
+                                       double nirho, double np, int nt, double2 nb,
+                                       unsigned &npair) {
   const double h = k.h;
   const double drx = ar.x - nr.x, dry = ar.y - nr.y;
-  const double r2 = (drx * drx) + (dry * dry);
-  if (r2 > 4.0 * h * h * (1.0 + 1e-12)) return;
-  const double drs = sqrt(r2);
-  if (drs / h > 2.0) return;
-  if (drs / h < 2.0) ++npair;
-  const KW64 kw = wendland64(drs, h, k.awen, k.bwen);
+  const Root64 rt = sqrt64((drx * drx) + (dry * dry));
+  // beyond the exact support (qq > 2) the kernel is 0 and so is every term
+  const double drs = rt.s, qq = quot64(drs, h, k.ih);
+  npair += qq < 2.0;
+  const KW64 kw = wendland64(rt, qq, k.awen, k.bwen);
   const double dvx = av.x - nv.x, dvy = av.y - nv.y;
   const double drdv = drx * dvx + dry * dvy;
   const double dWx = drx * kw.f, dWy = dry * kw.f;
   const double dvdW = dvx * dWx + dvy * dWy;
   const double drdW = drx * dWx + dry * dWy;
-  const double p_temp = (ap + np) / (arho * nrho);
-  const double visco = art_visc64(h, drs, drdv, 0.5 * (arho + nrho), k.cs, k.avisc);
+  // 1 / (arho nrho) from the two reciprocals and a Newton iteration
+  const double rr = arho * nrho, yy = airho * nirho;
+  const double p_temp = quot64_any(ap + np, rr, __builtin_fma(yy, __builtin_fma(-rr, yy, 1.0), yy));
+  const double d = drs * drs + kEps * h * h, yd = recip64(d);
+  const double visco = art_visc64(h, d, yd, drdv, 0.5 * (arho + nrho), k.cs, k.avisc);
   if (VAR == TSPH_FORCES_BT && nt == TSPH_WALL) {
     s.accx += kw.w * (p_temp + visco) * k.dp * nb.x * nrho;
     s.accy += kw.w * (p_temp + visco) * k.dp * nb.y * nrho;
     const double dvnb = dvx * nb.x + dvy * nb.y;
     s.drho_sum -= dvnb * kw.w * nrho * k.dp;
   } else {
-    const double diff =
-        diff_fourtakas64(h, drs, dry, drdW, arho, nrho, k.rho0, k.cs, k.delta, k.m, k.gy);
+    const double diff = diff_fourtakas64(h, d, yd, dry, drdW, arho, nrho, nirho, k.rho0, k.cb,
+                                         k.icb, k.cs, k.delta, k.m, k.gy);
     s.accx -= dWx * (p_temp + visco) * k.m;
     s.accy -= dWy * (p_temp + visco) * k.m;
     s.drho_sum += dvdW * k.m;
     s.diff_sum -= diff;
   }
-  if (VAR == TSPH_FORCES_BT && nt == TSPH_FLUID) s.gamma += kw.w * k.m / nrho;
+  if (VAR == TSPH_FORCES_BT && nt == TSPH_FLUID) s.gamma += quot64_any(kw.w * k.m, nrho, nirho);
 }
 
 // final assignment, src/SPH_interaction.h:134-136, src/SPH_interactionDBC.h:137-142,
@@ -222,7 +226,7 @@ __device__ void particle64_global(const Soa &d, const int *__restrict__ cell_sta
                                   unsigned &npair, unsigned &ncand) {
   const int at = d.type[i];
   const double2 ar = d.r[i], av = d.v[i];
-  const double arho = d.rho[i], ap = d.p[i];
+  const double arho = d.rho[i], airho = recip64(arho), ap = d.p[i];
   const int c = cellof[i] - k.cell_base;
   const int cx = c / k.ncy, cy = c - cx * k.ncy;
   Acc64 s;
@@ -238,7 +242,9 @@ __device__ void particle64_global(const Soa &d, const int *__restrict__ cell_sta
       if (VAR == TSPH_FORCES_DBC && at == TSPH_WALL && nt == TSPH_WALL) continue;
       ++ncand;
       const double2 nb = (VAR == TSPH_FORCES_BT) ? d.n[j] : make_double2(0., 0.);
-      pair64<VAR>(k, s, ar, av, arho, ap, d.r[j], d.v[j], d.rho[j], d.p[j], nt, nb, npair);
+      const double nrho = d.rho[j];
+      pair64<VAR>(k, s, ar, av, arho, airho, ap, d.r[j], d.v[j], nrho, recip64(nrho), d.p[j], nt, nb,
+                  npair);
     }
   }
   double2 a;
@@ -447,6 +453,7 @@ __global__ __launch_bounds__(kWave * kPoolWaves) void k_tile64(Soa d, const int 
     }
     nact += act;
     const double2 ar = s_r[li], av = s_v[li], arp = s_rp[li];
+    const double airho = recip64(arp.x);
     // walk of the 9 stencil cells in reference order: cell q, LDS range [lj, lend).
     // A cell's candidates are tested kGroup at a time (their LDS loads in
     // flight together) and appended without branches: every slot of the group
@@ -474,6 +481,7 @@ __global__ __launch_bounds__(kWave * kPoolWaves) void k_tile64(Soa d, const int 
           const int bq = sel3(t.base, dx + 1);
           lj = tab[e] + bq;
           lend = tab[e + 1] + bq;
+          if (VAR != TSPH_FORCES_DBC) ncand += lend - lj - (q == 0);
           continue;
         }
         const int m = min(kGroup, lend - lj);
@@ -483,22 +491,28 @@ __global__ __launch_bounds__(kWave * kPoolWaves) void k_tile64(Soa d, const int 
 #pragma unroll
         for (int u = 0; u < kGroup; ++u) {
           const int j = lj + u;
-          bool cand = u < m && j != li;
-          if (VAR == TSPH_FORCES_DBC) cand = cand && !(dbc_wall && s_t[j] == TSPH_WALL);
-          ncand += cand;
+          bool cand = (u < m) & (j != li);
+          if (VAR == TSPH_FORCES_DBC) {
+            cand &= !(dbc_wall & (s_t[j] == TSPH_WALL));
+            ncand += cand;
+          }
           const double drx = ar.x - pp[u].x, dry = ar.y - pp[u].y;
-          const bool in = cand && (drx * drx) + (dry * dry) <= c2;
+          const bool in = cand & ((drx * drx) + (dry * dry) <= c2);
           my_list[cnt * kWave] = (uint16_t)j;
           cnt += in;
         }
         lj += m;
       }
+      int jn = my_list[0];
       for (int e = 0; e < cnt; ++e) {
-        const int j = my_list[e * kWave];
+        const int j = jn;
+        // read unconditionally (past cnt it is an unused entry of the list)
+        jn = my_list[min(e + 1, kList - 1) * kWave];
         const double2 nrp = s_rp[j];
         const int nt = VAR != TSPH_FORCES_WCSPH ? s_t[j] : 0;
         const double2 nb = VAR == TSPH_FORCES_BT ? s_n[j] : make_double2(0., 0.);
-        pair64<VAR>(k, s, ar, av, arp.x, arp.y, s_r[j], s_v[j], nrp.x, nrp.y, nt, nb, npair);
+        pair64<VAR>(k, s, ar, av, arp.x, airho, arp.y, s_r[j], s_v[j], nrp.x, recip64(nrp.x), nrp.y,
+                    nt, nb, npair);
       }
     }
     if (act) {

@@ -7,6 +7,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include "tsph_fp64.h"
 #include "tsph_internal.h"
 #include "tsph_pow7.h"
 #include "tsph_root7.h"
@@ -59,28 +60,40 @@ __device__ __forceinline__ KW64 wendland64(double r, double h, double awen, doub
   return k;
 }
 
-// Artificial_Viscosity, src/SPH_viscouse_forces.h:7-25 (rhobar = 0.5*(rho_i+rho_j))
-__device__ __forceinline__ double art_visc64(double h, double drs, double drdv, double rhobar,
-                                             double c0, double alpha) {
-  double av = 0.0;
-  const double visco = drdv > alpha ? drdv : alpha;
-  if (drdv < 0) {
-    const double mu = h * drdv / (drs * drs + kEps * h * h);
-    av = -visco * c0 * mu / rhobar;
-  }
-  return av;
+// the same for a pair loop, without branches: r with its square root's
+// by-product, qq = r/h
+__device__ __forceinline__ KW64 wendland64(const Root64 &rt, double qq, double awen, double bwen) {
+  const double r = rt.s;
+  const float wqq1 = (float)(1.0 - 0.5 * qq);
+  const float wqq2 = wqq1 * wqq1;
+  const float wqq = (float)(qq + qq + 1.0);
+  const bool in = qq <= 2.0;
+  const double w = awen * (double)wqq * (double)wqq2 * (double)wqq2;
+  const double f = quot64(bwen * qq * (double)wqq2 * (double)wqq1, r, recip_of_root64(rt));
+  return {in ? w : 0.0, (in & (r != 0.0)) ? f : 0.0};  // r = 0: qq = 0, w = awen
 }
 
-// Density_Diffusion_term_FOURTAKAS, src/SPH_viscouse_forces.h:45-61
-__device__ __forceinline__ double diff_fourtakas64(double h, double drs, double dr_z, double drdW,
-                                                   double arho, double nrho, double rho0,
+// Artificial_Viscosity, src/SPH_viscouse_forces.h:7-25 (rhobar = 0.5*(rho_i+rho_j);
+// d = drs^2 + eps h^2, yd = recip64(d))
+__device__ __forceinline__ double art_visc64(double h, double d, double yd, double drdv,
+                                             double rhobar, double c0, double alpha) {
+  const double visco = drdv > alpha ? drdv : alpha;
+  const double mu = quot64(h * drdv, d, yd);
+  const double av = quot64_any(-visco * c0 * mu, rhobar, recip64(rhobar));
+  return drdv < 0 ? av : 0.0;
+}
+
+// Density_Diffusion_term_FOURTAKAS, src/SPH_viscouse_forces.h:45-61 (d, yd as
+// above; cb = c0^2 rho0 / 7 and icb = 1/cb; inrho = 1/nrho)
+__device__ __forceinline__ double diff_fourtakas64(double h, double d, double yd, double dr_z,
+                                                   double drdW, double arho, double nrho,
+                                                   double inrho, double rho0, double cb, double icb,
                                                    double c0, double delta, double m,
                                                    double gravity) {
-  const double cb = c0 * c0 * rho0 / 7.;
-  const double dpH = 1. + dr_z * rho0 * gravity / cb;
+  const double dpH = 1. + quot64(dr_z * rho0 * gravity, cb, icb);
   const double drhoH = rho0 * root7(dpH) - rho0;  // pow(dpH, 1/7), tsph_root7.h
-  const double psi = 2. * c0 * h * delta * ((nrho - arho) - drhoH) / (drs * drs + kEps * h * h);
-  return psi * drdW * m / nrho;
+  const double psi = quot64(2. * c0 * h * delta * ((nrho - arho) - drhoH), d, yd);
+  return quot64_any(psi * drdW * m, nrho, inrho);
 }
 
 // Compute_Pressure (Tait, gamma = 7), src/SPH_pressure.h:7-19
