@@ -1811,6 +1811,7 @@ int tsph_autotune(tsph_ctx *c, int variant, int *tile_rows, int *waves_per_cu, i
     // the chosen depth's particles per lane: every particle belongs to one
     // tile of the list, whose 64 lanes take its particles in turn
     int ntiles = 0, np = 0;
+    if ((e = ensure_tile_list(c, 0))) return e;  // (a pass by cells needs no list)
     TSPH_HIP(hipMemcpyAsync(&ntiles, c->scal + S_NTILES, sizeof(int), hipMemcpyDeviceToHost, c->stream));
     TSPH_HIP(hipMemcpyAsync(&np, c->scal + S_NP, sizeof(int), hipMemcpyDeviceToHost, c->stream));
     TSPH_HIP(hipStreamSynchronize(c->stream));

@@ -68,9 +68,17 @@ struct Acc64 {
 };
 
 
+// the constants of the FP64 pair terms
+struct PairConsts {
+  double h, ih, awen, bwen, cs, avisc, delta, m, gx, gy, rho0, cb, icb, dp;
+};
+__host__ __device__ __forceinline__ PairConsts pair_consts(const Consts &k) {
+  return {k.h, k.ih, k.awen, k.bwen, k.cs, k.avisc, k.delta, k.m, k.gx, k.gy, k.rho0, k.cb, k.icb, k.dp};
+}
+
 // (airho, nirho = recip64 of the densities)
-template <int VAR>
-__device__ __forceinline__ void pair64(const Consts &k, Acc64 &s, double2 ar, double2 av, double arho,
+template <int VAR, class K>
+__device__ __forceinline__ void pair64(const K &k, Acc64 &s, double2 ar, double2 av, double arho,
                                        double airho, double ap, double2 nr, double2 nv, double nrho,
                                        double nirho, double np, int nt, double2 nb,
                                        unsigned &npair) {
@@ -109,8 +117,8 @@ __device__ __forceinline__ void pair64(const Consts &k, Acc64 &s, double2 ar, do
 
 // final assignment, src/SPH_interaction.h:134-136, src/SPH_interactionDBC.h:137-142,
 // src/SPH_interactionBT.h:166-178
-template <int VAR>
-__device__ __forceinline__ void finish64(const Consts &k, const Acc64 &s, int at, double2 &a, double &dr) {
+template <int VAR, class K>
+__device__ __forceinline__ void finish64(const K &k, const Acc64 &s, int at, double2 &a, double &dr) {
   if (VAR == TSPH_FORCES_BT) {
     if (s.gamma > kEps) {
       a = make_double2(s.accx / s.gamma - k.gx, s.accy / s.gamma - k.gy);
@@ -220,21 +228,20 @@ __device__ __forceinline__ void finish32(const Consts &k, const Acc32 &s, int at
 // --------------------------------------------------------------------------
 // global-memory forms (tiles whose neighbourhood overflows the LDS budget)
 // --------------------------------------------------------------------------
-template <int VAR>
-__device__ void particle64_global(const Soa &d, const int *__restrict__ cell_start,
-                                  const int *__restrict__ cellof, const Consts &k, int i,
-                                  unsigned &npair, unsigned &ncand) {
+template <int VAR, class D, class K>
+__device__ void particle64_global(const D &d, const int *__restrict__ cell_start, const K &k,
+                                  const CellGrid &g, int c, int i, unsigned &npair,
+                                  unsigned &ncand) {
   const int at = d.type[i];
   const double2 ar = d.r[i], av = d.v[i];
   const double arho = d.rho[i], airho = recip64(arho), ap = d.p[i];
-  const int c = cellof[i] - k.cell_base;
-  const int cx = c / k.ncy, cy = c - cx * k.ncy;
+  const int cx = c / g.ncy, cy = c - cx * g.ncy;
   Acc64 s;
   for (int q = 0; q < 9; ++q) {
     int dx, dy;
     stencil_dxy(q, dx, dy);
-    if (cx + dx < 0 || cx + dx >= k.ncx || cy + dy < 0 || cy + dy >= k.ncy) continue;
-    const int cl = c + dy + dx * k.ncy;
+    if (cx + dx < 0 || cx + dx >= g.ncx || cy + dy < 0 || cy + dy >= g.ncy) continue;
+    const int cl = c + dy + dx * g.ncy;
     const int j1 = cell_start[cl + 1];
     for (int j = cell_start[cl]; j < j1; ++j) {
       if (j == i) continue;
@@ -421,7 +428,7 @@ __global__ __launch_bounds__(kWave * kPoolWaves) void k_tile64(Soa d, const int 
     for (int i = t.own0 + tile_lane(); i < t.own1; i += kWave) {
       if (!is_active<VAR>(d.type[i])) continue;
       ++nact;
-      particle64_global<VAR>(d, cs, cellof, k, i, npair, ncand);
+      particle64_global<VAR>(d, cs, k, cell_grid(k), cellof[i] - k.cell_base, i, npair, ncand);
     }
     it = next;
     continue;
@@ -527,6 +534,109 @@ __global__ __launch_bounds__(kWave * kPoolWaves) void k_tile64(Soa d, const int 
   }  // tiles
   tq_mark(tq, -1);
   wave_count(npair, ncand, nact, counters);
+}
+
+// --------------------------------------------------------------------------
+// FP64 cell kernel (cells64, tsph_tiles.h): the same sums, for systems too
+// small to fill the chip with tiles
+// --------------------------------------------------------------------------
+// the fields and constants a pair pass reads (kept few: they live in scalar
+// registers)
+struct Pair64 {
+  const double2 *r, *v, *n;
+  const double *rho, *p;
+  const uint8_t *type;
+  double2 *a;
+  double *drho;
+};
+
+template <int VAR>
+struct Cell64 {
+  Pair64 d;
+  PairConsts k;
+  static constexpr int kSums = VAR == TSPH_FORCES_BT ? 5 : 4;
+  static constexpr int kSlotBytes = (VAR == TSPH_FORCES_BT ? 4 : 3) * 16 + 9;
+  struct Lds {
+    double2 *r, *v, *rp, *n;  // rp = {rho, p}; n: BT only
+    double *ir;               // recip64(rho)
+    uint8_t *t;
+  };
+  struct Rec {
+    double2 r, v, rp, n;
+    uint8_t t;
+  };
+  static __device__ __forceinline__ Lds lds(unsigned char *b, int cap) {
+    double2 *p = reinterpret_cast<double2 *>(b);
+    Lds L;
+    L.r = p; L.v = p + cap; L.rp = p + 2 * cap; L.n = p + 3 * cap;
+    L.ir = reinterpret_cast<double *>(p + (VAR == TSPH_FORCES_BT ? 4 : 3) * cap);
+    L.t = reinterpret_cast<uint8_t *>(L.ir + cap);
+    return L;
+  }
+  __device__ __forceinline__ void set(const Consts &c) { k = pair_consts(c); }
+  __device__ __forceinline__ Rec load(int j) const {
+    Rec q;
+    q.r = d.r[j];
+    q.v = d.v[j];
+    q.rp = make_double2(d.rho[j], d.p[j]);
+    q.t = d.type[j];
+    if (VAR == TSPH_FORCES_BT) q.n = d.n[j];
+    return q;
+  }
+  __device__ __forceinline__ void store(const Lds &L, int l, const Rec &q) const {
+    L.r[l] = q.r;
+    L.v[l] = q.v;
+    L.rp[l] = q.rp;
+    L.ir[l] = recip64(q.rp.x);
+    L.t[l] = q.t;
+    if (VAR == TSPH_FORCES_BT) L.n[l] = q.n;
+  }
+  __device__ __forceinline__ bool act_lds(const Lds &L, int l) const { return is_active<VAR>(L.t[l]); }
+  static constexpr bool kSkip = VAR == TSPH_FORCES_DBC;
+  __device__ __forceinline__ bool skip_lds(const Lds &L, int l) const { return L.t[l] == TSPH_WALL; }
+  __device__ __forceinline__ double2 pos_lds(const Lds &L, int l) const { return L.r[l]; }
+  __device__ __forceinline__ int terms(const Lds &L, int p, int l, double (&t)[kSums]) const {
+    const double2 arp = L.rp[p], nrp = L.rp[l];
+    const int nt = VAR != TSPH_FORCES_WCSPH ? L.t[l] : 0;
+    const double2 nb = VAR == TSPH_FORCES_BT ? L.n[l] : make_double2(0., 0.);
+    Acc64 s;
+    unsigned np = 0;
+    pair64<VAR>(k, s, L.r[p], L.v[p], arp.x, L.ir[p], arp.y, L.r[l], L.v[l], nrp.x, L.ir[l], nrp.y,
+                nt, nb, np);
+    t[0] = s.accx;
+    t[1] = s.accy;
+    t[2] = s.drho_sum;
+    t[3] = s.diff_sum;
+    if (VAR == TSPH_FORCES_BT) t[kSums - 1] = s.gamma;
+    return (int)np;
+  }
+  __device__ __forceinline__ void sums(const Lds &L, int p, int i, const double (&t)[kSums]) const {
+    Acc64 s;
+    s.accx = t[0];
+    s.accy = t[1];
+    s.drho_sum = t[2];
+    s.diff_sum = t[3];
+    if (VAR == TSPH_FORCES_BT) s.gamma = t[kSums - 1];
+    double2 a;
+    double dr;
+    finish64<VAR>(k, s, L.t[p], a, dr);
+    d.a[i] = a;
+    d.drho[i] = dr;
+  }
+  __device__ __forceinline__ void far(int i, const int *cs, const CellGrid &g, int c,
+                                      unsigned &npair, unsigned &ncand, unsigned &nact) const {
+    if (!is_active<VAR>(d.type[i])) return;
+    ++nact;
+    particle64_global<VAR>(d, cs, k, g, c, i, npair, ncand);
+  }
+};
+
+template <class P>
+__global__ __launch_bounds__(kCellBlock, 3) void k_cells64(P pol, CellGrid g, const int *__restrict__ cell_start,
+                                                        const Consts *__restrict__ cases,
+                                                        int ncases, int ncells_tot,
+                                                        unsigned long long *__restrict__ counters) {
+  cells64(pol, g, cell_start, cases, ncases, ncells_tot, counters);
 }
 
 // --------------------------------------------------------------------------
@@ -887,6 +997,18 @@ TileGrid tile_grid(tsph_ctx *c, bool fp32, size_t lds_wave, bool may_pool) {
   return tg;
 }
 
+// The FP64 pair pass walks cells instead of tiles for systems of up to
+// kCellsMax particles.  A tile's wavefront takes about 25 us however small the
+// system is, a cell's 8 us, while a full chip does more pairs per second by
+// tiles (a dam break, us per pass, cells and tiles: 6k particles 9 / 41, 23k
+// 14 / 23, 50k 24 / 34, 92k 39 / 36, 740k 259 / 204).  The walk looks at every
+// cell of the grid, so grids of more than kCellsGrid cells keep the list of
+// non-empty tiles.
+constexpr int kCellsMax = 70000, kCellsGrid = 1 << 18;
+static bool cells_walk(const tsph_ctx *c) {
+  return c->prm.precision == TSPH_PREC_FP64 && c->n_ub <= kCellsMax && c->ncells_tot <= kCellsGrid;
+}
+
 // LDS bytes per wavefront of the pair pass of `variant` at the current tile rows
 static size_t forces_lds_wave(const tsph_ctx *c, int variant) {
   const int cap = 3 * (c->tile_rows + 2) * kCellCap;
@@ -899,6 +1021,7 @@ static size_t forces_lds_wave(const tsph_ctx *c, int variant) {
 }
 
 int pass_groups(tsph_ctx *c, int variant) {
+  if (cells_walk(c)) return 0;
   const TileGrid tg = tile_grid(c, c->prm.precision == TSPH_PREC_MIXED, forces_lds_wave(c, variant));
   return tg.pooled ? tg.groups : 0;
 }
@@ -927,6 +1050,18 @@ void pair_launch(tsph_ctx *c, const TileGrid &tg, int rows, int cap, bool corr, 
 }
 
 template <int VAR>
+void cell_launch(tsph_ctx *c) {
+  using P = Cell64<VAR>;
+  constexpr int lds = cell_lds_bytes<P>();
+  const Soa &d = c->cur;
+  const int groups = cell_groups(c, k_cells64<P>, lds, c->cells_fit[VAR]);
+  hipLaunchKernelGGL(k_cells64<P>, dim3(groups), dim3(kCellBlock), lds, c->stream,
+                     P{{d.r, d.v, d.n, d.rho, d.p, d.type, d.a, d.drho}, pair_consts(c->k)},
+                     cell_grid(c->k), c->cell_start, c->cases, c->ncases,
+                     c->ncells_tot, c->counters);
+}
+
+template <int VAR>
 void pair_launch(tsph_ctx *c, const TileGrid &tg, int rows, int cap, bool corr, double corr_dt) {
   if (tg.pooled) pair_launch<VAR, true>(c, tg, rows, cap, corr, corr_dt);
   else pair_launch<VAR, false>(c, tg, rows, cap, corr, corr_dt);
@@ -942,6 +1077,14 @@ int launch_forces(tsph_ctx *c, int variant, bool corr, double corr_dt) {
     if (int e = launch_mixed_records(c)) return e;
     c->records_valid = true;
   }
+  if (cells_walk(c))
+    return launch_timed(c, [&] {
+      switch (variant) {
+        case TSPH_FORCES_WCSPH: cell_launch<TSPH_FORCES_WCSPH>(c); break;
+        case TSPH_FORCES_DBC: cell_launch<TSPH_FORCES_DBC>(c); break;
+        default: cell_launch<TSPH_FORCES_BT>(c);
+      }
+    });
   const TileGrid tg = tile_grid(c, mixed, forces_lds_wave(c, variant));
   if (int e = ensure_tile_list(c, tg.pooled ? tg.groups : 0, mixed && corr ? 1 : 0)) return e;
   const int e = launch_timed(c, [&] {

@@ -4,6 +4,8 @@
 // of the three neighbour slices in LDS, and the lane-private neighbour lists.
 #pragma once
 
+#include <algorithm>
+
 #include "tsph_internal.h"
 #include "tsph_physics.h"
 
@@ -559,6 +561,309 @@ __device__ __forceinline__ void walk64(const P &pol, const Consts &k, const int 
   wave_count(npair, ncand, nact, counters);
 }
 
+// --------------------------------------------------------------------------
+// Cell walk (FP64): one wavefront per cell, its pairs spread over all lanes
+// --------------------------------------------------------------------------
+// The tile walks give each lane a particle and its ~20 pairs one after the
+// other, so a pass lasts at least that chain however few tiles there are, and
+// its lanes wait for the longest list.  Here a wavefront takes one cell
+// (about nine particles):
+//   1. the particles of the 9 stencil cells are staged in LDS in the reference
+//      order (cell order, ascending index), so slot order is candidate order
+//      and the cell's own particles are the first slots;
+//   2. for each own particle the lanes test all candidate slots at once (two
+//      per lane) and append the pairs, in order, to one flat list (ballots and
+//      prefix counts; the bookkeeping is scalar);
+//   3. the lanes evaluate 64 pairs of that list at a time, whichever particles
+//      they belong to, and leave each pair's kSums terms in LDS;
+//   4. lane (particle, term) adds its particle's terms in list order.
+// Every sum is formed in the reference order from the same terms (a term
+// leaves the pair function as 0 + x or 0 - x, exactly x or -x), so the results
+// are the tile walks', bit for bit.
+//
+// A policy P supplies kSums, kSlotBytes, Lds and lds(base, cap), and
+//   set(k)                        constants of the case (batched grids)
+//   Rec load(j), store(L, l, rec) slot l <- particle j, in two halves
+//   act_lds(L, l)                 slot l is active
+//   kSkip, skip_lds(L, l)         pairs of two slots with skip_lds are no
+//                                 candidates (DBC walls)
+//   terms(L, p, l, double (&t)[kSums])  the terms of pair (p, l), zeros
+//                                 beyond the exact support (the lists hold
+//                                 r^2 <= 4h^2 (1 + 1e-12)); returns whether it
+//                                 counts as a pair interaction
+//   sums(L, p, i, const double (&s)[kSums])  writes particle i, slot p
+//   far(i, cs, g, c, counts...)   particle i of cell c from global memory
+constexpr int kCellSlots = 104;  // staged slots of a cell's neighbourhood
+constexpr int kCellFlat = 640;   // flat list entries (own particles listed together x candidates)
+constexpr double kFar64 = 1e150;  // coordinate of slots past the last (its square is finite)
+constexpr int kCellBlock = 4 * kWave;  // one wavefront per SIMD
+constexpr int kCellRun = 64;     // consecutive cells of one XCD
+template <class P>
+constexpr int cell_terms() { return P::kSums <= 4 ? 184 : 128; }  // pairs whose terms are in LDS together
+// a workgroup's non-empty cells (and their cases), and the next to take
+struct CellQueue {
+  int count, next, pad[2];
+  int cell[kCellBlock];
+  uint8_t cse[kCellBlock];
+};
+// LDS bytes of a wavefront of a cell walk
+template <class P>
+constexpr int cell_wave_bytes() {
+  return (cell_terms<P>() * P::kSums * 8 + kCellFlat * 2 + kCellSlots * P::kSlotBytes + 15) / 16 * 16;
+}
+template <class P>
+constexpr int cell_lds_bytes() {
+  return (int)sizeof(CellQueue) + kCellBlock / kWave * cell_wave_bytes<P>();
+}
+
+// what a cell walk knows of a case's grid
+struct CellGrid {
+  int ncx, ncy, cell_base;
+  double c2;  // 4h^2 (1 + 1e-12)
+};
+__host__ __device__ __forceinline__ CellGrid cell_grid(const Consts &k) {
+  return {k.ncx, k.ncy, k.cell_base, 4.0 * k.h * k.h * (1.0 + 1e-12)};
+}
+
+// case whose cell range holds global cell c
+__device__ __forceinline__ int case_of_cell(const Consts *__restrict__ cases, int ncases, int c) {
+  int lo = 0, hi = ncases;
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1;
+    if (cases[mid].cell_base <= c) lo = mid;
+    else hi = mid;
+  }
+  return lo;
+}
+
+struct CellItem {
+  int c, cse;  // global cell (-1: none left), its case
+};
+__device__ __forceinline__ CellItem cell_take(CellQueue &cq, int todo) {
+  int at = 0;
+  if (tile_lane() == 0) at = atomicAdd(&cq.next, 1);
+  at = __builtin_amdgcn_readfirstlane(at);
+  if (at >= todo) return {-1, 0};
+  return {__builtin_amdgcn_readfirstlane(cq.cell[at]), __builtin_amdgcn_readfirstlane((int)cq.cse[at])};
+}
+
+// the 9 stencil cells of global cell gc, one per lane: first particle and
+// count (cells the reference reaches by wrapping into the neighbouring column
+// are not visited)
+__device__ __forceinline__ void cell_ranges(const CellGrid &g, const int *__restrict__ cell_start,
+                                            int gc, int &lo, int &cnt) {
+  const int *cs = cell_start + g.cell_base;
+  const int c = gc - g.cell_base;
+  const int cx = c / g.ncy, cy = c - cx * g.ncy;
+  lo = cnt = 0;
+  if (tile_lane() < 9) {
+    int dx, dy;
+    stencil_dxy(tile_lane(), dx, dy);
+    if (cx + dx >= 0 && cx + dx < g.ncx && cy + dy >= 0 && cy + dy < g.ncy) {
+      const int cl = c + dy + dx * g.ncy;
+      lo = cs[cl];
+      cnt = cs[cl + 1] - lo;
+    }
+  }
+}
+
+// the slots of those cells (lo, cnt: cell_ranges), and the loads of the
+// lane's two slots, in flight together
+struct CellSlots {
+  int own0, nown, tot;
+};
+template <class P>
+__device__ __forceinline__ CellSlots cell_slots(int lo, int cnt, typename P::Rec &r0,
+                                                typename P::Rec &r1, const P &pol) {
+  const int lane = tile_lane();
+  // slot l of cell q holds particle l + dj[q], for l in [pre[q], pre[q + 1])
+  int pre[9], dj[9], tot = 0;
+#pragma unroll
+  for (int q = 0; q < 9; ++q) {
+    pre[q] = tot;
+    dj[q] = __builtin_amdgcn_readlane(lo, q) - tot;
+    tot += __builtin_amdgcn_readlane(cnt, q);
+  }
+  int j[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int l = h * kWave + lane;
+    j[h] = l + dj[0];
+#pragma unroll
+    for (int q = 1; q < 9; ++q) j[h] = l >= pre[q] ? l + dj[q] : j[h];
+    if (l >= tot) j[h] = dj[0];
+  }
+  r0 = pol.load(j[0]);
+  r1 = pol.load(j[1]);
+  return {dj[0], __builtin_amdgcn_readlane(cnt, 0), tot};
+}
+
+template <class P>
+__device__ __forceinline__ void cells64(P &pol, CellGrid g, const int *__restrict__ cell_start,
+                                        const Consts *__restrict__ cases, int ncases,
+                                        int ncells_tot, unsigned long long *__restrict__ counters) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  constexpr int NS = P::kSums;
+  constexpr int NT = cell_terms<P>();
+  constexpr int kOwn = 64 / NS;  // particles whose sums are formed together
+  CellQueue &cq = *reinterpret_cast<CellQueue *>(smem);
+  unsigned char *wl = smem + sizeof(CellQueue) + (threadIdx.x >> 6) * cell_wave_bytes<P>();
+  double *terms = reinterpret_cast<double *>(wl);
+  uint16_t *flat = reinterpret_cast<uint16_t *>(terms + NT * NS);
+  const typename P::Lds L = P::lds(reinterpret_cast<unsigned char *>(flat + kCellFlat), kCellSlots);
+  const int lane = tile_lane();
+  if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&counters[C_PASSES], 1ull);
+  unsigned npair = 0, ncand = 0, nact = 0, scand = 0, snact = 0;
+  // Runs of kCellRun cells are dealt to the 8 XCDs in turn, so that a run's
+  // cells share staged particles through one L2 while every XCD gets a share
+  // of each part of the domain.  The workgroups of an XCD stride through its
+  // cells, a thread per cell to find the non-empty ones, which the workgroup's
+  // wavefronts take from a counter in LDS.  (No tile list: its length, entry
+  // and cell offsets would be three dependent loads before the first cell.)
+  const int band = blockIdx.x & 7, nwb = gridDim.x >> 3, wb = blockIdx.x >> 3;
+  const int mine = (ncells_tot + 8 * kCellRun - 1) / (8 * kCellRun) * kCellRun;  // cells per XCD
+  for (int j0 = wb; j0 < mine; j0 += nwb * kCellBlock) {
+    __syncthreads();
+    if (threadIdx.x == 0) cq.count = cq.next = 0;
+    __syncthreads();
+    const int u = j0 + (int)threadIdx.x * nwb;
+    const int gc = ((u / kCellRun) * 8 + band) * kCellRun + u % kCellRun;
+    if (u < mine && gc < ncells_tot && cell_start[gc + 1] > cell_start[gc]) {
+      const int at = atomicAdd(&cq.count, 1);
+      cq.cell[at] = gc;
+      if (cases) cq.cse[at] = (uint8_t)case_of_cell(cases, ncases, gc);
+    }
+    __syncthreads();
+    const int todo = cq.count;
+    for (;;) {
+      const CellItem it = cell_take(cq, todo);
+      if (it.c < 0) break;
+      if (cases) {
+        g = cell_grid(cases[it.cse]);
+        pol.set(cases[it.cse]);
+      }
+      int lo, cnt;
+      cell_ranges(g, cell_start, it.c, lo, cnt);
+      typename P::Rec r0, r1;
+      const CellSlots sl = cell_slots(lo, cnt, r0, r1, pol);
+      const int own0 = sl.own0, nown = sl.nown, tot = sl.tot;
+      if (tot > kCellSlots || nown > kWave) {
+        // neighbourhood beyond the LDS budget: gather from global memory
+        for (int p = lane; p < nown; p += kWave)
+          pol.far(own0 + p, cell_start + g.cell_base, g, it.c - g.cell_base, npair, ncand, nact);
+        continue;
+      }
+      wave_sync();  // the previous cell's LDS is no longer read
+      if (lane < tot) pol.store(L, lane, r0);
+      if (kWave + lane < tot) pol.store(L, kWave + lane, r1);
+      wave_sync();
+      // candidate slots lane and 64 + lane in registers (slots past the last:
+      // far away); the active own particles, and the slots that skip each
+      // other, as bit masks
+      double2 cp[2];
+      unsigned long long skp[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int l = h * kWave + lane;
+        const bool real = l < tot;
+        const double2 r = pol.pos_lds(L, real ? l : 0);
+        cp[h] = real ? r : make_double2(kFar64, kFar64);
+        skp[h] = P::kSkip ? __ballot(real && pol.skip_lds(L, real ? l : 0)) : 0ull;
+      }
+      const unsigned long long act =
+          __ballot(lane < nown && pol.act_lds(L, lane < nown ? lane : 0));
+      snact += __popcll(act);
+      scand += __popcll(act & ~skp[0]) * (tot - 1);
+      if (P::kSkip) scand += __popcll(act & skp[0]) * (tot - __popcll(skp[0]) - __popcll(skp[1]));
+      if (!act) continue;
+      const int most = min(kOwn, kCellFlat / tot);  // own particles listed together
+      for (int p0 = 0; p0 < nown; p0 += most) {
+        const int np = min(most, nown - p0);
+        int e = 0, st = 0;  // st: lane p's first list position (lane np: the list's length)
+        double2 pr = pol.pos_lds(L, p0);
+        for (int p = 0; p < np; ++p) {
+          const int q = p0 + p;
+          const double2 own = pr;
+          pr = pol.pos_lds(L, q + 1);  // the next one's (slot q + 1 exists or is unused LDS)
+          st = lane == p ? e : st;
+          if (!((act >> q) & 1ull)) continue;
+          const bool skips = P::kSkip && ((skp[0] >> q) & 1ull);
+          unsigned long long m[2];
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            // (fused: the superset's margin covers the rounding)
+            const double drx = own.x - cp[h].x, dry = own.y - cp[h].y;
+            m[h] = __ballot(__builtin_fma(drx, drx, dry * dry) <= g.c2);
+            if (skips) m[h] &= ~skp[h];
+          }
+          m[0] &= ~(1ull << q);
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            if (__builtin_amdgcn_inverse_ballot_w64(m[h]))
+              flat[__builtin_amdgcn_mbcnt_hi((unsigned)(m[h] >> 32),
+                                             __builtin_amdgcn_mbcnt_lo((unsigned)m[h], e))] =
+                  (uint16_t)(p << 8 | h << 6 | lane);
+            e += __popcll(m[h]);
+          }
+        }
+        st = lane == np ? e : st;
+        wave_sync();
+        // lane (particle pc, term tc) sums particle pc's list range
+        const int pc = lane / NS, tc = lane - pc * NS;
+        const int x0 = __shfl(st, pc, kWave), x1 = pc < np ? __shfl(st, min(pc + 1, 63), kWave) : 0;
+        double acc = 0.;
+        for (int w0 = 0; w0 < e; w0 += NT) {
+          const int we = min(NT, e - w0);
+          for (int w = lane; w < we; w += kWave) {
+            const unsigned en = flat[w0 + w];
+            double t[NS];
+            npair += pol.terms(L, p0 + (int)(en >> 8), (int)(en & 255u), t);
+#pragma unroll
+            for (int q = 0; q < NS; ++q) terms[q * NT + w] = t[q];
+          }
+          wave_sync();
+          // eight terms at a time, their loads in flight together
+          const double *tp = terms + tc * NT;
+          const int hi = min(x1 - w0, NT);
+          int x = max(x0 - w0, 0);
+          for (; x + 8 <= hi; x += 8) {
+            double v[8];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) v[q] = tp[x + q];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) acc += v[q];
+          }
+          // the rest with one more batch of loads (reads past the range stay
+          // in the wavefront's LDS; +0 leaves a sum that starts at +0 unchanged)
+          if (x < hi) {
+            double v[7];
+#pragma unroll
+            for (int q = 0; q < 7; ++q) v[q] = tp[x + q];
+#pragma unroll
+            for (int q = 0; q < 7; ++q) acc += x + q < hi ? v[q] : 0.;
+          }
+          wave_sync();
+        }
+        // lane p takes its particle's sums and writes the particle
+        terms[lane] = acc;
+        wave_sync();
+        if (lane < np && pol.act_lds(L, p0 + lane)) {
+          double sum[NS];
+#pragma unroll
+          for (int q = 0; q < NS; ++q) sum[q] = terms[lane * NS + q];
+          pol.sums(L, p0 + lane, own0 + p0 + lane, sum);
+        }
+        wave_sync();
+      }
+    }
+  }
+  if (lane == 0) {
+    ncand += scand;
+    nact += snact;
+  }
+  wave_count(npair, ncand, nact, counters);
+}
+
 template <bool DYN, class P>
 __device__ __forceinline__ void walk32(const P &pol, const Consts &k, const int *__restrict__ cell_start,
                                        const int *__restrict__ cellof, int rows,
@@ -673,6 +978,20 @@ __device__ __forceinline__ void walk32(const P &pol, const Consts &k, const int 
   }
   tq_mark(tq, -1);
   wave_count(npair, ncand, nact, counters);
+}
+
+// workgroups of a cell-walk launch: those that are resident at once (the walk
+// strides, so a workgroup that waits for a slot would run its whole share
+// after the others'), fewer for a system that has not a cell for each
+// wavefront of those.  fit: the context's record of the kernel's occupancy
+// (0: not asked yet).
+template <typename K>
+int cell_groups(const tsph_ctx *c, K kernel, int lds, int &fit) {
+  if (fit < 1 &&
+      (hipOccupancyMaxActiveBlocksPerMultiprocessor(&fit, kernel, kCellBlock, lds) != hipSuccess || fit < 1))
+    fit = 1;
+  const int most = c->num_cu * std::min(fit, 8), want = std::max(c->num_cu, c->n_ub / 12);
+  return 8 * ((std::min(most, want) + 7) / 8);
 }
 
 // a pair-loop launch, bracketed by HIP events while pair timing is enabled
