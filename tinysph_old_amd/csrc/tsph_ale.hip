@@ -6,9 +6,10 @@
 // with the particle volume variables of ALESPH_Add_particle
 // (src/SPH_particle_system.h:51-108).
 //
-// The pair loop reuses the tile machinery of the WCSPH loops (persistent
-// waves over XCD-banded tiles, neighbour slices staged in LDS, lane-private
-// neighbour lists).  Per pair it solves the linearised Riemann problem along
+// The pair loop is the cell walk of tsph_tiles.h in FP64 and reuses the tile
+// machinery of the WCSPH loops in the mixed form (persistent waves over
+// XCD-banded tiles, neighbour slices staged in LDS, lane-private neighbour
+// lists).  Per pair it solves the linearised Riemann problem along
 // the pair normal (src/ALESPH_riemann_solver.h:20-34, 86-96), with a
 // one-sided wall state for BT wall neighbours (src/RALESPH_interaction.h:217-253).
 //
@@ -29,57 +30,76 @@ namespace {
 
 using namespace tiles;
 
-struct AccA64 {
-  double dom = 0, domrho = 0, dovx = 0, dovy = 0, gamma = 0;
+// constants of the FP64 pass
+struct Rale64 {
+  double h, ih, awen, bwen, cs, ics, cs2, ics2, rho0, irho0, cb, dp, gx, gy;
+};
+__host__ __device__ __forceinline__ Rale64 rale64(const Consts &k) {
+  return {k.h, k.ih, k.awen, k.bwen, k.cs, 1. / k.cs, k.cs * k.cs, 1. / (k.cs * k.cs), k.rho0,
+          1. / k.rho0, k.cb, k.dp, k.gx, k.gy};
+}
+
+// one particle of the FP64 pass
+struct RaleP {
+  double2 r, v, n;
+  double rho, omega;
+  int t;
 };
 
-// one RALE pair in the reference operand order
-__device__ __forceinline__ void rale_pair64(const Consts &k, AccA64 &s, double2 ar, double2 av,
-                                            double arho, double2 nr, double2 nv, double nrho,
-                                            double no, int nt, double2 n) {
-  const double h = k.h, c0 = k.cs, dp = k.dp, m = k.m, rho0 = k.rho0;
-  const double drx = ar.x - nr.x, dry = ar.y - nr.y;
-  const double drs = sqrt((drx * drx) + (dry * dry));
-  const KW64 kw = wendland64(drs, h, k.awen, k.bwen);
+// the terms of one RALE pair (d omega, d omega rho, d omega v) in the reference
+// operand order, zeros beyond the exact support; bit 0 of the result: inside
+// it, bit 1: its gamma term W m / rho_j is not 0 (W is 0 only at qq = 2)
+__device__ __forceinline__ int rale_pair64(const Rale64 &k, const RaleP &o, const RaleP &b,
+                                           double (&t)[4]) {
+  const double c0 = k.cs, dp = k.dp, rho0 = k.rho0;
+  const double drx = o.r.x - b.r.x, dry = o.r.y - b.r.y;
+  const Root64 rt = sqrt64((drx * drx) + (dry * dry));
+  const double qq = quot64(rt.s, k.h, k.ih);
+  const KW64 kw = wendland64(rt, qq, k.awen, k.bwen);
   const double W = kw.w;
   const double dWx = drx * kw.f, dWy = dry * kw.f;
-  const double dvx = av.x - nv.x, dvy = av.y - nv.y;
+  const double dvx = o.v.x - b.v.x, dvy = o.v.y - b.v.y;
   const double dvdW = dvx * dWx + dvy * dWy;
-  const double inv = 1 / drs;
+  const double inv = quot64(1., rt.s, recip_of_root64(rt));
   const double drnx = drx * inv * (-1), drny = dry * inv * (-1);
-  const double vL = av.x * drnx + av.y * drny;
-  const double vR = nv.x * drnx + nv.y * drny;
-  const double avgrho = 0.5 * (arho + nrho);
-  const double vss = 0.5 * (vR + vL) - 0.5 * (nrho - arho) * c0 / avgrho;
+  const double vL = o.v.x * drnx + o.v.y * drny;
+  const double vR = b.v.x * drnx + b.v.y * drny;
+  const double avgrho = 0.5 * (o.rho + b.rho);
+  const double vss = 0.5 * (vR + vL) - quot64_any(0.5 * (b.rho - o.rho) * c0, avgrho, recip64(avgrho));
   const double dd = vL - vR;
   const double mx = dd > 0 ? dd : 0;
   const double e = 3. * mx;
   const double beta = e < c0 ? e : c0;
-  const double rhos = 0.5 * (arho + nrho) + 0.5 * beta * (vL - vR) * (0.5 * (arho + nrho)) / (c0 * c0);
-  const double vsx = drnx * vss + ((av.x + nv.x) * 0.5 - drnx * (vL + vR) * 0.5);
-  const double vsy = drny * vss + ((av.y + nv.y) * 0.5 - drny * (vL + vR) * 0.5);
-  if (nt == TSPH_WALL) {
-    const double nbx = n.x * (-1), nby = n.y * (-1);
-    const double rw = arho - ((0 - av.x) * nbx + (0 - av.y) * nby) * arho / c0;
+  const double rhos = 0.5 * (o.rho + b.rho) +
+                      quot64_any(0.5 * beta * (vL - vR) * (0.5 * (o.rho + b.rho)), k.cs2, k.ics2);
+  const double vsx = drnx * vss + ((o.v.x + b.v.x) * 0.5 - drnx * (vL + vR) * 0.5);
+  const double vsy = drny * vss + ((o.v.y + b.v.y) * 0.5 - drny * (vL + vR) * 0.5);
+  if (b.t == TSPH_WALL) {
+    const double nbx = b.n.x * (-1), nby = b.n.y * (-1);
+    const double rw = o.rho - quot64_any(((0 - o.v.x) * nbx + (0 - o.v.y) * nby) * o.rho, c0, k.ics);
     const double pw = c0 * c0 * (rw - rho0) * 1;
-    s.dovx -= 2 * W * dp * (pw * nbx);
-    s.dovy -= 2 * W * dp * (pw * nby);
     const double dvn = dvx * nbx + dvy * nby;
-    s.dom -= dvn * W * dp;
+    t[0] = 0. - dvn * W * dp;
+    t[1] = 0.;
+    t[2] = 0. - 2 * W * dp * (pw * nbx);
+    t[3] = 0. - 2 * W * dp * (pw * nby);
   } else {
-    const double ps = tait64(rhos, rho0, c0);
-    s.dovx -= 2 * no * ((rhos * vsx * (vsx - av.x) + ps) * dWx + (rhos * vsx * (vsy - av.y)) * dWy);
-    s.dovy -= 2 * no * ((rhos * vsy * (vsx - av.x)) * dWx + (rhos * vsy * (vsy - av.y) + ps) * dWy);
-    const double vsdW = (vsx - av.x) * dWx + (vsy - av.y) * dWy;
-    s.dom -= dvdW * no;
-    s.domrho -= 2 * rhos * no * vsdW;
+    // Compute_Pressure (tait64)
+    const double ps = k.cb * (pow7(quot64_any(rhos, rho0, k.irho0)) - 1);
+    const double vsdW = (vsx - o.v.x) * dWx + (vsy - o.v.y) * dWy;
+    t[0] = 0. - dvdW * b.omega;
+    t[1] = 0. - 2 * rhos * b.omega * vsdW;
+    t[2] = 0. - 2 * b.omega * ((rhos * vsx * (vsx - o.v.x) + ps) * dWx + (rhos * vsx * (vsy - o.v.y)) * dWy);
+    t[3] = 0. - 2 * b.omega * ((rhos * vsy * (vsx - o.v.x)) * dWx + (rhos * vsy * (vsy - o.v.y) + ps) * dWy);
   }
-  s.gamma += W * m / nrho;
+  if (!(qq <= 2.0)) t[0] = t[1] = t[2] = t[3] = 0.;
+  return (int)(qq <= 2.0) | ((int)((qq < 2.0) & (fabs(b.rho) != INFINITY)) << 1);
 }
 
 // outputs for a particle whose own gamma sum is non-zero (:271-273), or the
 // all-zero branch (:265-267) pending k_rale_isolated
-__device__ __forceinline__ void rale_finish(const Soa &d, const Consts &k, int i, double ao,
+template <class D, class K>
+__device__ __forceinline__ void rale_finish(const D &d, const K &k, int i, double ao,
                                            double arho, double dom, double domrho, double dovx,
                                            double dovy, bool nonzero, uint8_t *gflag) {
   if (nonzero) {
@@ -94,123 +114,90 @@ __device__ __forceinline__ void rale_finish(const Soa &d, const Consts &k, int i
   gflag[i] = nonzero;
 }
 
-// FP64 tile kernel, reference summation order (9 cells, ascending index)
-template <bool DYN>
-__global__ __launch_bounds__(kWave * kPoolWaves) void k_rale64(Soa d, const int *__restrict__ cell_start,
-                                                  const int *__restrict__ cellof, Consts k, int rows,
-                                                  int *__restrict__ scal,
-                                                  const int *__restrict__ tile_list, int cap,
-                                                  const int *__restrict__ bound, int lds_wave,
-                                                  uint8_t *__restrict__ gflag,
-                                                  unsigned long long *__restrict__ counters) {
-  extern __shared__ __align__(16) unsigned char smem[];
-  unsigned char *wl = wave_lds<DYN>(smem, lds_wave);
-  int *tab = reinterpret_cast<int *>(wl);
-  double2 *s_r = reinterpret_cast<double2 *>(wl + kTabBytes);
-  double2 *s_v = s_r + cap;
-  double2 *s_rw = s_v + cap;  // {rho, omega}
-  double2 *s_n = s_rw + cap;
-  uint16_t *s_list = reinterpret_cast<uint16_t *>(s_n + cap);
-  uint8_t *s_t = reinterpret_cast<uint8_t *>(s_list + kList * kWave);
+// FP64: the cell walk's policy (cells64, tsph_tiles.h)
+struct RalePtr {
+  const double2 *r, *v, *n;
+  const double *rho, *omega;
+  const uint8_t *type;
+  double *domega, *domegarho;
+  double2 *domegav;
+  uint8_t *gflag;
+};
 
-  if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&counters[C_PASSES], 1ull);
-  unsigned npair = 0, ncand = 0, nact = 0;
-  TileQueue tq = tq_begin<DYN>(scal, bound, tile_list, smem);
-  for (int it = tq_take<DYN>(tq, tq_ticket<DYN>(tq)); it >= 0;) {
-    wave_sync();
-    const int ticket = tq_ticket<DYN>(tq);  // read once this tile's loads are waited for
-    Tile t;
-    tile_begin(k, cell_start, tile_list[it], rows, tab, t);
-    tq_mark(tq, tile_list[it]);
-    const bool staged = t.lq[3] <= cap;
-    if (staged) {
-      for (int l = tile_lane(); l < t.lq[3]; l += kWave) {
-        const int j = l - sel3(t.base, slice_of(t, l));
-        s_r[l] = d.r[j];
-        s_v[l] = d.v[j];
-        s_rw[l] = make_double2(d.rho[j], d.omega[j]);
-        s_t[l] = d.type[j];
-        s_n[l] = d.n ? d.n[j] : make_double2(0., 0.);
-      }
-    }
-    wave_sync();
-    const int next = tq_take<DYN>(tq, ticket);
-    const int lane = tile_lane();
-    uint16_t *my_list = s_list + lane;
-    for (int i0 = t.own0; i0 < t.own1; i0 += kWave) {
-      const int i = i0 + lane;
-      int li = 0, cy = 0;
-      bool act = false;
-      if (i < t.own1) {
-        li = i + t.base[1];
-        act = d.type[i] == TSPH_FLUID;
-        cy = cellof[i] - t.cx * k.ncy;
-      }
-      nact += act;
-      const double2 ar = act ? d.r[i] : make_double2(0., 0.);
-      const double2 av = act ? d.v[i] : make_double2(0., 0.);
-      const double arho = act ? d.rho[i] : 1.;
-      const double ao = act ? d.omega[i] : 0.;
-      AccA64 s;
-      if (!staged) {
-        // neighbourhood beyond the LDS budget: gather from global memory
-        if (act) {
-          const int c = cellof[i];
-          for (int q = 0; q < 9; ++q) {
-            int dx, dy;
-            stencil_dxy(q, dx, dy);
-            if (t.cx + dx < 0 || t.cx + dx >= k.ncx || cy + dy < 0 || cy + dy >= k.ncy) continue;
-            const int cl = c + dy + dx * k.ncy;
-            for (int j = cell_start[cl]; j < cell_start[cl + 1]; ++j) {
-              if (j == i) continue;
-              ++ncand;
-              const double2 nr = d.r[j];
-              if (!in_support64(ar.x - nr.x, ar.y - nr.y, k.h)) continue;
-              ++npair;
-              rale_pair64(k, s, ar, av, arho, nr, d.v[j], d.rho[j], d.omega[j], d.type[j],
-                          d.n ? d.n[j] : make_double2(0., 0.));
-            }
-          }
-        }
-      } else {
-        int q = -1, lj = 0, lend = 0;
-        bool more = act;
-        while (__any(more)) {
-          int cnt = 0;
-          while (more && cnt < kList) {
-            if (lj >= lend) {
-              ++q;
-              if (q == 9) { more = false; break; }
-              int dx, dy;
-              stencil_dxy(q, dx, dy);
-              const int row = cy + dy;
-              if (row < 0 || row >= k.ncy) { lend = lj; continue; }
-              const int e = (dx + 1) * t.w + (row - t.row_lo);
-              const int bq = sel3(t.base, dx + 1);
-              lj = tab[e] + bq;
-              lend = tab[e + 1] + bq;
-              continue;
-            }
-            const int j = lj++;
-            if (j == li) continue;
-            ++ncand;
-            const double2 nr = s_r[j];
-            if (in_support64(ar.x - nr.x, ar.y - nr.y, k.h)) my_list[(cnt++) * kWave] = (uint16_t)j;
-          }
-          npair += cnt;
-          for (int e = 0; e < cnt; ++e) {
-            const int j = my_list[e * kWave];
-            const double2 rw = s_rw[j];
-            rale_pair64(k, s, ar, av, arho, s_r[j], s_v[j], rw.x, rw.y, s_t[j], s_n[j]);
-          }
-        }
-      }
-      if (act) rale_finish(d, k, i, ao, arho, s.dom, s.domrho, s.dovx, s.dovy, s.gamma != 0, gflag);
-    }
-    it = next;
+struct RaleCell64 {
+  RalePtr d;
+  Rale64 k;
+  static constexpr int kSums = 4, kSlotBytes = 4 * 16 + 1, kWaves = 4;
+  static constexpr bool kFlag = true, kSkip = false;
+  struct Lds {
+    double2 *r, *v, *rw, *n;  // rw = {rho, omega}
+    uint8_t *t;
+  };
+  using Rec = RaleP;
+  static __device__ __forceinline__ Lds lds(unsigned char *b, int cap) {
+    double2 *p = reinterpret_cast<double2 *>(b);
+    return {p, p + cap, p + 2 * cap, p + 3 * cap, reinterpret_cast<uint8_t *>(p + 4 * cap)};
   }
-  tq_mark(tq, -1);
-  wave_count(npair, ncand, nact, counters);
+  __device__ __forceinline__ void set(const Consts &) {}  // (no batched ALE contexts)
+  __device__ __forceinline__ Rec load(int j) const {
+    return {d.r[j], d.v[j], d.n ? d.n[j] : make_double2(0., 0.), d.rho[j], d.omega[j], d.type[j]};
+  }
+  __device__ __forceinline__ void store(const Lds &L, int l, const Rec &q) const {
+    L.r[l] = q.r;
+    L.v[l] = q.v;
+    L.rw[l] = make_double2(q.rho, q.omega);
+    L.n[l] = q.n;
+    L.t[l] = (uint8_t)q.t;
+  }
+  static __device__ __forceinline__ Rec slot(const Lds &L, int l) {
+    const double2 rw = L.rw[l];
+    return {L.r[l], L.v[l], L.n[l], rw.x, rw.y, L.t[l]};
+  }
+  __device__ __forceinline__ bool act_lds(const Lds &L, int l) const { return L.t[l] == TSPH_FLUID; }
+  __device__ __forceinline__ bool skip_lds(const Lds &, int) const { return false; }
+  __device__ __forceinline__ double2 pos_lds(const Lds &L, int l) const { return L.r[l]; }
+  __device__ __forceinline__ int terms(const Lds &L, int p, int l, double (&t)[kSums]) const {
+    return rale_pair64(k, slot(L, p), slot(L, l), t);
+  }
+  __device__ __forceinline__ void sums(const Lds &L, int p, int i, const double (&s)[kSums],
+                                       bool some) const {
+    const double2 rw = L.rw[p];
+    rale_finish(d, k, i, rw.y, rw.x, s[0], s[1], s[2], s[3], some, d.gflag);
+  }
+  __device__ __forceinline__ void far(int i, const int *cs, const CellGrid &g, int c, unsigned &npair,
+                                      unsigned &ncand, unsigned &nact) const {
+    const Rec o = load(i);
+    if (o.t != TSPH_FLUID) return;
+    ++nact;
+    const int cx = c / g.ncy, cy = c - cx * g.ncy;
+    double s[kSums] = {0., 0., 0., 0.};
+    bool some = false;
+    for (int q = 0; q < 9; ++q) {
+      int dx, dy;
+      stencil_dxy(q, dx, dy);
+      if (cx + dx < 0 || cx + dx >= g.ncx || cy + dy < 0 || cy + dy >= g.ncy) continue;
+      const int cl = c + dy + dx * g.ncy;
+      for (int j = cs[cl]; j < cs[cl + 1]; ++j) {
+        if (j == i) continue;
+        ++ncand;
+        const Rec b = load(j);
+        const double drx = o.r.x - b.r.x, dry = o.r.y - b.r.y;
+        if (drx * drx + dry * dry > g.c2) continue;
+        double t[kSums];
+        const int got = rale_pair64(k, o, b, t);
+        npair += got & 1;
+        some |= (got & 2) != 0;
+        for (int u = 0; u < kSums; ++u) s[u] += t[u];
+      }
+    }
+    rale_finish(d, k, i, o.omega, o.rho, s[0], s[1], s[2], s[3], some, d.gflag);
+  }
+};
+
+__global__ __launch_bounds__(RaleCell64::kWaves * kWave, 3) void k_rale_cells64(
+    RaleCell64 pol, CellGrid g, const int *__restrict__ cell_start, CellSource src,
+    unsigned long long *__restrict__ counters) {
+  cells64(pol, g, cell_start, nullptr, 1, src, counters);
 }
 
 // --------------------------------------------------------------------------
@@ -522,30 +509,22 @@ int launch_rale_forces(tsph_ctx *c) {
     // the ALE passes stride (see launch_pass, tsph_alemuscl.hip)
     const TileGrid tg =
         tile_grid(c, true, kTabBytes + list + (size_t)cap * (4 * sizeof(float2) + 1), false);
-    if ((e = ensure_tile_list(c, tg.pooled ? tg.groups : 0))) return e;
+    if ((e = ensure_tile_list(c, 0))) return e;
     e = launch_timed(c, [&] {
-      if (tg.pooled)
-        hipLaunchKernelGGL(k_rale32<true>, tg.grid, tg.block, tg.lds, s, c->cur, c->cell_start,
-                           c->cellof, k, rows, c->scal, c->tile_list, cap, c->tile_bound,
-                           tg.lds_wave, c->ale_flag, c->counters);
-      else
-        hipLaunchKernelGGL(k_rale32<false>, tg.grid, tg.block, tg.lds, s, c->cur, c->cell_start,
+      hipLaunchKernelGGL(k_rale32<false>, tg.grid, tg.block, tg.lds, s, c->cur, c->cell_start,
                            c->cellof, k, rows, c->scal, c->tile_list, cap, c->tile_bound,
                            tg.lds_wave, c->ale_flag, c->counters);
     });
   } else {
-    const TileGrid tg =
-        tile_grid(c, false, kTabBytes + list + (size_t)cap * (4 * sizeof(double2) + 1), false);
-    if ((e = ensure_tile_list(c, tg.pooled ? tg.groups : 0))) return e;
+    constexpr int lds = cell_lds_bytes<RaleCell64>();
+    const Soa &d = c->cur;
+    if (!cells_direct(c) && (e = ensure_tile_list(c, 0))) return e;
+    const int groups = cell_groups(c, k_rale_cells64, RaleCell64::kWaves, lds, c->ale_fit[7]);
     e = launch_timed(c, [&] {
-      if (tg.pooled)
-        hipLaunchKernelGGL(k_rale64<true>, tg.grid, tg.block, tg.lds, s, c->cur, c->cell_start,
-                           c->cellof, k, rows, c->scal, c->tile_list, cap, c->tile_bound,
-                           tg.lds_wave, c->ale_flag, c->counters);
-      else
-        hipLaunchKernelGGL(k_rale64<false>, tg.grid, tg.block, tg.lds, s, c->cur, c->cell_start,
-                           c->cellof, k, rows, c->scal, c->tile_list, cap, c->tile_bound,
-                           tg.lds_wave, c->ale_flag, c->counters);
+      hipLaunchKernelGGL(k_rale_cells64, dim3(groups), dim3(RaleCell64::kWaves * kWave), lds, s,
+                         RaleCell64{{d.r, d.v, d.n, d.rho, d.omega, d.type, d.domega, d.domegarho,
+                                     d.domegav, c->ale_flag}, rale64(k)},
+                         cell_grid(k), c->cell_start, cell_source(c), c->counters);
     });
   }
   if (e) return e;

@@ -7,9 +7,10 @@
 //   Compute_Acceleration_BT            src/ALESPH_acceleration_bt.h:12-295
 //   Integrate_LeapFrog_partTwo_ALESPH  src/ALESPH_integration.h:33-83
 //
-// The three pair passes are policies over the generic tile walks of
-// tsph_tiles.h: FP64 in the reference's neighbour and operand order, and a
-// mixed form with FP32 fluxes on tile-frame positions and densities carried as
+// The three pair passes are policies: in FP64 of the cell walk of tsph_tiles.h
+// (the reference's neighbour and operand order; the tile walk's 27 KB of
+// records per wavefront left a compute unit four wavefronts, and each of them
+// two or three tiles of 183k particles), and of its tile walk in a mixed form with FP32 fluxes on tile-frame positions and densities carried as
 // deviations from rho0 (the linear EOS makes the pressure of a deviation exact).
 //
 // MUSCL states (src/ALESPH_riemann_solver.h:195-235): A_L = A_i + a/2 gA_i.dr,
@@ -39,19 +40,48 @@ constexpr int kOutletF = 17;  // outletf, src/SPH_defs.h:44-65
 // ---------------------------------------------------------------------------
 // shared pieces
 // ---------------------------------------------------------------------------
-// velRiemannLinearized, src/ALESPH_riemann_solver.h:86-96
-__device__ __forceinline__ double vel_riemann64(double rhoL, double rhoR, double vL, double vR,
-                                                double rhoAvg, double c) {
-  return 0.5 * (vR + vL) - 0.5 * (rhoR - rhoL) * c / rhoAvg;
+// constants of the FP64 passes
+struct Ale64 {
+  double h, ih, awen, bwen, cs, ics, cs2, ics2, rho0, irho0, m, dp, gx, gy;
+};
+__host__ __device__ __forceinline__ Ale64 ale64(const Consts &k) {
+  return {k.h, k.ih, k.awen, k.bwen, k.cs, 1. / k.cs, k.cs * k.cs, 1. / (k.cs * k.cs), k.rho0,
+          1. / k.rho0, k.m, k.dp, k.gx, k.gy};
 }
-// densRiemannLinearizedWithLimiter, src/ALESPH_riemann_solver.h:20-34
+
+// velRiemannLinearized, src/ALESPH_riemann_solver.h:86-96 (iavg: recip64(rhoAvg))
+__device__ __forceinline__ double vel_riemann64(double rhoL, double rhoR, double vL, double vR,
+                                                double rhoAvg, double iavg, double c) {
+  return 0.5 * (vR + vL) - quot64_any(0.5 * (rhoR - rhoL) * c, rhoAvg, iavg);
+}
+// densRiemannLinearizedWithLimiter, src/ALESPH_riemann_solver.h:20-34 (c2 = c c, ic2 = 1/c2)
 __device__ __forceinline__ double dens_riemann_lim64(double rhoL, double rhoR, double vL, double vR,
-                                                     double rhoAvg, double c) {
+                                                     double rhoAvg, double c, double c2, double ic2) {
   const double d = vL - vR;
   const double mx = d > 0 ? d : 0;
   const double e = 3. * mx;
   const double beta = e < c ? e : c;
-  return 0.5 * (rhoL + rhoR) + 0.5 * beta * (vL - vR) * rhoAvg / (c * c);
+  return 0.5 * (rhoL + rhoR) + quot64_any(0.5 * beta * (vL - vR) * rhoAvg, c2, ic2);
+}
+// minmod weights of a pair's two sides for one variable
+// (src/ALESPH_riemann_solver.h:161-191): r = 2 (grad.r_CD) / (aD - aC) - 1 on
+// either side; the two denominators are each other's negative, so one
+// reciprocal serves both.  r_CD: rij from o to b, dr back.  (A denominator so
+// small that its reciprocal overflows takes the general division.)
+__device__ __forceinline__ void minmod_weights64(double ao, double ab, double2 go, double2 gb,
+                                                 double2 rij, double2 dr, double &po, double &pb) {
+  const double d = ab - ao;
+  const double no = 2. * (go.x * rij.x + go.y * rij.y), nb = 2. * (gb.x * dr.x + gb.y * dr.y);
+  const double y = recip64(d);
+  double qo = quot64_any(no, d, y), qb = quot64_any(nb, -d, -y);
+  if (fabs(d) < 0x1p-960) {
+    qo = no / d;
+    qb = nb / -d;
+  }
+  const double ro = qo - 1., rb = qb - 1.;
+  const double mo = 1. < ro ? 1. : ro, mb = 1. < rb ? 1. : rb;
+  po = d == 0. ? 0. : (0. > mo ? 0. : mo);
+  pb = d == 0. ? 0. : (0. > mb ? 0. : mb);
 }
 template <typename T, typename V>
 __device__ __forceinline__ T minmod_phi(T aC, T aD, V g, V rCD) {
@@ -61,80 +91,47 @@ __device__ __forceinline__ T minmod_phi(T aC, T aD, V g, V rCD) {
   return T(0) > mn ? T(0) : mn;
 }
 
-// LDS slots of the FP64 passes: r, v, {rho, omega}, n [, grad rho, grad vx, grad vy], type
-template <bool G>
-struct Lds64 {
-  double2 *r, *v, *ro, *n, *gr, *gx, *gy;
-  uint8_t *t;
+// the fields the FP64 passes read and write
+struct AlePtr {
+  const double2 *r, *v, *n;
+  const double *rho, *omega;
+  const uint8_t *type;
+  double2 *gradrho, *gradvx, *gradvy;
+  double *domega, *domegarho;
+  double2 *domegav;
 };
-template <bool G>
-__device__ __forceinline__ Lds64<G> carve64(unsigned char *b, int cap) {
-  double2 *p = reinterpret_cast<double2 *>(b);
-  Lds64<G> L;
-  L.r = p; L.v = p + cap; L.ro = p + 2 * cap; L.n = p + 3 * cap;
-  L.gr = G ? p + 4 * cap : nullptr;
-  L.gx = G ? p + 5 * cap : nullptr;
-  L.gy = G ? p + 6 * cap : nullptr;
-  L.t = reinterpret_cast<uint8_t *>(p + (G ? 7 : 4) * cap);
-  return L;
-}
-template <bool G>
-constexpr int slot_bytes64() { return (G ? 7 : 4) * 16 + 1; }
 
+// one particle of the FP64 passes (own or neighbour; G: with its gradients)
 template <bool G>
-__device__ __forceinline__ void stage64(const Soa &d, const Lds64<G> &L, int l, int j) {
-  L.r[l] = d.r[j];
-  L.v[l] = d.v[j];
-  L.ro[l] = make_double2(d.rho[j], d.omega[j]);
-  L.n[l] = d.n ? d.n[j] : make_double2(0., 0.);
-  L.t[l] = d.type[j];
-  if (G) {
-    L.gr[l] = d.gradrho[j];
-    L.gx[l] = d.gradvx[j];
-    L.gy[l] = d.gradvy[j];
-  }
-}
-
-// one neighbour's data
-struct Nb64 {
-  double2 r, v, n, gr, gx, gy;
+struct P64;
+template <>
+struct P64<false> {
+  double2 r, v, n;
   double rho, omega;
   int t;
 };
-template <bool G>
-__device__ __forceinline__ Nb64 nb_lds64(const Lds64<G> &L, int l) {
-  Nb64 b;
-  b.r = L.r[l]; b.v = L.v[l]; b.n = L.n[l];
-  const double2 ro = L.ro[l];
-  b.rho = ro.x; b.omega = ro.y; b.t = L.t[l];
-  if (G) { b.gr = L.gr[l]; b.gx = L.gx[l]; b.gy = L.gy[l]; }
-  return b;
-}
-template <bool G>
-__device__ __forceinline__ Nb64 nb_glob64(const Soa &d, int j) {
-  Nb64 b;
-  b.r = d.r[j]; b.v = d.v[j]; b.n = d.n ? d.n[j] : make_double2(0., 0.);
-  b.rho = d.rho[j]; b.omega = d.omega[j]; b.t = d.type[j];
-  if (G) { b.gr = d.gradrho[j]; b.gx = d.gradvx[j]; b.gy = d.gradvy[j]; }
-  return b;
-}
-
-struct Own64 {
-  double2 r, v, gr, gx, gy;
-  double rho, omega;
+template <>
+struct P64<true> : P64<false> {
+  double2 gr, gx, gy;
 };
-template <bool G>
-__device__ __forceinline__ Own64 own64(const Soa &d, int i) {
-  Own64 o;
-  if (i >= 0) {
-    o.r = d.r[i]; o.v = d.v[i]; o.rho = d.rho[i]; o.omega = d.omega[i];
-    if (G) { o.gr = d.gradrho[i]; o.gx = d.gradvx[i]; o.gy = d.gradvy[i]; }
-  } else {
-    o.r = o.v = make_double2(0., 0.);
-    o.rho = 1.; o.omega = 0.;
-    o.gr = o.gx = o.gy = make_double2(0., 0.);
-  }
-  return o;
+
+// a pair's geometry: dr = r_i - r_j, its length, the kernel (0 beyond the
+// exact support) and whether the pair is inside it (qq <= 2)
+struct Geo64 {
+  double2 dr;
+  Root64 rt;
+  KW64 kw;
+  bool in, some;  // some: the kernel is not 0 (qq < 2)
+};
+__device__ __forceinline__ Geo64 geometry64(const Ale64 &k, double2 a, double2 b) {
+  Geo64 g;
+  g.dr = make_double2(a.x - b.x, a.y - b.y);
+  g.rt = sqrt64((g.dr.x * g.dr.x) + (g.dr.y * g.dr.y));
+  const double qq = quot64(g.rt.s, k.h, k.ih);
+  g.in = qq <= 2.0;
+  g.some = qq < 2.0;
+  g.kw = wendland64(g.rt, qq, k.awen, k.bwen);
+  return g;
 }
 
 // reconstructed left/right states (FP64, reference operand order)
@@ -142,22 +139,19 @@ struct LR64 {
   double rhoL, rhoR;
   double2 vL, vR;
 };
-template <bool G, bool LIM>
-__device__ __forceinline__ LR64 states64(const Own64 &o, const Nb64 &b, double2 dr) {
+template <bool LIM>
+__device__ __forceinline__ LR64 states64(const P64<false> &o, const P64<false> &b, double2) {
+  return {o.rho, b.rho, o.v, b.v};
+}
+template <bool LIM>
+__device__ __forceinline__ LR64 states64(const P64<true> &o, const P64<true> &b, double2 dr) {
   LR64 s;
-  if (!G) {
-    s.rhoL = o.rho; s.rhoR = b.rho; s.vL = o.v; s.vR = b.v;
-    return s;
-  }
   double a1 = 1, a2 = 1, a3 = 1, a4 = 1, a5 = 1, a6 = 1;
   if (LIM) {
     const double2 rij = make_double2(0. - dr.x, 0. - dr.y);
-    a1 = minmod_phi(o.rho, b.rho, o.gr, rij);
-    a2 = minmod_phi(b.rho, o.rho, b.gr, dr);
-    a3 = minmod_phi(o.v.x, b.v.x, o.gx, rij);
-    a4 = minmod_phi(o.v.y, b.v.y, o.gy, rij);
-    a5 = minmod_phi(b.v.x, o.v.x, b.gx, dr);
-    a6 = minmod_phi(b.v.y, o.v.y, b.gy, dr);
+    minmod_weights64(o.rho, b.rho, o.gr, b.gr, rij, dr, a1, a2);
+    minmod_weights64(o.v.x, b.v.x, o.gx, b.gx, rij, dr, a3, a5);
+    minmod_weights64(o.v.y, b.v.y, o.gy, b.gy, rij, dr, a4, a6);
   }
   s.rhoL = o.rho + a1 * 0.5 * (o.gr.x * dr.x + o.gr.y * dr.y);
   s.rhoR = b.rho - a2 * 0.5 * (b.gr.x * dr.x + b.gr.y * dr.y);
@@ -169,176 +163,260 @@ __device__ __forceinline__ LR64 states64(const Own64 &o, const Nb64 &b, double2 
 }
 
 // ---------------------------------------------------------------------------
-// FP64 passes
+// FP64 passes: policies of the cell walk (cells64, tsph_tiles.h).  The
+// reference's gamma sum is only compared with zero; its terms W m / rho are
+// zero exactly where W is (qq = 2) or rho is infinite, so a flag stands for it.
 // ---------------------------------------------------------------------------
 // Kernel_gradient_approx (fluid only): gradients of rho, vx, vy
 struct Grad64 {
-  Soa d;
-  Consts k;
-  using Lds = Lds64<false>;
-  using Own = Own64;
-  struct Acc {
-    double grx = 0, gry = 0, gxx = 0, gxy = 0, gyx = 0, gyy = 0, gamma = 0;
-  };
-  static __device__ Lds lds(unsigned char *b, int cap) { return carve64<false>(b, cap); }
-  __device__ void stage(const Lds &L, int l, int j) const { stage64<false>(d, L, l, j); }
-  __device__ bool active(int i) const { return d.type[i] == TSPH_FLUID; }
-  __device__ Own own(int i) const { return own64<false>(d, i); }
-  __device__ double2 pos_lds(const Lds &L, int l) const { return L.r[l]; }
-  __device__ double2 pos_glob(int j) const { return d.r[j]; }
-  __device__ void pair(Acc &a, const Own &o, const Nb64 &b) const {
-    const double2 dr = make_double2(o.r.x - b.r.x, o.r.y - b.r.y);
-    const double drs = sqrt((dr.x * dr.x) + (dr.y * dr.y));
-    const KW64 kw = wendland64(drs, k.h, k.awen, k.bwen);
-    const double W = kw.w;
-    const double dWx = dr.x * kw.f, dWy = dr.y * kw.f;
+  static constexpr bool kG = false, kSound = false;
+  static constexpr int kSums = 6;
+  static __device__ __forceinline__ bool active(int t) { return t == TSPH_FLUID; }
+  static __device__ __forceinline__ void pair(const Ale64 &k, const P64<false> &o, const P64<false> &b,
+                                              const Geo64 &g, double, double, double (&s)[kSums]) {
+    const double W = g.kw.w;
+    const double dWx = g.dr.x * g.kw.f, dWy = g.dr.y * g.kw.f;
     const double drho = b.rho - o.rho, dvx = b.v.x - o.v.x, dvy = b.v.y - o.v.y;
     if (b.t == TSPH_WALL) {
       const double nbx = b.n.x * (-1), nby = b.n.y * (-1);
-      a.grx += drho * nbx * W * k.dp;
-      a.gry += drho * nby * W * k.dp;
-      a.gxx += dvx * nbx * W * k.dp;
-      a.gxy += dvx * nby * W * k.dp;
-      a.gyx += dvy * nbx * W * k.dp;
-      a.gyy += dvy * nby * W * k.dp;
+      s[0] = drho * nbx * W * k.dp;
+      s[1] = drho * nby * W * k.dp;
+      s[2] = dvx * nbx * W * k.dp;
+      s[3] = dvx * nby * W * k.dp;
+      s[4] = dvy * nbx * W * k.dp;
+      s[5] = dvy * nby * W * k.dp;
     } else {
-      a.grx += drho * b.omega * dWx;
-      a.gry += drho * b.omega * dWy;
-      a.gxx += dvx * b.omega * dWx;
-      a.gxy += dvx * b.omega * dWy;
-      a.gyx += dvy * b.omega * dWx;
-      a.gyy += dvy * b.omega * dWy;
+      s[0] = drho * b.omega * dWx;
+      s[1] = drho * b.omega * dWy;
+      s[2] = dvx * b.omega * dWx;
+      s[3] = dvx * b.omega * dWy;
+      s[4] = dvy * b.omega * dWx;
+      s[5] = dvy * b.omega * dWy;
     }
-    a.gamma += W * k.m / b.rho;
   }
-  __device__ void pair_lds(Acc &a, const Own &o, const Lds &L, int l) const { pair(a, o, nb_lds64<false>(L, l)); }
-  __device__ void pair_glob(Acc &a, const Own &o, int j) const { pair(a, o, nb_glob64<false>(d, j)); }
-  __device__ void finish(const Acc &a, const Own &, int i) const {
-    if (a.gamma == 0) {
-      d.gradrho[i] = d.gradvx[i] = d.gradvy[i] = make_double2(0., 0.);
-    } else {
-      d.gradrho[i] = make_double2(a.grx * 2., a.gry * 2.);
-      d.gradvx[i] = make_double2(a.gxx * 2., a.gxy * 2.);
-      d.gradvy[i] = make_double2(a.gyx * 2., a.gyy * 2.);
+  static __device__ __forceinline__ void write(const Ale64 &, const AlePtr &d, const P64<false> &, int i,
+                                               const double (&s)[kSums], bool some) {
+    double2 gr = make_double2(0., 0.), gx = gr, gy = gr;
+    if (some) {
+      gr = make_double2(s[0] * 2., s[1] * 2.);
+      gx = make_double2(s[2] * 2., s[3] * 2.);
+      gy = make_double2(s[4] * 2., s[5] * 2.);
     }
+    d.gradrho[i] = gr;
+    d.gradvx[i] = gx;
+    d.gradvy[i] = gy;
   }
 };
 
 // Compute_Density: d(omega), d(omega rho)
 template <bool G, bool LIM>
 struct Dens64 {
-  Soa d;
-  Consts k;
-  using Lds = Lds64<G>;
-  using Own = Own64;
-  struct Acc {
-    double dom = 0, domrho = 0, gamma = 0;
-  };
-  static __device__ Lds lds(unsigned char *b, int cap) { return carve64<G>(b, cap); }
-  __device__ void stage(const Lds &L, int l, int j) const { stage64<G>(d, L, l, j); }
-  __device__ bool active(int i) const {
-    const int t = d.type[i];
+  static constexpr bool kG = G, kSound = false;
+  static constexpr int kSums = 2;
+  static __device__ __forceinline__ bool active(int t) {
     return t != kOutletF && t != TSPH_OUTLET && t != TSPH_INLET && t != TSPH_WALL && t != kRemoved;
   }
-  __device__ Own own(int i) const { return own64<G>(d, i); }
-  __device__ double2 pos_lds(const Lds &L, int l) const { return L.r[l]; }
-  __device__ double2 pos_glob(int j) const { return d.r[j]; }
-  __device__ void pair(Acc &a, const Own &o, const Nb64 &b) const {
-    const double c0 = k.cs;
-    const double2 dr = make_double2(o.r.x - b.r.x, o.r.y - b.r.y);
+  static __device__ __forceinline__ void pair(const Ale64 &k, const P64<G> &o, const P64<G> &b,
+                                              const Geo64 &g, double, double, double (&t)[kSums]) {
+    const double2 dr = g.dr;
     const double dvx = o.v.x - b.v.x, dvy = o.v.y - b.v.y;
-    const double drs = sqrt((dr.x * dr.x) + (dr.y * dr.y));
-    const double inv = 1 / drs;
+    const double inv = quot64(1., g.rt.s, recip_of_root64(g.rt));
     const double drnx = dr.x * inv * (-1), drny = dr.y * inv * (-1);
-    const KW64 kw = wendland64(drs, k.h, k.awen, k.bwen);
-    const double W = kw.w;
-    const double dWx = dr.x * kw.f, dWy = dr.y * kw.f;
-    const LR64 s = states64<G, LIM>(o, b, dr);
+    const double W = g.kw.w;
+    const double dWx = dr.x * g.kw.f, dWy = dr.y * g.kw.f;
+    const LR64 s = states64<LIM>(o, b, dr);
     const double vl = s.vL.x * drnx + s.vL.y * drny;
     const double vr = s.vR.x * drnx + s.vR.y * drny;
-    const double rhos = dens_riemann_lim64(s.rhoL, s.rhoR, vl, vr, 0.5 * (s.rhoL + s.rhoR), c0);
-    const double vss = vel_riemann64(s.rhoL, s.rhoR, vl, vr, 0.5 * (s.rhoL + s.rhoR), c0);
+    const double avg = 0.5 * (s.rhoL + s.rhoR);
+    const double rhos = dens_riemann_lim64(s.rhoL, s.rhoR, vl, vr, avg, k.cs, k.cs2, k.ics2);
+    const double vss = vel_riemann64(s.rhoL, s.rhoR, vl, vr, avg, recip64(avg), k.cs);
     const double vsx = drnx * vss + ((o.v.x + b.v.x) * 0.5 - drnx * (vl + vr) * 0.5);
     const double vsy = drny * vss + ((o.v.y + b.v.y) * 0.5 - drny * (vl + vr) * 0.5);
     const double vsdW = (vsx - o.v.x) * dWx + (vsy - o.v.y) * dWy;
-    if (b.t == TSPH_WALL) {
-      const double nbx = b.n.x * (-1), nby = b.n.y * (-1);
-      const double dvn = dvx * nbx + dvy * nby;
-      a.dom -= dvn * W * k.dp;
-    } else {
-      // the fluid volume flux term is zero as the reference build evaluates it
-      a.domrho -= 2 * rhos * b.omega * vsdW;
-    }
-    a.gamma += W * k.m / b.rho;
+    const bool wall = b.t == TSPH_WALL;
+    const double nbx = b.n.x * (-1), nby = b.n.y * (-1);
+    const double dvn = dvx * nbx + dvy * nby;
+    // the fluid volume flux term is zero as the reference build evaluates it
+    t[0] = wall ? 0. - dvn * W * k.dp : 0.;
+    t[1] = wall ? 0. : 0. - 2 * rhos * b.omega * vsdW;
   }
-  __device__ void pair_lds(Acc &a, const Own &o, const Lds &L, int l) const { pair(a, o, nb_lds64<G>(L, l)); }
-  __device__ void pair_glob(Acc &a, const Own &o, int j) const { pair(a, o, nb_glob64<G>(d, j)); }
-  __device__ void finish(const Acc &a, const Own &o, int i) const {
-    if (a.gamma == 0) {
-      d.domega[i] = 0.;
-      d.domegarho[i] = 0.;
-    } else {
-      d.domega[i] = a.dom * o.omega;
-      d.domegarho[i] = a.domrho * o.omega;
-    }
+  static __device__ __forceinline__ void write(const Ale64 &, const AlePtr &d, const P64<false> &o, int i,
+                                               const double (&s)[kSums], bool some) {
+    d.domega[i] = some ? s[0] * o.omega : 0.;
+    d.domegarho[i] = some ? s[1] * o.omega : 0.;
   }
 };
 
 // Compute_Acceleration_BT: d(omega v)
 template <bool G, bool LIM>
 struct Acc64P {
-  Soa d;
-  Consts k;
-  using Lds = Lds64<G>;
-  using Own = Own64;
-  struct Acc {
-    double ax = 0, ay = 0, gamma = 0;
-  };
-  static __device__ Lds lds(unsigned char *b, int cap) { return carve64<G>(b, cap); }
-  __device__ void stage(const Lds &L, int l, int j) const { stage64<G>(d, L, l, j); }
-  __device__ bool active(int i) const { return d.type[i] == TSPH_FLUID; }
-  __device__ Own own(int i) const { return own64<G>(d, i); }
-  __device__ double2 pos_lds(const Lds &L, int l) const { return L.r[l]; }
-  __device__ double2 pos_glob(int j) const { return d.r[j]; }
-  __device__ void pair(Acc &a, const Own &o, const Nb64 &b) const {
+  static constexpr bool kG = G, kSound = true;
+  static constexpr int kSums = 2;
+  static __device__ __forceinline__ bool active(int t) { return t == TSPH_FLUID; }
+  // co, cb: the particles' sound speeds c0 (rho/rho0)^(1/2)
+  // (src/ALESPH_riemann_solver.h:148-159), summed (:178)
+  static __device__ __forceinline__ void pair(const Ale64 &k, const P64<G> &o, const P64<G> &b,
+                                              const Geo64 &g, double co, double cb,
+                                              double (&t)[kSums]) {
     const double c0 = k.cs, rho0 = k.rho0;
-    const double2 dr = make_double2(o.r.x - b.r.x, o.r.y - b.r.y);
-    const double drs = sqrt((dr.x * dr.x) + (dr.y * dr.y));
-    const double inv = 1 / drs;
+    const double2 dr = g.dr;
+    const double inv = quot64(1., g.rt.s, recip_of_root64(g.rt));
     const double drnx = dr.x * inv * (-1), drny = dr.y * inv * (-1);
-    const KW64 kw = wendland64(drs, k.h, k.awen, k.bwen);
-    const double W = kw.w;
-    const double dWx = dr.x * kw.f, dWy = dr.y * kw.f;
-    const LR64 s = states64<G, LIM>(o, b, dr);
+    const double W = g.kw.w;
+    const double dWx = dr.x * g.kw.f, dWy = dr.y * g.kw.f;
+    const LR64 s = states64<LIM>(o, b, dr);
     const double vl = s.vL.x * drnx + s.vL.y * drny;
     const double vr = s.vR.x * drnx + s.vR.y * drny;
-    // cs(rho) = c0 (rho/rho0)^(1/2) (src/ALESPH_riemann_solver.h:148-159), summed (:178)
-    const double avgc = c0 * sqrt(o.rho / rho0) + c0 * sqrt(b.rho / rho0);
-    const double rhos = dens_riemann_lim64(s.rhoL, s.rhoR, vl, vr, 0.5 * (s.rhoL + s.rhoR), avgc);
-    const double vss = vel_riemann64(o.rho, b.rho, vl, vr, 0.5 * (s.rhoL + s.rhoR), avgc);
+    const double avgc = co + cb, c2 = avgc * avgc;
+    const double avg = 0.5 * (s.rhoL + s.rhoR);
+    const double rhos = dens_riemann_lim64(s.rhoL, s.rhoR, vl, vr, avg, avgc, c2, recip64(c2));
+    const double vss = vel_riemann64(o.rho, b.rho, vl, vr, avg, recip64(avg), avgc);
     const double vsx = drnx * vss + ((o.v.x + b.v.x) * 0.5 - drnx * (vl + vr) * 0.5);
     const double vsy = drny * vss + ((o.v.y + b.v.y) * 0.5 - drny * (vl + vr) * 0.5);
     if (b.t == TSPH_WALL) {
       const double nbx = b.n.x * (-1), nby = b.n.y * (-1);
-      const double rw = s.rhoL - ((0 - s.vL.x) * nbx + (0 - s.vL.y) * nby) * s.rhoL / c0;
+      const double rw = s.rhoL - quot64_any(((0 - s.vL.x) * nbx + (0 - s.vL.y) * nby) * s.rhoL, c0, k.ics);
       const double pw = c0 * c0 * (rw - 1000.) * 1;
-      a.ax -= 2 * W * k.dp * (pw * nbx);
-      a.ay -= 2 * W * k.dp * (pw * nby);
+      t[0] = 0. - 2 * W * k.dp * (pw * nbx);
+      t[1] = 0. - 2 * W * k.dp * (pw * nby);
     } else {
       const double ps = c0 * c0 * (rhos - rho0);
-      a.ax -= 2 * b.omega * ((rhos * vsx * (vsx - o.v.x) + ps) * dWx + (rhos * vsx * (vsy - o.v.y)) * dWy);
-      a.ay -= 2 * b.omega * ((rhos * vsy * (vsx - o.v.x)) * dWx + (rhos * vsy * (vsy - o.v.y) + ps) * dWy);
+      t[0] = 0. - 2 * b.omega * ((rhos * vsx * (vsx - o.v.x) + ps) * dWx + (rhos * vsx * (vsy - o.v.y)) * dWy);
+      t[1] = 0. - 2 * b.omega * ((rhos * vsy * (vsx - o.v.x)) * dWx + (rhos * vsy * (vsy - o.v.y) + ps) * dWy);
     }
-    a.gamma += W * k.m / b.rho;
   }
-  __device__ void pair_lds(Acc &a, const Own &o, const Lds &L, int l) const { pair(a, o, nb_lds64<G>(L, l)); }
-  __device__ void pair_glob(Acc &a, const Own &o, int j) const { pair(a, o, nb_glob64<G>(d, j)); }
-  __device__ void finish(const Acc &a, const Own &o, int i) const {
+  static __device__ __forceinline__ void write(const Ale64 &k, const AlePtr &d, const P64<false> &o, int i,
+                                               const double (&s)[kSums], bool some) {
     const double gx = k.gx * o.omega * o.rho, gy = k.gy * o.omega * o.rho;
-    if (a.gamma == 0)
-      d.domegav[i] = make_double2(0. - gx, 0. - gy);
-    else
-      d.domegav[i] = make_double2(a.ax * o.omega - gx, a.ay * o.omega - gy);
+    d.domegav[i] = some ? make_double2(s[0] * o.omega - gx, s[1] * o.omega - gy)
+                        : make_double2(0. - gx, 0. - gy);
+  }
+};
+
+// the cell walk's policy of pass A
+template <class A>
+struct AleCell64 {
+  AlePtr d;
+  Ale64 k;
+  static constexpr bool G = A::kG;
+  static constexpr int kSums = A::kSums;
+  static constexpr int kSlotBytes = (G ? 7 : 4) * 16 + (A::kSound ? 8 : 0) + 1;
+  static constexpr int kWaves = G ? 2 : 4;
+  static constexpr bool kFlag = true, kSkip = false;
+  struct Lds {
+    double2 *r, *v, *ro, *n, *gr, *gx, *gy;  // ro = {rho, omega}
+    double *cs;
+    uint8_t *t;
+  };
+  using Rec = P64<G>;
+  static __device__ __forceinline__ Lds lds(unsigned char *b, int cap) {
+    double2 *p = reinterpret_cast<double2 *>(b);
+    Lds L;
+    L.r = p; L.v = p + cap; L.ro = p + 2 * cap; L.n = p + 3 * cap;
+    L.gr = p + 4 * cap; L.gx = p + 5 * cap; L.gy = p + 6 * cap;
+    L.cs = reinterpret_cast<double *>(p + (G ? 7 : 4) * cap);
+    L.t = reinterpret_cast<uint8_t *>(L.cs + (A::kSound ? cap : 0));
+    return L;
+  }
+  __device__ __forceinline__ void set(const Consts &) {}  // (no batched ALE contexts)
+  __device__ __forceinline__ Rec load(int j) const {
+    Rec q;
+    q.r = d.r[j];
+    q.v = d.v[j];
+    q.rho = d.rho[j];
+    q.omega = d.omega[j];
+    q.n = d.n ? d.n[j] : make_double2(0., 0.);
+    q.t = d.type[j];
+    if constexpr (G) {
+      q.gr = d.gradrho[j];
+      q.gx = d.gradvx[j];
+      q.gy = d.gradvy[j];
+    }
+    return q;
+  }
+  __device__ __forceinline__ double sound(double rho) const {
+    return A::kSound ? k.cs * sqrt(quot64_any(rho, k.rho0, k.irho0)) : 0.;
+  }
+  __device__ __forceinline__ void store(const Lds &L, int l, const Rec &q) const {
+    L.r[l] = q.r;
+    L.v[l] = q.v;
+    L.ro[l] = make_double2(q.rho, q.omega);
+    L.n[l] = q.n;
+    L.t[l] = (uint8_t)q.t;
+    if (A::kSound) L.cs[l] = sound(q.rho);
+    if constexpr (G) {
+      L.gr[l] = q.gr;
+      L.gx[l] = q.gx;
+      L.gy[l] = q.gy;
+    }
+  }
+  static __device__ __forceinline__ Rec slot(const Lds &L, int l) {
+    Rec q;
+    q.r = L.r[l];
+    q.v = L.v[l];
+    q.n = L.n[l];
+    const double2 ro = L.ro[l];
+    q.rho = ro.x;
+    q.omega = ro.y;
+    q.t = L.t[l];
+    if constexpr (G) {
+      q.gr = L.gr[l];
+      q.gx = L.gx[l];
+      q.gy = L.gy[l];
+    }
+    return q;
+  }
+  __device__ __forceinline__ bool act_lds(const Lds &L, int l) const { return A::active(L.t[l]); }
+  __device__ __forceinline__ bool skip_lds(const Lds &, int) const { return false; }
+  __device__ __forceinline__ double2 pos_lds(const Lds &L, int l) const { return L.r[l]; }
+  // the terms; bit 0: inside the support, bit 1: its gamma term is not 0
+  __device__ __forceinline__ int pair(const Rec &o, const Rec &b, double co, double cb,
+                                      double (&t)[kSums]) const {
+    const Geo64 g = geometry64(k, o.r, b.r);
+    A::pair(k, o, b, g, co, cb, t);
+    if (!g.in) {
+#pragma unroll
+      for (int q = 0; q < kSums; ++q) t[q] = 0.;
+    }
+    return (int)g.in | ((int)(g.some & (fabs(b.rho) != INFINITY)) << 1);
+  }
+  __device__ __forceinline__ int terms(const Lds &L, int p, int l, double (&t)[kSums]) const {
+    return pair(slot(L, p), slot(L, l), A::kSound ? L.cs[p] : 0., A::kSound ? L.cs[l] : 0., t);
+  }
+  __device__ __forceinline__ void sums(const Lds &L, int p, int i, const double (&s)[kSums],
+                                       bool some) const {
+    A::write(k, d, slot(L, p), i, s, some);
+  }
+  __device__ __forceinline__ void far(int i, const int *cs, const CellGrid &g, int c, unsigned &npair,
+                                      unsigned &ncand, unsigned &nact) const {
+    const Rec o = load(i);
+    if (!A::active(o.t)) return;
+    ++nact;
+    const int cx = c / g.ncy, cy = c - cx * g.ncy;
+    double s[kSums];
+#pragma unroll
+    for (int q = 0; q < kSums; ++q) s[q] = 0.;
+    bool some = false;
+    for (int q = 0; q < 9; ++q) {
+      int dx, dy;
+      stencil_dxy(q, dx, dy);
+      if (cx + dx < 0 || cx + dx >= g.ncx || cy + dy < 0 || cy + dy >= g.ncy) continue;
+      const int cl = c + dy + dx * g.ncy;
+      for (int j = cs[cl]; j < cs[cl + 1]; ++j) {
+        if (j == i) continue;
+        ++ncand;
+        const Rec b = load(j);
+        const double drx = o.r.x - b.r.x, dry = o.r.y - b.r.y;
+        if (drx * drx + dry * dry > g.c2) continue;
+        double t[kSums];
+        const int got = pair(o, b, sound(o.rho), sound(b.rho), t);
+        npair += got & 1;
+        some |= (got & 2) != 0;
+#pragma unroll
+        for (int u = 0; u < kSums; ++u) s[u] += t[u];
+      }
+    }
+    A::write(k, d, o, i, s, some);
   }
 };
 
@@ -679,15 +757,11 @@ struct Acc32P {
 // ---------------------------------------------------------------------------
 // kernels
 // ---------------------------------------------------------------------------
-template <class P, bool DYN>
-__global__ __launch_bounds__(kWave * kPoolWaves) void k_ale_pass64(P pol, const int *__restrict__ cell_start,
-                                                      const int *__restrict__ cellof, int rows,
-                                                      int *__restrict__ scal,
-                                                      const int *__restrict__ tile_list,
-                                                      const int *__restrict__ bound, int cap,
-                                                      int lds_wave,
-                                                      unsigned long long *__restrict__ counters) {
-  walk64<DYN>(pol, pol.k, cell_start, cellof, rows, scal, tile_list, bound, cap, lds_wave, counters);
+template <class P>
+__global__ __launch_bounds__(P::kWaves * kWave, 2) void k_ale_cells64(
+    P pol, CellGrid g, const int *__restrict__ cell_start, CellSource src,
+    unsigned long long *__restrict__ counters) {
+  cells64(pol, g, cell_start, nullptr, 1, src, counters);
 }
 
 template <class P, bool DYN>
@@ -752,46 +826,46 @@ __global__ void k_ale_lf2(Soa d, const int *__restrict__ scal, double dt, int fi
   }
 }
 
-// launch of one pair pass on the persistent tile grid
-template <class P, int SLOT, bool FP32>
-int launch_pass(tsph_ctx *c, const P &pol) {
+// launch of one mixed pair pass on the persistent tile grid
+template <class P, int SLOT>
+int launch_pass32(tsph_ctx *c, const P &pol) {
   const int rows = c->tile_rows;
   // slots budgeted per tile, within 64 KiB of LDS per wavefront; a tile whose
   // neighbourhood does not fit is gathered from global memory instead.  The
-  // ALE records are large (57 B mixed, 113 B FP64 with the MUSCL gradients),
-  // so the budget is kAleCellCap records per cell, about a full cell's count
-  // at the configured resolutions: the fullest tiles then take the global
-  // path, and the smaller LDS area lets a compute unit hold more waves, which
-  // pays more than staging every tile does
+  // ALE records are large (57 B with the MUSCL gradients), so the budget is
+  // kAleCellCap records per cell, about a full cell's count at the configured
+  // resolutions: the fullest tiles then take the global path, and the smaller
+  // LDS area lets a compute unit hold more waves, which pays more than staging
+  // every tile does
   constexpr int kAleCellCap = 9;
   constexpr int kFixed = kTabBytes + sizeof(uint16_t) * kList * kWave;
   const int cap = std::min(3 * (rows + 2) * kAleCellCap, (65536 - kPoolHdr - kFixed) / SLOT);
   // the static walk: a cell build serves several passes of different cost
   // profiles, and the dam breaks these passes run on give each wave about ten
-  // tiles, too few for the pooled walk to pay for its chunk cut (183k
-  // particles, FP64: 0.56 ms per step pooled against 0.51 static)
-  const TileGrid tg = tile_grid(c, FP32, kFixed + (size_t)cap * SLOT, false);
-  if (int e = ensure_tile_list(c, tg.pooled ? tg.groups : 0)) return e;
+  // tiles, too few for the pooled walk to pay for its chunk cut
+  const TileGrid tg = tile_grid(c, true, kFixed + (size_t)cap * SLOT, false);
+  if (int e = ensure_tile_list(c, 0)) return e;
   return launch_timed(c, [&] {
-    if constexpr (FP32) {
-      if (tg.pooled)
-        hipLaunchKernelGGL((k_ale_pass32<P, true>), tg.grid, tg.block, tg.lds, c->stream, pol,
-                           c->cell_start, c->cellof, rows, c->scal, c->tile_list, c->tile_bound,
-                           cap, tg.lds_wave, c->counters);
-      else
-        hipLaunchKernelGGL((k_ale_pass32<P, false>), tg.grid, tg.block, tg.lds, c->stream, pol,
-                           c->cell_start, c->cellof, rows, c->scal, c->tile_list, c->tile_bound,
-                           cap, tg.lds_wave, c->counters);
-    } else {
-      if (tg.pooled)
-        hipLaunchKernelGGL((k_ale_pass64<P, true>), tg.grid, tg.block, tg.lds, c->stream, pol,
-                           c->cell_start, c->cellof, rows, c->scal, c->tile_list, c->tile_bound,
-                           cap, tg.lds_wave, c->counters);
-      else
-        hipLaunchKernelGGL((k_ale_pass64<P, false>), tg.grid, tg.block, tg.lds, c->stream, pol,
-                           c->cell_start, c->cellof, rows, c->scal, c->tile_list, c->tile_bound,
-                           cap, tg.lds_wave, c->counters);
-    }
+    hipLaunchKernelGGL((k_ale_pass32<P, false>), tg.grid, tg.block, tg.lds, c->stream, pol,
+                       c->cell_start, c->cellof, rows, c->scal, c->tile_list, c->tile_bound, cap,
+                       tg.lds_wave, c->counters);
+  });
+}
+
+// launch of one FP64 pair pass by cells
+template <class A>
+int launch_pass64(tsph_ctx *c, int slot) {
+  using P = AleCell64<A>;
+  constexpr int lds = cell_lds_bytes<P>();
+  const Soa &d = c->cur;
+  if (!cells_direct(c))
+    if (int e = ensure_tile_list(c, 0)) return e;
+  const int groups = cell_groups(c, k_ale_cells64<P>, P::kWaves, lds, c->ale_fit[slot]);
+  return launch_timed(c, [&] {
+    hipLaunchKernelGGL(k_ale_cells64<P>, dim3(groups), dim3(P::kWaves * kWave), lds, c->stream,
+                       P{{d.r, d.v, d.n, d.rho, d.omega, d.type, d.gradrho, d.gradvx, d.gradvy,
+                          d.domega, d.domegarho, d.domegav}, ale64(c->k)},
+                       cell_grid(c->k), c->cell_start, cell_source(c), c->counters);
   });
 }
 
@@ -802,32 +876,32 @@ int launch_ale_density(tsph_ctx *c, int muscl) {
   const bool mixed = c->prm.precision == TSPH_PREC_MIXED;
   if (mixed) {
     const C32A cc = make_c32a(c->k);
-    if (muscl == 0) return launch_pass<Dens32<false, false>, slot_bytes32<false>(), true>(c, {c->cur, c->k, cc});
-    if (muscl == 1) return launch_pass<Dens32<true, false>, slot_bytes32<true>(), true>(c, {c->cur, c->k, cc});
-    return launch_pass<Dens32<true, true>, slot_bytes32<true>(), true>(c, {c->cur, c->k, cc});
+    if (muscl == 0) return launch_pass32<Dens32<false, false>, slot_bytes32<false>()>(c, {c->cur, c->k, cc});
+    if (muscl == 1) return launch_pass32<Dens32<true, false>, slot_bytes32<true>()>(c, {c->cur, c->k, cc});
+    return launch_pass32<Dens32<true, true>, slot_bytes32<true>()>(c, {c->cur, c->k, cc});
   }
-  if (muscl == 0) return launch_pass<Dens64<false, false>, slot_bytes64<false>(), false>(c, {c->cur, c->k});
-  if (muscl == 1) return launch_pass<Dens64<true, false>, slot_bytes64<true>(), false>(c, {c->cur, c->k});
-  return launch_pass<Dens64<true, true>, slot_bytes64<true>(), false>(c, {c->cur, c->k});
+  if (muscl == 0) return launch_pass64<Dens64<false, false>>(c, 0);
+  if (muscl == 1) return launch_pass64<Dens64<true, false>>(c, 1);
+  return launch_pass64<Dens64<true, true>>(c, 2);
 }
 
 int launch_ale_acceleration(tsph_ctx *c, int muscl) {
   const bool mixed = c->prm.precision == TSPH_PREC_MIXED;
   if (mixed) {
     const C32A cc = make_c32a(c->k);
-    if (muscl == 0) return launch_pass<Acc32P<false, false>, slot_bytes32<false>(), true>(c, {c->cur, c->k, cc});
-    if (muscl == 1) return launch_pass<Acc32P<true, false>, slot_bytes32<true>(), true>(c, {c->cur, c->k, cc});
-    return launch_pass<Acc32P<true, true>, slot_bytes32<true>(), true>(c, {c->cur, c->k, cc});
+    if (muscl == 0) return launch_pass32<Acc32P<false, false>, slot_bytes32<false>()>(c, {c->cur, c->k, cc});
+    if (muscl == 1) return launch_pass32<Acc32P<true, false>, slot_bytes32<true>()>(c, {c->cur, c->k, cc});
+    return launch_pass32<Acc32P<true, true>, slot_bytes32<true>()>(c, {c->cur, c->k, cc});
   }
-  if (muscl == 0) return launch_pass<Acc64P<false, false>, slot_bytes64<false>(), false>(c, {c->cur, c->k});
-  if (muscl == 1) return launch_pass<Acc64P<true, false>, slot_bytes64<true>(), false>(c, {c->cur, c->k});
-  return launch_pass<Acc64P<true, true>, slot_bytes64<true>(), false>(c, {c->cur, c->k});
+  if (muscl == 0) return launch_pass64<Acc64P<false, false>>(c, 3);
+  if (muscl == 1) return launch_pass64<Acc64P<true, false>>(c, 4);
+  return launch_pass64<Acc64P<true, true>>(c, 5);
 }
 
 int launch_ale_gradient(tsph_ctx *c) {
   if (c->prm.precision == TSPH_PREC_MIXED)
-    return launch_pass<Grad32, slot_bytes32<false>(), true>(c, {c->cur, c->k, make_c32a(c->k)});
-  return launch_pass<Grad64, slot_bytes64<false>(), false>(c, {c->cur, c->k});
+    return launch_pass32<Grad32, slot_bytes32<false>()>(c, {c->cur, c->k, make_c32a(c->k)});
+  return launch_pass64<Grad64>(c, 6);
 }
 
 int launch_ale_density_pressure(tsph_ctx *c, double dt) {

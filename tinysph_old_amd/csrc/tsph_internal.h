@@ -171,7 +171,8 @@ struct tsph_ctx {
   int num_cu = 256;      // compute units of the device
   int max_lds_block = 65536;  // LDS bytes a workgroup may allocate
   int lds_cu = 163840;        // LDS bytes of one compute unit
-  int cells_fit[3] = {0, 0, 0};  // workgroups per compute unit of the cell walks (0: not asked yet)
+  // workgroups per compute unit of the cell walks, by kernel (0: not asked yet)
+  int cells_fit[3] = {}, ale_fit[8] = {};
   // pair-loop tile walk per precision (FP64, mixed): pooled (work-balanced
   // chunks per workgroup, tiles taken from an LDS counter by the workgroup's
   // waves) or the plain static walk; defaults set at creation

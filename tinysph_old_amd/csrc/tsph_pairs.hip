@@ -554,7 +554,8 @@ template <int VAR>
 struct Cell64 {
   Pair64 d;
   PairConsts k;
-  static constexpr int kSums = VAR == TSPH_FORCES_BT ? 5 : 4;
+  static constexpr int kSums = VAR == TSPH_FORCES_BT ? 5 : 4, kWaves = 4;
+  static constexpr bool kFlag = false;
   static constexpr int kSlotBytes = (VAR == TSPH_FORCES_BT ? 4 : 3) * 16 + 9;
   struct Lds {
     double2 *r, *v, *rp, *n;  // rp = {rho, p}; n: BT only
@@ -610,7 +611,7 @@ struct Cell64 {
     if (VAR == TSPH_FORCES_BT) t[kSums - 1] = s.gamma;
     return (int)np;
   }
-  __device__ __forceinline__ void sums(const Lds &L, int p, int i, const double (&t)[kSums]) const {
+  __device__ __forceinline__ void sums(const Lds &L, int p, int i, const double (&t)[kSums], bool) const {
     Acc64 s;
     s.accx = t[0];
     s.accy = t[1];
@@ -632,11 +633,11 @@ struct Cell64 {
 };
 
 template <class P>
-__global__ __launch_bounds__(kCellBlock, 3) void k_cells64(P pol, CellGrid g, const int *__restrict__ cell_start,
+__global__ __launch_bounds__(P::kWaves * kWave, 3) void k_cells64(P pol, CellGrid g, const int *__restrict__ cell_start,
                                                         const Consts *__restrict__ cases,
-                                                        int ncases, int ncells_tot,
+                                                        int ncases, CellSource src,
                                                         unsigned long long *__restrict__ counters) {
-  cells64(pol, g, cell_start, cases, ncases, ncells_tot, counters);
+  cells64(pol, g, cell_start, cases, ncases, src, counters);
 }
 
 // --------------------------------------------------------------------------
@@ -1001,12 +1002,12 @@ TileGrid tile_grid(tsph_ctx *c, bool fp32, size_t lds_wave, bool may_pool) {
 // kCellsMax particles.  A tile's wavefront takes about 25 us however small the
 // system is, a cell's 8 us, while a full chip does more pairs per second by
 // tiles (a dam break, us per pass, cells and tiles: 6k particles 9 / 41, 23k
-// 14 / 23, 50k 24 / 34, 92k 39 / 36, 740k 259 / 204).  The walk looks at every
-// cell of the grid, so grids of more than kCellsGrid cells keep the list of
-// non-empty tiles.
-constexpr int kCellsMax = 70000, kCellsGrid = 1 << 18;
+// 14 / 23, 50k 24 / 34, 92k 39 / 36, 740k 259 / 204).  A batch's grids
+// are walked whole (its tile list runs over all cases), so only up to
+// kCellsDirect cells.
+constexpr int kCellsMax = 70000;
 static bool cells_walk(const tsph_ctx *c) {
-  return c->prm.precision == TSPH_PREC_FP64 && c->n_ub <= kCellsMax && c->ncells_tot <= kCellsGrid;
+  return c->prm.precision == TSPH_PREC_FP64 && c->n_ub <= kCellsMax && (!c->cases || cells_direct(c));
 }
 
 // LDS bytes per wavefront of the pair pass of `variant` at the current tile rows
@@ -1054,11 +1055,11 @@ void cell_launch(tsph_ctx *c) {
   using P = Cell64<VAR>;
   constexpr int lds = cell_lds_bytes<P>();
   const Soa &d = c->cur;
-  const int groups = cell_groups(c, k_cells64<P>, lds, c->cells_fit[VAR]);
-  hipLaunchKernelGGL(k_cells64<P>, dim3(groups), dim3(kCellBlock), lds, c->stream,
+  const int groups = cell_groups(c, k_cells64<P>, P::kWaves, lds, c->cells_fit[VAR]);
+  hipLaunchKernelGGL(k_cells64<P>, dim3(groups), dim3(P::kWaves * kWave), lds, c->stream,
                      P{{d.r, d.v, d.n, d.rho, d.p, d.type, d.a, d.drho}, pair_consts(c->k)},
                      cell_grid(c->k), c->cell_start, c->cases, c->ncases,
-                     c->ncells_tot, c->counters);
+                     cell_source(c), c->counters);
 }
 
 template <int VAR>
@@ -1077,7 +1078,9 @@ int launch_forces(tsph_ctx *c, int variant, bool corr, double corr_dt) {
     if (int e = launch_mixed_records(c)) return e;
     c->records_valid = true;
   }
-  if (cells_walk(c))
+  if (cells_walk(c)) {
+    if (!cells_direct(c))
+      if (int e = ensure_tile_list(c, 0)) return e;
     return launch_timed(c, [&] {
       switch (variant) {
         case TSPH_FORCES_WCSPH: cell_launch<TSPH_FORCES_WCSPH>(c); break;
@@ -1085,6 +1088,7 @@ int launch_forces(tsph_ctx *c, int variant, bool corr, double corr_dt) {
         default: cell_launch<TSPH_FORCES_BT>(c);
       }
     });
+  }
   const TileGrid tg = tile_grid(c, mixed, forces_lds_wave(c, variant));
   if (int e = ensure_tile_list(c, tg.pooled ? tg.groups : 0, mixed && corr ? 1 : 0)) return e;
   const int e = launch_timed(c, [&] {

@@ -434,132 +434,17 @@ __device__ __forceinline__ int slice_of(const Tile &t, int l) {
 }
 
 // --------------------------------------------------------------------------
-// Generic tile walks.  A pass supplies a policy P:
+// Generic tile walk of the mixed passes (walk32).  A pass supplies a policy P:
 //   P::Lds            pointers into the staged-slot area of LDS
-//   P::lds(base, cap) carves that area (double2 / float2 arrays first)
+//   P::lds(base, cap) carves that area (float2 arrays first)
 //   P::kSlotBytes     bytes per staged slot
-//   stage(L, l, j[, ox, oy])  slot l <- particle j (FP32 walk: tile-frame origin)
+//   stage(L, l, j, ox, oy)  slot l <- particle j (tile-frame origin)
 //   active(i)         whether particle i is active in the pass
-//   Own own(i[, ox, oy]); Acc{} accumulators
-//   pair_lds(acc, own, L, l[, drx, dry, r2]) / pair_glob(acc, own, j[, ...])
+//   Own own(i, ox, oy); Acc{} accumulators
+//   pair_lds(acc, own, L, l, drx, dry, r2) / pair_glob(acc, own, j, ...)
 //   finish(acc, own, i)
-// walk64 visits neighbours in the reference order (9-cell stencil order,
-// ascending index in a cell) and tests support exactly as the reference does;
-// walk32 visits the three column slices in memory order with an FP32 test.
+// It visits the three column slices in memory order with an FP32 test.
 // --------------------------------------------------------------------------
-template <bool DYN, class P>
-__device__ __forceinline__ void walk64(const P &pol, const Consts &k, const int *__restrict__ cell_start,
-                                       const int *__restrict__ cellof, int rows,
-                                       int *__restrict__ scal, const int *__restrict__ tile_list,
-                                       const int *__restrict__ bound, int cap, int lds_wave,
-                                       unsigned long long *__restrict__ counters) {
-  extern __shared__ __align__(16) unsigned char smem[];
-  unsigned char *wl = wave_lds<DYN>(smem, lds_wave);
-  int *tab = reinterpret_cast<int *>(wl);
-  uint16_t *s_list = reinterpret_cast<uint16_t *>(wl + kTabBytes);
-  const typename P::Lds L = P::lds(wl + kTabBytes + sizeof(uint16_t) * kList * kWave, cap);
-  const int lane = tile_lane();
-  if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&counters[C_PASSES], 1ull);
-  unsigned npair = 0, ncand = 0, nact = 0;
-  TileQueue tq = tq_begin<DYN>(scal, bound, tile_list, smem);
-  for (int it = tq_take<DYN>(tq, tq_ticket<DYN>(tq)); it >= 0;) {
-    wave_sync();
-    const int ticket = tq_ticket<DYN>(tq);  // read once this tile's loads are waited for
-    Tile t;
-    tile_begin(k, cell_start, tile_list[it], rows, tab, t);
-    tq_mark(tq, tile_list[it]);
-    const bool staged = t.lq[3] <= cap;
-    if (staged)
-      for (int l = lane; l < t.lq[3]; l += kWave) pol.stage(L, l, l - sel3(t.base, slice_of(t, l)));
-    wave_sync();
-    const int next = tq_take<DYN>(tq, ticket);
-    uint16_t *my_list = s_list + lane;
-    for (int i0 = t.own0; i0 < t.own1; i0 += kWave) {
-      const int i = i0 + lane;
-      int li = 0, cy = 0;
-      bool act = false;
-      if (i < t.own1) {
-        li = i + t.base[1];
-        act = pol.active(i);
-        cy = cellof[i] - t.cx * k.ncy;
-      }
-      nact += act;
-      const typename P::Own o = pol.own(act ? i : -1);
-      typename P::Acc acc{};
-      if (!staged) {
-        if (act) {
-          const int c = cellof[i];
-          for (int q = 0; q < 9; ++q) {
-            int dx, dy;
-            stencil_dxy(q, dx, dy);
-            if (t.cx + dx < 0 || t.cx + dx >= k.ncx || cy + dy < 0 || cy + dy >= k.ncy) continue;
-            const int cl = c + dy + dx * k.ncy;
-            for (int j = cell_start[cl]; j < cell_start[cl + 1]; ++j) {
-              if (j == i) continue;
-              ++ncand;
-              const double2 nr = pol.pos_glob(j);
-              if (!in_support64(o.r.x - nr.x, o.r.y - nr.y, k.h)) continue;
-              ++npair;
-              pol.pair_glob(acc, o, j);
-            }
-          }
-        }
-      } else {
-        // a cell's candidates kGroup at a time, their LDS loads in flight
-        // together, appended without branches (every slot of the group is
-        // written, the count advances by the test); the exact test of
-        // in_support64, with its rounded square root only for the rare
-        // candidates within a relative 1e-12 of the boundary.  Slots past the
-        // cell's end are masked; they lie in the staged area or the next
-        // array of the wave's slots (positions come first).
-        const double c2 = 4.0 * k.h * k.h, c2lo = c2 * (1.0 - 1e-12), c2hi = c2 * (1.0 + 1e-12);
-        int q = -1, lj = 0, lend = 0;
-        bool more = act;
-        while (__any(more)) {
-          int cnt = 0;
-          while (more && cnt <= kList - kGroup) {
-            if (lj >= lend) {
-              ++q;
-              if (q == 9) { more = false; break; }
-              int dx, dy;
-              stencil_dxy(q, dx, dy);
-              const int row = cy + dy;
-              if (row < 0 || row >= k.ncy) { lend = lj; continue; }
-              const int e = (dx + 1) * t.w + (row - t.row_lo);
-              const int bq = sel3(t.base, dx + 1);
-              lj = tab[e] + bq;
-              lend = tab[e + 1] + bq;
-              continue;
-            }
-            const int m = min(kGroup, lend - lj);
-            double2 pp[kGroup];
-#pragma unroll
-            for (int u = 0; u < kGroup; ++u) pp[u] = pol.pos_lds(L, lj + u);
-#pragma unroll
-            for (int u = 0; u < kGroup; ++u) {
-              const int j = lj + u;
-              const bool cand = u < m && j != li;
-              ncand += cand;
-              const double drx = o.r.x - pp[u].x, dry = o.r.y - pp[u].y;
-              const double r2 = (drx * drx) + (dry * dry);
-              bool in = cand && r2 < c2lo;
-              if (cand && !in && r2 <= c2hi) in = sqrt(r2) / k.h <= 2.0;
-              my_list[cnt * kWave] = (uint16_t)j;
-              cnt += in;
-            }
-            lj += m;
-          }
-          npair += cnt;
-          for (int e = 0; e < cnt; ++e) pol.pair_lds(acc, o, L, my_list[e * kWave]);
-        }
-      }
-      if (act) pol.finish(acc, o, i);
-    }
-    it = next;
-  }
-  tq_mark(tq, -1);
-  wave_count(npair, ncand, nact, counters);
-}
 
 // --------------------------------------------------------------------------
 // Cell walk (FP64): one wavefront per cell, its pairs spread over all lanes
@@ -587,16 +472,19 @@ __device__ __forceinline__ void walk64(const P &pol, const Consts &k, const int 
 //   act_lds(L, l)                 slot l is active
 //   kSkip, skip_lds(L, l)         pairs of two slots with skip_lds are no
 //                                 candidates (DBC walls)
+//   kWaves                        wavefronts of a workgroup
+//   kFlag                         sums() wants to know whether any of the
+//                                 particle's pairs has bit 1 set (below)
 //   terms(L, p, l, double (&t)[kSums])  the terms of pair (p, l), zeros
 //                                 beyond the exact support (the lists hold
-//                                 r^2 <= 4h^2 (1 + 1e-12)); returns whether it
-//                                 counts as a pair interaction
-//   sums(L, p, i, const double (&s)[kSums])  writes particle i, slot p
+//                                 r^2 <= 4h^2 (1 + 1e-12)); bit 0 of the result:
+//                                 it counts as a pair interaction, bit 1: a flag
+//   sums(L, p, i, const double (&s)[kSums], flag)  writes particle i, slot p
 //   far(i, cs, g, c, counts...)   particle i of cell c from global memory
 constexpr int kCellSlots = 104;  // staged slots of a cell's neighbourhood
 constexpr int kCellFlat = 640;   // flat list entries (own particles listed together x candidates)
 constexpr double kFar64 = 1e150;  // coordinate of slots past the last (its square is finite)
-constexpr int kCellBlock = 4 * kWave;  // one wavefront per SIMD
+constexpr int kCellBlock = 4 * kWave;  // most threads of a workgroup
 constexpr int kCellRun = 64;     // consecutive cells of one XCD
 template <class P>
 constexpr int cell_terms() { return P::kSums <= 4 ? 184 : 128; }  // pairs whose terms are in LDS together
@@ -613,7 +501,7 @@ constexpr int cell_wave_bytes() {
 }
 template <class P>
 constexpr int cell_lds_bytes() {
-  return (int)sizeof(CellQueue) + kCellBlock / kWave * cell_wave_bytes<P>();
+  return (int)sizeof(CellQueue) + P::kWaves * cell_wave_bytes<P>();
 }
 
 // what a cell walk knows of a case's grid
@@ -698,14 +586,25 @@ __device__ __forceinline__ CellSlots cell_slots(int lo, int cnt, typename P::Rec
   return {dj[0], __builtin_amdgcn_readlane(cnt, 0), tot};
 }
 
+// where a cell walk finds its cells: among all cells of the grid, or (tiles
+// set; a single case) among those of the listed tiles
+struct CellSource {
+  int ncells;        // cells of all cases
+  const int *tiles;  // the list of non-empty tiles, of `rows` cells each
+  const int *ntiles;
+  int rows;
+};
+
 template <class P>
 __device__ __forceinline__ void cells64(P &pol, CellGrid g, const int *__restrict__ cell_start,
                                         const Consts *__restrict__ cases, int ncases,
-                                        int ncells_tot, unsigned long long *__restrict__ counters) {
+                                        const CellSource src,
+                                        unsigned long long *__restrict__ counters) {
   extern __shared__ __align__(16) unsigned char smem[];
   constexpr int NS = P::kSums;
   constexpr int NT = cell_terms<P>();
-  constexpr int kOwn = 64 / NS;  // particles whose sums are formed together
+  constexpr int kBlock = P::kWaves * kWave;
+  constexpr int kOwn = NS < 4 ? 16 : 64 / NS;  // particles whose sums are formed together
   CellQueue &cq = *reinterpret_cast<CellQueue *>(smem);
   unsigned char *wl = smem + sizeof(CellQueue) + (threadIdx.x >> 6) * cell_wave_bytes<P>();
   double *terms = reinterpret_cast<double *>(wl);
@@ -718,17 +617,25 @@ __device__ __forceinline__ void cells64(P &pol, CellGrid g, const int *__restric
   // cells share staged particles through one L2 while every XCD gets a share
   // of each part of the domain.  The workgroups of an XCD stride through its
   // cells, a thread per cell to find the non-empty ones, which the workgroup's
-  // wavefronts take from a counter in LDS.  (No tile list: its length, entry
-  // and cell offsets would be three dependent loads before the first cell.)
+  // wavefronts take from a counter in LDS.
   const int band = blockIdx.x & 7, nwb = gridDim.x >> 3, wb = blockIdx.x >> 3;
-  const int mine = (ncells_tot + 8 * kCellRun - 1) / (8 * kCellRun) * kCellRun;  // cells per XCD
-  for (int j0 = wb; j0 < mine; j0 += nwb * kCellBlock) {
+  const int all = src.tiles ? *src.ntiles * src.rows : src.ncells;
+  const int mine = (all + 8 * kCellRun - 1) / (8 * kCellRun) * kCellRun;  // cells per XCD
+  for (int j0 = wb; j0 < mine; j0 += nwb * kBlock) {
     __syncthreads();
     if (threadIdx.x == 0) cq.count = cq.next = 0;
     __syncthreads();
     const int u = j0 + (int)threadIdx.x * nwb;
-    const int gc = ((u / kCellRun) * 8 + band) * kCellRun + u % kCellRun;
-    if (u < mine && gc < ncells_tot && cell_start[gc + 1] > cell_start[gc]) {
+    int gc = ((u / kCellRun) * 8 + band) * kCellRun + u % kCellRun;
+    bool take = u < mine && gc < all;
+    if (take && src.tiles) {
+      const int tl = gc / src.rows, r = gc - tl * src.rows;
+      const int tile = src.tiles[tl], nty = (g.ncy + src.rows - 1) / src.rows;
+      const int cx = tile / nty, cy = (tile - cx * nty) * src.rows + r;
+      take = cy < g.ncy;
+      gc = cx * g.ncy + cy;
+    }
+    if (take && cell_start[gc + 1] > cell_start[gc]) {
       const int at = atomicAdd(&cq.count, 1);
       cq.cell[at] = gc;
       if (cases) cq.cse[at] = (uint8_t)case_of_cell(cases, ncases, gc);
@@ -812,14 +719,25 @@ __device__ __forceinline__ void cells64(P &pol, CellGrid g, const int *__restric
         const int pc = lane / NS, tc = lane - pc * NS;
         const int x0 = __shfl(st, pc, kWave), x1 = pc < np ? __shfl(st, min(pc + 1, 63), kWave) : 0;
         double acc = 0.;
+        bool flag = false;
         for (int w0 = 0; w0 < e; w0 += NT) {
           const int we = min(NT, e - w0);
-          for (int w = lane; w < we; w += kWave) {
-            const unsigned en = flat[w0 + w];
-            double t[NS];
-            npair += pol.terms(L, p0 + (int)(en >> 8), (int)(en & 255u), t);
+          for (int w = 0; w < we; w += kWave) {
+            int got = 0;
+            if (w + lane < we) {
+              const unsigned en = flat[w0 + w + lane];
+              double t[NS];
+              got = pol.terms(L, p0 + (int)(en >> 8), (int)(en & 255u), t);
 #pragma unroll
-            for (int q = 0; q < NS; ++q) terms[q * NT + w] = t[q];
+              for (int q = 0; q < NS; ++q) terms[q * NT + w + lane] = t[q];
+            }
+            npair += got & 1;
+            if (P::kFlag) {
+              // this window's part of the particle's list range
+              const unsigned long long m = __ballot(got & 2);
+              const int a = max(x0 - w0 - w, 0), b = min(x1 - w0 - w, kWave);
+              if (a < b) flag |= (m >> a & (~0ull >> (kWave - (b - a)))) != 0;
+            }
           }
           wave_sync();
           // eight terms at a time, their loads in flight together
@@ -846,12 +764,13 @@ __device__ __forceinline__ void cells64(P &pol, CellGrid g, const int *__restric
         }
         // lane p takes its particle's sums and writes the particle
         terms[lane] = acc;
+        const bool mine_flag = P::kFlag && __shfl((int)flag, min(lane * NS, 63), kWave);
         wave_sync();
         if (lane < np && pol.act_lds(L, p0 + lane)) {
           double sum[NS];
 #pragma unroll
           for (int q = 0; q < NS; ++q) sum[q] = terms[lane * NS + q];
-          pol.sums(L, p0 + lane, own0 + p0 + lane, sum);
+          pol.sums(L, p0 + lane, own0 + p0 + lane, sum, mine_flag);
         }
         wave_sync();
       }
@@ -986,12 +905,23 @@ __device__ __forceinline__ void walk32(const P &pol, const Consts &k, const int 
 // wavefront of those.  fit: the context's record of the kernel's occupancy
 // (0: not asked yet).
 template <typename K>
-int cell_groups(const tsph_ctx *c, K kernel, int lds, int &fit) {
-  if (fit < 1 &&
-      (hipOccupancyMaxActiveBlocksPerMultiprocessor(&fit, kernel, kCellBlock, lds) != hipSuccess || fit < 1))
+int cell_groups(const tsph_ctx *c, K kernel, int waves, int lds, int &fit) {
+  if (fit < 1 && (hipOccupancyMaxActiveBlocksPerMultiprocessor(&fit, kernel, waves * kWave, lds) !=
+                      hipSuccess || fit < 1))
     fit = 1;
-  const int most = c->num_cu * std::min(fit, 8), want = std::max(c->num_cu, c->n_ub / 12);
+  const int most = c->num_cu * std::min(fit, 32 / waves), want = std::max(c->num_cu, c->n_ub / (3 * waves));
   return 8 * ((std::min(most, want) + 7) / 8);
+}
+
+// A cell walk looks at every cell of grids of up to kCellsDirect cells (a
+// tile list's length, its entry and the cell's offsets would be three
+// dependent loads before the first cell, 2 us more per pass on small grids);
+// on larger ones, which may be mostly empty, at those of the listed tiles.
+constexpr int kCellsDirect = 1 << 20;
+inline bool cells_direct(const tsph_ctx *c) { return c->ncells_tot <= kCellsDirect; }
+inline CellSource cell_source(const tsph_ctx *c) {
+  if (cells_direct(c)) return {c->ncells_tot, nullptr, nullptr, 1};
+  return {c->ncells_tot, c->tile_list, c->scal + S_NTILES, c->tile_rows};
 }
 
 // a pair-loop launch, bracketed by HIP events while pair timing is enabled
