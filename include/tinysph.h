@@ -423,8 +423,10 @@ int tsph_autotune(tsph_ctx *ctx, int variant, int *tile_rows, int *waves_per_cu,
  * default: workgroups of up to 4 wavefronts, each with a chunk of the tile
  * list of about equal cost, cut by the time each tile took in the previous
  * pass, whose tiles its wavefronts take from a counter in LDS, the costliest
- * first), 0 = static striding, one wavefront per workgroup.  Grids with fewer
- * than 16 tiles per persistent wave, and the ALE passes, always stride.
+ * first), 0 = static striding, one wavefront per workgroup.  Systems
+ * with fewer than 80 (mixed) or 200 (FP64) particles per persistent wave, and
+ * the ALE passes, always stride; FP64 passes over at most 70,000 particles go
+ * by cells instead of tiles and do not depend on the setting.
  * Results do not depend on it.  No counterpart in the reference. */
 int tsph_set_balanced(tsph_ctx *ctx, int balanced);
 /* Per-cell order of the cell-list build (Particle_To_Cell's push_back in

@@ -38,14 +38,19 @@ def state(preset, dx, seed, delta=0.0):
     return case, fluid, g
 
 
-def compare(case, what):
+def compare(case, what, waves=0):
     print(f"[case] {what} np={case.np}", flush=True)
     O = oracle_for(case)
     oracle_init(O)
     O.call("compute_forces", oracle_variant(case.wall))
     with T.system_for_case(case) as ps:
+        if waves:
+            ps.set_waves_per_cu(waves)
         ps.particle_to_cell()
         ps.compute_forces(T.forces_variant(case.wall))
+        if waves:  # once more, its chunks cut by the times the first pass recorded
+            ps.particle_to_cell()
+            ps.compute_forces(T.forces_variant(case.wall))
         got = ps.download(("a", "drho"))
     assert np.array_equal(got["a"], O.get(po.F_A), equal_nan=True)
     if case.params["delta"] == 0.0:
@@ -60,6 +65,14 @@ def compare(case, what):
 def test_pair_pass_equals_oracle_bit_for_bit(preset, dx, delta):
     case, _, _ = state(preset, dx, 7, delta)
     compare(case, f"preset {preset} dx {dx} delta {delta}")
+
+
+@pytest.mark.parametrize("preset,dx", [(T.CASE_STILL_WATER_DBC, 0.0026), (T.CASE_DAM_BREAK_MDBC, 0.003),
+                                       (T.CASE_DAM_BREAK_BT, 0.0015)])
+def test_pooled_walk_equals_oracle_bit_for_bit(preset, dx):
+    """One wavefront per compute unit: enough particles for each that tiles are pooled."""
+    case, _, _ = state(preset, dx, 9)
+    compare(case, f"preset {preset} dx {dx} pooled", waves=1)
 
 
 @pytest.mark.parametrize("preset", [T.CASE_STILL_WATER_DBC, T.CASE_DAM_BREAK_MDBC, T.CASE_DAM_BREAK_BT])

@@ -285,11 +285,13 @@ inline int total_tiles(const tsph_ctx *c) {
 }
 
 // whether a pair launch of `waves` persistent waves takes the pooled walk:
-// the precision's setting, for grids of at least 16 tiles per wave (below that
-// the waves have a few tiles each and little to balance: a 183k-particle ALE
-// dam break with 8-10 tiles per wave ran 0.35 ms per step pooled, 0.28 static)
+// the precision's setting, for systems that give each wave enough particles to
+// balance.  Dam breaks, us per step pooled and static: mixed (3072 waves) 190k
+// particles 139 and 133, 333k 172 and 189; FP64 (2048 waves) 333k 314 and 287,
+// 517k 409 and 422; 16 tanks of 879k particles in all, mixed, 354 and 432.
+constexpr int kPoolMixed = 80, kPoolFp64 = 200;  // particles per wave
 inline bool walk_balanced(const tsph_ctx *c, bool fp32, int waves) {
-  return c->balanced[fp32 ? 1 : 0] && total_tiles(c) >= 16 * waves;
+  return c->balanced[fp32 ? 1 : 0] && c->n_ub >= (long long)(fp32 ? kPoolMixed : kPoolFp64) * waves;
 }
 
 // launch geometry of a tile kernel: `groups` workgroups (a multiple of 8) of
