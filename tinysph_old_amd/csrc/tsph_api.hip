@@ -139,7 +139,10 @@ static int replay_step(tsph_ctx *c, Graph *slots, int tag, double dt, int nsteps
       hipGraph_t graph = nullptr;
       TSPH_HIP(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
       int e = 0;
-      for (int j = 0; j < k && !e; ++j) e = record();
+      c->rec_steps = k;
+      for (c->rec_step = 0; c->rec_step < k && !e; ++c->rec_step) e = record();
+      c->rec_step = 0;
+      c->rec_steps = 1;
       const hipError_t ce = hipStreamEndCapture(c->stream, &graph);
       if (e || ce != hipSuccess) {
         if (graph) (void)hipGraphDestroy(graph);
@@ -266,7 +269,7 @@ static int record_step(tsph_ctx *c, int wall, double dt, int inlet = -1, int out
     if (outlet >= 0 && (e = launch_bz_outlet(c, outlet, dt))) return e;
     if ((e = launch_cell_list(c, true, false, 0., active))) return e;
   } else if ((e = launch_cell_list(c, true, true, dt, active, false, false,
-                                   walls_in_build ? wall : 0, true))) {
+                                   walls_in_build ? wall : 0, true, c->rec_step > 0))) {
     return e;  // (the predictor is applied by the build)
   }
   // the corrector writes the removal states; the build takes the removal
@@ -278,10 +281,13 @@ static int record_step(tsph_ctx *c, int wall, double dt, int inlet = -1, int out
     return e;
   }
   // r_o, v_o, rho_o are dead after the corrector until the next predictor
-  // rewrites them: this build leaves them behind
+  // rewrites them: this build leaves them behind.  Where another step follows
+  // in the same graph it also takes the hash of that step's first build (a
+  // step's last pair pass changes neither positions nor velocities).
+  const bool more = !zones && c->rec_step + 1 < c->rec_steps;
   c->cut_groups = groups;
   c->cut_table = 0;
-  if ((e = launch_cell_list(c, true, false, 0., active, true, true)) ||
+  if ((e = launch_cell_list(c, true, false, dt, active, true, true, 0, false, false, more)) ||
       (e = launch_forces(c, variant)))
     return e;
   return 0;
@@ -376,7 +382,8 @@ static int alloc_context(tsph_ctx *c) {
   if ((e = alloc_soa(c->cur, cap, false, false)) || (e = alloc_soa(c->alt, cap, false, false)))
     return e;
   if ((e = dalloc(&c->scal, S_NSCAL + (size_t)kCostTables * (nct + 8))) ||
-      (e = dalloc(&c->cell_count, nct + 1)) || (e = dalloc(&c->cell_start, nct + 2)) ||
+      (e = dalloc(&c->cell_count, nct + 1)) || (e = dalloc(&c->cell_count_next, nct + 1)) ||
+      (e = dalloc(&c->cell_start, nct + 2)) ||
       (e = dalloc(&c->cell_start_next, nct + 2)) ||
       (e = dalloc(&c->cellof, cap)) ||
       // (hcell and hrank also serve the download's bitmap over the positions)
@@ -395,6 +402,7 @@ static int alloc_context(tsph_ctx *c) {
   // the per-cell counters and removal states start cleared; later builds clear
   // them as they consume them (the single-pass scan's words likewise)
   if (hipMemsetAsync(c->cell_count, 0, sizeof(int) * (nct + 1), c->stream) != hipSuccess ||
+      hipMemsetAsync(c->cell_count_next, 0, sizeof(int) * (nct + 1), c->stream) != hipSuccess ||
       hipMemsetAsync(c->scan_state, 0, sizeof(unsigned long long) * ((nct + 1) / 1024 + 2),
                      c->stream) != hipSuccess ||
       hipMemsetAsync(c->seqstate, 0, (size_t)c->seq_cap, c->stream) != hipSuccess)
@@ -486,7 +494,7 @@ int tsph_destroy(tsph_ctx *c) {
   drop_graph(c);
   free_soa(c->cur);
   free_soa(c->alt);
-  void *ps[] = {c->scal, c->counters, c->cell_count, c->cell_start, c->cell_start_next, c->cellof, c->hrank,
+  void *ps[] = {c->scal, c->counters, c->cell_count, c->cell_count_next, c->cell_start, c->cell_start_next, c->cellof, c->hrank,
                 c->hcell, c->perm, c->arrival, c->arrival_seq, c->arrival_span, c->scan_state, c->scan_cost, c->scan_tile0, c->seqstate, c->probe_out, c->mx.rv,
                 c->mx.rp, c->mx.nrm, c->tile_list, c->list_cost, c->wall_list, c->bz_list,
                 c->cases, c->tile_base, c->list_part, c->tile_bound};

@@ -58,15 +58,66 @@ __device__ __forceinline__ unsigned long long lanemask_lt() {
 // no decision in this pass reads a state that this pass changes.
 // The wall-density pass that precedes a build in the symplectic step (WALLS:
 // TSPH_WALL_MDBC or TSPH_WALL_BT; 0: none) runs in the first wb.walls +
-// wb.sweep workgroups of the hash launch (64 threads each), beside the hash
-// rather than before it: it reads the previous cell list and writes wall
-// densities, the hash reads positions and writes the new cell counts.
+// wb.sweep wavefronts of the hash launch, or of the scan launch where the
+// build needs no hash, beside that pass rather than before it: it reads the
+// previous cell list and writes wall densities, the hash reads positions and
+// writes the new cell counts, the scan the new cell offsets.
 struct WallPass {
   Soa d;
   const int *cell_start, *nwall, *wall_list;
-  int walls, sweep;  // wall and sweep workgroups
+  int walls, sweep;  // wall and sweep wavefronts
   unsigned long long *counters;  // the density count (or nullptr)
 };
+
+// wavefront b of the wall pass; terms: walls::kTerms doubles of LDS
+template <int WALLS>
+__device__ __forceinline__ void wall_wave(int b, const WallPass &wp, const Consts &k0,
+                                          const Consts *__restrict__ cases,
+                                          const int *__restrict__ scal, double *terms) {
+  if (WALLS == TSPH_WALL_MDBC)
+    walls::mdbc_wave(b, wp.walls, wp.sweep, wp.d, wp.cell_start, wp.nwall, wp.wall_list, k0, cases,
+                     wp.counters, scal, terms);
+  else
+    walls::bt_wave(b, wp.walls, wp.sweep, wp.d, wp.cell_start, wp.nwall, wp.wall_list, k0, cases,
+                   wp.counters, scal, terms);
+}
+
+// global cell of a particle at r (counted and clamped beyond its case's grid)
+__device__ __forceinline__ int hash_cell(const Consts &k, double2 r,
+                                         unsigned long long *__restrict__ counters) {
+  const int cx = cell_coord(r.x, k.x0, k.of, k.kh);
+  const int cy = cell_coord(r.y, k.y0, k.of, k.kh);
+  int c = cy + cx * k.ncy;  // POS(x,y) = y + x*Y, src/SPH_defs.h:36
+  if (c < 0 || c >= k.ncells) {
+    // undefined behaviour in the reference; counted and clamped here
+    atomicAdd(&counters[C_OUTGRID], 1ull);
+    c = c < 0 ? 0 : k.ncells - 1;
+  }
+  return c + k.cell_base;  // the case's segment of the global cell range
+}
+
+// counts the lanes' particles (live lanes) into their cells c and returns each
+// one's arrival rank: the lanes of a wavefront that share a cell are grouped,
+// and the lowest lane of each group does the atomic
+__device__ __forceinline__ int count_cell(bool live, int c, int *__restrict__ cell_count) {
+  const int lane = threadIdx.x & 63;
+  unsigned long long rem = __ballot(live);
+  int leader = 0;
+  unsigned long long grp = 0;
+  while (rem) {
+    const int l = __builtin_ctzll(rem);
+    const int key = __shfl(c, l, 64);
+    const unsigned long long m = __ballot(c == key) & rem;
+    if ((m >> lane) & 1ull) {
+      leader = l;
+      grp = m;
+    }
+    rem &= ~m;
+  }
+  int base = 0;
+  if (live && lane == leader) base = atomicAdd(&cell_count[c], __popcll(grp));
+  return __shfl(base, leader, 64) + __popcll(grp & lanemask_lt());
+}
 
 template <bool PRED, bool DECIDE, int WALLS>
 __global__ void k_hash(const double2 *__restrict__ r, const double2 *__restrict__ v,
@@ -78,14 +129,10 @@ __global__ void k_hash(const double2 *__restrict__ r, const double2 *__restrict_
                        unsigned long long *__restrict__ counters, WallPass wp) {
   int hb = blockIdx.x;  // hash workgroup
   if (WALLS) {
-    const int b = blockIdx.x;
+    __shared__ __align__(16) double s_terms[walls::kTerms];
+    const int b = blockIdx.x;  // (64 threads)
     if (b < wp.walls + wp.sweep) {
-      if (WALLS == TSPH_WALL_MDBC)
-        walls::mdbc_block(b, wp.walls, wp.sweep, wp.d, wp.cell_start, wp.nwall, wp.wall_list, k0,
-                          cases, wp.counters, scal);
-      else
-        walls::bt_block(b, wp.walls, wp.sweep, wp.d, wp.cell_start, wp.nwall, wp.wall_list, k0,
-                        cases, wp.counters, scal);
+      wall_wave<WALLS>(b, wp, k0, cases, scal, s_terms);
       return;
     }
     hb = b - wp.walls - wp.sweep;
@@ -107,38 +154,13 @@ __global__ void k_hash(const double2 *__restrict__ r, const double2 *__restrict_
       const Consts k = case_consts(k0, cases, cid, i);
       double2 ri = r[i];
       if (PRED) ri = predicted_r(ri, v[i], cases ? k.dt : dt0);
-      const int cx = cell_coord(ri.x, k.x0, k.of, k.kh);
-      const int cy = cell_coord(ri.y, k.y0, k.of, k.kh);
-      c = cy + cx * k.ncy;  // POS(x,y) = y + x*Y, src/SPH_defs.h:36
-      if (c < 0 || c >= k.ncells) {
-        // undefined behaviour in the reference; counted and clamped here
-        atomicAdd(&counters[C_OUTGRID], 1ull);
-        c = c < 0 ? 0 : k.ncells - 1;
-      }
-      c += k.cell_base;  // the case's segment of the global cell range
+      c = hash_cell(k, ri, counters);
     }
   }
-  // group the lanes by cell; the lowest lane of each group does the atomic
-  const int lane = threadIdx.x & 63;
-  unsigned long long rem = __ballot(live);
-  int leader = 0;
-  unsigned long long grp = 0;
-  while (rem) {
-    const int l = __builtin_ctzll(rem);
-    const int key = __shfl(c, l, 64);
-    const unsigned long long m = __ballot(c == key) & rem;
-    if ((m >> lane) & 1ull) {
-      leader = l;
-      grp = m;
-    }
-    rem &= ~m;
-  }
-  int base = 0;
-  if (live && lane == leader) base = atomicAdd(&cell_count[c], __popcll(grp));
-  base = __shfl(base, leader, 64);
+  const int rank = count_cell(live, c, cell_count);
   if (live) {
     hcell[i] = c;
-    hrank[i] = base + __popcll(grp & lanemask_lt());
+    hrank[i] = rank;
   }
 }
 
@@ -328,17 +350,29 @@ __device__ __forceinline__ void block_reduce3(int &a, int &b, int &m, int *lds) 
   __syncthreads();
 }
 
-template <int IT>
+template <int IT, int WALLS>
 __global__ __launch_bounds__(kScanBlock) void k_scan(const int *__restrict__ in, int len,
                                                      unsigned long long *__restrict__ state,
                                                      int *__restrict__ out, int *__restrict__ scal,
                                                      unsigned long long *__restrict__ counters,
-                                                     TileScan ts, int spin_limit, int nwall_idx) {
+                                                     TileScan ts, int spin_limit, int nwall_idx,
+                                                     int wall_groups, WallPass wp, Consts k0) {
   __shared__ int lds[3 * kScanBlock / 64];
   constexpr int kTile = kScanBlock * IT;
   __shared__ int s_cnt[kTile + kMaxTileRows];
   __shared__ int s_case;
-  const int nb = gridDim.x, blk = blockIdx.x;
+  // the wall pass (WALLS) in the last wall_groups workgroups, a wavefront's
+  // share per wavefront
+  const int nb = gridDim.x - (WALLS ? wall_groups : 0), blk = blockIdx.x;
+  if (WALLS && blk >= nb) {
+    constexpr int kWaves = kScanBlock / 64;
+    __shared__ __align__(16) double s_terms[kWaves * walls::kTerms];
+    const int wid = threadIdx.x >> 6, b = (blk - nb) * kWaves + wid;
+    if (b < wp.walls + wp.sweep)
+      wall_wave<WALLS ? WALLS : TSPH_WALL_MDBC>(b, wp, k0, ts.cases, scal,
+                                                s_terms + wid * walls::kTerms);
+    return;
+  }
   int v[IT], tl[IT], own[IT], halo;
   load_counts<IT>(in, len, blk, v, halo);
   const int nt = stage_counts<IT>(len, blk, ts, v, halo, tl, own, s_cnt, &s_case);
@@ -671,10 +705,13 @@ __device__ __forceinline__ int ranked_slot(const int *__restrict__ cell_start,
 // written, for the step sequences in which that stage follows the cell build.
 // With PRED the symplectic predictor (src/SPH_integration.h:266-287) is
 // applied to the moved particles, for the step sequences in which it
-// immediately precedes the cell build.  ad_skip (a type mask): a and drho of
+// immediately precedes the cell build.  With NEXT the hash of the next step's
+// first build is taken on the way: that build sorts by the positions the
+// predictor will give, which need no forces, so a step inside a run of steps
+// starts with its scan (next_count: the next build's cell counts).  ad_skip (a type mask): a and drho of
 // those types are not moved, for the step sequences in which a pair pass that
 // overwrites them for exactly those types follows the build.
-template <bool EOS, bool PRED, bool RANK>
+template <bool EOS, bool PRED, bool RANK, bool NEXT>
 __global__ void k_reorder(const int *__restrict__ cell_start, int ncells,
                           const int *__restrict__ arrival, const uint32_t *__restrict__ arrival_seq,
                           const uint32_t *__restrict__ arrival_span, int *__restrict__ perm,
@@ -683,14 +720,15 @@ __global__ void k_reorder(const int *__restrict__ cell_start, int ncells,
                           const int *__restrict__ cellof, Consts k0,
                           const Consts *__restrict__ cases, Mixed mx, double dt0,
                           unsigned ad_skip, unsigned long long *__restrict__ counters,
-                          int nwall_idx, bool move_olds) {
+                          int nwall_idx, bool move_olds, int *__restrict__ next_count,
+                          int *__restrict__ hcell, int *__restrict__ hrank) {
   const int n_new = cell_start[ncells];
   const int x = blockIdx.x * blockDim.x + threadIdx.x;  // arrival position
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     scal[S_NP] = n_new;
     if (RANK) cell_count[ncells] = 0;  // the removed bucket
   }
-  int wall = 0, k = x;
+  int wall = 0, k = x, next_c = -1;
   unsigned bad = 0;
   if (x < n_new) {
     const int j = arrival[x];
@@ -726,6 +764,7 @@ __global__ void k_reorder(const int *__restrict__ cell_start, int ncells,
     }
     dst.r[k] = r;
     dst.v[k] = v;
+    if (NEXT) next_c = hash_cell(kc, predicted_r(r, v, cases ? kc.dt : dt0), counters);
     if (move_ad) {
       dst.a[k] = a;
       dst.drho[k] = drho;
@@ -777,6 +816,14 @@ __global__ void k_reorder(const int *__restrict__ cell_start, int ncells,
       dst.rhoc[k] = src.rhoc[j];
     }
   }
+  if (NEXT) {
+    const bool live = x < n_new;
+    const int rank = count_cell(live, next_c, next_count);
+    if (live) {
+      hcell[k] = next_c;
+      hrank[k] = rank;
+    }
+  }
   const unsigned long long m = __ballot(wall);
   if (m) {
     const int lane = threadIdx.x & 63;
@@ -805,8 +852,10 @@ __global__ void k_gather_olds(const int *__restrict__ scal, const int *__restric
 }
 
 // exclusive scan of the cell counts into cell_start, with the tile list of the
-// current tile_rows (and, for cost_table >= 0, the listed tiles' costs)
-int scan_cells(tsph_ctx *c, hipStream_t s, int *cs, int nwall_idx, int cost_table) {
+// current tile_rows (and, for cost_table >= 0, the listed tiles' costs); with
+// walls (TSPH_WALL_*; 0: none) the wall pass wp beside it
+int scan_cells(tsph_ctx *c, hipStream_t s, const int *count, int *cs, int nwall_idx, int cost_table,
+               int walls, const WallPass &wp) {
   const int len = c->ncells_tot + 1;
   const TileScan ts{c->k.ncy, c->k.ncells, c->k.cell_base, c->cases, c->tile_base, c->ncases,
                     c->tile_rows, c->tile_list,
@@ -814,12 +863,22 @@ int scan_cells(tsph_ctx *c, hipStream_t s, int *cs, int nwall_idx, int cost_tabl
                     cost_table >= 0 ? c->list_cost : nullptr,
                     cost_estimate(c->prm.precision == TSPH_PREC_MIXED), c->scan_cost,
                     c->scan_tile0};
-  if (scan_items(c) == 4)
-    hipLaunchKernelGGL(k_scan<4>, dim3(scan_blocks(c)), dim3(kScanBlock), 0, s, c->cell_count,
-                       len, c->scan_state, cs, c->scal, c->counters, ts, c->scan_wait, nwall_idx);
-  else
-    hipLaunchKernelGGL(k_scan<16>, dim3(scan_blocks(c)), dim3(kScanBlock), 0, s, c->cell_count,
-                       len, c->scan_state, cs, c->scal, c->counters, ts, c->scan_wait, nwall_idx);
+  const int wg = walls ? grid_for(wp.walls + wp.sweep, kScanBlock / 64) : 0;
+#define TSPH_SCAN(IT, W)                                                                       \
+  hipLaunchKernelGGL((k_scan<IT, W>), dim3(scan_blocks(c) + wg), dim3(kScanBlock), 0, s, count, len, \
+                     c->scan_state, cs, c->scal, c->counters, ts, c->scan_wait, nwall_idx, wg, wp, \
+                     c->k)
+#define TSPH_SCAN_W(IT)                                                                        \
+  if (walls == TSPH_WALL_MDBC) TSPH_SCAN(IT, TSPH_WALL_MDBC);                                 \
+  else if (walls == TSPH_WALL_BT) TSPH_SCAN(IT, TSPH_WALL_BT);                                \
+  else TSPH_SCAN(IT, 0)
+  if (scan_items(c) == 4) {
+    TSPH_SCAN_W(4);
+  } else {
+    TSPH_SCAN_W(16);
+  }
+#undef TSPH_SCAN_W
+#undef TSPH_SCAN
   TSPH_HIP(hipGetLastError());
   c->list_groups = 0;  // a pooled pass cuts the new list
   c->list_cost_table = cost_table;
@@ -838,7 +897,8 @@ int ensure_olds(tsph_ctx *c) {
 }
 
 int launch_cell_list(tsph_ctx *c, bool eos, bool predict, double dt, unsigned ad_skip,
-                     bool decide, bool skip_olds, int walls, bool count_density) {
+                     bool decide, bool skip_olds, int walls, bool count_density, bool hashed,
+                     bool hash_next) {
   // a build that moves r_o, v_o, rho_o needs them current (the predictor's
   // build rewrites them instead)
   if (!predict && !skip_olds)
@@ -862,6 +922,10 @@ int launch_cell_list(tsph_ctx *c, bool eos, bool predict, double dt, unsigned ad
     hg = wp.walls + wp.sweep + grid_for(c->n_ub, hbs);
     c->records_valid = false;
   }
+  // counts of a build whose hash the previous build took (hash_next) are kept
+  // apart from those of the builds between
+  int *count = hashed ? c->cell_count_next : c->cell_count;
+  if (!hashed) {
 #define TSPH_HASH(P, D, W)                                                                     \
   hipLaunchKernelGGL((k_hash<P, D, W>), dim3(hg), dim3(hbs), 0, s, c->cur.r, c->cur.v,            \
                      c->cur.type, c->cur.seq, c->scal, k, c->cases, c->cur.cid, dt, nct,          \
@@ -879,6 +943,7 @@ int launch_cell_list(tsph_ctx *c, bool eos, bool predict, double dt, unsigned ad
   } else {
     TSPH_HASH_W(false, false);
   }
+  }
 #undef TSPH_HASH_W
 #undef TSPH_HASH
   // the pooled pair pass that follows (if any) has its chunks cut in the
@@ -890,7 +955,8 @@ int launch_cell_list(tsph_ctx *c, bool eos, bool predict, double dt, unsigned ad
     set_error("tile list: more pooled workgroups than allocated");
     return TSPH_ESTATE;
   }
-  if (int e = scan_cells(c, s, cs, wslot, cut > 0 ? c->cut_table : -1)) return e;
+  if (int e = scan_cells(c, s, count, cs, wslot, cut > 0 ? c->cut_table : -1, hashed ? walls : 0, wp))
+    return e;
   const int sg = grid_for(c->n_ub, kScatterBlock);
   // the per-cell order: ranked by the reorder (one launch fewer), or by its
   // own pass (fewer bytes moved); by size, up to kRankMax particles ranked
@@ -916,21 +982,25 @@ int launch_cell_list(tsph_ctx *c, bool eos, bool predict, double dt, unsigned ad
   if (!rank) {
     if (c->cases)
       hipLaunchKernelGGL(k_order, dim3(grid_for(nct + 1, nb)), dim3(nb), 0, s, cs, nct, c->cur.seq,
-                         c->perm, c->cell_count);
+                         c->perm, count);
     else
       hipLaunchKernelGGL(k_order_tiles, dim3(kOrderWaves * std::max(1, c->num_cu)), dim3(nb), 0, s,
                          cs, c->scal, c->tile_list, c->tile_rows, k.ncy, nct, c->cur.seq, c->perm,
-                         c->cell_count);
+                         count);
   }
   const Mixed mx = c->prm.precision == TSPH_PREC_MIXED ? c->mx : Mixed{};
-#define TSPH_REORDER(E, P, R)                                                                 \
-  hipLaunchKernelGGL((k_reorder<E, P, R>), dim3(g), dim3(nb), 0, s, cs, nct, arrival,              \
-                     c->arrival_seq, c->arrival_span, c->perm, c->cell_count, c->cur, c->alt,     \
-                     c->scal, c->wall_list, c->cellof, k, c->cases, mx, dt, ad_skip, c->counters, \
-                     wslot, !skip_olds)
+#define TSPH_REORDER(E, P, R, N)                                                              \
+  hipLaunchKernelGGL((k_reorder<E, P, R, N>), dim3(g), dim3(nb), 0, s, cs, nct, arrival,           \
+                     c->arrival_seq, c->arrival_span, c->perm, count, c->cur, c->alt, c->scal,     \
+                     c->wall_list, c->cellof, k, c->cases, mx, dt, ad_skip, c->counters, wslot,    \
+                     !skip_olds, c->cell_count_next, c->hcell, c->hrank)
 #define TSPH_REORDER_R(E, P)                                                                  \
-  if (rank) TSPH_REORDER(E, P, true);                                                         \
-  else TSPH_REORDER(E, P, false)
+  if (rank) TSPH_REORDER(E, P, true, false);                                                  \
+  else TSPH_REORDER(E, P, false, false)
+  if (hash_next) {
+    if (rank) TSPH_REORDER(true, false, true, true);
+    else TSPH_REORDER(true, false, false, true);
+  } else
   if (eos && predict) {
     TSPH_REORDER_R(true, true);
   } else if (eos) {

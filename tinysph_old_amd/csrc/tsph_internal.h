@@ -211,6 +211,7 @@ struct tsph_ctx {
   int *scal = nullptr;                 // S_* slots, then the per-tile costs
   unsigned long long *counters = nullptr;
   int *cell_count = nullptr;           // ncells+1 (last = removed bucket)
+  int *cell_count_next = nullptr;      // the counts of a hash taken by the build before
   int *cell_start = nullptr;           // ncells+2
   // Every build writes its cell offsets and wall count into the buffers the
   // previous build did not (cell_start_next, the other wall-count slot) and
@@ -244,6 +245,8 @@ struct tsph_ctx {
   // symplectic step, by parity at the step's start: one step ([0], [1]) or
   // kGraphSteps steps ([2], [3])
   tsph::Graph graph[4];
+  // the step being recorded of the run that one graph holds
+  int rec_step = 0, rec_steps = 1;
   tsph::Graph rale_graph[2];  // Riemann-ALE step, by parity at the step's start
   tsph::Graph ale_graph[2];   // ALE-SPH MUSCL step, by parity at the step's start
   tsph::Graph inflow_graph[2];  // symplectic step with buffer zones
@@ -319,10 +322,14 @@ struct TileGrid {
 // walls (TSPH_WALL_MDBC or TSPH_WALL_BT; 0: none): the wall densities of that
 // treatment are computed first, from the previous cell list, in the same
 // launch as the build's hash (as launch_mdbc / launch_bt_density with
-// count_density)
+// count_density), or as its scan where it has none
+// hash_next (with eos, without predict): the build's reorder also takes the
+// hash of the predict build that follows it with nothing but a pair pass
+// between them (the next step's first, with time step dt); hashed: that build
 int launch_cell_list(tsph_ctx *c, bool eos = false, bool predict = false, double dt = 0.,
                      unsigned ad_skip = 0, bool decide = false, bool skip_olds = false,
-                     int walls = 0, bool count_density = false);
+                     int walls = 0, bool count_density = false, bool hashed = false,
+                     bool hash_next = false);
 // r_o, v_o, rho_o of the current generation, gathered from the previous one
 // through the last build's permutation if that build left them behind; every
 // launch that reads or moves them calls this first

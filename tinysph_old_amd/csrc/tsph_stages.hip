@@ -86,8 +86,9 @@ __global__ __launch_bounds__(64) void k_mdbc(Soa d, const int *__restrict__ cell
                                              const Consts *__restrict__ cases,
                                              unsigned long long *__restrict__ counters,
                                              const int *__restrict__ scal, int wall_blocks) {
-  mdbc_block(blockIdx.x, wall_blocks, gridDim.x - wall_blocks, d, cell_start, nwall, wall_list, k0,
-             cases, counters, scal);
+  __shared__ __align__(16) double s_terms[walls::kTerms];
+  mdbc_wave(blockIdx.x, wall_blocks, gridDim.x - wall_blocks, d, cell_start, nwall, wall_list, k0,
+            cases, counters, scal, s_terms);
 }
 
 __global__ __launch_bounds__(64) void k_bt_density(Soa d, const int *__restrict__ cell_start,
@@ -96,8 +97,9 @@ __global__ __launch_bounds__(64) void k_bt_density(Soa d, const int *__restrict_
                                                    const Consts *__restrict__ cases,
                                                    unsigned long long *__restrict__ counters,
                                                    const int *__restrict__ scal, int wall_blocks) {
-  bt_block(blockIdx.x, wall_blocks, gridDim.x - wall_blocks, d, cell_start, nwall, wall_list, k0,
-           cases, counters, scal);
+  __shared__ __align__(16) double s_terms[walls::kTerms];
+  bt_wave(blockIdx.x, wall_blocks, gridDim.x - wall_blocks, d, cell_start, nwall, wall_list, k0,
+          cases, counters, scal, s_terms);
 }
 
 // Removal.  The reference erases inside an ascending loop without stepping

@@ -1,6 +1,6 @@
-// Wall densities (mDBC, BT) by workgroups of 64 threads, shared by their own
-// launches (tsph_stages.hip) and the first cell build of a symplectic step,
-// whose hash pass runs them in workgroups of its own (tsph_cells.hip):
+// Wall densities (mDBC, BT) by wavefronts, shared by their own launches
+// (tsph_stages.hip) and the first cell build of a symplectic step, whose hash
+// or scan launch runs them in wavefronts of its own (tsph_cells.hip):
 //   mDBC_compute_density_mdbcGeo   src/SPH_mDBC.h:9-50 with
 //                                  Kernel_density_approximation_MATRIX_mDBC,
 //                                  src/SPH_kernel_approx.h:1141-1342
@@ -32,6 +32,7 @@ __device__ __forceinline__ int point_cell(const Consts &k, double x, double y) {
 constexpr int kWG = 16;
 constexpr int kWPre = 3;
 constexpr int kWallsPerWave = 64 / kWG;
+constexpr int kTerms = 64 * 12;  // doubles of LDS of a wavefront of the pass
 
 template <int NS, typename Term>
 __device__ __forceinline__ void wall_sums(const Soa &d, const int *__restrict__ cell_start,
@@ -155,13 +156,13 @@ __device__ __forceinline__ void count_walls(bool wall_bad, unsigned long long *_
   if (w && (threadIdx.x & 63) == 0) atomicAdd(&counters[C_BADRHO], (unsigned long long)__popcll(w));
 }
 
-// sweep workgroup sb of nsb (64 threads each)
+// sweep wavefront sb of nsb
 __device__ __forceinline__ void sweep_density(const Soa &d, const int *__restrict__ scal, int sb,
                                               int nsb, unsigned long long *__restrict__ counters) {
   const int n = scal[S_NP];
   const int stride = nsb * 64;
   unsigned bad = 0;
-  for (int p0 = sb * 64 + (int)threadIdx.x; p0 < n; p0 += kSweep * stride) {
+  for (int p0 = sb * 64 + (int)(threadIdx.x & 63); p0 < n; p0 += kSweep * stride) {
     int t[kSweep];
     double rho[kSweep];
 #pragma unroll
@@ -176,29 +177,28 @@ __device__ __forceinline__ void sweep_density(const Soa &d, const int *__restric
         bad += rho[q] > 1500. || rho[q] < 0.;
   }
   for (int o = 32; o > 0; o >>= 1) bad += __shfl_xor(bad, o, 64);
-  if (bad && threadIdx.x == 0) atomicAdd(&counters[C_BADRHO], (unsigned long long)bad);
+  if (bad && (threadIdx.x & 63) == 0) atomicAdd(&counters[C_BADRHO], (unsigned long long)bad);
 }
 
 // sweep workgroups that follow wall_blocks wall workgroups for n particles
 inline int sweep_blocks(int n) { return grid_for(n, 64 * kSweep); }
 
-// The wall-density passes by workgroups of 64 threads: workgroup b < wall_blocks
-// takes walls kWallsPerWave b ..., workgroup wall_blocks + s (s < nsweep) the
+// The wall-density passes by wavefronts: wavefront b < wall_blocks takes walls
+// kWallsPerWave b ..., wavefront wall_blocks + s (s < nsweep) the
 // density sweep's share s (counters set).  nwall: the wall count of the cell
 // list in use (one of the two alternating slots).
-__device__ __forceinline__ void mdbc_block(int b, int wall_blocks, int nsweep, const Soa &d,
+__device__ __forceinline__ void mdbc_wave(int b, int wall_blocks, int nsweep, const Soa &d,
                                            const int *__restrict__ cell_start,
                                            const int *__restrict__ nwall,
                                            const int *__restrict__ wall_list, const Consts &k0,
                                            const Consts *__restrict__ cases,
                                            unsigned long long *__restrict__ counters,
-                                           const int *__restrict__ scal) {
+                                           const int *__restrict__ scal, double *s_terms) {
   if (b >= wall_blocks) {
     sweep_density(d, scal, b - wall_blocks, nsweep, counters);
     return;
   }
-  __shared__ __align__(16) double s_terms[64 * 12];
-  const int w = b * kWallsPerWave + (int)(threadIdx.x / kWG);
+  const int w = b * kWallsPerWave + (int)(threadIdx.x & 63) / kWG;
   const bool live = w < *nwall;
   const int i = live ? wall_list[w] : 0;
   const Consts k = live ? case_consts(k0, cases, d.cid, i) : k0;
@@ -259,19 +259,18 @@ __device__ __forceinline__ void mdbc_block(int b, int wall_blocks, int nsweep, c
   if (counters) count_walls(wall_bad, counters);
 }
 
-__device__ __forceinline__ void bt_block(int b, int wall_blocks, int nsweep, const Soa &d,
+__device__ __forceinline__ void bt_wave(int b, int wall_blocks, int nsweep, const Soa &d,
                                          const int *__restrict__ cell_start,
                                          const int *__restrict__ nwall,
                                          const int *__restrict__ wall_list, const Consts &k0,
                                          const Consts *__restrict__ cases,
                                          unsigned long long *__restrict__ counters,
-                                         const int *__restrict__ scal) {
+                                         const int *__restrict__ scal, double *s_terms) {
   if (b >= wall_blocks) {
     sweep_density(d, scal, b - wall_blocks, nsweep, counters);
     return;
   }
-  __shared__ __align__(16) double s_terms[64 * 2];
-  const int w = b * kWallsPerWave + (int)(threadIdx.x / kWG);
+  const int w = b * kWallsPerWave + (int)(threadIdx.x & 63) / kWG;
   const bool live = w < *nwall;
   const int i = live ? wall_list[w] : 0;
   const Consts k = live ? case_consts(k0, cases, d.cid, i) : k0;
