@@ -432,9 +432,11 @@ int tsph_set_balanced(tsph_ctx *ctx, int balanced);
 /* Per-cell order of the cell-list build (Particle_To_Cell's push_back in
  * ascending particle index, src/SPH_find_pairs.h:45-92): 1 = ranked by the
  * pass that moves the particles (each particle counts those of its cell with
- * a lower index: one launch fewer), 2 = a separate ordering pass over the
- * cells (fewer bytes moved), 0 = by size (the default: 1 up to 2,000,000
- * particles, 2 above).  Results do not depend on it.  No counterpart in the
+ * a lower index, from a row of indices per cell: two launches fewer), 2 =
+ * placed and ordered by passes of their own, 0 = the default: 1.  Grids of
+ * more than about a cell per particle slot (the rows would outgrow the
+ * particles) or with over 85 lattice particles in a cell always take 2.
+ * Results do not depend on it.  No counterpart in the
  * reference. */
 int tsph_set_cell_order(tsph_ctx *ctx, int mode);
 

@@ -122,18 +122,10 @@ static int replay_step(tsph_ctx *c, Graph *slots, int tag, double dt, int nsteps
     if (!g.exec || g.wall != tag || g.dt != dt || g.n_ub != c->n_ub || g.steps != k) {
       if (g.exec) (void)hipGraphExecDestroy(g.exec);
       g = Graph{};
-      const Soa cur0 = c->cur, alt0 = c->alt;
-      int *const cs0 = c->cell_start, *const csn0 = c->cell_start_next;
-      const int nwall0 = c->nwall_idx;
       const int parity0 = c->parity;
       const HostState h0 = host_state(c);
       auto undo = [&] {  // nothing was launched: restore the host view
-        c->cur = cur0;
-        c->alt = alt0;
-        c->cell_start = cs0;
-        c->cell_start_next = csn0;
-        c->nwall_idx = nwall0;
-        c->parity = parity0;
+        if (c->parity != parity0) flip_build(c);
         set_host_state(c, h0);
       };
       hipGraph_t graph = nullptr;
@@ -164,12 +156,8 @@ static int replay_step(tsph_ctx *c, Graph *slots, int tag, double dt, int nsteps
       g.post = host_state(c);
       g.steps = k;
     } else {
-      if (g.flips) {  // what an odd number of cell builds leaves (launch_cell_list)
-        std::swap(c->cur, c->alt);
-        std::swap(c->cell_start, c->cell_start_next);
-        c->nwall_idx = c->nwall_idx == S_NWALL ? S_NWALL_B : S_NWALL;
-        c->parity ^= 1;
-      }
+      if (g.flips)  // what an odd number of cell builds leaves (launch_cell_list)
+        flip_build(c);
       set_host_state(c, g.post);
     }
     TSPH_HIP(hipGraphLaunch(g.exec, c->stream));
@@ -371,6 +359,21 @@ static int make_consts(const tsph_params *prm, Consts &k) {
   return 0;
 }
 
+// entries of a cell's row: one and a half times the particles that a lattice of
+// spacing dp puts in a cell (the reference cases: 8 in a cell of 2.83 dp), as a
+// power of two, so that only cells packed well beyond the lattice are chained;
+// 0: cells too full for rows
+static int row_width_of(const tsph_ctx *c) {
+  double most = 0.;
+  for (int q = 0; q < c->ncases; ++q) {
+    const Consts &k = c->host_cases.empty() ? c->k : c->host_cases[q];
+    most = std::max(most, k.kh / k.dp * (k.kh / k.dp));
+  }
+  int w = 16;
+  while (w < 1.5 * most && w <= 128) w *= 2;
+  return w <= 128 ? w : 0;
+}
+
 // device buffers of a context holding `cap` particles over `ncells_tot` cells
 static int alloc_context(tsph_ctx *c) {
   int e = 0;
@@ -379,6 +382,7 @@ static int alloc_context(tsph_ctx *c) {
     return fail(TSPH_EHIP, "hipStreamCreate failed");
   const int cap = c->capacity, nct = c->ncells_tot;
   c->seq_cap = 2 * cap + kBzMax + c->ncases;
+  const size_t slots = std::max<size_t>(cap, dl_words(c->seq_cap));
   if ((e = alloc_soa(c->cur, cap, false, false)) || (e = alloc_soa(c->alt, cap, false, false)))
     return e;
   if ((e = dalloc(&c->scal, S_NSCAL + (size_t)kCostTables * (nct + 8))) ||
@@ -387,10 +391,9 @@ static int alloc_context(tsph_ctx *c) {
       (e = dalloc(&c->cell_start_next, nct + 2)) ||
       (e = dalloc(&c->cellof, cap)) ||
       // (hcell and hrank also serve the download's bitmap over the positions)
-      (e = dalloc(&c->hrank, std::max<size_t>(cap, dl_words(c->seq_cap)))) ||
-      (e = dalloc(&c->hcell, std::max<size_t>(cap, dl_words(c->seq_cap)))) ||
-      (e = dalloc(&c->perm, cap)) || (e = dalloc(&c->arrival, cap)) ||
-      (e = dalloc(&c->arrival_seq, cap)) || (e = dalloc(&c->arrival_span, cap)) ||
+      (e = dalloc(&c->hrank, slots)) || (e = dalloc(&c->hrank_next, slots)) ||
+      (e = dalloc(&c->hcell, slots)) || (e = dalloc(&c->hcell_next, slots)) ||
+      (e = dalloc(&c->perm, cap)) ||
       (e = dalloc(&c->seqstate, (size_t)c->seq_cap)) || (e = dalloc(&c->probe_out, 4)) ||
       (e = dalloc(&c->bz_list, 2 * kBzMax)) ||
       (e = dalloc(&c->tile_list, nct + 8)) || (e = dalloc(&c->list_cost, nct + 8)) ||
@@ -399,6 +402,18 @@ static int alloc_context(tsph_ctx *c) {
       (e = dalloc(&c->scan_cost, (nct + 1) / 1024 + 2)) ||
       (e = dalloc(&c->scan_tile0, (nct + 1) / 1024 + 2)))
     return e;
+  // the cells' rows (row_width), where they take no more than about what the
+  // particles do
+  const size_t rows = (size_t)nct * row_width_of(c);
+  if (rows && 2 * rows * sizeof(uint32_t) <= (64u << 20) + 512 * (size_t)cap) {
+    c->row_width = row_width_of(c);
+    if ((e = dalloc(&c->row_seq, rows)) || (e = dalloc(&c->row_seq_next, rows)) ||
+        (e = dalloc(&c->row_head, kRowHeads)) || (e = dalloc(&c->row_head_next, kRowHeads)))
+      return e;
+    if (hipMemsetAsync(c->row_head, 0, sizeof(int) * kRowHeads, c->stream) != hipSuccess ||
+        hipMemsetAsync(c->row_head_next, 0, sizeof(int) * kRowHeads, c->stream) != hipSuccess)
+      return fail(TSPH_EHIP, "initialisation failed");
+  }
   // the per-cell counters and removal states start cleared; later builds clear
   // them as they consume them (the single-pass scan's words likewise)
   if (hipMemsetAsync(c->cell_count, 0, sizeof(int) * (nct + 1), c->stream) != hipSuccess ||
@@ -495,7 +510,7 @@ int tsph_destroy(tsph_ctx *c) {
   free_soa(c->cur);
   free_soa(c->alt);
   void *ps[] = {c->scal, c->counters, c->cell_count, c->cell_count_next, c->cell_start, c->cell_start_next, c->cellof, c->hrank,
-                c->hcell, c->perm, c->arrival, c->arrival_seq, c->arrival_span, c->scan_state, c->scan_cost, c->scan_tile0, c->seqstate, c->probe_out, c->mx.rv,
+                c->hcell, c->hrank_next, c->hcell_next, c->row_seq, c->row_seq_next, c->row_head, c->row_head_next, c->perm, c->scan_state, c->scan_cost, c->scan_tile0, c->seqstate, c->probe_out, c->mx.rv,
                 c->mx.rp, c->mx.nrm, c->tile_list, c->list_cost, c->wall_list, c->bz_list,
                 c->cases, c->tile_base, c->list_part, c->tile_bound};
   for (void *p : ps)

@@ -5,26 +5,28 @@
 //                 arrival rank in the cell; lanes of a wavefront that fall in
 //                 the same cell share one atomic increment (the input is in
 //                 cell order from the previous build, so a wavefront spans only
-//                 a handful of cells); removed particles go to the extra
-//                 bucket `ncells`
+//                 a handful of cells); the particle's seq goes to that place
+//                 in the cell's row; removed particles go to the extra bucket
+//                 `ncells`
 //   2. scan       exclusive scan of the per-cell counts -> cell_start (CSR);
 //                 also lists the non-empty pair-loop tiles
-//   3. k_scatter  arrival position = cell_start[cell] + rank, with the seq
-//                 of the particle placed there
-//   4. k_reorder  each arrival position ranks its seq among those of its cell
+//   3. k_reorder  each particle ranks its seq among those in its cell's row
 //                 (reference particle order), which makes the result identical
 //                 to the reference's serial push_back in ascending particle
 //                 index and independent of the atomic arrival order, and moves
 //                 the SoA fields to the ranked slot; also lists the wall
 //                 particles for the wall-density gathers and clears the counts
 //
-// Steps 1-3 are a one-digit counting sort on the cell key (the key range is
-// the cell count, so a single digit covers it and its scan is the cell-start
-// table the pair loops need anyway); the rank in step 4 supplies the
-// stability.  All passes read the particle count from device memory, so the
-// sequence can be captured in a HIP graph.  The per-cell counters are cleared
-// by the reorder that follows their scan, so no separate clearing pass is
-// needed.  The scan also lists the pair loops' non-empty tiles.
+// This is a one-digit counting sort on the cell key (the key range is the cell
+// count, so a single digit covers it and its scan is the cell-start table the
+// pair loops need anyway); the rank in step 3 supplies the stability.  With the
+// rows a build is three launches, or two where the build before took its hash;
+// a placement pass between scan and reorder (each slot's source, then the
+// reorder as a gather) measured 4.7 us more per build on 6k to 50k particles
+// and 8 of 271 us per step on 740k (the FP32-pair dam break: 271 -> 259 us).
+// All passes read the particle count from device memory, so the sequence can
+// be captured in a HIP graph.  The per-cell counters are cleared by the reorder
+// that follows their scan, so no separate clearing pass is needed.
 #include "tsph_internal.h"
 #include "tsph_physics.h"
 #include "tsph_tiles.h"
@@ -119,13 +121,29 @@ __device__ __forceinline__ int count_cell(bool live, int c, int *__restrict__ ce
   return __shfl(base, leader, 64) + __popcll(grp & lanemask_lt());
 }
 
+// The rows in which a hash leaves the seqs of every cell's particles, in arrival
+// order, for the reorder to rank: `width` entries per cell, the rest of a
+// fuller cell chained by input slot (link, one more than the slot; 0 ends) from
+// one of kRowHeads heads.  width == 0: no rows (the hash stores arrival ranks).
+struct CellRows {
+  uint32_t *seq;
+  int *head, *link;
+  int width;
+};
+
+// slot i (seq q) as the rank-th arrival of cell c
+__device__ __forceinline__ void put_row(const CellRows &rw, int c, int rank, int i, uint32_t q) {
+  if (rank < rw.width) rw.seq[(size_t)c * rw.width + rank] = q;
+  else rw.link[i] = atomicExch(&rw.head[c & (kRowHeads - 1)], i + 1);
+}
+
 template <bool PRED, bool DECIDE, int WALLS>
 __global__ void k_hash(const double2 *__restrict__ r, const double2 *__restrict__ v,
                        uint8_t *__restrict__ type,
                        const uint32_t *__restrict__ seq, const int *__restrict__ scal, Consts k0,
                        const Consts *__restrict__ cases, const uint8_t *__restrict__ cid, double dt0,
                        int ncells_tot, int *__restrict__ cell_count, int *__restrict__ hcell,
-                       int *__restrict__ hrank, uint8_t *__restrict__ seqstate,
+                       int *__restrict__ hrank, CellRows rows, uint8_t *__restrict__ seqstate,
                        unsigned long long *__restrict__ counters, WallPass wp) {
   int hb = blockIdx.x;  // hash workgroup
   if (WALLS) {
@@ -160,7 +178,8 @@ __global__ void k_hash(const double2 *__restrict__ r, const double2 *__restrict_
   const int rank = count_cell(live, c, cell_count);
   if (live) {
     hcell[i] = c;
-    hrank[i] = rank;
+    if (!rows.width) hrank[i] = rank;
+    else if (c != ncells_tot) put_row(rows, c, rank, i, seq[i]);
   }
 }
 
@@ -356,7 +375,8 @@ __global__ __launch_bounds__(kScanBlock) void k_scan(const int *__restrict__ in,
                                                      int *__restrict__ out, int *__restrict__ scal,
                                                      unsigned long long *__restrict__ counters,
                                                      TileScan ts, int spin_limit, int nwall_idx,
-                                                     int wall_groups, WallPass wp, Consts k0) {
+                                                     int wall_groups, WallPass wp, Consts k0,
+                                                     int *__restrict__ old_heads) {
   __shared__ int lds[3 * kScanBlock / 64];
   constexpr int kTile = kScanBlock * IT;
   __shared__ int s_cnt[kTile + kMaxTileRows];
@@ -373,6 +393,10 @@ __global__ __launch_bounds__(kScanBlock) void k_scan(const int *__restrict__ in,
                                                 s_terms + wid * walls::kTerms);
     return;
   }
+  // the chains of the build before this one, which nothing reads any more
+  if (old_heads)
+    for (int h = blk * kScanBlock + threadIdx.x; h < kRowHeads; h += nb * kScanBlock)
+      old_heads[h] = 0;
   int v[IT], tl[IT], own[IT], halo;
   load_counts<IT>(in, len, blk, v, halo);
   const int nt = stage_counts<IT>(len, blk, ts, v, halo, tl, own, s_cnt, &s_case);
@@ -515,58 +539,45 @@ __global__ __launch_bounds__(kScanBlock) void k_scan(const int *__restrict__ in,
   }
 }
 
-// Arrival position of every particle: cell_start[cell] + its rank from the
-// hash.  RANK (the reorder ranks the cells' particles by seq): with the seq of
-// the particle placed there and the span of its cell (arrival rank | cell
-// count << 16; all ones for a cell of more than 0xffff particles), so that the
-// reorder needs no cell offsets; otherwise k_order / k_order_tiles order
-// `arrival` (then perm) in place.  Also marks the reference positions of removed particles (the trailing
-// bucket) absent in the removal states, and clears k_scan's words for the
-// next build.  CUT: the first `cuts` workgroups (one wavefront per scan block)
+// Placement without rows: arrival position of every particle (cell_start[cell]
+// + its arrival rank from the hash), whose cells k_order / k_order_tiles order
+// in place.  Also marks the reference positions of removed particles (the
+// trailing bucket) absent in the removal states, and clears k_scan's words for
+// the next build.  The first `cuts` workgroups (one wavefront per scan block)
 // cut the new tile list into the chunks of the pooled pair pass that follows
 // from the scan's per-block sums (cut_chunks_scan), beside the placement.
 constexpr int kScatterBlock = 256;
-// particles up to which the reorder ranks the cells' particles itself (on the
-// 740k-particle dam break that saves 6 us of a 0.28 ms step; on 4M and 7.8M
-// particles the 12 more bytes per particle it moves cost 2-3% of the step)
-constexpr int kRankMax = 2000000;
 // ordering workgroups (of 256 threads) per compute unit, single case
 constexpr int kOrderWaves = 4;
-template <bool CUT, bool RANK>
+// the chunk cut's share of a launch of kScatterBlock-thread workgroups
+struct ChunkCut {
+  int cuts;  // cutting workgroups (0: no cut)
+  int scan_blocks, groups;
+  const int *list_cost, *blk_cost, *blk_tile0;
+  int *bound;
+};
+__device__ __forceinline__ void cut_wave(const ChunkCut &cc, const int *__restrict__ scal) {
+  __shared__ long long red[kScatterBlock / 64], pfx[kScatterBlock / 64];
+  tiles::cut_chunks_scan(scal, cc.list_cost, cc.blk_cost, cc.blk_tile0, cc.scan_blocks, cc.groups,
+                         cc.bound, blockIdx.x, red, pfx);
+}
 __global__ __launch_bounds__(kScatterBlock) void k_scatter(
     const int *__restrict__ scal, const int *__restrict__ hcell, const int *__restrict__ hrank,
-    const int *__restrict__ cell_start, int *__restrict__ arrival,
-    uint32_t *__restrict__ arrival_seq, uint32_t *__restrict__ arrival_span,
-    int *__restrict__ cellof, int ncells_tot,
-    const uint32_t *__restrict__ seq, uint8_t *__restrict__ seqstate,
-    unsigned long long *__restrict__ scan_state, int scan_blocks, int groups, int cuts,
-    const int *__restrict__ list_cost, const int *__restrict__ blk_cost,
-    const int *__restrict__ blk_tile0, int *__restrict__ bound) {
-  int blk = blockIdx.x, nblk = gridDim.x;
-  if constexpr (CUT) {
-    __shared__ long long red[kScatterBlock / 64], pfx[kScatterBlock / 64];
-    if (blk < cuts) {
-      tiles::cut_chunks_scan(scal, list_cost, blk_cost, blk_tile0, scan_blocks, groups, bound,
-                             blk, red, pfx);
-      return;
-    }
-    blk -= cuts;
-    nblk -= cuts;
+    const int *__restrict__ cell_start, int *__restrict__ arrival, int *__restrict__ cellof,
+    int ncells_tot, const uint32_t *__restrict__ seq, uint8_t *__restrict__ seqstate,
+    unsigned long long *__restrict__ scan_state, ChunkCut cc) {
+  if ((int)blockIdx.x < cc.cuts) {
+    cut_wave(cc, scal);
+    return;
   }
-  const int n = scal[S_NP];
-  const int i = blk * blockDim.x + threadIdx.x;
-  for (int b = i; b < scan_blocks; b += nblk * blockDim.x) scan_state[b] = 0;
+  const int n = scal[S_NP], blk = blockIdx.x - cc.cuts;
+  const int i = blk * kScatterBlock + threadIdx.x;
+  for (int b = i; b < cc.scan_blocks; b += (gridDim.x - cc.cuts) * kScatterBlock) scan_state[b] = 0;
   if (i >= n) return;
   const int c = hcell[i];
   if (c == ncells_tot) seqstate[seq[i]] = 0;
-  const int s0 = cell_start[c], rank = hrank[i];
-  const int pos = s0 + rank;
+  const int pos = cell_start[c] + hrank[i];
   arrival[pos] = i;
-  if (RANK) {
-    const int cnt = cell_start[c + 1] - s0;
-    arrival_seq[pos] = seq[i];
-    arrival_span[pos] = cnt <= 0xffff ? (uint32_t)rank | (uint32_t)cnt << 16 : 0xffffffffu;
-  }
   cellof[pos] = c;
 }
 
@@ -659,84 +670,109 @@ __global__ void k_order_tiles(const int *__restrict__ cell_start, const int *__r
   }
 }
 
-// slot of arrival position x in (cell, seq) order: the cell's first slot plus
-// the number of the cell's particles that precede x's in seq (ties, which
-// distinct seqs never give, broken by arrival position so that every arrival
-// position of the cell gets a slot of its own).  The cell's keys are read
-// kRankBatch at a time, all of them in flight together (one round for all
-// but the fullest cells).
-constexpr int kRankBatch = 16;
-__device__ __forceinline__ int ranked_slot(const int *__restrict__ cell_start,
-                                           const int *__restrict__ cellof,
-                                           const uint32_t *__restrict__ span,
-                                           const uint32_t *__restrict__ key, int x) {
-  const uint32_t sp = span[x];
-  int s, e;
-  if (sp != 0xffffffffu) {
-    s = x - (int)(sp & 0xffffu);
-    e = s + (int)(sp >> 16);
-  } else {
-    const int c = cellof[x];
-    s = cell_start[c];
-    e = cell_start[c + 1];
-  }
-  const uint32_t mine = key[x];
+// slot of the particle with seq `mine` in cell c, in (cell, seq) order: the
+// cell's first slot plus the number of the cell's particles that precede it in
+// seq.  The row is read 16 entries at a time, all of them in flight together
+// (one round for all but the fullest cells); the chained ones cell by seq.
+__device__ __forceinline__ int ranked_slot(const int *__restrict__ cell_start, const CellRows &rw,
+                                           const int *__restrict__ hcell,
+                                           const uint32_t *__restrict__ seq, int n, int c,
+                                           uint32_t mine) {
+  const int s = cell_start[c], cnt = cell_start[c + 1] - s;
+  const uint4 *row = reinterpret_cast<const uint4 *>(rw.seq + (size_t)c * rw.width);
+  const int in_row = min(cnt, rw.width);
   int slot = s;
-  for (int a0 = s; a0 < e; a0 += kRankBatch) {
-    uint32_t kv[kRankBatch];
+  for (int a = 0; a < in_row; a += 16) {
+    uint4 q[4];
 #pragma unroll
-    for (int u = 0; u < kRankBatch; ++u) kv[u] = a0 + u < e ? key[a0 + u] : 0u;
+    for (int u = 0; u < 4; ++u)
+      q[u] = a + 4 * u < in_row ? row[a / 4 + u] : make_uint4(0u, 0u, 0u, 0u);
 #pragma unroll
-    for (int u = 0; u < kRankBatch; ++u) {
-      const int a = a0 + u;
-      slot += a < e && (kv[u] < mine || (kv[u] == mine && a < x));
+    for (int u = 0; u < 4; ++u) {
+      const int o = a + 4 * u;
+      slot += (o < in_row && q[u].x < mine) + (o + 1 < in_row && q[u].y < mine) +
+              (o + 2 < in_row && q[u].z < mine) + (o + 3 < in_row && q[u].w < mine);
+    }
+  }
+  if (cnt > rw.width) {
+    int y = rw.head[c & (kRowHeads - 1)];
+    for (int left = n; y > 0 && left > 0; --left) {
+      slot += hcell[y - 1] == c && seq[y - 1] < mine;
+      y = rw.link[y - 1];
     }
   }
   return slot;
 }
 
-// Moves every field from its arrival position to its ranked slot (the state
-// after the build is the reference's state, permuted; perm records the
-// permutation), lists the wall particles, clears the cell counts for the next
-// build and sets the new particle count (removed particles sit after n_new and
-// are dropped).
+// Moves every field to its slot of the new order (the state after the build is
+// the reference's state, permuted; perm records the permutation), lists the
+// wall particles and sets the new particle count (removed particles are
+// dropped).  RANK: thread x moves input slot x to the slot that the hash's rows
+// give it (reads in a row, writes nearly so: few particles change cells in a
+// step), and does the placement's other work: the cell of each slot, the cell
+// counts and the scan's words cleared for the next build, removed particles
+// marked absent, the pooled pass's chunk cut (cc) in the first workgroups.
+// Otherwise thread x fills slot x from where the placement says.
 // With EOS the pressure is recomputed as Density_to_pressure does
 // (src/SPH_pressure.h:65-89) and the FP32 records of the mixed path are
 // written, for the step sequences in which that stage follows the cell build.
 // With PRED the symplectic predictor (src/SPH_integration.h:266-287) is
 // applied to the moved particles, for the step sequences in which it
 // immediately precedes the cell build.  With NEXT the hash of the next step's
-// first build is taken on the way: that build sorts by the positions the
-// predictor will give, which need no forces, so a step inside a run of steps
-// starts with its scan (next_count: the next build's cell counts).  ad_skip (a type mask): a and drho of
-// those types are not moved, for the step sequences in which a pair pass that
-// overwrites them for exactly those types follows the build.
+// first build is taken on the way (next_count, next_hcell, next_rows or
+// next_hrank): that build sorts by the positions the predictor will give,
+// which need no forces, so a step inside a run of steps starts with its scan.
+// ad_skip (a type mask): a and drho of those types are not moved, for the step
+// sequences in which a pair pass that overwrites them for exactly those types
+// follows the build.
 template <bool EOS, bool PRED, bool RANK, bool NEXT>
-__global__ void k_reorder(const int *__restrict__ cell_start, int ncells,
-                          const int *__restrict__ arrival, const uint32_t *__restrict__ arrival_seq,
-                          const uint32_t *__restrict__ arrival_span, int *__restrict__ perm,
-                          int *__restrict__ cell_count,
-                          Soa src, Soa dst, int *__restrict__ scal, int *__restrict__ wall_list,
-                          const int *__restrict__ cellof, Consts k0,
-                          const Consts *__restrict__ cases, Mixed mx, double dt0,
-                          unsigned ad_skip, unsigned long long *__restrict__ counters,
-                          int nwall_idx, bool move_olds, int *__restrict__ next_count,
-                          int *__restrict__ hcell, int *__restrict__ hrank) {
+__global__ __launch_bounds__(kScatterBlock) void k_reorder(
+    const int *__restrict__ cell_start, int ncells, const int *__restrict__ hcell, CellRows rows,
+    int *__restrict__ perm, int *__restrict__ cell_count, uint8_t *__restrict__ seqstate,
+    unsigned long long *__restrict__ scan_state, ChunkCut cc, Soa src, Soa dst,
+    int *__restrict__ scal, int *__restrict__ wall_list, int *__restrict__ cellof, Consts k0,
+    const Consts *__restrict__ cases, Mixed mx, double dt0, unsigned ad_skip,
+    unsigned long long *__restrict__ counters, int nwall_idx, bool move_olds,
+    int *__restrict__ next_count, int *__restrict__ next_hcell, int *__restrict__ next_hrank,
+    CellRows next_rows) {
+  int blk = blockIdx.x;
+  if (RANK) {
+    if (blk < cc.cuts) {
+      cut_wave(cc, scal);
+      return;
+    }
+    blk -= cc.cuts;
+  }
   const int n_new = cell_start[ncells];
-  const int x = blockIdx.x * blockDim.x + threadIdx.x;  // arrival position
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
+  const int n = RANK ? cell_start[ncells + 1] : n_new;  // RANK: with the removed ones
+  const int x = blk * kScatterBlock + threadIdx.x;
+  if (blk == 0 && threadIdx.x == 0) {
     scal[S_NP] = n_new;
     if (RANK) cell_count[ncells] = 0;  // the removed bucket
   }
+  if (RANK)
+    for (int b = x; b < cc.scan_blocks; b += (gridDim.x - cc.cuts) * kScatterBlock)
+      scan_state[b] = 0;
   int wall = 0, k = x, next_c = -1;
   unsigned bad = 0;
-  if (x < n_new) {
-    const int j = arrival[x];
-    const int cell = RANK || (EOS && mx.rv) ? cellof[x] : 0;
+  bool live = x < n;
+  int cell = 0;
+  if (RANK && live) {
+    cell = hcell[x];
+    if (cell == ncells) {
+      seqstate[src.seq[x]] = 0;
+      live = false;
+    }
+  }
+  if (live) {
+    const int j = RANK ? x : perm[x];
     if (RANK) {
-      k = ranked_slot(cell_start, cellof, arrival_span, arrival_seq, x);
+      k = ranked_slot(cell_start, rows, hcell, src.seq, n, cell, src.seq[x]);
       cell_count[cell] = 0;
       perm[k] = j;
+      cellof[k] = cell;
+    } else if (EOS && mx.rv) {
+      cell = cellof[x];
     }
     const uint8_t t = src.type[j];
     wall = t == TSPH_WALL;
@@ -817,11 +853,11 @@ __global__ void k_reorder(const int *__restrict__ cell_start, int ncells,
     }
   }
   if (NEXT) {
-    const bool live = x < n_new;
     const int rank = count_cell(live, next_c, next_count);
     if (live) {
-      hcell[k] = next_c;
-      hrank[k] = rank;
+      next_hcell[k] = next_c;
+      if (RANK) put_row(next_rows, next_c, rank, k, src.seq[x]);
+      else next_hrank[k] = rank;
     }
   }
   const unsigned long long m = __ballot(wall);
@@ -851,6 +887,13 @@ __global__ void k_gather_olds(const int *__restrict__ scal, const int *__restric
   dst.rho_o[k] = src.rho_o[j];
 }
 
+// The builds' cells are ordered from rows by the reorder: wherever the context
+// has rows.  Ranked against placement and ordering passes, us per step of the
+// dam break: FP32 pairs 258 / 276 at 740k particles, 670 / 692 at 2.0M, 1232 /
+// 1253 at 3.9M, 2279 / 2306 at 7.6M; FP64 511 / 533, 1336 / 1346, 2561 / 2574,
+// 4788 / 4776 (within the runs' spread).
+bool cells_ranked(const tsph_ctx *c) { return c->row_width > 0 && c->cell_order != 2; }
+
 // exclusive scan of the cell counts into cell_start, with the tile list of the
 // current tile_rows (and, for cost_table >= 0, the listed tiles' costs); with
 // walls (TSPH_WALL_*; 0: none) the wall pass wp beside it
@@ -867,7 +910,7 @@ int scan_cells(tsph_ctx *c, hipStream_t s, const int *count, int *cs, int nwall_
 #define TSPH_SCAN(IT, W)                                                                       \
   hipLaunchKernelGGL((k_scan<IT, W>), dim3(scan_blocks(c) + wg), dim3(kScanBlock), 0, s, count, len, \
                      c->scan_state, cs, c->scal, c->counters, ts, c->scan_wait, nwall_idx, wg, wp, \
-                     c->k)
+                     c->k, c->row_width ? c->row_head_next : nullptr)
 #define TSPH_SCAN_W(IT)                                                                        \
   if (walls == TSPH_WALL_MDBC) TSPH_SCAN(IT, TSPH_WALL_MDBC);                                 \
   else if (walls == TSPH_WALL_BT) TSPH_SCAN(IT, TSPH_WALL_BT);                                \
@@ -886,6 +929,18 @@ int scan_cells(tsph_ctx *c, hipStream_t s, const int *count, int *cs, int nwall_
 }
 
 }  // namespace
+
+void flip_build(tsph_ctx *c) {
+  std::swap(c->cur, c->alt);
+  std::swap(c->cell_start, c->cell_start_next);
+  std::swap(c->cell_count, c->cell_count_next);
+  std::swap(c->hcell, c->hcell_next);
+  std::swap(c->hrank, c->hrank_next);
+  std::swap(c->row_seq, c->row_seq_next);
+  std::swap(c->row_head, c->row_head_next);
+  c->nwall_idx = c->nwall_idx == S_NWALL ? S_NWALL_B : S_NWALL;
+  c->parity ^= 1;
+}
 
 int ensure_olds(tsph_ctx *c) {
   if (!c->olds_stale) return 0;
@@ -922,14 +977,17 @@ int launch_cell_list(tsph_ctx *c, bool eos, bool predict, double dt, unsigned ad
     hg = wp.walls + wp.sweep + grid_for(c->n_ub, hbs);
     c->records_valid = false;
   }
-  // counts of a build whose hash the previous build took (hash_next) are kept
-  // apart from those of the builds between
-  int *count = hashed ? c->cell_count_next : c->cell_count;
+  // the per-cell order: ranked by the reorder from rows that the hash leaves (two
+  // launches and a hash), or by passes of its own
+  const bool rank = cells_ranked(c);
+  const CellRows rw{c->row_seq, c->row_head, rank ? c->hrank : nullptr, rank ? c->row_width : 0};
+  const CellRows rw_next{c->row_seq_next, c->row_head_next, rank ? c->hrank_next : nullptr,
+                         rank ? c->row_width : 0};
   if (!hashed) {
 #define TSPH_HASH(P, D, W)                                                                     \
   hipLaunchKernelGGL((k_hash<P, D, W>), dim3(hg), dim3(hbs), 0, s, c->cur.r, c->cur.v,            \
                      c->cur.type, c->cur.seq, c->scal, k, c->cases, c->cur.cid, dt, nct,          \
-                     c->cell_count, c->hcell, c->hrank, c->seqstate, c->counters, wp)
+                     c->cell_count, c->hcell, c->hrank, rw, c->seqstate, c->counters, wp)
 #define TSPH_HASH_W(P, D)                                                                      \
   if (walls == TSPH_WALL_MDBC) TSPH_HASH(P, D, TSPH_WALL_MDBC);                               \
   else if (walls == TSPH_WALL_BT) TSPH_HASH(P, D, TSPH_WALL_BT);                              \
@@ -955,45 +1013,36 @@ int launch_cell_list(tsph_ctx *c, bool eos, bool predict, double dt, unsigned ad
     set_error("tile list: more pooled workgroups than allocated");
     return TSPH_ESTATE;
   }
-  if (int e = scan_cells(c, s, count, cs, wslot, cut > 0 ? c->cut_table : -1, hashed ? walls : 0, wp))
+  if (int e = scan_cells(c, s, c->cell_count, cs, wslot, cut > 0 ? c->cut_table : -1, hashed ? walls : 0, wp))
     return e;
   const int sg = grid_for(c->n_ub, kScatterBlock);
-  // the per-cell order: ranked by the reorder (one launch fewer), or by its
-  // own pass (fewer bytes moved); by size, up to kRankMax particles ranked
-  const bool rank = c->cell_order == 1 || (c->cell_order == 0 && c->n_ub <= kRankMax);
-  int *arrival = rank ? c->arrival : c->perm;
-#define TSPH_SCATTER(CUT, RANK, GRID, CUTS, GROUPS)                                            \
-  hipLaunchKernelGGL((k_scatter<CUT, RANK>), dim3(GRID), dim3(kScatterBlock), 0, s, c->scal,       \
-                     c->hcell, c->hrank, cs, arrival, c->arrival_seq, c->arrival_span, c->cellof,   \
-                     nct, c->cur.seq, c->seqstate, c->scan_state, scan_blocks(c), GROUPS, CUTS,     \
-                     c->list_cost, c->scan_cost, c->scan_tile0, c->tile_bound)
+  // one cutting wavefront per scan block, in the first workgroups
+  const int cuts = cut > 0 ? grid_for(scan_blocks(c), kScatterBlock / 64) : 0;
+  const ChunkCut cc{cuts, scan_blocks(c), cut, c->list_cost, c->scan_cost, c->scan_tile0,
+                    c->tile_bound};
   if (cut > 0) {
-    // one cutting wavefront per scan block, in the first workgroups
-    const int cuts = (scan_blocks(c) + kScatterBlock / 64 - 1) / (kScatterBlock / 64);
-    if (rank) TSPH_SCATTER(true, true, cuts + sg, cuts, cut);
-    else TSPH_SCATTER(true, false, cuts + sg, cuts, cut);
     c->list_groups = cut;
     c->list_table = c->cut_table;
-  } else {
-    if (rank) TSPH_SCATTER(false, true, sg, 0, 0);
-    else TSPH_SCATTER(false, false, sg, 0, 0);
   }
-#undef TSPH_SCATTER
   if (!rank) {
+    hipLaunchKernelGGL(k_scatter, dim3(cuts + sg), dim3(kScatterBlock), 0, s, c->scal, c->hcell,
+                       c->hrank, cs, c->perm, c->cellof, nct, c->cur.seq, c->seqstate,
+                       c->scan_state, cc);
     if (c->cases)
       hipLaunchKernelGGL(k_order, dim3(grid_for(nct + 1, nb)), dim3(nb), 0, s, cs, nct, c->cur.seq,
-                         c->perm, count);
+                         c->perm, c->cell_count);
     else
       hipLaunchKernelGGL(k_order_tiles, dim3(kOrderWaves * std::max(1, c->num_cu)), dim3(nb), 0, s,
                          cs, c->scal, c->tile_list, c->tile_rows, k.ncy, nct, c->cur.seq, c->perm,
-                         count);
+                         c->cell_count);
   }
   const Mixed mx = c->prm.precision == TSPH_PREC_MIXED ? c->mx : Mixed{};
 #define TSPH_REORDER(E, P, R, N)                                                              \
-  hipLaunchKernelGGL((k_reorder<E, P, R, N>), dim3(g), dim3(nb), 0, s, cs, nct, arrival,           \
-                     c->arrival_seq, c->arrival_span, c->perm, count, c->cur, c->alt, c->scal,     \
-                     c->wall_list, c->cellof, k, c->cases, mx, dt, ad_skip, c->counters, wslot,    \
-                     !skip_olds, c->cell_count_next, c->hcell, c->hrank)
+  hipLaunchKernelGGL((k_reorder<E, P, R, N>), dim3(R ? cuts + sg : sg), dim3(kScatterBlock), 0, s,  \
+                     cs, nct, c->hcell, rw, c->perm, c->cell_count, c->seqstate, c->scan_state, cc, \
+                     c->cur, c->alt, c->scal, c->wall_list, c->cellof, k, c->cases, mx, dt,        \
+                     ad_skip, c->counters, wslot, !skip_olds, c->cell_count_next, c->hcell_next,    \
+                     c->hrank_next, rw_next)
 #define TSPH_REORDER_R(E, P)                                                                  \
   if (rank) TSPH_REORDER(E, P, true, false);                                                  \
   else TSPH_REORDER(E, P, false, false)
@@ -1013,11 +1062,8 @@ int launch_cell_list(tsph_ctx *c, bool eos, bool predict, double dt, unsigned ad
 #undef TSPH_REORDER_R
 #undef TSPH_REORDER
   TSPH_HIP(hipGetLastError());
-  std::swap(c->cur, c->alt);
-  std::swap(c->cell_start, c->cell_start_next);
-  c->nwall_idx = wslot;
+  flip_build(c);
   c->olds_stale = skip_olds && !predict;
-  c->parity ^= 1;
   c->cells_valid = true;
   c->tiles_valid = true;  // listed by the scan
   c->records_valid = eos && c->prm.precision == TSPH_PREC_MIXED;

@@ -177,7 +177,7 @@ struct tsph_ctx {
   // chunks per workgroup, tiles taken from an LDS counter by the workgroup's
   // waves) or the plain static walk; defaults set at creation
   bool balanced[2] = {false, false};
-  int cell_order = 0;  // tsph_set_cell_order: 0 by size, 1 ranked, 2 separate pass
+  int cell_order = 0;  // tsph_set_cell_order: 0 and 1 ranked, 2 separate passes
   int *tile_list = nullptr;  // non-empty tiles of the current cell list, in tile order
   bool tiles_valid = false;  // tile_list matches the cell list and tile_rows
   int *list_part = nullptr;  // per list-build block: tiles, work
@@ -211,7 +211,7 @@ struct tsph_ctx {
   int *scal = nullptr;                 // S_* slots, then the per-tile costs
   unsigned long long *counters = nullptr;
   int *cell_count = nullptr;           // ncells+1 (last = removed bucket)
-  int *cell_count_next = nullptr;      // the counts of a hash taken by the build before
+  int *cell_count_next = nullptr;      // the next build's
   int *cell_start = nullptr;           // ncells+2
   // Every build writes its cell offsets and wall count into the buffers the
   // previous build did not (cell_start_next, the other wall-count slot) and
@@ -220,14 +220,20 @@ struct tsph_ctx {
   int *cell_start_next = nullptr;      // ncells+2
   int nwall_idx = 3;                   // S_NWALL or S_NWALL_B: the current wall count
   int *cellof = nullptr;               // cell of each slot (sorted order)
-  int *hrank = nullptr;                // rank inside the cell from the hash pass
+  int *hrank = nullptr;                // rank inside the cell from the hash pass, or row links
   int *hcell = nullptr;                // cell from the hash pass (pre-sort order)
   int *perm = nullptr;                 // sorted position -> old slot
-  // the scatter's placement (cell, then arrival order) and the seq of each
-  // placed particle, which the reorder ranks within the cell
-  int *arrival = nullptr;              // arrival position -> old slot
-  uint32_t *arrival_seq = nullptr;     // arrival position -> seq
-  uint32_t *arrival_span = nullptr;    // arrival rank | cell count << 16
+  // the seqs of each cell's particles as the hash leaves them for the reorder
+  // to rank (row_width per cell, fuller cells chained from row_head; 0: the
+  // builds order the cells in passes of their own)
+  int row_width = 0;
+  uint32_t *row_seq = nullptr;
+  int *row_head = nullptr;
+  // the next build's (flip_build swaps them in), so that a build's reorder can
+  // take the hash of the build after it
+  int *hcell_next = nullptr, *hrank_next = nullptr;
+  uint32_t *row_seq_next = nullptr;
+  int *row_head_next = nullptr;
   // cell-list scan: one published word per block (zero: not yet published),
   // and the polls a block makes for an earlier block's word (-1: none)
   unsigned long long *scan_state = nullptr;
@@ -326,6 +332,11 @@ struct TileGrid {
 // hash_next (with eos, without predict): the build's reorder also takes the
 // hash of the predict build that follows it with nothing but a pair pass
 // between them (the next step's first, with time step dt); hashed: that build
+// heads of the chains that hold what the cells' rows do not (a power of two)
+constexpr int kRowHeads = 4096;
+// the buffers that change places with every cell build: cur and alt, and this
+// build's cell-list buffers and the next one's
+void flip_build(tsph_ctx *c);
 int launch_cell_list(tsph_ctx *c, bool eos = false, bool predict = false, double dt = 0.,
                      unsigned ad_skip = 0, bool decide = false, bool skip_olds = false,
                      int walls = 0, bool count_density = false, bool hashed = false,
