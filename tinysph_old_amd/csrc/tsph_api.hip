@@ -386,7 +386,8 @@ static int alloc_context(tsph_ctx *c) {
   if ((e = alloc_soa(c->cur, cap, false, false)) || (e = alloc_soa(c->alt, cap, false, false)))
     return e;
   if ((e = dalloc(&c->scal, S_NSCAL + (size_t)kCostTables * (nct + 8))) ||
-      (e = dalloc(&c->cell_count, nct + 1)) || (e = dalloc(&c->cell_count_next, nct + 1)) ||
+      (e = dalloc(&c->cell_count, count_words(c))) ||
+      (e = dalloc(&c->cell_count_next, count_words(c))) ||
       (e = dalloc(&c->cell_start, nct + 2)) ||
       (e = dalloc(&c->cell_start_next, nct + 2)) ||
       (e = dalloc(&c->cellof, cap)) ||
@@ -399,6 +400,7 @@ static int alloc_context(tsph_ctx *c) {
       (e = dalloc(&c->tile_list, nct + 8)) || (e = dalloc(&c->list_cost, nct + 8)) ||
       (e = dalloc(&c->wall_list, cap)) ||
       (e = dalloc(&c->scan_state, (nct + 1) / 1024 + 2)) ||
+      (e = dalloc(&c->scan_state_next, (nct + 1) / 1024 + 2)) ||
       (e = dalloc(&c->scan_cost, (nct + 1) / 1024 + 2)) ||
       (e = dalloc(&c->scan_tile0, (nct + 1) / 1024 + 2)))
     return e;
@@ -414,11 +416,20 @@ static int alloc_context(tsph_ctx *c) {
         hipMemsetAsync(c->row_head_next, 0, sizeof(int) * kRowHeads, c->stream) != hipSuccess)
       return fail(TSPH_EHIP, "initialisation failed");
   }
+  if (c->row_width && bin_words(c) <= kBinMax) {
+    if ((e = dalloc(&c->bin_count, bin_words(c))) || (e = dalloc(&c->bin_count_next, bin_words(c))))
+      return e;
+    if (hipMemsetAsync(c->bin_count, 0, sizeof(int) * bin_words(c), c->stream) != hipSuccess ||
+        hipMemsetAsync(c->bin_count_next, 0, sizeof(int) * bin_words(c), c->stream) != hipSuccess)
+      return fail(TSPH_EHIP, "initialisation failed");
+  }
   // the per-cell counters and removal states start cleared; later builds clear
   // them as they consume them (the single-pass scan's words likewise)
-  if (hipMemsetAsync(c->cell_count, 0, sizeof(int) * (nct + 1), c->stream) != hipSuccess ||
-      hipMemsetAsync(c->cell_count_next, 0, sizeof(int) * (nct + 1), c->stream) != hipSuccess ||
+  if (hipMemsetAsync(c->cell_count, 0, sizeof(int) * count_words(c), c->stream) != hipSuccess ||
+      hipMemsetAsync(c->cell_count_next, 0, sizeof(int) * count_words(c), c->stream) != hipSuccess ||
       hipMemsetAsync(c->scan_state, 0, sizeof(unsigned long long) * ((nct + 1) / 1024 + 2),
+                     c->stream) != hipSuccess ||
+      hipMemsetAsync(c->scan_state_next, 0, sizeof(unsigned long long) * ((nct + 1) / 1024 + 2),
                      c->stream) != hipSuccess ||
       hipMemsetAsync(c->seqstate, 0, (size_t)c->seq_cap, c->stream) != hipSuccess)
     return fail(TSPH_EHIP, "initialisation failed");
@@ -510,7 +521,7 @@ int tsph_destroy(tsph_ctx *c) {
   free_soa(c->cur);
   free_soa(c->alt);
   void *ps[] = {c->scal, c->counters, c->cell_count, c->cell_count_next, c->cell_start, c->cell_start_next, c->cellof, c->hrank,
-                c->hcell, c->hrank_next, c->hcell_next, c->row_seq, c->row_seq_next, c->row_head, c->row_head_next, c->perm, c->scan_state, c->scan_cost, c->scan_tile0, c->seqstate, c->probe_out, c->mx.rv,
+                c->hcell, c->hrank_next, c->hcell_next, c->row_seq, c->row_seq_next, c->row_head, c->row_head_next, c->bin_count, c->bin_count_next, c->perm, c->scan_state, c->scan_state_next, c->scan_cost, c->scan_tile0, c->seqstate, c->probe_out, c->mx.rv,
                 c->mx.rp, c->mx.nrm, c->tile_list, c->list_cost, c->wall_list, c->bz_list,
                 c->cases, c->tile_base, c->list_part, c->tile_bound};
   for (void *p : ps)

@@ -20,7 +20,9 @@
 // This is a one-digit counting sort on the cell key (the key range is the cell
 // count, so a single digit covers it and its scan is the cell-start table the
 // pair loops need anyway); the rank in step 3 supplies the stability.  With the
-// rows a build is three launches, or two where the build before took its hash;
+// rows a build is three launches, one fewer where the build before took its
+// hash, and one fewer on grids of up to 65k cells, whose scan runs beside the
+// reorder (the bins: kBinMax);
 // a placement pass between scan and reorder (each slot's source, then the
 // reorder as a gather) measured 4.7 us more per build on 6k to 50k particles
 // and 8 of 271 us per step on 740k (the FP32-pair dam break: 271 -> 259 us).
@@ -98,27 +100,57 @@ __device__ __forceinline__ int hash_cell(const Consts &k, double2 r,
   return c + k.cell_base;  // the case's segment of the global cell range
 }
 
-// counts the lanes' particles (live lanes) into their cells c and returns each
-// one's arrival rank: the lanes of a wavefront that share a cell are grouped,
-// and the lowest lane of each group does the atomic
-__device__ __forceinline__ int count_cell(bool live, int c, int *__restrict__ cell_count) {
-  const int lane = threadIdx.x & 63;
-  unsigned long long rem = __ballot(live);
-  int leader = 0;
-  unsigned long long grp = 0;
-  while (rem) {
-    const int l = __builtin_ctzll(rem);
-    const int key = __shfl(c, l, 64);
-    const unsigned long long m = __ballot(c == key) & rem;
-    if ((m >> lane) & 1ull) {
-      leader = l;
-      grp = m;
+// counts the lanes' particles (live lanes) into their cells c: the lanes of a
+// wavefront that share a cell are grouped, and the lowest lane of each group
+// does the atomic.  rank() gives each particle's arrival rank once the atomic
+// has returned.
+struct CellCount {
+  int leader, base;
+  unsigned before;  // lanes of the group before this one
+  __device__ __forceinline__ CellCount(bool live, int c, int *__restrict__ cell_count,
+                                       int *__restrict__ bin) {
+    const int lane = threadIdx.x & 63;
+    unsigned long long rem = __ballot(live);
+    leader = 0;
+    unsigned long long grp = 0;
+    while (rem) {
+      const int l = __builtin_ctzll(rem);
+      const int key = __shfl(c, l, 64);
+      const unsigned long long m = __ballot(c == key) & rem;
+      if ((m >> lane) & 1ull) {
+        leader = l;
+        grp = m;
+      }
+      rem &= ~m;
     }
-    rem &= ~m;
+    before = __popcll(grp & lanemask_lt());
+    base = 0;
+    if (live && lane == leader) base = atomicAdd(&cell_count[c], __popcll(grp));
+    if (bin) {  // one add per bin and wavefront: few addresses, many wavefronts
+      const int b = c / kBinCells;
+      for (rem = __ballot(live); rem;) {
+        const int l = __builtin_ctzll(rem);
+        const unsigned long long m = __ballot(b == __shfl(b, l, 64)) & rem;
+        if (lane == l) atomicAdd(&bin[b], __popcll(m));
+        rem &= ~m;
+      }
+    }
   }
-  int base = 0;
-  if (live && lane == leader) base = atomicAdd(&cell_count[c], __popcll(grp));
-  return __shfl(base, leader, 64) + __popcll(grp & lanemask_lt());
+  __device__ __forceinline__ int rank() const { return __shfl(base, leader, 64) + before; }
+};
+
+// What a build clears for the one after it, which shares its buffers with the
+// one before: in its hash, or in its reorder if the build before took its hash
+// (that reorder takes no hash itself).
+struct Clear {
+  int *word[3];  // cell counts, bins, row heads
+  int n4[3];     // int4 words of each
+};
+__device__ __forceinline__ void clear_next(const Clear &cl, int i, int stride) {
+#pragma unroll
+  for (int a = 0; a < 3; ++a)
+    for (int k = i; k < cl.n4[a]; k += stride)
+      reinterpret_cast<int4 *>(cl.word[a])[k] = make_int4(0, 0, 0, 0);
 }
 
 // The rows in which a hash leaves the seqs of every cell's particles, in arrival
@@ -143,7 +175,8 @@ __global__ void k_hash(const double2 *__restrict__ r, const double2 *__restrict_
                        const uint32_t *__restrict__ seq, const int *__restrict__ scal, Consts k0,
                        const Consts *__restrict__ cases, const uint8_t *__restrict__ cid, double dt0,
                        int ncells_tot, int *__restrict__ cell_count, int *__restrict__ hcell,
-                       int *__restrict__ hrank, CellRows rows, uint8_t *__restrict__ seqstate,
+                       int *__restrict__ hrank, CellRows rows, int *__restrict__ bin, Clear cl,
+                       uint8_t *__restrict__ seqstate,
                        unsigned long long *__restrict__ counters, WallPass wp) {
   int hb = blockIdx.x;  // hash workgroup
   if (WALLS) {
@@ -159,9 +192,11 @@ __global__ void k_hash(const double2 *__restrict__ r, const double2 *__restrict_
   const int i = hb * blockDim.x + threadIdx.x;
   const bool live = i < n;
   int c = -1;
+  uint32_t mine = 0;
   if (live) {
+    mine = seq[i];
     bool removed = type[i] == kRemoved;
-    if (DECIDE && !removed && removal_decided(seqstate, seq[i])) {
+    if (DECIDE && !removed && removal_decided(seqstate, mine)) {
       removed = true;
       type[i] = kRemoved;
       atomicAdd(&counters[C_REMOVED], 1ull);
@@ -175,12 +210,13 @@ __global__ void k_hash(const double2 *__restrict__ r, const double2 *__restrict_
       c = hash_cell(k, ri, counters);
     }
   }
-  const int rank = count_cell(live, c, cell_count);
+  const int rank = CellCount(live, c, cell_count, bin).rank();
   if (live) {
     hcell[i] = c;
     if (!rows.width) hrank[i] = rank;
-    else if (c != ncells_tot) put_row(rows, c, rank, i, seq[i]);
+    else if (c != ncells_tot) put_row(rows, c, rank, i, mine);
   }
+  clear_next(cl, i, (gridDim.x - (WALLS ? wp.walls + wp.sweep : 0)) * blockDim.x);
 }
 
 template <int NT>
@@ -329,8 +365,8 @@ __device__ __forceinline__ int stage_counts(int len, int block, const TileScan t
 // (a grid of at most 1024 blocks reads all its words in one round and
 // publishes no inclusive prefixes).  Blocks cover 256 IT cells: IT = 16 above
 // 1M cells keeps grids of up to 4M cells in one round.
-// k_scatter clears the words for the next build.  Blocks are dispatched in
-// index order, so a block waits only for blocks that have started, and those
+// Every scan clears the words of the next (two sets take turns).  Blocks are
+// dispatched in index order, so a block waits only for blocks that have started, and those
 // publish their own sums before they wait themselves.  A block whose wait
 // exceeds spin_limit polls (the context's scan_wait; -1: it does not poll)
 // forms its sums from the counts of the cells before it instead (and counts
@@ -369,34 +405,29 @@ __device__ __forceinline__ void block_reduce3(int &a, int &b, int &m, int *lds) 
   __syncthreads();
 }
 
-template <int IT, int WALLS>
-__global__ __launch_bounds__(kScanBlock) void k_scan(const int *__restrict__ in, int len,
-                                                     unsigned long long *__restrict__ state,
-                                                     int *__restrict__ out, int *__restrict__ scal,
-                                                     unsigned long long *__restrict__ counters,
-                                                     TileScan ts, int spin_limit, int nwall_idx,
-                                                     int wall_groups, WallPass wp, Consts k0,
-                                                     int *__restrict__ old_heads) {
+struct ScanArgs {
+  const int *in;  // the cells' counts, len of them
+  int len;
+  unsigned long long *state, *state_next;
+  int *out;
+  TileScan ts;
+  int spin_limit;
+};
+
+// block blk of nb
+template <int IT>
+__device__ __forceinline__ void scan_block(const ScanArgs &sa, int blk, int nb,
+                                           int *__restrict__ scal,
+                                           unsigned long long *__restrict__ counters) {
   __shared__ int lds[3 * kScanBlock / 64];
   constexpr int kTile = kScanBlock * IT;
   __shared__ int s_cnt[kTile + kMaxTileRows];
   __shared__ int s_case;
-  // the wall pass (WALLS) in the last wall_groups workgroups, a wavefront's
-  // share per wavefront
-  const int nb = gridDim.x - (WALLS ? wall_groups : 0), blk = blockIdx.x;
-  if (WALLS && blk >= nb) {
-    constexpr int kWaves = kScanBlock / 64;
-    __shared__ __align__(16) double s_terms[kWaves * walls::kTerms];
-    const int wid = threadIdx.x >> 6, b = (blk - nb) * kWaves + wid;
-    if (b < wp.walls + wp.sweep)
-      wall_wave<WALLS ? WALLS : TSPH_WALL_MDBC>(b, wp, k0, ts.cases, scal,
-                                                s_terms + wid * walls::kTerms);
-    return;
-  }
-  // the chains of the build before this one, which nothing reads any more
-  if (old_heads)
-    for (int h = blk * kScanBlock + threadIdx.x; h < kRowHeads; h += nb * kScanBlock)
-      old_heads[h] = 0;
+  const int *__restrict__ in = sa.in;
+  const int len = sa.len, spin_limit = sa.spin_limit;
+  unsigned long long *__restrict__ state = sa.state;
+  int *__restrict__ out = sa.out;
+  const TileScan &ts = sa.ts;
   int v[IT], tl[IT], own[IT], halo;
   load_counts<IT>(in, len, blk, v, halo);
   const int nt = stage_counts<IT>(len, blk, ts, v, halo, tl, own, s_cnt, &s_case);
@@ -530,20 +561,36 @@ __global__ __launch_bounds__(kScanBlock) void k_scan(const int *__restrict__ in,
       ts.blk_tile0[blk] = pt;
     }
   }
-  if (threadIdx.x == 0) {
-    if (blk == 0) scal[nwall_idx] = 0;  // the reorder that follows counts the walls
-    if (blk == nb - 1) {
-      out[len] = pc + total;
-      scal[S_NTILES] = pt + tiles;
-    }
+  if (threadIdx.x == 0) sa.state_next[blk] = 0;
+  if (threadIdx.x == 0 && blk == nb - 1) {
+    out[len] = pc + total;
+    scal[S_NTILES] = pt + tiles;
   }
+}
+
+// the scan, with the wall pass (WALLS) in the last wall_groups workgroups, a
+// wavefront's share per wavefront
+template <int IT, int WALLS>
+__global__ __launch_bounds__(kScanBlock) void k_scan(ScanArgs sa, int *__restrict__ scal,
+                                                     unsigned long long *__restrict__ counters,
+                                                     int wall_groups, WallPass wp, Consts k0) {
+  const int nb = gridDim.x - (WALLS ? wall_groups : 0), blk = blockIdx.x;
+  if (WALLS && blk >= nb) {
+    constexpr int kWaves = kScanBlock / 64;
+    __shared__ __align__(16) double s_terms[kWaves * walls::kTerms];
+    const int wid = threadIdx.x >> 6, b = (blk - nb) * kWaves + wid;
+    if (b < wp.walls + wp.sweep)
+      wall_wave<WALLS ? WALLS : TSPH_WALL_MDBC>(b, wp, k0, sa.ts.cases, scal,
+                                                s_terms + wid * walls::kTerms);
+    return;
+  }
+  scan_block<IT>(sa, blk, nb, scal, counters);
 }
 
 // Placement without rows: arrival position of every particle (cell_start[cell]
 // + its arrival rank from the hash), whose cells k_order / k_order_tiles order
 // in place.  Also marks the reference positions of removed particles (the
-// trailing bucket) absent in the removal states, and clears k_scan's words for
-// the next build.  The first `cuts` workgroups (one wavefront per scan block)
+// trailing bucket) absent in the removal states.  The first `cuts` workgroups (one wavefront per scan block)
 // cut the new tile list into the chunks of the pooled pair pass that follows
 // from the scan's per-block sums (cut_chunks_scan), beside the placement.
 constexpr int kScatterBlock = 256;
@@ -565,14 +612,13 @@ __global__ __launch_bounds__(kScatterBlock) void k_scatter(
     const int *__restrict__ scal, const int *__restrict__ hcell, const int *__restrict__ hrank,
     const int *__restrict__ cell_start, int *__restrict__ arrival, int *__restrict__ cellof,
     int ncells_tot, const uint32_t *__restrict__ seq, uint8_t *__restrict__ seqstate,
-    unsigned long long *__restrict__ scan_state, ChunkCut cc) {
+    ChunkCut cc) {
   if ((int)blockIdx.x < cc.cuts) {
     cut_wave(cc, scal);
     return;
   }
   const int n = scal[S_NP], blk = blockIdx.x - cc.cuts;
   const int i = blk * kScatterBlock + threadIdx.x;
-  for (int b = i; b < cc.scan_blocks; b += (gridDim.x - cc.cuts) * kScatterBlock) scan_state[b] = 0;
   if (i >= n) return;
   const int c = hcell[i];
   if (c == ncells_tot) seqstate[seq[i]] = 0;
@@ -670,18 +716,16 @@ __global__ void k_order_tiles(const int *__restrict__ cell_start, const int *__r
   }
 }
 
-// slot of the particle with seq `mine` in cell c, in (cell, seq) order: the
-// cell's first slot plus the number of the cell's particles that precede it in
-// seq.  The row is read 16 entries at a time, all of them in flight together
-// (one round for all but the fullest cells); the chained ones cell by seq.
-__device__ __forceinline__ int ranked_slot(const int *__restrict__ cell_start, const CellRows &rw,
-                                           const int *__restrict__ hcell,
-                                           const uint32_t *__restrict__ seq, int n, int c,
-                                           uint32_t mine) {
-  const int s = cell_start[c], cnt = cell_start[c + 1] - s;
+// rank of the particle with seq `mine` in cell c (of cnt particles): the number
+// of the cell's particles that precede it in seq.  The row is read 16 entries
+// at a time, all of them in flight together (one round for all but the fullest
+// cells); the chained ones one by one.
+__device__ __forceinline__ int rank_in_cell(const CellRows &rw, const int *__restrict__ hcell,
+                                            const uint32_t *__restrict__ seq, int n, int c, int cnt,
+                                            uint32_t mine) {
   const uint4 *row = reinterpret_cast<const uint4 *>(rw.seq + (size_t)c * rw.width);
   const int in_row = min(cnt, rw.width);
-  int slot = s;
+  int rank = 0;
   for (int a = 0; a < in_row; a += 16) {
     uint4 q[4];
 #pragma unroll
@@ -690,18 +734,85 @@ __device__ __forceinline__ int ranked_slot(const int *__restrict__ cell_start, c
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const int o = a + 4 * u;
-      slot += (o < in_row && q[u].x < mine) + (o + 1 < in_row && q[u].y < mine) +
+      rank += (o < in_row && q[u].x < mine) + (o + 1 < in_row && q[u].y < mine) +
               (o + 2 < in_row && q[u].z < mine) + (o + 3 < in_row && q[u].w < mine);
     }
   }
   if (cnt > rw.width) {
     int y = rw.head[c & (kRowHeads - 1)];
     for (int left = n; y > 0 && left > 0; --left) {
-      slot += hcell[y - 1] == c && seq[y - 1] < mine;
+      rank += hcell[y - 1] == c && seq[y - 1] < mine;
       y = rw.link[y - 1];
     }
   }
-  return slot;
+  return rank;
+}
+
+// exclusive prefix of the bins (a multiple of kBinChunk of them) into pre, by
+// one workgroup; returns their sum
+__device__ __forceinline__ int scan_bins(const int *__restrict__ bin, int bins, int *pre) {
+  constexpr int kU = 4, kWaves = kScanBlock / 64;
+  __shared__ int tot[kU * kWaves];
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, chunks = bins / kBinChunk;
+  int carry = 0;
+  for (int c0 = 0; c0 < chunks; c0 += kU) {
+    int4 q[kU];
+    int inc[kU], off[kU];
+#pragma unroll
+    for (int u = 0; u < kU; ++u)
+      q[u] = c0 + u < chunks
+                 ? reinterpret_cast<const int4 *>(bin)[(c0 + u) * kScanBlock + threadIdx.x]
+                 : make_int4(0, 0, 0, 0);
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      if (c0 + u >= chunks) break;
+      q[u].y += q[u].x;
+      q[u].z += q[u].y;
+      q[u].w += q[u].z;
+      int x = q[u].w;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(x, o, 64);
+        if (lane >= o) x += y;
+      }
+      inc[u] = x;
+      if (lane == 63) tot[u * kWaves + wid] = x;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      if (c0 + u >= chunks) break;
+#pragma unroll
+      for (int w = 0; w < kWaves; ++w) {
+        if (w == wid) off[u] = carry;
+        carry += tot[u * kWaves + w];
+      }
+      const int ex = off[u] + inc[u] - q[u].w;
+      reinterpret_cast<int4 *>(pre)[(c0 + u) * kScanBlock + threadIdx.x] =
+          make_int4(ex, ex + q[u].x, ex + q[u].y, ex + q[u].z);
+    }
+    __syncthreads();
+  }
+  return carry;
+}
+
+// particles in the cells of c's bin before c; cnt: those in c
+__device__ __forceinline__ int bin_offset(const int *__restrict__ cell_count, int c, int &cnt) {
+  const int4 *q = reinterpret_cast<const int4 *>(cell_count) + c / kBinCells * (kBinCells / 4);
+  const int m = c % kBinCells;
+  int4 v[kBinCells / 4];
+#pragma unroll
+  for (int u = 0; u < kBinCells / 4; ++u) v[u] = q[u];
+  int s = 0;
+  cnt = 0;
+#pragma unroll
+  for (int u = 0; u < kBinCells; ++u) {
+    const int4 &w = v[u / 4];
+    const int x = u % 4 == 0 ? w.x : u % 4 == 1 ? w.y : u % 4 == 2 ? w.z : w.w;
+    s += u < m ? x : 0;
+    cnt = u == m ? x : cnt;
+  }
+  return s;
 }
 
 // Moves every field to its slot of the new order (the state after the build is
@@ -710,9 +821,12 @@ __device__ __forceinline__ int ranked_slot(const int *__restrict__ cell_start, c
 // dropped).  RANK: thread x moves input slot x to the slot that the hash's rows
 // give it (reads in a row, writes nearly so: few particles change cells in a
 // step), and does the placement's other work: the cell of each slot, the cell
-// counts and the scan's words cleared for the next build, removed particles
-// marked absent, the pooled pass's chunk cut (cc) in the first workgroups.
+// counts cleared for the next build, removed particles marked absent, the
+// pooled pass's chunk cut (cc) in the first workgroups.
 // Otherwise thread x fills slot x from where the placement says.
+// SCAN (with RANK): the scan runs in the first workgroups of the launch; the
+// others find their cells' offsets from the bins, which every workgroup scans
+// in LDS.
 // With EOS the pressure is recomputed as Density_to_pressure does
 // (src/SPH_pressure.h:65-89) and the FP32 records of the mixed path are
 // written, for the step sequences in which that stage follows the cell build.
@@ -725,16 +839,18 @@ __device__ __forceinline__ int ranked_slot(const int *__restrict__ cell_start, c
 // ad_skip (a type mask): a and drho of those types are not moved, for the step
 // sequences in which a pair pass that overwrites them for exactly those types
 // follows the build.
-template <bool EOS, bool PRED, bool RANK, bool NEXT>
-__global__ __launch_bounds__(kScatterBlock) void k_reorder(
-    const int *__restrict__ cell_start, int ncells, const int *__restrict__ hcell, CellRows rows,
-    int *__restrict__ perm, int *__restrict__ cell_count, uint8_t *__restrict__ seqstate,
-    unsigned long long *__restrict__ scan_state, ChunkCut cc, Soa src, Soa dst,
+template <bool EOS, bool PRED, bool RANK, bool NEXT, bool SCAN>
+__global__ __launch_bounds__(kScatterBlock, SCAN ? 1 : 6) void k_reorder(
+    const int *__restrict__ cell_start, int ncells, int n_ub, const int *__restrict__ hcell,
+    CellRows rows, const int *__restrict__ bin, int nbins, Clear cl, ScanArgs sa,
+    int *__restrict__ perm,
+    int *__restrict__ cell_count, uint8_t *__restrict__ seqstate, ChunkCut cc, Soa src, Soa dst,
     int *__restrict__ scal, int *__restrict__ wall_list, int *__restrict__ cellof, Consts k0,
     const Consts *__restrict__ cases, Mixed mx, double dt0, unsigned ad_skip,
-    unsigned long long *__restrict__ counters, int nwall_idx, bool move_olds,
-    int *__restrict__ next_count, int *__restrict__ next_hcell, int *__restrict__ next_hrank,
-    CellRows next_rows) {
+    unsigned long long *__restrict__ counters, int nwall_idx, int nwall_next, bool move_olds,
+    int *__restrict__ next_count, int *__restrict__ next_bin, int *__restrict__ next_hcell,
+    int *__restrict__ next_hrank, CellRows next_rows) {
+  extern __shared__ __align__(16) int s_pre[];  // SCAN: the bins' offsets
   int blk = blockIdx.x;
   if (RANK) {
     if (blk < cc.cuts) {
@@ -743,123 +859,177 @@ __global__ __launch_bounds__(kScatterBlock) void k_reorder(
     }
     blk -= cc.cuts;
   }
-  const int n_new = cell_start[ncells];
-  const int n = RANK ? cell_start[ncells + 1] : n_new;  // RANK: with the removed ones
+  if (SCAN) {
+    if (blk < cc.scan_blocks) {
+      scan_block<4>(sa, blk, cc.scan_blocks, scal, counters);
+      return;
+    }
+    blk -= cc.scan_blocks;
+  }
+  // Every load before the first store (loads and stores complete in order, so
+  // a load behind a store would wait for the store's acknowledgement too), and
+  // those of the particle's fields beside those that find its slot.
   const int x = blk * kScatterBlock + threadIdx.x;
-  if (blk == 0 && threadIdx.x == 0) {
-    scal[S_NP] = n_new;
-    if (RANK) cell_count[ncells] = 0;  // the removed bucket
-  }
-  if (RANK)
-    for (int b = x; b < cc.scan_blocks; b += (gridDim.x - cc.cuts) * kScatterBlock)
-      scan_state[b] = 0;
-  int wall = 0, k = x, next_c = -1;
-  unsigned bad = 0;
-  bool live = x < n;
-  int cell = 0;
-  if (RANK && live) {
-    cell = hcell[x];
-    if (cell == ncells) {
-      seqstate[src.seq[x]] = 0;
-      live = false;
-    }
-  }
-  if (live) {
-    const int j = RANK ? x : perm[x];
+  int cell = 0, j = x;
+  uint32_t mine = 0;
+  uint8_t t = kRemoved;
+  bool move_ad = false;
+  double2 r = {}, v = {}, a = {}, r_o = {}, v_o = {}, gnr = {}, nv = {};
+  double rho = 0., drho = 0., rho_o = 0., p = 0.;
+  int index = 0, cid = 0;
+  if (x < n_ub) {
     if (RANK) {
-      k = ranked_slot(cell_start, rows, hcell, src.seq, n, cell, src.seq[x]);
-      cell_count[cell] = 0;
-      perm[k] = j;
-      cellof[k] = cell;
-    } else if (EOS && mx.rv) {
-      cell = cellof[x];
+      cell = hcell[x];
+    } else {
+      j = min((unsigned)perm[x], (unsigned)(n_ub - 1));  // (slots past the last hold any value)
+      if (EOS && mx.rv) cell = cellof[x];
     }
-    const uint8_t t = src.type[j];
-    wall = t == TSPH_WALL;
-    double2 r = src.r[j], v = src.v[j];
-    const bool move_ad = !((ad_skip >> t) & 1u);
-    double2 a = make_double2(0., 0.);
-    double drho = 0.;
-    if (PRED || move_ad) {
+    mine = src.seq[j];
+    t = src.type[j];
+    r = src.r[j];
+    v = src.v[j];
+    rho = src.rho[j];
+    index = src.index[j];
+    if (src.cid) cid = src.cid[j];
+    if (PRED) {
+      a = src.a[j];
+      drho = src.drho[j];
+    } else if (move_olds) {
+      r_o = src.r_o[j];
+      v_o = src.v_o[j];
+      rho_o = src.rho_o[j];
+    }
+    if (src.gnr) gnr = src.gnr[j];
+    if (src.n) nv = src.n[j];
+  }
+  int n_new, n;  // RANK: n with the removed ones
+  if (SCAN) {
+    n = scan_bins(bin, nbins, s_pre);
+    n_new = n - cell_count[ncells];
+  } else {
+    n_new = cell_start[ncells];
+    n = RANK ? cell_start[ncells + 1] : n_new;
+  }
+  bool live = x < n, gone = false;
+  if (RANK) {
+    gone = live && cell == ncells;
+    live = live && !gone;
+  }
+  int k = x, next_c = -1;
+  unsigned bad = 0;
+  Consts kc = k0;
+  if (live) {
+    if (RANK) {
+      int cnt;
+      if (SCAN) {
+        k = s_pre[cell / kBinCells] + bin_offset(cell_count, cell, cnt);
+      } else {
+        k = cell_start[cell];
+        cnt = cell_start[cell + 1] - k;
+      }
+      k += rank_in_cell(rows, hcell, src.seq, n, cell, cnt, mine);
+    }
+    if (cases && (EOS || PRED)) kc = cases[cid];
+    move_ad = !((ad_skip >> t) & 1u);
+    if (!PRED && move_ad) {
       a = src.a[j];
       drho = src.drho[j];
     }
-    double rho = src.rho[j];
-    const Consts kc = EOS || PRED ? case_consts(k0, cases, src.cid, j) : k0;
-    if (src.cid) dst.cid[k] = src.cid[j];
+    // with the EOS the old pressure is read only where it is kept
+    if (!EOS || t == TSPH_OUTLET || t == TSPH_INLET) p = src.p[j];
+    if (src.omega) {
+      const double w0 = src.omega[j], w1 = src.omegarho[j], w2 = src.omega_o[j],
+                   w3 = src.omegarho_o[j], w4 = src.domega[j], w5 = src.domegarho[j];
+      const double2 u0 = src.omegav[j], u1 = src.omegav_o[j], u2 = src.domegav[j];
+      dst.omega[k] = w0;
+      dst.omegarho[k] = w1;
+      dst.omega_o[k] = w2;
+      dst.omegarho_o[k] = w3;
+      dst.domega[k] = w4;
+      dst.domegarho[k] = w5;
+      dst.omegav[k] = u0;
+      dst.omegav_o[k] = u1;
+      dst.domegav[k] = u2;
+      if (src.gradrho) {
+        const double2 g0 = src.gradrho[j], g1 = src.gradvx[j], g2 = src.gradvy[j];
+        dst.gradrho[k] = g0;
+        dst.gradvx[k] = g1;
+        dst.gradvy[k] = g2;
+      }
+    }
+    if (src.v_oo) {
+      const double2 u0 = src.v_oo[j];
+      const double w0 = src.rho_oo[j], w1 = src.rho_tmp[j];
+      dst.v_oo[k] = u0;
+      dst.rho_oo[k] = w0;
+      dst.rho_tmp[k] = w1;
+    }
+    if (src.rc) {
+      const double2 u0 = src.rc[j];
+      const double w0 = src.rhoc[j];
+      dst.rc[k] = u0;
+      dst.rhoc[k] = w0;
+    }
     if (PRED) {
-      const double dt = cases ? kc.dt : dt0;
-      dst.r_o[k] = r;
-      dst.v_o[k] = v;
-      dst.rho_o[k] = rho;
-      predict(r, v, rho, a, drho, dt);
-    } else if (move_olds) {
-      dst.r_o[k] = src.r_o[j];
-      dst.v_o[k] = src.v_o[j];
-      dst.rho_o[k] = src.rho_o[j];
+      r_o = r;
+      v_o = v;
+      rho_o = rho;
+      predict(r, v, rho, a, drho, cases ? kc.dt : dt0);
+    }
+    if (NEXT) next_c = hash_cell(kc, predicted_r(r, v, cases ? kc.dt : dt0), counters);
+    if (EOS && t != TSPH_OUTLET && t != TSPH_INLET) {
+      bad = rho > 1500. || rho < 0.;
+      p = tait64(rho, kc.rho0, kc.cs);
+    }
+  }
+  const bool wall = live && t == TSPH_WALL;
+  auto store = [&] {
+    if (PRED || move_olds) {
+      dst.r_o[k] = r_o;
+      dst.v_o[k] = v_o;
+      dst.rho_o[k] = rho_o;
     }
     dst.r[k] = r;
     dst.v[k] = v;
-    if (NEXT) next_c = hash_cell(kc, predicted_r(r, v, cases ? kc.dt : dt0), counters);
     if (move_ad) {
       dst.a[k] = a;
       dst.drho[k] = drho;
     }
     dst.rho[k] = rho;
-    dst.type[k] = t;
-    dst.seq[k] = src.seq[j];
-    dst.index[k] = src.index[j];
-    // with the EOS the old pressure is read only where it is kept
-    double p;
-    if (EOS && t != TSPH_OUTLET && t != TSPH_INLET) {
-      bad = rho > 1500. || rho < 0.;
-      p = tait64(rho, kc.rho0, kc.cs);
-    } else {
-      p = src.p[j];
-    }
     dst.p[k] = p;
-    if (src.gnr) dst.gnr[k] = src.gnr[j];
-    double2 nv = make_double2(0., 0.);
-    if (src.n) {
-      nv = src.n[j];
-      dst.n[k] = nv;
-    }
+    dst.type[k] = t;
+    dst.seq[k] = mine;
+    dst.index[k] = index;
+    if (src.cid) dst.cid[k] = cid;
+    if (src.gnr) dst.gnr[k] = gnr;
+    if (src.n) dst.n[k] = nv;
     if (EOS && mx.rv)
       write_mixed_record(mx, kc, cell - kc.cell_base, k, r, v, rho, p, src.n != nullptr, nv);
-    if (src.omega) {
-      dst.omega[k] = src.omega[j];
-      dst.omegarho[k] = src.omegarho[j];
-      dst.omegav[k] = src.omegav[j];
-      dst.omega_o[k] = src.omega_o[j];
-      dst.omegarho_o[k] = src.omegarho_o[j];
-      dst.omegav_o[k] = src.omegav_o[j];
-      dst.domega[k] = src.domega[j];
-      dst.domegarho[k] = src.domegarho[j];
-      dst.domegav[k] = src.domegav[j];
-      if (src.gradrho) {
-        dst.gradrho[k] = src.gradrho[j];
-        dst.gradvx[k] = src.gradvx[j];
-        dst.gradvy[k] = src.gradvy[j];
-      }
+    if (RANK) {
+      perm[k] = j;
+      cellof[k] = cell;
+      if (!SCAN && !bin) cell_count[cell] = 0;
     }
-    if (src.v_oo) {
-      dst.v_oo[k] = src.v_oo[j];
-      dst.rho_oo[k] = src.rho_oo[j];
-      dst.rho_tmp[k] = src.rho_tmp[j];
-    }
-    if (src.rc) {
-      dst.rc[k] = src.rc[j];
-      dst.rhoc[k] = src.rhoc[j];
-    }
-  }
+  };
   if (NEXT) {
-    const int rank = count_cell(live, next_c, next_count);
+    const CellCount cn(live, next_c, next_count, next_bin);
+    if (live) store();
+    const int rank = cn.rank();
     if (live) {
       next_hcell[k] = next_c;
-      if (RANK) put_row(next_rows, next_c, rank, k, src.seq[x]);
+      if (RANK) put_row(next_rows, next_c, rank, k, mine);
       else next_hrank[k] = rank;
     }
+  } else if (live) {
+    store();
   }
+  if (gone) seqstate[mine] = 0;
+  if (blk == 0 && threadIdx.x == 0) {
+    scal[S_NP] = n_new;
+    scal[nwall_next] = 0;
+    if (RANK && !bin) cell_count[ncells] = 0;  // the removed bucket
+  }
+  clear_next(cl, x, (gridDim.x - (blockIdx.x - blk)) * kScatterBlock);
   const unsigned long long m = __ballot(wall);
   if (m) {
     const int lane = threadIdx.x & 63;
@@ -894,26 +1064,30 @@ __global__ void k_gather_olds(const int *__restrict__ scal, const int *__restric
 // 4788 / 4776 (within the runs' spread).
 bool cells_ranked(const tsph_ctx *c) { return c->row_width > 0 && c->cell_order != 2; }
 
-// exclusive scan of the cell counts into cell_start, with the tile list of the
-// current tile_rows (and, for cost_table >= 0, the listed tiles' costs); with
-// walls (TSPH_WALL_*; 0: none) the wall pass wp beside it
-int scan_cells(tsph_ctx *c, hipStream_t s, const int *count, int *cs, int nwall_idx, int cost_table,
-               int walls, const WallPass &wp) {
-  const int len = c->ncells_tot + 1;
+// the arguments of the scan of the cell counts into cs, with the tile list of
+// the current tile_rows (and, for cost_table >= 0, the listed tiles' costs)
+ScanArgs scan_args(tsph_ctx *c, int *cs, int cost_table) {
   const TileScan ts{c->k.ncy, c->k.ncells, c->k.cell_base, c->cases, c->tile_base, c->ncases,
                     c->tile_rows, c->tile_list,
                     cost_table >= 0 ? c->scal + S_NSCAL + cost_table : nullptr,
                     cost_table >= 0 ? c->list_cost : nullptr,
                     cost_estimate(c->prm.precision == TSPH_PREC_MIXED), c->scan_cost,
                     c->scan_tile0};
+  c->list_groups = 0;  // a pooled pass cuts the new list
+  c->list_cost_table = cost_table;
+  return {c->cell_count, c->ncells_tot + 1, c->scan_state, c->scan_state_next, cs, ts, c->scan_wait};
+}
+
+// the scan in a launch of its own, with walls (TSPH_WALL_*; 0: none) the wall
+// pass wp beside it
+int launch_scan(tsph_ctx *c, const ScanArgs &sa, int walls, const WallPass &wp) {
   const int wg = walls ? grid_for(wp.walls + wp.sweep, kScanBlock / 64) : 0;
-#define TSPH_SCAN(IT, W)                                                                       \
-  hipLaunchKernelGGL((k_scan<IT, W>), dim3(scan_blocks(c) + wg), dim3(kScanBlock), 0, s, count, len, \
-                     c->scan_state, cs, c->scal, c->counters, ts, c->scan_wait, nwall_idx, wg, wp, \
-                     c->k, c->row_width ? c->row_head_next : nullptr)
-#define TSPH_SCAN_W(IT)                                                                        \
-  if (walls == TSPH_WALL_MDBC) TSPH_SCAN(IT, TSPH_WALL_MDBC);                                 \
-  else if (walls == TSPH_WALL_BT) TSPH_SCAN(IT, TSPH_WALL_BT);                                \
+#define TSPH_SCAN(IT, W)                                                                        \
+  hipLaunchKernelGGL((k_scan<IT, W>), dim3(scan_blocks(c) + wg), dim3(kScanBlock), 0, c->stream, \
+                     sa, c->scal, c->counters, wg, wp, c->k)
+#define TSPH_SCAN_W(IT)                                                                         \
+  if (walls == TSPH_WALL_MDBC) TSPH_SCAN(IT, TSPH_WALL_MDBC);                                  \
+  else if (walls == TSPH_WALL_BT) TSPH_SCAN(IT, TSPH_WALL_BT);                                 \
   else TSPH_SCAN(IT, 0)
   if (scan_items(c) == 4) {
     TSPH_SCAN_W(4);
@@ -923,8 +1097,6 @@ int scan_cells(tsph_ctx *c, hipStream_t s, const int *count, int *cs, int nwall_
 #undef TSPH_SCAN_W
 #undef TSPH_SCAN
   TSPH_HIP(hipGetLastError());
-  c->list_groups = 0;  // a pooled pass cuts the new list
-  c->list_cost_table = cost_table;
   return 0;
 }
 
@@ -934,6 +1106,8 @@ void flip_build(tsph_ctx *c) {
   std::swap(c->cur, c->alt);
   std::swap(c->cell_start, c->cell_start_next);
   std::swap(c->cell_count, c->cell_count_next);
+  std::swap(c->bin_count, c->bin_count_next);
+  std::swap(c->scan_state, c->scan_state_next);
   std::swap(c->hcell, c->hcell_next);
   std::swap(c->hrank, c->hrank_next);
   std::swap(c->row_seq, c->row_seq_next);
@@ -981,13 +1155,23 @@ int launch_cell_list(tsph_ctx *c, bool eos, bool predict, double dt, unsigned ad
   // launches and a hash), or by passes of its own
   const bool rank = cells_ranked(c);
   const CellRows rw{c->row_seq, c->row_head, rank ? c->hrank : nullptr, rank ? c->row_width : 0};
+  // (without bins a build's reorder clears the counts it has used)
+  const bool binned = c->bin_count != nullptr;
+  const Clear clear{{c->cell_count_next, c->bin_count_next, c->row_head_next},
+                    {binned ? count_words(c) / 4 : 0, binned ? bin_words(c) / 4 : 0,
+                     c->row_width ? kRowHeads / 4 : 0}};
+  if (hashed && hash_next) {
+    set_error("cell list: a build whose hash was taken takes no next hash");
+    return TSPH_ESTATE;
+  }
   const CellRows rw_next{c->row_seq_next, c->row_head_next, rank ? c->hrank_next : nullptr,
                          rank ? c->row_width : 0};
   if (!hashed) {
 #define TSPH_HASH(P, D, W)                                                                     \
   hipLaunchKernelGGL((k_hash<P, D, W>), dim3(hg), dim3(hbs), 0, s, c->cur.r, c->cur.v,            \
                      c->cur.type, c->cur.seq, c->scal, k, c->cases, c->cur.cid, dt, nct,          \
-                     c->cell_count, c->hcell, c->hrank, rw, c->seqstate, c->counters, wp)
+                     c->cell_count, c->hcell, c->hrank, rw, c->bin_count, clear, c->seqstate,   \
+                     c->counters, wp)
 #define TSPH_HASH_W(P, D)                                                                      \
   if (walls == TSPH_WALL_MDBC) TSPH_HASH(P, D, TSPH_WALL_MDBC);                               \
   else if (walls == TSPH_WALL_BT) TSPH_HASH(P, D, TSPH_WALL_BT);                              \
@@ -1013,8 +1197,10 @@ int launch_cell_list(tsph_ctx *c, bool eos, bool predict, double dt, unsigned ad
     set_error("tile list: more pooled workgroups than allocated");
     return TSPH_ESTATE;
   }
-  if (int e = scan_cells(c, s, c->cell_count, cs, wslot, cut > 0 ? c->cut_table : -1, hashed ? walls : 0, wp))
-    return e;
+  const ScanArgs sa = scan_args(c, cs, cut > 0 ? c->cut_table : -1);
+  const bool own_scan = !(rank && binned) || cut > 0 || (hashed && walls);
+  if (own_scan)
+    if (int e = launch_scan(c, sa, hashed ? walls : 0, wp)) return e;
   const int sg = grid_for(c->n_ub, kScatterBlock);
   // one cutting wavefront per scan block, in the first workgroups
   const int cuts = cut > 0 ? grid_for(scan_blocks(c), kScatterBlock / 64) : 0;
@@ -1026,8 +1212,7 @@ int launch_cell_list(tsph_ctx *c, bool eos, bool predict, double dt, unsigned ad
   }
   if (!rank) {
     hipLaunchKernelGGL(k_scatter, dim3(cuts + sg), dim3(kScatterBlock), 0, s, c->scal, c->hcell,
-                       c->hrank, cs, c->perm, c->cellof, nct, c->cur.seq, c->seqstate,
-                       c->scan_state, cc);
+                       c->hrank, cs, c->perm, c->cellof, nct, c->cur.seq, c->seqstate, cc);
     if (c->cases)
       hipLaunchKernelGGL(k_order, dim3(grid_for(nct + 1, nb)), dim3(nb), 0, s, cs, nct, c->cur.seq,
                          c->perm, c->cell_count);
@@ -1037,27 +1222,29 @@ int launch_cell_list(tsph_ctx *c, bool eos, bool predict, double dt, unsigned ad
                          c->cell_count);
   }
   const Mixed mx = c->prm.precision == TSPH_PREC_MIXED ? c->mx : Mixed{};
-#define TSPH_REORDER(E, P, R, N)                                                              \
-  hipLaunchKernelGGL((k_reorder<E, P, R, N>), dim3(R ? cuts + sg : sg), dim3(kScatterBlock), 0, s,  \
-                     cs, nct, c->hcell, rw, c->perm, c->cell_count, c->seqstate, c->scan_state, cc, \
-                     c->cur, c->alt, c->scal, c->wall_list, c->cellof, k, c->cases, mx, dt,        \
-                     ad_skip, c->counters, wslot, !skip_olds, c->cell_count_next, c->hcell_next,    \
-                     c->hrank_next, rw_next)
-#define TSPH_REORDER_R(E, P)                                                                  \
-  if (rank) TSPH_REORDER(E, P, true, false);                                                  \
-  else TSPH_REORDER(E, P, false, false)
+  const Clear cl = hashed ? clear : Clear{};
+#define TSPH_REORDER(E, P, R, N, S)                                                           \
+  hipLaunchKernelGGL((k_reorder<E, P, R, N, S>),                                              \
+                     dim3((R ? cuts : 0) + (S ? cc.scan_blocks : 0) + sg), dim3(kScatterBlock),    \
+                     S ? sizeof(int) * bin_words(c) : 0, s, cs, nct, c->n_ub, c->hcell, rw,         \
+                     c->bin_count, bin_words(c), cl, sa, c->perm, c->cell_count, c->seqstate, cc, c->cur, c->alt,     \
+                     c->scal, c->wall_list, c->cellof, k, c->cases, mx, dt, ad_skip, c->counters,   \
+                     wslot, c->nwall_idx, !skip_olds, c->cell_count_next, c->bin_count_next,        \
+                     c->hcell_next, c->hrank_next, rw_next)
+#define TSPH_REORDER_R(E, P, N)                                                               \
+  if (!rank) TSPH_REORDER(E, P, false, N, false);                                             \
+  else if (own_scan) TSPH_REORDER(E, P, true, N, false);                                      \
+  else TSPH_REORDER(E, P, true, N, true)
   if (hash_next) {
-    if (rank) TSPH_REORDER(true, false, true, true);
-    else TSPH_REORDER(true, false, false, true);
-  } else
-  if (eos && predict) {
-    TSPH_REORDER_R(true, true);
+    TSPH_REORDER_R(true, false, true);
+  } else if (eos && predict) {
+    TSPH_REORDER_R(true, true, false);
   } else if (eos) {
-    TSPH_REORDER_R(true, false);
+    TSPH_REORDER_R(true, false, false);
   } else if (predict) {
-    TSPH_REORDER_R(false, true);
+    TSPH_REORDER_R(false, true, false);
   } else {
-    TSPH_REORDER_R(false, false);
+    TSPH_REORDER_R(false, false, false);
   }
 #undef TSPH_REORDER_R
 #undef TSPH_REORDER
