@@ -160,7 +160,8 @@ int tsph_interpolate_point(tsph_ctx *ctx, double x, double y, double *out4);
 int tsph_get_counters(tsph_ctx *ctx, tsph_counters *out);
 int tsph_reset_counters(tsph_ctx *ctx);
 /* Pair-loop tile: one wavefront handles `rows` consecutive cells of a grid
- * column (1..24, default 7). */
+ * column (1..24; default 7, or 6 in FP64 for systems with fewer than 150
+ * particles per persistent wave, from the upload on). */
 int tsph_set_tile_rows(tsph_ctx *ctx, int rows);
 int tsph_get_tile_rows(tsph_ctx *ctx, int *rows);
 /* Pair-loop waves launched per compute unit (1..32; default 12 on the mixed
@@ -424,7 +425,7 @@ int tsph_autotune(tsph_ctx *ctx, int variant, int *tile_rows, int *waves_per_cu,
  * list of about equal cost, cut by the time each tile took in the previous
  * pass, whose tiles its wavefronts take from a counter in LDS, the costliest
  * first), 0 = static striding, one wavefront per workgroup.  Systems
- * with fewer than 80 (mixed) or 200 (FP64) particles per persistent wave, and
+ * with fewer than 80 (mixed) or 150 (FP64) particles per persistent wave, and
  * the ALE passes, always stride; FP64 passes over at most 70,000 particles go
  * by cells instead of tiles and do not depend on the setting.
  * Results do not depend on it.  No counterpart in the reference. */

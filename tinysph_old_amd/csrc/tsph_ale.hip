@@ -258,17 +258,16 @@ __device__ __forceinline__ void rale_pair32(const CA32 &c, AccA32 &s, float drx,
   s.gamma += W * c.m * __builtin_amdgcn_rcpf(nrho);
 }
 
-template <bool DYN>
 __global__ __launch_bounds__(kWave * kPoolWaves) void k_rale32(Soa d, const int *__restrict__ cell_start,
                                                   const int *__restrict__ cellof, Consts k, int rows,
                                                   int *__restrict__ scal,
                                                   const int *__restrict__ tile_list, int cap,
-                                                  const int *__restrict__ bound, int lds_wave,
+                                                  int lds_wave,
                                                   uint8_t *__restrict__ gflag,
                                                   unsigned long long *__restrict__ counters) {
 #pragma clang fp contract(fast)
   extern __shared__ __align__(16) unsigned char smem[];
-  unsigned char *wl = wave_lds<DYN>(smem, lds_wave);
+  unsigned char *wl = wave_lds<false>(smem, lds_wave);
   int *tab = reinterpret_cast<int *>(wl);
   float2 *s_pos = reinterpret_cast<float2 *>(wl + kTabBytes);
   float2 *s_vel = s_pos + cap;
@@ -284,13 +283,13 @@ __global__ __launch_bounds__(kWave * kPoolWaves) void k_rale32(Soa d, const int 
 
   if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&counters[C_PASSES], 1ull);
   unsigned npair = 0, ncand = 0, nact = 0;
-  TileQueue tq = tq_begin<DYN>(scal, bound, tile_list, smem);
-  for (int it = tq_take<DYN>(tq, tq_ticket<DYN>(tq)); it >= 0;) {
+  TileQueue tq = tq_begin<false>(scal, nullptr, tile_list, smem);
+  for (int it = tq_take<false>(tq, 0); it >= 0;) {
     wave_sync();
-    const int ticket = tq_ticket<DYN>(tq);  // read once this tile's loads are waited for
+    const int entry = tile_list[it];
     Tile t;
-    tile_begin(k, cell_start, tile_list[it], rows, tab, t);
-    tq_mark(tq, tile_list[it]);
+    tile_begin(k, cell_start, entry_tile(entry), rows, tab, t);
+    entry_part(entry, t);
     const bool staged = t.lq[3] <= cap;
     const int mid = t.row_lo + (t.nrows >> 1);
     const double ox = k.x0 - k.of + t.cx * k.kh, oy = k.y0 - k.of + mid * k.kh;
@@ -306,7 +305,7 @@ __global__ __launch_bounds__(kWave * kPoolWaves) void k_rale32(Soa d, const int 
       }
     }
     wave_sync();
-    const int next = tq_take<DYN>(tq, ticket);
+    const int next = tq_take<false>(tq, 0);
     const int lane = tile_lane();
     uint16_t *my_list = s_list + lane;
     for (int i0 = t.own0; i0 < t.own1; i0 += kWave) {
@@ -387,7 +386,6 @@ __global__ __launch_bounds__(kWave * kPoolWaves) void k_rale32(Soa d, const int 
     }
     it = next;
   }
-  tq_mark(tq, -1);
   wave_count(npair, ncand, nact, counters);
 }
 
@@ -511,9 +509,9 @@ int launch_rale_forces(tsph_ctx *c) {
         tile_grid(c, true, kTabBytes + list + (size_t)cap * (4 * sizeof(float2) + 1), false);
     if ((e = ensure_tile_list(c, 0))) return e;
     e = launch_timed(c, [&] {
-      hipLaunchKernelGGL(k_rale32<false>, tg.grid, tg.block, tg.lds, s, c->cur, c->cell_start,
-                           c->cellof, k, rows, c->scal, c->tile_list, cap, c->tile_bound,
-                           tg.lds_wave, c->ale_flag, c->counters);
+      hipLaunchKernelGGL(k_rale32, tg.grid, tg.block, tg.lds, s, c->cur, c->cell_start,
+                           c->cellof, k, rows, c->scal, c->tile_list, cap, tg.lds_wave,
+                            c->ale_flag, c->counters);
     });
   } else {
     constexpr int lds = cell_lds_bytes<RaleCell64>();

@@ -764,15 +764,14 @@ __global__ __launch_bounds__(P::kWaves * kWave, 2) void k_ale_cells64(
   cells64(pol, g, cell_start, nullptr, 1, src, counters);
 }
 
-template <class P, bool DYN>
+template <class P>
 __global__ __launch_bounds__(kWave * kPoolWaves) void k_ale_pass32(P pol, const int *__restrict__ cell_start,
                                                       const int *__restrict__ cellof, int rows,
                                                       int *__restrict__ scal,
                                                       const int *__restrict__ tile_list,
-                                                      const int *__restrict__ bound, int cap,
-                                                      int lds_wave,
+                                                      int cap, int lds_wave,
                                                       unsigned long long *__restrict__ counters) {
-  walk32<DYN>(pol, pol.k, cell_start, cellof, rows, scal, tile_list, bound, cap, lds_wave, counters);
+  walk32(pol, pol.k, cell_start, cellof, rows, scal, tile_list, cap, lds_wave, counters);
 }
 
 // Integrate_density_compute_pressure, src/ALESPH_integration.h:86-135 (fluid
@@ -830,25 +829,34 @@ __global__ void k_ale_lf2(Soa d, const int *__restrict__ scal, double dt, int fi
 template <class P, int SLOT>
 int launch_pass32(tsph_ctx *c, const P &pol) {
   const int rows = c->tile_rows;
-  // slots budgeted per tile, within 64 KiB of LDS per wavefront; a tile whose
-  // neighbourhood does not fit is gathered from global memory instead.  The
-  // ALE records are large (57 B with the MUSCL gradients), so the budget is
-  // kAleCellCap records per cell, about a full cell's count at the configured
-  // resolutions: the fullest tiles then take the global path, and the smaller
-  // LDS area lets a compute unit hold more waves, which pays more than staging
-  // every tile does
-  constexpr int kAleCellCap = 9;
+  // Slots per tile.  The ALE records are large (57 B with the MUSCL
+  // gradients) and the waves that a compute unit holds pay, so systems that
+  // fill the chip are budgeted kAleCellCap records per cell, which the fullest
+  // tiles of a running dam break just need: us per step with 9 and 10 records,
+  // at the start and after some thousand steps, 727k particles 770 and 807, 841
+  // and 811; 183k 236 and 238, 284 and 247 (a tile beyond the budget is taken
+  // in two runs; gathered from global memory instead, 183k took 467).  What
+  // those waves leave over, and all that fewer waves leave over in a system
+  // without a tile for each of them, goes to the tiles, up to kCellCap records
+  // per cell (47k particles after 1300 steps: 135, 357 with 9 records).
+  constexpr int kAleCellCap = 10;
   constexpr int kFixed = kTabBytes + sizeof(uint16_t) * kList * kWave;
-  const int cap = std::min(3 * (rows + 2) * kAleCellCap, (65536 - kPoolHdr - kFixed) / SLOT);
+  const int most = std::min(3 * (rows + 2) * kCellCap, (65536 - kPoolHdr - kFixed) / SLOT);
+  const int base = std::min(3 * (rows + 2) * kAleCellCap, most);
+  const int lds = kStaticHdr + kFixed + 32;  // (with the rounding to allocation granules below)
+  const int fit = std::max(1, c->lds_cu / (lds + base * SLOT));
+  const int want = std::max(1, grid_for(c->n_ub, 48 * c->num_cu));
+  const int share = c->lds_cu / std::min(fit, want) / kLdsGranule * kLdsGranule;
+  const int cap = std::max(base, std::min(most, (share - lds) / SLOT));
   // the static walk: a cell build serves several passes of different cost
   // profiles, and the dam breaks these passes run on give each wave about ten
   // tiles, too few for the pooled walk to pay for its chunk cut
   const TileGrid tg = tile_grid(c, true, kFixed + (size_t)cap * SLOT, false);
   if (int e = ensure_tile_list(c, 0)) return e;
   return launch_timed(c, [&] {
-    hipLaunchKernelGGL((k_ale_pass32<P, false>), tg.grid, tg.block, tg.lds, c->stream, pol,
-                       c->cell_start, c->cellof, rows, c->scal, c->tile_list, c->tile_bound, cap,
-                       tg.lds_wave, c->counters);
+    hipLaunchKernelGGL(k_ale_pass32<P>, tg.grid, tg.block, tg.lds, c->stream, pol,
+                       c->cell_start, c->cellof, rows, c->scal, c->tile_list, cap, tg.lds_wave,
+                        c->counters);
   });
 }
 

@@ -397,7 +397,7 @@ static int alloc_context(tsph_ctx *c) {
       (e = dalloc(&c->perm, cap)) ||
       (e = dalloc(&c->seqstate, (size_t)c->seq_cap)) || (e = dalloc(&c->probe_out, 4)) ||
       (e = dalloc(&c->bz_list, 2 * kBzMax)) ||
-      (e = dalloc(&c->tile_list, nct + 8)) || (e = dalloc(&c->list_cost, nct + 8)) ||
+      (e = dalloc(&c->tile_list, 2 * ((size_t)nct + 8))) || (e = dalloc(&c->list_cost, nct + 8)) ||
       (e = dalloc(&c->wall_list, cap)) ||
       (e = dalloc(&c->scan_state, (nct + 1) / 1024 + 2)) ||
       (e = dalloc(&c->scan_state_next, (nct + 1) / 1024 + 2)) ||
@@ -483,6 +483,23 @@ static int update_tile_base(tsph_ctx *c) {
   return 0;
 }
 
+static int change_tile_rows(tsph_ctx *c, int rows) {
+  if (rows != c->tile_rows) {
+    drop_graph(c);
+    c->tiles_valid = false;
+    c->tile_rows = rows;
+    if (int e = clear_tile_costs(c)) return e;  // costs of the old tile layout
+  }
+  return update_tile_base(c);
+}
+
+// the tile rows of a context that has chosen none, for its particle count
+static int default_tile_rows(tsph_ctx *c) {
+  if (c->rows_set || c->prm.precision != TSPH_PREC_FP64) return 0;
+  const long long pool = (long long)kPoolFp64 * c->num_cu * c->waves_per_cu;
+  return change_tile_rows(c, c->n_ub < pool ? kTileRowsFp64 : kTileRows);
+}
+
 }  // namespace tsph
 
 extern "C" {
@@ -495,7 +512,7 @@ int tsph_create(const tsph_params *prm, tsph_ctx **out) {
   tsph_ctx *c = new tsph_ctx();
   c->prm = *prm;
   c->capacity = prm->capacity;
-  c->tile_rows = 7;
+  c->tile_rows = kTileRows;
   set_walk_defaults(c);
   c->k = k;
   c->ncells_tot = k.ncells;
@@ -613,6 +630,7 @@ static int upload_impl(tsph_ctx *c, const tsph_particles *h, const uint32_t *seq
   TSPH_HIP(hipMemsetAsync(c->seqstate, 0, (size_t)c->seq_cap, c->stream));
   TSPH_HIP(hipStreamSynchronize(c->stream));
   c->n_ub = n;
+  if (int e = default_tile_rows(c)) return e;
   c->n_wall = 0;
   for (int i = 0; i < n; ++i) c->n_wall += t[i] == TSPH_WALL;
   c->olds_stale = false;
@@ -1082,7 +1100,10 @@ int tsph_step_inflow(tsph_ctx *c, int wall, double dt, int nsteps, int inlet, in
   if (!c->cells_valid) return fail(TSPH_ESTATE, "no cell list: call tsph_particle_to_cell first");
   if (wall == TSPH_WALL_MDBC && !c->has_gnr) return fail(TSPH_ESTATE, "mDBC needs ghost nodes (gnr)");
   if (wall == TSPH_WALL_BT && !c->has_n) return fail(TSPH_ESTATE, "BT needs wall normals (n)");
-  if (inlet >= 0) c->n_ub = c->capacity;
+  if (inlet >= 0) {
+    c->n_ub = c->capacity;
+    if (int e = default_tile_rows(c)) return e;
+  }
   // one inlet pass per step: replay in runs that cannot exhaust the reference
   // positions, relabelling them in between when needed
   for (int done = 0; done < nsteps;) {
@@ -1155,13 +1176,8 @@ int tsph_reset_counters(tsph_ctx *c) {
 int tsph_set_tile_rows(tsph_ctx *c, int rows) {
   if (!c) return fail(TSPH_EINVAL, "null argument");
   if (rows < 1 || rows > kMaxTileRows) return fail(TSPH_EINVAL, "tile rows must be 1..24");
-  if (rows != c->tile_rows) {
-    drop_graph(c);
-    c->tiles_valid = false;
-    c->tile_rows = rows;
-    if (int e = clear_tile_costs(c)) return e;  // costs of the old tile layout
-  }
-  return update_tile_base(c);
+  c->rows_set = true;
+  return change_tile_rows(c, rows);
 }
 
 int tsph_set_waves_per_cu(tsph_ctx *c, int waves) {
@@ -1591,7 +1607,7 @@ int tsph_batch_create(const tsph_params *prm, const double *dt, int ncases, tsph
   c->prm = prm[0];
   c->prm.capacity = (int)cap;
   c->capacity = (int)cap;
-  c->tile_rows = 7;
+  c->tile_rows = kTileRows;
   set_walk_defaults(c);
   c->k = ks[0];
   c->ncells_tot = (int)cells;
@@ -1845,7 +1861,9 @@ int tsph_autotune(tsph_ctx *c, int variant, int *tile_rows, int *waves_per_cu, i
     // the chosen depth's particles per lane: every particle belongs to one
     // tile of the list, whose 64 lanes take its particles in turn
     int ntiles = 0, np = 0;
-    if ((e = ensure_tile_list(c, 0))) return e;  // (a pass by cells needs no list)
+    // (a pass by cells needs no list, a static one lists fuller tiles twice)
+    if (c->list_split) c->tiles_valid = false;
+    if ((e = ensure_tile_list(c, 0))) return e;
     TSPH_HIP(hipMemcpyAsync(&ntiles, c->scal + S_NTILES, sizeof(int), hipMemcpyDeviceToHost, c->stream));
     TSPH_HIP(hipMemcpyAsync(&np, c->scal + S_NP, sizeof(int), hipMemcpyDeviceToHost, c->stream));
     TSPH_HIP(hipStreamSynchronize(c->stream));

@@ -263,6 +263,7 @@ struct TileScan {
   const int *cost_in;
   int *cost_list;
   CostEstimate cm;  // the estimate for a tile without a recorded cost
+  bool split;  // list the entries of a static walk (tiles::entry_part)
   // with cost_list: per scan block, the listed tiles' summed cost and the
   // list position of the first (tiles::cut_chunks_scan)
   int *blk_cost, *blk_tile0;
@@ -312,6 +313,11 @@ __device__ __forceinline__ int2 tile_at(const TileScan &ts, int c, const CaseGri
   return make_int2(t, min(ts.rows, g.ncy - cy));
 }
 
+// entries of a tile with `own` particles
+__device__ __forceinline__ int tile_entries(const TileScan &ts, int own) {
+  return own == 0 ? 0 : ts.split && own > tiles::kWave ? 2 : 1;
+}
+
 // the thread's counts (v) and, for the first kMaxTileRows threads, one count
 // of the next block (halo)
 template <int IT>
@@ -351,7 +357,7 @@ __device__ __forceinline__ int stage_counts(int len, int block, const TileScan t
     for (int r = 0; r < tn.y; ++r) o += s_cnt[threadIdx.x * IT + j + r];
     tl[j] = o ? tn.x : -1;
     own[j] = o;
-    nt += o != 0;
+    nt += tile_entries(ts, o);
   }
   return nt;
 }
@@ -527,7 +533,7 @@ __device__ __forceinline__ void scan_block(const ScanArgs &sa, int blk, int nb,
       const int2 tn = tile_at(ts, c, case_grid(ts, ts.cases ? case_of(ts, c) : 0));
       int own = 0;
       for (int r = 0; r < tn.y; ++r) own += in[c + r];
-      pt += own != 0;
+      pt += tile_entries(ts, own);
     }
     int unused = 0;
     block_reduce3(pc, pt, unused, lds);
@@ -550,7 +556,12 @@ __device__ __forceinline__ void scan_block(const ScanArgs &sa, int blk, int nb,
         ts.cost_list[et] = wc;
         csum += wc;
       }
-      ts.list[et++] = tl[j];
+      if (ts.split && own[j] > tiles::kWave) {
+        ts.list[et++] = tl[j] | tiles::kTileFirst;
+        ts.list[et++] = tl[j] | tiles::kTileRest;
+      } else {
+        ts.list[et++] = tl[j];
+      }
     }
   }
   if (ts.cost_list) {
@@ -1066,13 +1077,14 @@ bool cells_ranked(const tsph_ctx *c) { return c->row_width > 0 && c->cell_order 
 
 // the arguments of the scan of the cell counts into cs, with the tile list of
 // the current tile_rows (and, for cost_table >= 0, the listed tiles' costs)
-ScanArgs scan_args(tsph_ctx *c, int *cs, int cost_table) {
+ScanArgs scan_args(tsph_ctx *c, int *cs, int cost_table, bool split) {
   const TileScan ts{c->k.ncy, c->k.ncells, c->k.cell_base, c->cases, c->tile_base, c->ncases,
                     c->tile_rows, c->tile_list,
                     cost_table >= 0 ? c->scal + S_NSCAL + cost_table : nullptr,
                     cost_table >= 0 ? c->list_cost : nullptr,
-                    cost_estimate(c->prm.precision == TSPH_PREC_MIXED), c->scan_cost,
+                    cost_estimate(c->prm.precision == TSPH_PREC_MIXED), split, c->scan_cost,
                     c->scan_tile0};
+  c->list_split = split;
   c->list_groups = 0;  // a pooled pass cuts the new list
   c->list_cost_table = cost_table;
   return {c->cell_count, c->ncells_tot + 1, c->scan_state, c->scan_state_next, cs, ts, c->scan_wait};
@@ -1197,7 +1209,10 @@ int launch_cell_list(tsph_ctx *c, bool eos, bool predict, double dt, unsigned ad
     set_error("tile list: more pooled workgroups than allocated");
     return TSPH_ESTATE;
   }
-  const ScanArgs sa = scan_args(c, cs, cut > 0 ? c->cut_table : -1);
+  // two entries for the fuller tiles where static tile walks follow (the FP64
+  // lists also serve the cell walks, and k_order_tiles takes each tile once)
+  const bool split = rank && cut == 0 && c->prm.precision == TSPH_PREC_MIXED;
+  const ScanArgs sa = scan_args(c, cs, cut > 0 ? c->cut_table : -1, split);
   const bool own_scan = !(rank && binned) || cut > 0 || (hashed && walls);
   if (own_scan)
     if (int e = launch_scan(c, sa, hashed ? walls : 0, wp)) return e;

@@ -167,6 +167,7 @@ struct tsph_ctx {
   bool has_gnr = false, has_n = false;
   bool cells_valid = false;
   int tile_rows = 16;  // cells per pair-loop tile (one grid-column run)
+  bool rows_set = false;  // by tsph_set_tile_rows
   int waves_per_cu = 8;  // persistent pair-loop waves per compute unit
   int num_cu = 256;      // compute units of the device
   int max_lds_block = 65536;  // LDS bytes a workgroup may allocate
@@ -178,7 +179,10 @@ struct tsph_ctx {
   // waves) or the plain static walk; defaults set at creation
   bool balanced[2] = {false, false};
   int cell_order = 0;  // tsph_set_cell_order: 0 and 1 ranked, 2 separate passes
-  int *tile_list = nullptr;  // non-empty tiles of the current cell list, in tile order
+  // the entries of the static walks and the tiles of the pooled ones: non-empty
+  // tiles of the current cell list, in tile order (tiles::part of each)
+  int *tile_list = nullptr;
+  bool list_split = false;  // tiles of more than a wavefront of particles have two entries
   bool tiles_valid = false;  // tile_list matches the cell list and tile_rows
   int *list_part = nullptr;  // per list-build block: tiles, work
   int list_part_cap = 0;     // list-build blocks list_part holds
@@ -297,10 +301,21 @@ inline int total_tiles(const tsph_ctx *c) {
 
 // whether a pair launch of `waves` persistent waves takes the pooled walk:
 // the precision's setting, for systems that give each wave enough particles to
-// balance.  Dam breaks, us per step pooled and static: mixed (3072 waves) 190k
-// particles 139 and 133, 333k 172 and 189; FP64 (2048 waves) 333k 314 and 287,
-// 517k 409 and 422; 16 tanks of 879k particles in all, mixed, 354 and 432.
-constexpr int kPoolMixed = 80, kPoolFp64 = 200;  // particles per wave
+// balance.  Dam breaks, us per step pooled and static, on the first 400 steps
+// and after 1500: mixed (3072 waves) 210k particles 130 and 130, 143 and 131,
+// 333k 155 and 177, 167 and 182; FP64 (2048 waves; static with 6 rows) 233k 227
+// and 222, 266 and 225, 333k 294 and 291, 298 and 312, 517k 390 and 427, 392
+// and 428; 16 tanks of 879k particles in all, mixed, 354 and 432.
+constexpr int kPoolMixed = 80, kPoolFp64 = 150;  // particles per wave
+// Rows of a tile unless tsph_set_tile_rows chose them: 7, about a wavefront of
+// particles, or 6 in FP64 systems too small for the pooled walk.  There, with
+// about a tile per resident wavefront, the tiles of more than 64 particles set
+// the pass's time by their second round (after 1500 steps: 92k particles 187
+// us per step with 7 rows and 135 with 6, 233k 292 and 225; at the start both
+// alike), and FP64 results do not depend on the rows.  The mixed path, whose
+// bits do (it rounds in the tile's frame), gives such tiles two list entries
+// instead.  Pooled FP64 passes hold fewer waves with 6 rows (740k: 520 and 862).
+constexpr int kTileRows = 7, kTileRowsFp64 = 6;
 inline bool walk_balanced(const tsph_ctx *c, bool fp32, int waves) {
   return c->balanced[fp32 ? 1 : 0] && c->n_ub >= (long long)(fp32 ? kPoolMixed : kPoolFp64) * waves;
 }

@@ -412,7 +412,8 @@ __global__ __launch_bounds__(kWave * kPoolWaves) void k_tile64(Soa d, const int 
   // and it is read once they have been waited for
   const int ticket = tq_ticket<DYN>(tq);
   // the tile's case: its constants and its segment of the cell range
-  int tile = tile_list[it];
+  const int entry = tile_list[it];
+  int tile = entry_tile(entry);
   Consts k = k0;
   if (cases) {
     const int cse = case_of_tile(tile_base, ncases, tile);
@@ -422,7 +423,8 @@ __global__ __launch_bounds__(kWave * kPoolWaves) void k_tile64(Soa d, const int 
   const int *cs = cell_start + k.cell_base;
   Tile t;
   tile_begin(k, cs, tile, rows, tab, t);
-  tq_mark(tq, tile_list[it]);
+  if (!DYN) entry_part(entry, t);
+  tq_mark(tq, DYN ? entry : -1);
   if (t.lq[3] > cap) {
     const int next = tq_take<DYN>(tq, ticket);
     for (int i = t.own0 + tile_lane(); i < t.own1; i += kWave) {
@@ -684,7 +686,8 @@ __global__ __launch_bounds__(kWave * kPoolWaves) void k_tile32(Soa d, Mixed mx, 
   // and it is read once they have been waited for
   const int ticket = tq_ticket<DYN>(tq);
   // the tile's case: its constants and its segment of the cell range
-  int tile = tile_list[it];
+  const int entry = tile_list[it];
+  int tile = entry_tile(entry);
   Consts k = k0;
   if (cases) {
     const int cse = case_of_tile(tile_base, ncases, tile);
@@ -695,7 +698,8 @@ __global__ __launch_bounds__(kWave * kPoolWaves) void k_tile32(Soa d, Mixed mx, 
   const C32 cc = make_c32(k);
   Tile t;
   tile_begin(k, cs, tile, rows, tab, t);
-  tq_mark(tq, tile_list[it]);
+  if (!DYN) entry_part(entry, t);
+  tq_mark(tq, DYN ? entry : -1);
   // LDS layout with kGroup sentinels after each column slice's records: a
   // candidate group may run past the end of its slice (the sentinels lie far
   // away and fail every distance test) and need not be masked
@@ -943,7 +947,7 @@ int ensure_tile_list(tsph_ctx *c, int groups, int table) {
   const Consts &k = c->k;
   const int rows = c->tile_rows;
   hipStream_t s = c->stream;
-  if (!c->tiles_valid) {
+  if (!c->tiles_valid || (groups > 0 && c->list_split)) {
     const int ntiles = total_tiles(c);
     const int nb = grid_for(ntiles, kListBlock);
     if (nb > c->list_part_cap) {
@@ -956,6 +960,7 @@ int ensure_tile_list(tsph_ctx *c, int groups, int table) {
                        c->tile_base, c->ncases, rows, ntiles, c->list_part, c->scal, c->tile_list);
     TSPH_HIP(hipGetLastError());
     c->tiles_valid = true;
+    c->list_split = false;
     c->list_groups = 0;
     c->list_cost_table = -1;
   }

@@ -14,6 +14,7 @@ namespace tiles {
 
 constexpr int kWave = 64;          // one wavefront per tile
 constexpr int kCellCap = 11;       // LDS records budgeted per cell of the slices
+constexpr int kLdsGranule = 1280;  // LDS bytes are allocated in units of
 constexpr int kList = 32;          // per-lane neighbour list entries in LDS
 constexpr int kGroup = 8;          // candidates tested together in the mixed pair loop
 constexpr int kStageU = 4;         // staged slots per lane whose loads are in flight together
@@ -224,11 +225,10 @@ __device__ __forceinline__ int tq_take(TileQueue &tq, int raw) {
 // Loads the cell offsets of the three slices (one global load per lane, all in
 // flight together) and derives the tile ranges.  False for an empty tile.
 __device__ __forceinline__ bool tile_begin(const Consts &k, const int *__restrict__ cell_start,
-                                           int tile, int rows, int *tab, Tile &t) {
-  const int nty = (k.ncy + rows - 1) / rows;
-  t.cx = tile / nty;
-  t.cy0 = (tile - t.cx * nty) * rows;
-  t.cy1 = min(t.cy0 + rows, k.ncy);
+                                           int cx, int cy0, int cy1, int *tab, Tile &t) {
+  t.cx = cx;
+  t.cy0 = cy0;
+  t.cy1 = cy1;
   t.row_lo = max(t.cy0 - 1, 0);
   t.nrows = min(t.cy1 + 1, k.ncy) - t.row_lo;
   t.w = t.nrows + 1;
@@ -250,6 +250,26 @@ __device__ __forceinline__ bool tile_begin(const Consts &k, const int *__restric
   }
   t.lq[3] = l;
   return t.own1 > t.own0;
+}
+__device__ __forceinline__ bool tile_begin(const Consts &k, const int *__restrict__ cell_start,
+                                           int tile, int rows, int *tab, Tile &t) {
+  const int nty = (k.ncy + rows - 1) / rows;
+  const int cx = tile / nty, cy0 = (tile - cx * nty) * rows;
+  return tile_begin(k, cell_start, cx, cy0, min(cy0 + rows, k.ncy), tab, t);
+}
+
+// Entries of a tile list.  The list of a static walk gives a tile of more than
+// kWave particles two entries, one for the first kWave and one for the rest,
+// so that another wavefront takes the second round: with about a tile per
+// resident wavefront the tiles of two rounds set the pass's time (they are
+// few on the lattice a run starts from, and up to a third later on).  The
+// tile's frame and each particle's sums are the same either way.
+constexpr int kTileFirst = 1 << 30, kTileRest = (int)(1u << 31), kTileMask = kTileFirst - 1;
+__device__ __forceinline__ int entry_tile(int e) { return e & kTileMask; }
+// the tile's own particles that entry e stands for
+__device__ __forceinline__ void entry_part(int e, Tile &t) {
+  if (e & kTileFirst) t.own1 = min(t.own1, t.own0 + kWave);
+  if (e & kTileRest) t.own0 = min(t.own1, t.own0 + kWave);
 }
 
 // case of global tile t in a batched ensemble (tile_base: ncases+1 bounds)
@@ -783,15 +803,15 @@ __device__ __forceinline__ void cells64(P &pol, CellGrid g, const int *__restric
   wave_count(npair, ncand, nact, counters);
 }
 
-template <bool DYN, class P>
+template <class P>
 __device__ __forceinline__ void walk32(const P &pol, const Consts &k, const int *__restrict__ cell_start,
                                        const int *__restrict__ cellof, int rows,
                                        int *__restrict__ scal, const int *__restrict__ tile_list,
-                                       const int *__restrict__ bound, int cap, int lds_wave,
+                                       int cap, int lds_wave,
                                        unsigned long long *__restrict__ counters) {
 #pragma clang fp contract(fast)
   extern __shared__ __align__(16) unsigned char smem[];
-  unsigned char *wl = wave_lds<DYN>(smem, lds_wave);
+  unsigned char *wl = wave_lds<false>(smem, lds_wave);
   int *tab = reinterpret_cast<int *>(wl);
   uint16_t *s_list = reinterpret_cast<uint16_t *>(wl + kTabBytes);
   const typename P::Lds L = P::lds(wl + kTabBytes + sizeof(uint16_t) * kList * kWave, cap);
@@ -799,21 +819,33 @@ __device__ __forceinline__ void walk32(const P &pol, const Consts &k, const int 
   const float r2cut = 4.f * (float)k.h * (float)k.h;
   if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&counters[C_PASSES], 1ull);
   unsigned npair = 0, ncand = 0, nact = 0;
-  TileQueue tq = tq_begin<DYN>(scal, bound, tile_list, smem);
-  for (int it = tq_take<DYN>(tq, tq_ticket<DYN>(tq)); it >= 0;) {
+  TileQueue tq = tq_begin<false>(scal, nullptr, tile_list, smem);
+  for (int it = tq_take<false>(tq, 0); it >= 0; it = tq_take<false>(tq, 0)) {
     wave_sync();
-    const int ticket = tq_ticket<DYN>(tq);  // read once this tile's loads are waited for
+    const int entry = tile_list[it];
     Tile t;
-    tile_begin(k, cell_start, tile_list[it], rows, tab, t);
-    tq_mark(tq, tile_list[it]);
-    const bool staged = t.lq[3] <= cap;
+    tile_begin(k, cell_start, entry_tile(entry), rows, tab, t);
+    entry_part(entry, t);
     const int mid = t.row_lo + (t.nrows >> 1);
     const double ox = k.x0 - k.of + t.cx * k.kh, oy = k.y0 - k.of + mid * k.kh;
+    // A tile whose slices do not fit is taken in runs of fewer rows (in the
+    // tile's frame, so with the same bits); one row's that do not fit either
+    // are gathered from global memory, which takes about ten times as long.
+    const int cy0 = t.cy0, cy1 = t.cy1, own0 = t.own0, own1 = t.own1;
+    const int sub = t.lq[3] <= cap ? cy1 - cy0
+                                   : max(1, (cy1 - cy0) / ((t.lq[3] + cap - 1) / cap));
+    for (int cy = cy0; cy < cy1; cy += sub) {
+    if (sub < cy1 - cy0) {
+      wave_sync();  // the previous run's LDS is no longer read
+      tile_begin(k, cell_start, t.cx, cy, min(cy + sub, cy1), tab, t);
+      t.own0 = max(t.own0, own0);
+      t.own1 = min(t.own1, own1);
+    }
+    const bool staged = t.lq[3] <= cap;
     if (staged)
       for (int l = lane; l < t.lq[3]; l += kWave)
         pol.stage(L, l, l - sel3(t.base, slice_of(t, l)), ox, oy);
     wave_sync();
-    const int next = tq_take<DYN>(tq, ticket);
     uint16_t *my_list = s_list + lane;
     for (int i0 = t.own0; i0 < t.own1; i0 += kWave) {
       const int i = i0 + lane;
@@ -893,9 +925,8 @@ __device__ __forceinline__ void walk32(const P &pol, const Consts &k, const int 
       }
       if (act) pol.finish(acc, o, i);
     }
-    it = next;
+    }  // runs of rows
   }
-  tq_mark(tq, -1);
   wave_count(npair, ncand, nact, counters);
 }
 
