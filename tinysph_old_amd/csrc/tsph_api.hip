@@ -36,15 +36,13 @@ static int dalloc(T **p, size_t count) {
   return 0;
 }
 
-static int alloc_soa(Soa &s, int cap, bool gnr, bool n) {
+static int alloc_soa(Soa &s, int cap) {
   int e = 0;
   if ((e = dalloc(&s.r, cap)) || (e = dalloc(&s.v, cap)) || (e = dalloc(&s.a, cap)) ||
       (e = dalloc(&s.r_o, cap)) || (e = dalloc(&s.v_o, cap)) || (e = dalloc(&s.rho, cap)) ||
       (e = dalloc(&s.drho, cap)) || (e = dalloc(&s.p, cap)) || (e = dalloc(&s.rho_o, cap)) ||
-      (e = dalloc(&s.type, cap)) || (e = dalloc(&s.seq, cap)) || (e = dalloc(&s.index, cap)))
+      (e = dalloc(&s.type, cap)) || (e = dalloc(&s.seq, cap)))
     return e;
-  if (gnr && (e = dalloc(&s.gnr, cap))) return e;
-  if (n && (e = dalloc(&s.n, cap))) return e;
   return 0;
 }
 
@@ -126,6 +124,7 @@ static int replay_step(tsph_ctx *c, Graph *slots, int tag, double dt, int nsteps
       const HostState h0 = host_state(c);
       auto undo = [&] {  // nothing was launched: restore the host view
         if (c->parity != parity0) flip_build(c);
+        c->olds_in_alt = false;
         set_host_state(c, h0);
       };
       hipGraph_t graph = nullptr;
@@ -170,7 +169,8 @@ static int replay_step(tsph_ctx *c, Graph *slots, int tag, double dt, int nsteps
 static int ensure_extras(tsph_ctx *c, bool gnr, bool n) {
   int e = 0;
   if (gnr && !c->has_gnr) {
-    if ((e = dalloc(&c->cur.gnr, c->capacity)) || (e = dalloc(&c->alt.gnr, c->capacity))) return e;
+    if ((e = dalloc(&c->cur.gnr, c->seq_cap)) || (e = dalloc(&c->pos_gnr, c->capacity))) return e;
+    c->alt.gnr = c->cur.gnr;
     c->has_gnr = true;
   }
   if (n && !c->has_n) {
@@ -247,6 +247,7 @@ static int record_step(tsph_ctx *c, int wall, double dt, int inlet = -1, int out
   }
   // each build cuts the chunks of the pooled pair pass that follows it
   const bool mixed = c->prm.precision == TSPH_PREC_MIXED;
+  const bool more = !zones && c->rec_step + 1 < c->rec_steps;  // another step in the same graph
   const int groups = pass_groups(c, variant);
   c->cut_groups = groups;
   c->cut_table = mixed ? 1 : 0;
@@ -255,9 +256,12 @@ static int record_step(tsph_ctx *c, int wall, double dt, int inlet = -1, int out
     if ((e = launch_predictor(c, dt))) return e;
     if (inlet >= 0 && (e = launch_bz_inlet(c, inlet, dt))) return e;
     if (outlet >= 0 && (e = launch_bz_outlet(c, outlet, dt))) return e;
-    if ((e = launch_cell_list(c, true, false, 0., active))) return e;
-  } else if ((e = launch_cell_list(c, true, true, dt, active, false, false,
-                                   walls_in_build ? wall : 0, true, c->rec_step > 0))) {
+    if ((e = launch_cell_list(c, true, false, 0., active, false, false, 0, false, false, false,
+                              mixed)))
+      return e;
+  } else if ((e = launch_cell_list(c, true, true, dt, active, false, more,
+                                   walls_in_build ? wall : 0, true, c->rec_step > 0, false,
+                                   mixed))) {
     return e;  // (the predictor is applied by the build)
   }
   // the corrector writes the removal states; the build takes the removal
@@ -272,10 +276,10 @@ static int record_step(tsph_ctx *c, int wall, double dt, int inlet = -1, int out
   // rewrites them: this build leaves them behind.  Where another step follows
   // in the same graph it also takes the hash of that step's first build (a
   // step's last pair pass changes neither positions nor velocities).
-  const bool more = !zones && c->rec_step + 1 < c->rec_steps;
   c->cut_groups = groups;
   c->cut_table = 0;
-  if ((e = launch_cell_list(c, true, false, dt, active, true, true, 0, false, false, more)) ||
+  if ((e = launch_cell_list(c, true, false, dt, active, true, true, 0, false, false, more,
+                            mixed && more)) ||
       (e = launch_forces(c, variant)))
     return e;
   return 0;
@@ -383,8 +387,10 @@ static int alloc_context(tsph_ctx *c) {
   const int cap = c->capacity, nct = c->ncells_tot;
   c->seq_cap = 2 * cap + kBzMax + c->ncases;
   const size_t slots = std::max<size_t>(cap, dl_words(c->seq_cap));
-  if ((e = alloc_soa(c->cur, cap, false, false)) || (e = alloc_soa(c->alt, cap, false, false)))
+  if ((e = alloc_soa(c->cur, cap)) || (e = alloc_soa(c->alt, cap)) ||
+      (e = dalloc(&c->cur.index, c->seq_cap)) || (e = dalloc(&c->pos_index, cap)))
     return e;
+  c->alt.index = c->cur.index;
   if ((e = dalloc(&c->scal, S_NSCAL + (size_t)kCostTables * (nct + 8))) ||
       (e = dalloc(&c->cell_count, count_words(c))) ||
       (e = dalloc(&c->cell_count_next, count_words(c))) ||
@@ -535,11 +541,13 @@ int tsph_destroy(tsph_ctx *c) {
   (void)tsph_io_wait(c);  // writer threads hold copies of this context's state
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   drop_graph(c);
+  c->alt.gnr = nullptr;  // (cur's)
+  c->alt.index = nullptr;
   free_soa(c->cur);
   free_soa(c->alt);
   void *ps[] = {c->scal, c->counters, c->cell_count, c->cell_count_next, c->cell_start, c->cell_start_next, c->cellof, c->hrank,
                 c->hcell, c->hrank_next, c->hcell_next, c->row_seq, c->row_seq_next, c->row_head, c->row_head_next, c->bin_count, c->bin_count_next, c->perm, c->scan_state, c->scan_state_next, c->scan_cost, c->scan_tile0, c->seqstate, c->probe_out, c->mx.rv,
-                c->mx.rp, c->mx.nrm, c->tile_list, c->list_cost, c->wall_list, c->bz_list,
+                c->mx.rp, c->mx.nrm, c->pos_gnr, c->pos_index, c->tile_list, c->list_cost, c->wall_list, c->bz_list,
                 c->cases, c->tile_base, c->list_part, c->tile_bound};
   for (void *p : ps)
     if (p) (void)hipFree(p);
@@ -612,10 +620,11 @@ static int upload_impl(tsph_ctx *c, const tsph_particles *h, const uint32_t *seq
     TSPH_HIP(cp(d.type, t.data(), n));
     if (seq_in) TSPH_HIP(cp(d.seq, seq_in, 4 * (size_t)n));
     else if ((e = launch_iota(c, reinterpret_cast<int *>(d.seq), n))) return e;
-    if (h->index) TSPH_HIP(cp(d.index, h->index, 4 * (size_t)n));
-    else if ((e = launch_iota(c, d.index, n))) return e;
     if (cid) TSPH_HIP(cp(d.cid, cid, n));
-    if (h->gnr || c->has_gnr) TSPH_HIP(put(d.gnr, h->gnr, nullptr, s2));
+    if (h->index) TSPH_HIP(cp(c->pos_index, h->index, 4 * (size_t)n));
+    else if ((e = launch_iota(c, c->pos_index, n))) return e;
+    if (c->has_gnr) TSPH_HIP(put(c->pos_gnr, h->gnr, nullptr, s2));
+    if ((e = launch_place(c, n, c->has_gnr))) return e;
     if (h->n || c->has_n) TSPH_HIP(put(d.n, h->n, nullptr, s2));
   }
   if (d.rc) {  // compensation starts from zero
@@ -699,11 +708,21 @@ static int renumber_seq(tsph_ctx *c) {
   std::vector<uint8_t> st((size_t)c->seq_cap), nst((size_t)c->seq_cap, 0);
   TSPH_HIP(hipMemcpy(st.data(), c->seqstate, (size_t)c->seq_cap, hipMemcpyDeviceToHost));
   std::vector<uint32_t> nseq((size_t)std::max(n, 1));
+  std::vector<int32_t> index((size_t)c->seq_cap);
+  std::vector<double2> gnr(c->has_gnr ? (size_t)c->seq_cap : 0);
+  TSPH_HIP(hipMemcpy(index.data(), c->cur.index, index.size() * sizeof(int32_t), hipMemcpyDeviceToHost));
+  if (c->has_gnr)
+    TSPH_HIP(hipMemcpy(gnr.data(), c->cur.gnr, gnr.size() * sizeof(double2), hipMemcpyDeviceToHost));
   uint32_t next = 0;
-  for (int i : order) {
+  for (int i : order) {  // (positions ascending, so none is read after it was written)
     nst[next] = st[seq[i]];
+    index[next] = index[seq[i]];
+    if (c->has_gnr) gnr[next] = gnr[seq[i]];
     nseq[i] = next++;
   }
+  TSPH_HIP(hipMemcpy(c->cur.index, index.data(), index.size() * sizeof(int32_t), hipMemcpyHostToDevice));
+  if (c->has_gnr)
+    TSPH_HIP(hipMemcpy(c->cur.gnr, gnr.data(), gnr.size() * sizeof(double2), hipMemcpyHostToDevice));
   for (int i = 0; i < n; ++i)
     if (type[i] == kRemoved) nseq[i] = next++;
   if (n > 0) TSPH_HIP(hipMemcpy(c->cur.seq, nseq.data(), 4 * (size_t)n, hipMemcpyHostToDevice));
@@ -745,7 +764,7 @@ static int download_impl(tsph_ctx *c, tsph_particles *h, int icase) {
                 {DL_DRHO, h->drho, d.drho, 1}, {DL_RHO_O, h->rho_o, d.rho_o, 1},
                 {DL_R, h->r, d.r, 2},          {DL_V, h->v, d.v, 2},
                 {DL_A, h->a, d.a, 2},          {DL_R_O, h->r_o, d.r_o, 2},
-                {DL_V_O, h->v_o, d.v_o, 2},    {DL_GNR, h->gnr, d.gnr, 2},
+                {DL_V_O, h->v_o, d.v_o, 2},    {DL_GNR, h->gnr, c->pos_gnr, 2},
                 {DL_N, h->n, d.n, 2}};
   unsigned mask = (h->type ? DL_TYPE : 0u) | (h->index ? DL_INDEX : 0u);
   for (const Field &f : fields)
@@ -767,7 +786,7 @@ static int download_impl(tsph_ctx *c, tsph_particles *h, int icase) {
   }
   std::vector<uint8_t> type(h->type ? m : 0);
   if (h->type) TSPH_HIP(get(type.data(), d.type, (size_t)m));
-  if (h->index) TSPH_HIP(get(h->index, d.index, 4 * (size_t)m));
+  if (h->index) TSPH_HIP(get(h->index, c->pos_index, 4 * (size_t)m));
   TSPH_HIP(hipStreamSynchronize(c->stream));
   for (size_t k = 0; k < type.size(); ++k) h->type[k] = type[k];
   return 0;

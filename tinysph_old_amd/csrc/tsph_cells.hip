@@ -68,7 +68,8 @@ __device__ __forceinline__ unsigned long long lanemask_lt() {
 // writes the new cell counts, the scan the new cell offsets.
 struct WallPass {
   Soa d;
-  const int *cell_start, *nwall, *wall_list;
+  const int *cell_start, *nwall;
+  const int2 *wall_list;
   int walls, sweep;  // wall and sweep wavefronts
   unsigned long long *counters;  // the density count (or nullptr)
 };
@@ -826,6 +827,11 @@ __device__ __forceinline__ int bin_offset(const int *__restrict__ cell_count, in
   return s;
 }
 
+// what a build moves beside the fields that every build does: the old state
+// (PRED: writes it), pressures (other than the inlet and outlet particles',
+// which no EOS rewrites), the permutation
+enum : unsigned { kMoveOlds = 1, kMoveP = 2, kMovePerm = 4 };
+
 // Moves every field to its slot of the new order (the state after the build is
 // the reference's state, permuted; perm records the permutation), lists the
 // wall particles and sets the new particle count (removed particles are
@@ -856,9 +862,9 @@ __global__ __launch_bounds__(kScatterBlock, SCAN ? 1 : 6) void k_reorder(
     CellRows rows, const int *__restrict__ bin, int nbins, Clear cl, ScanArgs sa,
     int *__restrict__ perm,
     int *__restrict__ cell_count, uint8_t *__restrict__ seqstate, ChunkCut cc, Soa src, Soa dst,
-    int *__restrict__ scal, int *__restrict__ wall_list, int *__restrict__ cellof, Consts k0,
+    int *__restrict__ scal, int2 *__restrict__ wall_list, int *__restrict__ cellof, Consts k0,
     const Consts *__restrict__ cases, Mixed mx, double dt0, unsigned ad_skip,
-    unsigned long long *__restrict__ counters, int nwall_idx, int nwall_next, bool move_olds,
+    unsigned long long *__restrict__ counters, int nwall_idx, int nwall_next, unsigned moves,
     int *__restrict__ next_count, int *__restrict__ next_bin, int *__restrict__ next_hcell,
     int *__restrict__ next_hrank, CellRows next_rows) {
   extern __shared__ __align__(16) int s_pre[];  // SCAN: the bins' offsets
@@ -885,9 +891,9 @@ __global__ __launch_bounds__(kScatterBlock, SCAN ? 1 : 6) void k_reorder(
   uint32_t mine = 0;
   uint8_t t = kRemoved;
   bool move_ad = false;
-  double2 r = {}, v = {}, a = {}, r_o = {}, v_o = {}, gnr = {}, nv = {};
+  double2 r = {}, v = {}, a = {}, r_o = {}, v_o = {}, nv = {};
   double rho = 0., drho = 0., rho_o = 0., p = 0.;
-  int index = 0, cid = 0;
+  int cid = 0;
   if (x < n_ub) {
     if (RANK) {
       cell = hcell[x];
@@ -900,17 +906,15 @@ __global__ __launch_bounds__(kScatterBlock, SCAN ? 1 : 6) void k_reorder(
     r = src.r[j];
     v = src.v[j];
     rho = src.rho[j];
-    index = src.index[j];
     if (src.cid) cid = src.cid[j];
     if (PRED) {
       a = src.a[j];
       drho = src.drho[j];
-    } else if (move_olds) {
+    } else if (moves & kMoveOlds) {
       r_o = src.r_o[j];
       v_o = src.v_o[j];
       rho_o = src.rho_o[j];
     }
-    if (src.gnr) gnr = src.gnr[j];
     if (src.n) nv = src.n[j];
   }
   int n_new, n;  // RANK: n with the removed ones
@@ -995,7 +999,7 @@ __global__ __launch_bounds__(kScatterBlock, SCAN ? 1 : 6) void k_reorder(
   }
   const bool wall = live && t == TSPH_WALL;
   auto store = [&] {
-    if (PRED || move_olds) {
+    if (moves & kMoveOlds) {
       dst.r_o[k] = r_o;
       dst.v_o[k] = v_o;
       dst.rho_o[k] = rho_o;
@@ -1007,17 +1011,15 @@ __global__ __launch_bounds__(kScatterBlock, SCAN ? 1 : 6) void k_reorder(
       dst.drho[k] = drho;
     }
     dst.rho[k] = rho;
-    dst.p[k] = p;
+    if ((moves & kMoveP) || t == TSPH_OUTLET || t == TSPH_INLET) dst.p[k] = p;
     dst.type[k] = t;
     dst.seq[k] = mine;
-    dst.index[k] = index;
     if (src.cid) dst.cid[k] = cid;
-    if (src.gnr) dst.gnr[k] = gnr;
     if (src.n) dst.n[k] = nv;
     if (EOS && mx.rv)
       write_mixed_record(mx, kc, cell - kc.cell_base, k, r, v, rho, p, src.n != nullptr, nv);
     if (RANK) {
-      perm[k] = j;
+      if (moves & kMovePerm) perm[k] = j;
       cellof[k] = cell;
       if (!SCAN && !bin) cell_count[cell] = 0;
     }
@@ -1047,7 +1049,7 @@ __global__ __launch_bounds__(kScatterBlock, SCAN ? 1 : 6) void k_reorder(
     int base = 0;
     if (lane == __builtin_ctzll(m)) base = atomicAdd(&scal[nwall_idx], __popcll(m));
     base = __shfl(base, __builtin_ctzll(m), 64);
-    if (wall) wall_list[base + __popcll(m & lanemask_lt())] = k;
+    if (wall) wall_list[base + __popcll(m & lanemask_lt())] = make_int2(k, (int)mine);
   }
   if (EOS) {
     const unsigned long long w = __ballot(bad);
@@ -1139,7 +1141,7 @@ int ensure_olds(tsph_ctx *c) {
 
 int launch_cell_list(tsph_ctx *c, bool eos, bool predict, double dt, unsigned ad_skip,
                      bool decide, bool skip_olds, int walls, bool count_density, bool hashed,
-                     bool hash_next) {
+                     bool hash_next, bool skip_p) {
   // a build that moves r_o, v_o, rho_o needs them current (the predictor's
   // build rewrites them instead)
   if (!predict && !skip_olds)
@@ -1238,13 +1240,15 @@ int launch_cell_list(tsph_ctx *c, bool eos, bool predict, double dt, unsigned ad
   }
   const Mixed mx = c->prm.precision == TSPH_PREC_MIXED ? c->mx : Mixed{};
   const Clear cl = hashed ? clear : Clear{};
+  const unsigned moves = (skip_olds ? 0 : kMoveOlds) | (skip_p ? 0 : kMoveP) |
+                         (skip_olds ? kMovePerm : 0);
 #define TSPH_REORDER(E, P, R, N, S)                                                           \
   hipLaunchKernelGGL((k_reorder<E, P, R, N, S>),                                              \
                      dim3((R ? cuts : 0) + (S ? cc.scan_blocks : 0) + sg), dim3(kScatterBlock),    \
                      S ? sizeof(int) * bin_words(c) : 0, s, cs, nct, c->n_ub, c->hcell, rw,         \
                      c->bin_count, bin_words(c), cl, sa, c->perm, c->cell_count, c->seqstate, cc, c->cur, c->alt,     \
                      c->scal, c->wall_list, c->cellof, k, c->cases, mx, dt, ad_skip, c->counters,   \
-                     wslot, c->nwall_idx, !skip_olds, c->cell_count_next, c->bin_count_next,        \
+                     wslot, c->nwall_idx, moves, c->cell_count_next, c->bin_count_next,        \
                      c->hcell_next, c->hrank_next, rw_next)
 #define TSPH_REORDER_R(E, P, N)                                                               \
   if (!rank) TSPH_REORDER(E, P, false, N, false);                                             \
@@ -1266,6 +1270,7 @@ int launch_cell_list(tsph_ctx *c, bool eos, bool predict, double dt, unsigned ad
   TSPH_HIP(hipGetLastError());
   flip_build(c);
   c->olds_stale = skip_olds && !predict;
+  c->olds_in_alt = skip_olds && predict;
   c->cells_valid = true;
   c->tiles_valid = true;  // listed by the scan
   c->records_valid = eos && c->prm.precision == TSPH_PREC_MIXED;

@@ -77,7 +77,10 @@ constexpr int kBzMax = 4096;  // zone particles an inlet pass may convert
 struct Soa {
   uint8_t *cid = nullptr;  // case of each particle (batched ensembles only)
   double2 *r = nullptr, *v = nullptr, *a = nullptr, *r_o = nullptr, *v_o = nullptr;
-  double2 *gnr = nullptr, *n = nullptr;
+  // by reference position (seq), as is index: nothing changes them, so the
+  // builds need not move them; cur's and alt's are the same arrays
+  double2 *gnr = nullptr;
+  double2 *n = nullptr;
   double *rho = nullptr, *drho = nullptr, *p = nullptr, *rho_o = nullptr;
   uint8_t *type = nullptr;
   uint32_t *seq = nullptr;
@@ -96,6 +99,8 @@ struct Soa {
   // density updates (allocated by tsph_set_compensated)
   double2 *rc = nullptr;
   double *rhoc = nullptr;
+  // where particle i's r_o, v_o, rho_o are (nullptr: at i), for the corrector
+  const int *old_at = nullptr;
 };
 
 // FP32 pair records of the mixed path, rebuilt after every reorder.
@@ -196,7 +201,8 @@ struct tsph_ctx {
   // a pooled pair pass of `cut_groups` workgroups and cost table `cut_table`
   // follows the next cell build (0: none): the build cuts its chunks
   int cut_groups = 0, cut_table = 0;
-  int *wall_list = nullptr;  // slots of the wall particles of the current cell list
+  // {slot, reference position} of the wall particles of the current cell list
+  int2 *wall_list = nullptr;
   int n_wall = 0;            // wall particles (walls are never created or removed)
   bool records_valid = false;  // mixed-path FP32 records match the FP64 state
   bool marks_valid = false;    // removal marks match the current positions
@@ -211,6 +217,9 @@ struct tsph_ctx {
   uint8_t *ale_flag = nullptr; // per particle: its own ALE gamma sum is non-zero
   hipStream_t stream = nullptr;
   tsph::Soa cur, alt;
+  // gnr and index in upload or download order, on their way
+  double2 *pos_gnr = nullptr;
+  int32_t *pos_index = nullptr;
   tsph::Mixed mx;
   int *scal = nullptr;                 // S_* slots, then the per-tile costs
   unsigned long long *counters = nullptr;
@@ -253,6 +262,7 @@ struct tsph_ctx {
   std::vector<hipEvent_t> tev;         // 2 per recorded launch
   int tev_used = 0;
   float last_pair_ms = 0.f;
+  bool olds_in_alt = false;   // the old state is alt's r, v, rho, through perm
   int parity = 0;             // flips whenever cur and alt are swapped
   // symplectic step, by parity at the step's start: one step ([0], [1]) or
   // kGraphSteps steps ([2], [3])
@@ -341,7 +351,11 @@ struct TileGrid {
 // place of a launch_remove immediately before (the removal states must be
 // current: a corrector precedes)
 // skip_olds: r_o, v_o, rho_o are not moved (olds_stale afterwards), for a build
-// after which they are dead until the next predictor rewrites them
+// after which they are dead until the next predictor rewrites them; with
+// predict they are not written: a corrector that follows takes them from the
+// previous generation (old_state), and they are dead after it
+// skip_p: pressures are not written where an EOS will rewrite them before
+// anything reads them (the mixed path's pair passes read its records)
 // walls (TSPH_WALL_MDBC or TSPH_WALL_BT; 0: none): the wall densities of that
 // treatment are computed first, from the previous cell list, in the same
 // launch as the build's hash (as launch_mdbc / launch_bt_density with
@@ -370,11 +384,22 @@ void flip_build(tsph_ctx *c);
 int launch_cell_list(tsph_ctx *c, bool eos = false, bool predict = false, double dt = 0.,
                      unsigned ad_skip = 0, bool decide = false, bool skip_olds = false,
                      int walls = 0, bool count_density = false, bool hashed = false,
-                     bool hash_next = false);
+                     bool hash_next = false, bool skip_p = false);
 // r_o, v_o, rho_o of the current generation, gathered from the previous one
 // through the last build's permutation if that build left them behind; every
 // launch that reads or moves them calls this first
 int ensure_olds(tsph_ctx *c);
+// cur, with the old state where the last build left it
+inline Soa old_state(const tsph_ctx *c) {
+  Soa d = c->cur;
+  if (c->olds_in_alt) {
+    d.r_o = c->alt.r;
+    d.v_o = c->alt.v;
+    d.rho_o = c->alt.rho;
+    d.old_at = c->perm;
+  }
+  return d;
+}
 // types whose a, drho a pair pass of `variant` writes (its active particles)
 inline unsigned forces_active_types(int variant) {
   return variant == TSPH_FORCES_DBC ? (1u << TSPH_FLUID) | (1u << TSPH_WALL) : 1u << TSPH_FLUID;
@@ -423,6 +448,9 @@ int launch_download_gather(tsph_ctx *c, int icase, unsigned fields);
 // p[i] = i for i < n
 int launch_iota(tsph_ctx *c, int *p, int n);
 // live particles of every case of a batch into counts[ncases] (device memory)
+// gnr (if gnr) and index of n uploaded particles from pos_gnr, pos_index to their
+// reference positions (cur.seq)
+int launch_place(tsph_ctx *c, int n, bool gnr);
 int launch_case_counts(tsph_ctx *c, int *counts);
 // words of the bitmap over reference positions that launch_download_gather
 // keeps in hcell (and its prefix in hrank)

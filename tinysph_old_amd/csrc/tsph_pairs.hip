@@ -1040,7 +1040,7 @@ template <int VAR, bool DYN>
 void pair_launch(tsph_ctx *c, const TileGrid &tg, int rows, int cap, bool corr, double corr_dt) {
   int *sc = c->scal;
   if (c->prm.precision == TSPH_PREC_MIXED && corr)
-    hipLaunchKernelGGL((k_tile32<VAR, DYN, true>), tg.grid, tg.block, tg.lds, c->stream, c->cur,
+    hipLaunchKernelGGL((k_tile32<VAR, DYN, true>), tg.grid, tg.block, tg.lds, c->stream, old_state(c),
                        c->mx, c->cell_start, c->cellof, c->k, c->cases, c->tile_base, c->ncases,
                        rows, sc, c->tile_list, cap, c->tile_bound, tg.lds_wave, c->counters,
                        corr_dt, c->seqstate);

@@ -140,12 +140,13 @@ __device__ __forceinline__ uint8_t removal_state(const Consts &k, int type, doub
 __device__ __forceinline__ void correct_particle(const Soa &d, const Consts &k, double dt, int i,
                                                  double2 a, double drho, uint8_t *__restrict__ state) {
   const double e = (-drho / d.rho[i]) * dt;
-  const double2 vo = d.v_o[i], ro = d.r_o[i];
+  const int o = d.old_at ? d.old_at[i] : i;
+  const double2 vo = d.v_o[o], ro = d.r_o[o];
   const double2 v = make_double2(vo.x + a.x * dt, vo.y + a.y * dt);
   d.v[i] = v;
   double2 r;
   if (!d.rc) {
-    d.rho[i] = d.rho_o[i] * ((2. - e) / (2. + e));
+    d.rho[i] = d.rho_o[o] * ((2. - e) / (2. + e));
     r = make_double2(ro.x + (v.x + vo.x) * dt * 0.5, ro.y + (v.y + vo.y) * dt * 0.5);
   } else {
     // Kahan-compensated form of the same updates: each is written as old value
@@ -153,7 +154,7 @@ __device__ __forceinline__ void correct_particle(const Soa &d, const Consts &k, 
     // of the increment that the rounded sum loses is carried to the next step
     double2 c = d.rc[i];
     double rc = d.rhoc[i];
-    const double rho_o = d.rho_o[i];
+    const double rho_o = d.rho_o[o];
     d.rho[i] = kahan_add(rho_o, rho_o * ((-2. * e) / (2. + e)), rc);
     r.x = kahan_add(ro.x, (v.x + vo.x) * dt * 0.5, c.x);
     r.y = kahan_add(ro.y, (v.y + vo.y) * dt * 0.5, c.y);

@@ -82,7 +82,7 @@ using namespace walls;
 // (counters set)
 __global__ __launch_bounds__(64) void k_mdbc(Soa d, const int *__restrict__ cell_start,
                                              const int *__restrict__ nwall,
-                                             const int *__restrict__ wall_list, Consts k0,
+                                             const int2 *__restrict__ wall_list, Consts k0,
                                              const Consts *__restrict__ cases,
                                              unsigned long long *__restrict__ counters,
                                              const int *__restrict__ scal, int wall_blocks) {
@@ -93,7 +93,7 @@ __global__ __launch_bounds__(64) void k_mdbc(Soa d, const int *__restrict__ cell
 
 __global__ __launch_bounds__(64) void k_bt_density(Soa d, const int *__restrict__ cell_start,
                                                    const int *__restrict__ nwall,
-                                                   const int *__restrict__ wall_list, Consts k0,
+                                                   const int2 *__restrict__ wall_list, Consts k0,
                                                    const Consts *__restrict__ cases,
                                                    unsigned long long *__restrict__ counters,
                                                    const int *__restrict__ scal, int wall_blocks) {
@@ -342,14 +342,14 @@ __global__ void k_dl_gather(Soa d, Soa o, const int *__restrict__ scal, int icas
   if (fields & DL_A) o.a[k] = d.a[i];
   if (fields & DL_R_O) o.r_o[k] = d.r_o[i];
   if (fields & DL_V_O) o.v_o[k] = d.v_o[i];
-  if (fields & DL_GNR) o.gnr[k] = d.gnr[i];
+  if (fields & DL_GNR) o.gnr[k] = d.gnr[s];
   if (fields & DL_N) o.n[k] = d.n[i];
   if (fields & DL_P) o.p[k] = d.p[i];
   if (fields & DL_RHO) o.rho[k] = d.rho[i];
   if (fields & DL_DRHO) o.drho[k] = d.drho[i];
   if (fields & DL_RHO_O) o.rho_o[k] = d.rho_o[i];
   if (fields & DL_TYPE) o.type[k] = d.type[i];
-  if (fields & DL_INDEX) o.index[k] = d.index[i];
+  if (fields & DL_INDEX) o.index[k] = d.index[s];
 }
 
 // live particles per case: a histogram in LDS per workgroup, then one atomic
@@ -381,18 +381,40 @@ __global__ void k_zero_ints(int *__restrict__ p, int n) {
 int launch_download_gather(tsph_ctx *c, int icase, unsigned fields) {
   uint32_t *bits = reinterpret_cast<uint32_t *>(c->hcell);
   const int g = grid_for(c->n_ub, 256);
+  Soa to = c->alt;
+  to.gnr = c->pos_gnr;
+  to.index = c->pos_index;
   const int wg = grid_for((int)std::min<size_t>(dl_words(c->seq_cap), 1 << 18), 256);
   hipLaunchKernelGGL(k_dl_clear, dim3(wg), dim3(256), 0, c->stream, c->scal, bits);
   hipLaunchKernelGGL(k_dl_mark, dim3(g), dim3(256), 0, c->stream, c->cur, c->scal, icase, bits);
   hipLaunchKernelGGL(k_dl_scan, dim3(1), dim3(kDlScan), 0, c->stream, c->scal, bits, c->hrank);
-  hipLaunchKernelGGL(k_dl_gather, dim3(g), dim3(256), 0, c->stream, c->cur, c->alt, c->scal, icase,
-                     fields, bits, c->hrank);
+  hipLaunchKernelGGL(k_dl_gather, dim3(g), dim3(256), 0, c->stream, c->cur, to, c->scal, icase, fields,
+                     bits, c->hrank);
   TSPH_HIP(hipGetLastError());
   return 0;
 }
 
 int launch_iota(tsph_ctx *c, int *p, int n) {
   hipLaunchKernelGGL(k_iota, dim3(grid_for(n, 256)), dim3(256), 0, c->stream, p, n);
+  TSPH_HIP(hipGetLastError());
+  return 0;
+}
+
+// k_place: to[at[i]] = from[i]
+namespace {
+template <typename V>
+__global__ void k_place(V *__restrict__ to, const V *__restrict__ from,
+                        const uint32_t *__restrict__ at, int n) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) to[at[i]] = from[i];
+}
+}  // namespace
+
+int launch_place(tsph_ctx *c, int n, bool gnr) {
+  const dim3 g(grid_for(n, 256)), b(256);
+  hipLaunchKernelGGL(k_place<int32_t>, g, b, 0, c->stream, c->cur.index, c->pos_index, c->cur.seq, n);
+  if (gnr)
+    hipLaunchKernelGGL(k_place<double2>, g, b, 0, c->stream, c->cur.gnr, c->pos_gnr, c->cur.seq, n);
   TSPH_HIP(hipGetLastError());
   return 0;
 }
@@ -427,7 +449,7 @@ int launch_predictor(tsph_ctx *c, double dt) {
 
 int launch_corrector(tsph_ctx *c, double dt) {
   if (int e = ensure_olds(c)) return e;
-  hipLaunchKernelGGL(k_corrector, dim3(grid_for(c->n_ub, 256)), dim3(256), 0, c->stream, c->cur,
+  hipLaunchKernelGGL(k_corrector, dim3(grid_for(c->n_ub, 256)), dim3(256), 0, c->stream, old_state(c),
                      c->scal, c->k, c->cases, dt, c->seqstate);
   TSPH_HIP(hipGetLastError());
   c->records_valid = false;

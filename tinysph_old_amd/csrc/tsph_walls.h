@@ -190,7 +190,7 @@ inline int sweep_blocks(int n) { return grid_for(n, 64 * kSweep); }
 __device__ __forceinline__ void mdbc_wave(int b, int wall_blocks, int nsweep, const Soa &d,
                                            const int *__restrict__ cell_start,
                                            const int *__restrict__ nwall,
-                                           const int *__restrict__ wall_list, const Consts &k0,
+                                           const int2 *__restrict__ wall_list, const Consts &k0,
                                            const Consts *__restrict__ cases,
                                            unsigned long long *__restrict__ counters,
                                            const int *__restrict__ scal, double *s_terms) {
@@ -200,9 +200,10 @@ __device__ __forceinline__ void mdbc_wave(int b, int wall_blocks, int nsweep, co
   }
   const int w = b * kWallsPerWave + (int)(threadIdx.x & 63) / kWG;
   const bool live = w < *nwall;
-  const int i = live ? wall_list[w] : 0;
+  const int2 wl = live ? wall_list[w] : make_int2(0, 0);
+  const int i = wl.x;
   const Consts k = live ? case_consts(k0, cases, d.cid, i) : k0;
-  const double2 gn = live ? d.gnr[i] : make_double2(0., 0.);
+  const double2 gn = live ? d.gnr[wl.y] : make_double2(0., 0.);
   const double2 r = live ? d.r[i] : make_double2(0., 0.);  // loaded with the ghost node
   const double m = k.m;
   // sums of src/SPH_kernel_approx.h:1141-1342 in its order:
@@ -262,7 +263,7 @@ __device__ __forceinline__ void mdbc_wave(int b, int wall_blocks, int nsweep, co
 __device__ __forceinline__ void bt_wave(int b, int wall_blocks, int nsweep, const Soa &d,
                                          const int *__restrict__ cell_start,
                                          const int *__restrict__ nwall,
-                                         const int *__restrict__ wall_list, const Consts &k0,
+                                         const int2 *__restrict__ wall_list, const Consts &k0,
                                          const Consts *__restrict__ cases,
                                          unsigned long long *__restrict__ counters,
                                          const int *__restrict__ scal, double *s_terms) {
@@ -272,7 +273,7 @@ __device__ __forceinline__ void bt_wave(int b, int wall_blocks, int nsweep, cons
   }
   const int w = b * kWallsPerWave + (int)(threadIdx.x & 63) / kWG;
   const bool live = w < *nwall;
-  const int i = live ? wall_list[w] : 0;
+  const int i = live ? wall_list[w].x : 0;
   const Consts k = live ? case_consts(k0, cases, d.cid, i) : k0;
   const double m = k.m;
   double acc[2];  // wsum, rhowsum (src/SPH_kernel_approx.h:1838-1953)

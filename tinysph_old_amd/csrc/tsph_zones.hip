@@ -111,7 +111,7 @@ __global__ __launch_bounds__(1024) void k_bz_inlet_append(Soa d, int *__restrict
     // Add_particle (src/SPH_particle_system.h:25-50): p 0, rho 1000, a 0, old
     // values = the new ones
     d.type[ns] = (uint8_t)z.btype;
-    d.index[ns] = np + q;
+    d.index[ms + q] = np + q;
     d.seq[ns] = (uint32_t)(ms + q);
     d.p[ns] = 0.;
     d.rho[ns] = 1000.;
@@ -121,7 +121,7 @@ __global__ __launch_bounds__(1024) void k_bz_inlet_append(Soa d, int *__restrict
     d.r_o[ns] = r0;
     d.v_o[ns] = vin;
     d.rho_o[ns] = 1000.;
-    if (d.gnr) d.gnr[ns] = make_double2(0., 0.);
+    if (d.gnr) d.gnr[ms + q] = make_double2(0., 0.);
     if (d.rc) {
       d.rc[ns] = make_double2(0., 0.);
       d.rhoc[ns] = 0.;
