@@ -583,7 +583,7 @@ __device__ __forceinline__ void scan_block(const ScanArgs &sa, int blk, int nb,
 // the scan, with the wall pass (WALLS) in the last wall_groups workgroups, a
 // wavefront's share per wavefront
 template <int IT, int WALLS>
-__global__ __launch_bounds__(kScanBlock) void k_scan(ScanArgs sa, int *__restrict__ scal,
+__global__ __launch_bounds__(kScanBlock, WALLS ? 4 : 1) void k_scan(ScanArgs sa, int *__restrict__ scal,
                                                      unsigned long long *__restrict__ counters,
                                                      int wall_groups, WallPass wp, Consts k0) {
   const int nb = gridDim.x - (WALLS ? wall_groups : 0), blk = blockIdx.x;

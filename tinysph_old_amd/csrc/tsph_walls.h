@@ -24,13 +24,20 @@ __device__ __forceinline__ int point_cell(const Consts &k, double x, double y) {
 // outside the grid skipped) form one candidate sequence in the reference order
 // (stencil order, ascending index within a cell); lane u of the group takes
 // candidates u, u + kWG, u + 2 kWG, ...  The records of kWPre such rounds are
-// loaded together (all in flight at once); then, round by round, the group's
-// lanes evaluate their candidates' terms at once, put them in LDS, and lane u
-// adds sums q = u, u + kWG, ... over the round's candidates in candidate
-// order, so every sum is formed in the reference order.  A candidate that is
-// not a fluid neighbour within the support adds nothing, as in the reference.
+// loaded together (all in flight at once).  The fluid neighbours among them (a
+// sixth to a third) are held in LDS in candidate order, and whenever there are
+// kWG of them the group's lanes evaluate their terms at once, put them in
+// LDS, and lane u adds sums q = u, u + kWG, ... over them in order, so every
+// sum is formed in the reference order.  A candidate that is not a fluid
+// neighbour within the support adds nothing, as in the reference.
+// The pass is bound by its loads (scattered over nine cells for each group) and
+// by FP64 issue: the cells' bounds by one load and broadcasts, rounds over the
+// neighbours instead of all candidates (two instead of five) and shared
+// reciprocals took it beside the scan, us, from 42 to 34 for the 57k walls of a
+// 16-tank ensemble, 22 to 19.5 for 20k and 10.7 to 9 for 5k.
 constexpr int kWG = 16;
 constexpr int kWPre = 3;
+constexpr int kWHeld = 2 * kWG;  // neighbours a group can hold
 constexpr int kWallsPerWave = 64 / kWG;
 constexpr int kTerms = 64 * 12;  // doubles of LDS of a wavefront of the pass
 
@@ -42,7 +49,10 @@ __device__ __forceinline__ void wall_sums(const Soa &d, const int *__restrict__ 
   constexpr int QPL = (NS + kWG - 1) / kWG;  // sums per lane
   const int u = threadIdx.x & (kWG - 1);
   const int g0 = threadIdx.x & 63 & ~(kWG - 1);  // the group's first lane
-  double *grp = terms + g0 * NS;                  // kWG x NS doubles of the group
+  // the group's LDS: held neighbours' {dx, dy, rho}, or a round's kWG x NS terms
+  constexpr int kArea = kWG * NS > kWHeld * 3 ? kWG * NS : kWHeld * 3;
+  static_assert(kArea * kWallsPerWave <= kTerms, "");
+  double *grp = terms + g0 / kWG * kArea;
   const double r2cut = 4.0 * k.h * k.h * (1.0 + 1e-12);
   // candidate f lies in the last cell s with pre[s] <= f, at index f + dj[s]
   int pre[9], dj[9], tot = 0;
@@ -51,24 +61,89 @@ __device__ __forceinline__ void wall_sums(const Soa &d, const int *__restrict__ 
     pre[s] = 0;
     dj[s] = 0;
   }
-  if (live) {
-    const int c = point_cell(k, ar.x, ar.y);
+  // The 12 offsets that bound the cells, one load by the group's first 12 lanes
+  // (4 for each of the 3 columns; outside the grid the nearest end, so that the
+  // cell is empty) and broadcast: 18 loads by every lane took a fourth of the
+  // pass.
+  static_assert(kWG == 16, "a group is a DPP row");
+  int edge = 0;
+  if (live && u < 12) {
+    const int c = point_cell(k, ar.x, ar.y) + (u / 4 - 1) * k.ncy + u % 4 - 1;
+    edge = cell_start[min(max(c, 0), k.ncells)];
+  }
+  int at[12];  // (lanes of groups that are not live: all 0)
+#define TSPH_EDGE(E) at[E] = __builtin_amdgcn_mov_dpp(edge, 0x150 + E, 0xf, 0xf, false);  // row_newbcast
+  TSPH_EDGE(0) TSPH_EDGE(1) TSPH_EDGE(2) TSPH_EDGE(3) TSPH_EDGE(4) TSPH_EDGE(5)
+  TSPH_EDGE(6) TSPH_EDGE(7) TSPH_EDGE(8) TSPH_EDGE(9) TSPH_EDGE(10) TSPH_EDGE(11)
+#undef TSPH_EDGE
 #pragma unroll
-    for (int s = 0; s < 9; ++s) {
-      const int cl = c + stencil_off(s, k.ncy);
-      int lo = 0, n = 0;
-      if (cl >= 0 && cl < k.ncells) {
-        lo = cell_start[cl];
-        n = cell_start[cl + 1] - lo;
-      }
-      pre[s] = tot;
-      dj[s] = lo - tot;
-      tot += n;
-    }
+  for (int s = 0; s < 9; ++s) {
+    int dx, dy;
+    stencil_dxy(s, dx, dy);
+    const int e = (dx + 1) * 4 + dy + 1;
+    pre[s] = tot;
+    dj[s] = at[e] - tot;
+    tot += at[e + 1] - at[e];
   }
   double mine[QPL];  // sums u + kWG x
 #pragma unroll
   for (int x = 0; x < QPL; ++x) mine[x] = 0.;
+  int held = 0;
+  // the terms of the first n (up to kWG) held neighbours into the sums
+  auto round = [&](int n) {
+    bool ok = false;
+    double drx = 0., dry = 0., nrho = 1., lx = 0., ly = 0., lr = 0.;
+    if (u < n) {
+      drx = grp[3 * u];
+      dry = grp[3 * u + 1];
+      nrho = grp[3 * u + 2];
+    }
+    const bool left = kWG + u < held;  // kept for the next round
+    if (left) {
+      lx = grp[3 * (kWG + u)];
+      ly = grp[3 * (kWG + u) + 1];
+      lr = grp[3 * (kWG + u) + 2];
+    }
+    const Root64 rt = sqrt64(drx * drx + dry * dry);
+    const double qq = quot64(rt.s, k.h, k.ih);
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    // the candidate's terms, straight into the group's LDS slots (the
+    // reference adds each to a running sum that starts at +0, which
+    // never turns -0, so the term x itself stands for 0 + x)
+    ok = u < n && qq <= 2.0;
+    if (ok) term(nrho, drx, dry, wendland64(rt, qq, k.awen, k.bwen), grp + u * NS);
+    const unsigned gm = (unsigned)(__ballot(ok) >> g0) & ((1u << kWG) - 1u);
+    // LDS accesses of one wavefront complete in issue order; the fences keep
+    // the compiler from moving them across the hand-over
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    // the round's terms of sum q = u + kWG x, read for all kWG candidates at
+    // once (the LDS reads in flight together), then added in candidate
+    // order; a candidate that is not a neighbour adds +0, which leaves the
+    // sum unchanged (a sum that starts at +0 and adds terms is never -0).
+    // Lanes past the last sum read sum NS - 1 and discard it.
+#pragma unroll
+    for (int x = 0; x < QPL; ++x) {
+      const int q = min(u + kWG * x, NS - 1);
+#pragma unroll
+      for (int h = 0; h < kWG; h += kWG / 2) {
+        double tv[kWG / 2];
+#pragma unroll
+        for (int w = 0; w < kWG / 2; ++w) tv[w] = grp[(h + w) * NS + q];
+#pragma unroll
+        for (int w = 0; w < kWG / 2; ++w) mine[x] += ((gm >> (h + w)) & 1u) ? tv[w] : 0.;
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    if (left) {
+      grp[3 * u] = lx;
+      grp[3 * u + 1] = ly;
+      grp[3 * u + 2] = lr;
+    }
+    held -= n;
+  };
   for (int base = 0; base < tot; base += kWG * kWPre) {  // uniform within the group
     int tt[kWPre];
     double2 rr[kWPre];
@@ -91,47 +166,22 @@ __device__ __forceinline__ void wall_sums(const Soa &d, const int *__restrict__ 
 #pragma unroll
     for (int v = 0; v < kWPre; ++v) {
       if (base + v * kWG >= tot) break;
-      bool ok = false;
-      if (tt[v] == TSPH_FLUID) {
-        const double drx = ar.x - rr[v].x, dry = ar.y - rr[v].y;
-        const double r2 = drx * drx + dry * dry;
-        if (r2 <= r2cut) {
-          const double drs = sqrt(r2);
-          if (drs / k.h <= 2.0) {
-            // the candidate's terms, straight into the group's LDS slots (the
-            // reference adds each to a running sum that starts at +0, which
-            // never turns -0, so the term x itself stands for 0 + x)
-            term(hh[v], drx, dry, drs, grp + u * NS);
-            ok = true;
-          }
-        }
+      const double drx = ar.x - rr[v].x, dry = ar.y - rr[v].y;
+      const bool near = tt[v] == TSPH_FLUID && drx * drx + dry * dry <= r2cut;
+      const unsigned gm = (unsigned)(__ballot(near) >> g0) & ((1u << kWG) - 1u);
+      if (near) {
+        double *e = grp + 3 * (held + __popc(gm & ((1u << u) - 1u)));
+        e[0] = drx;
+        e[1] = dry;
+        e[2] = hh[v];
       }
-      const unsigned gm = (unsigned)(__ballot(ok) >> g0) & ((1u << kWG) - 1u);
-      // LDS accesses of one wavefront complete in issue order; the fences keep
-      // the compiler from moving them across the hand-over
+      held += __popc(gm);
       __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
       __builtin_amdgcn_wave_barrier();
-      // the round's terms of sum q = u + kWG x, read for all kWG candidates at
-      // once (the LDS reads in flight together), then added in candidate
-      // order; a candidate that is not a neighbour adds +0, which leaves the
-      // sum unchanged (a sum that starts at +0 and adds terms is never -0).
-      // Lanes past the last sum read sum NS - 1 and discard it.
-#pragma unroll
-      for (int x = 0; x < QPL; ++x) {
-        const int q = min(u + kWG * x, NS - 1);
-#pragma unroll
-        for (int h = 0; h < kWG; h += kWG / 2) {
-          double tv[kWG / 2];
-#pragma unroll
-          for (int w = 0; w < kWG / 2; ++w) tv[w] = grp[(h + w) * NS + q];
-#pragma unroll
-          for (int w = 0; w < kWG / 2; ++w) mine[x] += ((gm >> (h + w)) & 1u) ? tv[w] : 0.;
-        }
-      }
-      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-      __builtin_amdgcn_wave_barrier();
+      if (held >= kWG) round(kWG);
     }
   }
+  if (held > 0) round(held);  // (fewer than kWG)
   // every lane of the group gets all NS sums
 #pragma unroll
   for (int x = 0; x < QPL; ++x)
@@ -183,6 +233,16 @@ __device__ __forceinline__ void sweep_density(const Soa &d, const int *__restric
 // sweep workgroups that follow wall_blocks wall workgroups for n particles
 inline int sweep_blocks(int n) { return grid_for(n, 64 * kSweep); }
 
+// the constants of particle i's case, by scalar loads where the wavefront's
+// particles are of one case (nearly all are)
+__device__ __forceinline__ Consts wave_consts(const Consts &k0, const Consts *__restrict__ cases,
+                                              const uint8_t *__restrict__ cid, int i, bool live) {
+  if (!cases) return k0;
+  const int c = live ? cid[i] : 0, first = __builtin_amdgcn_readfirstlane(c);
+  if (__all(!live || c == first)) return cases[first];
+  return cases[c];
+}
+
 // The wall-density passes by wavefronts: wavefront b < wall_blocks takes walls
 // kWallsPerWave b ..., wavefront wall_blocks + s (s < nsweep) the
 // density sweep's share s (counters set).  nwall: the wall count of the cell
@@ -202,7 +262,7 @@ __device__ __forceinline__ void mdbc_wave(int b, int wall_blocks, int nsweep, co
   const bool live = w < *nwall;
   const int2 wl = live ? wall_list[w] : make_int2(0, 0);
   const int i = wl.x;
-  const Consts k = live ? case_consts(k0, cases, d.cid, i) : k0;
+  const Consts k = wave_consts(k0, cases, d.cid, i, live);
   const double2 gn = live ? d.gnr[wl.y] : make_double2(0., 0.);
   const double2 r = live ? d.r[i] : make_double2(0., 0.);  // loaded with the ghost node
   const double m = k.m;
@@ -210,9 +270,8 @@ __device__ __forceinline__ void mdbc_wave(int b, int wall_blocks, int nsweep, co
   // rhowsum, drhodx, drhody, a11, a12, a13, a21, a22, a23, a31, a32, a33
   double acc[12];
   wall_sums<12>(d, cell_start + k.cell_base, k, gn, live, acc, s_terms,
-                [&](double nrho, double drx, double dry, double drs, double *a) {
-                  const KW64 kw = wendland64(drs, k.h, k.awen, k.bwen);
-                  const double mr = m / nrho;
+                [&](double nrho, double drx, double dry, const KW64 &kw, double *a) {
+                  const double mr = quot64_any(m, nrho, recip64(nrho));
                   a[0] = m * kw.w;
                   a[1] = drx * kw.f * m;
                   a[2] = dry * kw.f * m;
@@ -274,13 +333,12 @@ __device__ __forceinline__ void bt_wave(int b, int wall_blocks, int nsweep, cons
   const int w = b * kWallsPerWave + (int)(threadIdx.x & 63) / kWG;
   const bool live = w < *nwall;
   const int i = live ? wall_list[w].x : 0;
-  const Consts k = live ? case_consts(k0, cases, d.cid, i) : k0;
+  const Consts k = wave_consts(k0, cases, d.cid, i, live);
   const double m = k.m;
   double acc[2];  // wsum, rhowsum (src/SPH_kernel_approx.h:1838-1953)
   wall_sums<2>(d, cell_start + k.cell_base, k, live ? d.r[i] : make_double2(0., 0.), live, acc,
-               s_terms, [&](double nrho, double, double, double drs, double *a) {
-                 const KW64 kw = wendland64(drs, k.h, k.awen, k.bwen);
-                 a[0] = kw.w * m / nrho;
+               s_terms, [&](double nrho, double, double, const KW64 &kw, double *a) {
+                 a[0] = quot64_any(kw.w * m, nrho, recip64(nrho));
                  a[1] = m * kw.w;
                });
   bool wall_bad = false;
