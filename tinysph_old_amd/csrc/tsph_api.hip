@@ -401,7 +401,7 @@ static int alloc_context(tsph_ctx *c) {
       (e = dalloc(&c->hrank, slots)) || (e = dalloc(&c->hrank_next, slots)) ||
       (e = dalloc(&c->hcell, slots)) || (e = dalloc(&c->hcell_next, slots)) ||
       (e = dalloc(&c->perm, cap)) ||
-      (e = dalloc(&c->seqstate, (size_t)c->seq_cap)) || (e = dalloc(&c->probe_out, 4)) ||
+      (e = dalloc(&c->seqstate, (size_t)c->seq_cap)) || (e = dalloc(&c->probe_out, kProbeOut)) ||
       (e = dalloc(&c->bz_list, 2 * kBzMax)) ||
       (e = dalloc(&c->tile_list, 2 * ((size_t)nct + 8))) || (e = dalloc(&c->list_cost, nct + 8)) ||
       (e = dalloc(&c->wall_list, cap)) ||

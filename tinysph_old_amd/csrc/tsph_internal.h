@@ -256,7 +256,7 @@ struct tsph_ctx {
   int *scan_cost = nullptr, *scan_tile0 = nullptr;
   int scan_wait = 1 << 20;
   uint8_t *seqstate = nullptr;         // removal: per-seq state
-  double *probe_out = nullptr;         // 4 doubles for probe results
+  double *probe_out = nullptr;         // tsph::kProbeOut doubles for probe results
   // pair-kernel timing: one event pair per pair launch while enabled
   bool time_pairs = false;
   std::vector<hipEvent_t> tev;         // 2 per recorded launch
@@ -363,6 +363,7 @@ struct TileGrid {
 // hash_next (with eos, without predict): the build's reorder also takes the
 // hash of the predict build that follows it with nothing but a pair pass
 // between them (the next step's first, with time step dt); hashed: that build
+constexpr int kProbeOut = 65;
 // heads of the chains that hold what the cells' rows do not (a power of two)
 constexpr int kRowHeads = 4096;
 // cells per bin, bins per round of a workgroup's scan of them, and the most
