@@ -36,6 +36,20 @@ static int dalloc(T **p, size_t count) {
   return 0;
 }
 
+// arrays laid out in one allocation, at multiples of 256 bytes
+struct Arena {
+  std::vector<std::pair<void **, size_t>> at;
+  size_t bytes = 0;
+  template <typename T>
+  void add(T *&p, size_t count) {
+    at.push_back({reinterpret_cast<void **>(&p), bytes});
+    bytes += (count * sizeof(T) + 255) / 256 * 256;
+  }
+  void place(unsigned char *base) const {
+    for (const auto &a : at) *a.first = base + a.second;
+  }
+};
+
 static int alloc_soa(Soa &s, int cap) {
   int e = 0;
   if ((e = dalloc(&s.r, cap)) || (e = dalloc(&s.v, cap)) || (e = dalloc(&s.a, cap)) ||
@@ -391,53 +405,53 @@ static int alloc_context(tsph_ctx *c) {
       (e = dalloc(&c->cur.index, c->seq_cap)) || (e = dalloc(&c->pos_index, cap)))
     return e;
   c->alt.index = c->cur.index;
-  if ((e = dalloc(&c->scal, S_NSCAL + (size_t)kCostTables * (nct + 8))) ||
-      (e = dalloc(&c->cell_count, count_words(c))) ||
-      (e = dalloc(&c->cell_count_next, count_words(c))) ||
-      (e = dalloc(&c->cell_start, nct + 2)) ||
-      (e = dalloc(&c->cell_start_next, nct + 2)) ||
-      (e = dalloc(&c->cellof, cap)) ||
-      // (hcell and hrank also serve the download's bitmap over the positions)
-      (e = dalloc(&c->hrank, slots)) || (e = dalloc(&c->hrank_next, slots)) ||
-      (e = dalloc(&c->hcell, slots)) || (e = dalloc(&c->hcell_next, slots)) ||
-      (e = dalloc(&c->perm, cap)) ||
-      (e = dalloc(&c->seqstate, (size_t)c->seq_cap)) || (e = dalloc(&c->probe_out, kProbeOut)) ||
-      (e = dalloc(&c->bz_list, 2 * kBzMax)) ||
-      (e = dalloc(&c->tile_list, 2 * ((size_t)nct + 8))) || (e = dalloc(&c->list_cost, nct + 8)) ||
-      (e = dalloc(&c->wall_list, cap)) ||
-      (e = dalloc(&c->scan_state, (nct + 1) / 1024 + 2)) ||
-      (e = dalloc(&c->scan_state_next, (nct + 1) / 1024 + 2)) ||
-      (e = dalloc(&c->scan_cost, (nct + 1) / 1024 + 2)) ||
-      (e = dalloc(&c->scan_tile0, (nct + 1) / 1024 + 2)))
-    return e;
+  // The cell-list buffers, in one allocation (each costs 10 to 20 us); the ones
+  // that start cleared come first: later builds clear them as they consume them
+  // (and the single-pass scan its words).
+  const size_t words = (nct + 1) / 1024 + 2;  // scan blocks
+  Arena ar;
+  ar.add(c->scal, S_NSCAL + (size_t)kCostTables * (nct + 8));
+  ar.add(c->cell_count, count_words(c));
+  ar.add(c->cell_count_next, count_words(c));
+  ar.add(c->scan_state, words);
+  ar.add(c->scan_state_next, words);
+  ar.add(c->seqstate, (size_t)c->seq_cap);
   // the cells' rows (row_width), where they take no more than about what the
   // particles do
   const size_t rows = (size_t)nct * row_width_of(c);
   if (rows && 2 * rows * sizeof(uint32_t) <= (64u << 20) + 512 * (size_t)cap) {
     c->row_width = row_width_of(c);
-    if ((e = dalloc(&c->row_seq, rows)) || (e = dalloc(&c->row_seq_next, rows)) ||
-        (e = dalloc(&c->row_head, kRowHeads)) || (e = dalloc(&c->row_head_next, kRowHeads)))
-      return e;
-    if (hipMemsetAsync(c->row_head, 0, sizeof(int) * kRowHeads, c->stream) != hipSuccess ||
-        hipMemsetAsync(c->row_head_next, 0, sizeof(int) * kRowHeads, c->stream) != hipSuccess)
-      return fail(TSPH_EHIP, "initialisation failed");
+    ar.add(c->row_head, kRowHeads);
+    ar.add(c->row_head_next, kRowHeads);
+    if (bin_words(c) <= kBinMax) {
+      ar.add(c->bin_count, bin_words(c));
+      ar.add(c->bin_count_next, bin_words(c));
+    }
   }
-  if (c->row_width && bin_words(c) <= kBinMax) {
-    if ((e = dalloc(&c->bin_count, bin_words(c))) || (e = dalloc(&c->bin_count_next, bin_words(c))))
-      return e;
-    if (hipMemsetAsync(c->bin_count, 0, sizeof(int) * bin_words(c), c->stream) != hipSuccess ||
-        hipMemsetAsync(c->bin_count_next, 0, sizeof(int) * bin_words(c), c->stream) != hipSuccess)
-      return fail(TSPH_EHIP, "initialisation failed");
+  const size_t cleared = ar.bytes;
+  if (c->row_width) {
+    ar.add(c->row_seq, rows);
+    ar.add(c->row_seq_next, rows);
   }
-  // the per-cell counters and removal states start cleared; later builds clear
-  // them as they consume them (the single-pass scan's words likewise)
-  if (hipMemsetAsync(c->cell_count, 0, sizeof(int) * count_words(c), c->stream) != hipSuccess ||
-      hipMemsetAsync(c->cell_count_next, 0, sizeof(int) * count_words(c), c->stream) != hipSuccess ||
-      hipMemsetAsync(c->scan_state, 0, sizeof(unsigned long long) * ((nct + 1) / 1024 + 2),
-                     c->stream) != hipSuccess ||
-      hipMemsetAsync(c->scan_state_next, 0, sizeof(unsigned long long) * ((nct + 1) / 1024 + 2),
-                     c->stream) != hipSuccess ||
-      hipMemsetAsync(c->seqstate, 0, (size_t)c->seq_cap, c->stream) != hipSuccess)
+  ar.add(c->cell_start, nct + 2);
+  ar.add(c->cell_start_next, nct + 2);
+  ar.add(c->cellof, cap);
+  // (hcell and hrank also serve the download's bitmap over the positions)
+  ar.add(c->hrank, slots);
+  ar.add(c->hrank_next, slots);
+  ar.add(c->hcell, slots);
+  ar.add(c->hcell_next, slots);
+  ar.add(c->perm, cap);
+  ar.add(c->probe_out, kProbeOut);
+  ar.add(c->bz_list, 2 * kBzMax);
+  ar.add(c->tile_list, 2 * ((size_t)nct + 8));
+  ar.add(c->list_cost, nct + 8);
+  ar.add(c->wall_list, cap);
+  ar.add(c->scan_cost, words);
+  ar.add(c->scan_tile0, words);
+  if ((e = dalloc(&c->arena, ar.bytes))) return e;
+  ar.place(c->arena);
+  if (hipMemsetAsync(c->arena, 0, cleared, c->stream) != hipSuccess)
     return fail(TSPH_EHIP, "initialisation failed");
   {
     int dev = 0;
@@ -461,9 +475,7 @@ static int alloc_context(tsph_ctx *c) {
   if (c->prm.precision == TSPH_PREC_MIXED) {
     if ((e = dalloc(&c->mx.rv, cap)) || (e = dalloc(&c->mx.rp, cap))) return e;
   }
-  if (hipMemsetAsync(c->scal, 0, (S_NSCAL + (size_t)kCostTables * (nct + 8)) * sizeof(int),
-                     c->stream) != hipSuccess ||
-      hipMemsetAsync(c->counters, 0, counter_words(c) * sizeof(unsigned long long), c->stream) != hipSuccess ||
+  if (hipMemsetAsync(c->counters, 0, counter_words(c) * sizeof(unsigned long long), c->stream) != hipSuccess ||
       hipStreamSynchronize(c->stream) != hipSuccess)
     return fail(TSPH_EHIP, "initialisation failed");
   return 0;
@@ -545,9 +557,7 @@ int tsph_destroy(tsph_ctx *c) {
   c->alt.index = nullptr;
   free_soa(c->cur);
   free_soa(c->alt);
-  void *ps[] = {c->scal, c->counters, c->cell_count, c->cell_count_next, c->cell_start, c->cell_start_next, c->cellof, c->hrank,
-                c->hcell, c->hrank_next, c->hcell_next, c->row_seq, c->row_seq_next, c->row_head, c->row_head_next, c->bin_count, c->bin_count_next, c->perm, c->scan_state, c->scan_state_next, c->scan_cost, c->scan_tile0, c->seqstate, c->probe_out, c->mx.rv,
-                c->mx.rp, c->mx.nrm, c->pos_gnr, c->pos_index, c->tile_list, c->list_cost, c->wall_list, c->bz_list,
+  void *ps[] = {c->arena, c->counters, c->mx.rv, c->mx.rp, c->mx.nrm, c->pos_gnr, c->pos_index,
                 c->cases, c->tile_base, c->list_part, c->tile_bound};
   for (void *p : ps)
     if (p) (void)hipFree(p);

@@ -221,6 +221,7 @@ struct tsph_ctx {
   double2 *pos_gnr = nullptr;
   int32_t *pos_index = nullptr;
   tsph::Mixed mx;
+  unsigned char *arena = nullptr;      // holds scal and the cell-list buffers below
   int *scal = nullptr;                 // S_* slots, then the per-tile costs
   unsigned long long *counters = nullptr;
   int *cell_count = nullptr;           // ncells+1 (last = removed bucket)
