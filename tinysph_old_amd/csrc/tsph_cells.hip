@@ -66,26 +66,8 @@ __device__ __forceinline__ unsigned long long lanemask_lt() {
 // build needs no hash, beside that pass rather than before it: it reads the
 // previous cell list and writes wall densities, the hash reads positions and
 // writes the new cell counts, the scan the new cell offsets.
-struct WallPass {
-  Soa d;
-  const int *cell_start, *nwall;
-  const int2 *wall_list;
-  int walls, sweep;  // wall and sweep wavefronts
-  unsigned long long *counters;  // the density count (or nullptr)
-};
-
-// wavefront b of the wall pass; terms: walls::kTerms doubles of LDS
-template <int WALLS>
-__device__ __forceinline__ void wall_wave(int b, const WallPass &wp, const Consts &k0,
-                                          const Consts *__restrict__ cases,
-                                          const int *__restrict__ scal, double *terms) {
-  if (WALLS == TSPH_WALL_MDBC)
-    walls::mdbc_wave(b, wp.walls, wp.sweep, wp.d, wp.cell_start, wp.nwall, wp.wall_list, k0, cases,
-                     wp.counters, scal, terms);
-  else
-    walls::bt_wave(b, wp.walls, wp.sweep, wp.d, wp.cell_start, wp.nwall, wp.wall_list, k0, cases,
-                   wp.counters, scal, terms);
-}
+using walls::WallPass;
+using walls::wall_wave;
 
 // global cell of a particle at r (counted and clamped beyond its case's grid)
 __device__ __forceinline__ int hash_cell(const Consts &k, double2 r,
@@ -1155,12 +1137,10 @@ int launch_cell_list(tsph_ctx *c, bool eos, bool predict, double dt, unsigned ad
   // cell list does not use (swapped in at the end)
   int *cs = c->cell_start_next;
   const int wslot = c->nwall_idx == S_NWALL ? S_NWALL_B : S_NWALL;
-  WallPass wp{c->cur, c->cell_start, c->scal + c->nwall_idx, c->wall_list, 0, 0,
-               count_density ? c->counters : nullptr};
+  WallPass wp{};
   int hg = g, hbs = nb;
   if (walls) {
-    wp.walls = walls::wall_blocks(c);
-    wp.sweep = count_density ? walls::sweep_blocks(c->n_ub) : 0;
+    wp = walls::wall_pass(c, count_density);
     hbs = 64;
     hg = wp.walls + wp.sweep + grid_for(c->n_ub, hbs);
     c->records_valid = false;

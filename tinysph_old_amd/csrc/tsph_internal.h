@@ -423,7 +423,10 @@ int launch_cut(tsph_ctx *c, hipStream_t s, int groups, int table);
 int pass_groups(tsph_ctx *c, int variant);
 // corr (mixed path only): the pass also applies the symplectic corrector to
 // every particle, with time step corr_dt (batched contexts: each case's own)
-int launch_forces(tsph_ctx *c, int variant, bool corr = false, double corr_dt = 0.);
+// walls (mixed path, static walk, not with corr): the wall densities that the
+// next step begins with are computed beside the pass
+int launch_forces(tsph_ctx *c, int variant, bool corr = false, double corr_dt = 0.,
+                  bool walls = false);
 int launch_mixed_records(tsph_ctx *c);
 // tsph_stages.hip
 int launch_eos(tsph_ctx *c);

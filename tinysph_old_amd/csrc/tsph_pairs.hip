@@ -47,6 +47,7 @@
 #include "tsph_internal.h"
 #include "tsph_physics.h"
 #include "tsph_tiles.h"
+#include "tsph_walls.h"
 
 namespace tsph {
 
@@ -651,7 +652,11 @@ __global__ __launch_bounds__(P::kWaves * kWave, 3) void k_cells64(P pol, CellGri
 // in this kernel (neighbours come from the FP32 records), so the update may
 // land while the pass runs; it replaces the corrector pass that follows the
 // first pair pass of a symplectic step.
-template <int VAR, bool DYN, bool CORR>
+// WALLS (static walk, a step's last pass inside a run of steps): the wall
+// densities that the next step begins with (mDBC, or BT for the BT forces) run
+// in the workgroups after the first `groups`; they read the FP64 state and
+// write wall densities, the pair pass reads the FP32 records.
+template <int VAR, bool DYN, bool CORR, bool WALLS>
 __global__ __launch_bounds__(kWave * kPoolWaves) void k_tile32(Soa d, Mixed mx, const int *__restrict__ cell_start,
                                                   const int *__restrict__ cellof, Consts k0,
                                                   const Consts *__restrict__ cases,
@@ -660,9 +665,17 @@ __global__ __launch_bounds__(kWave * kPoolWaves) void k_tile32(Soa d, Mixed mx, 
                                                   const int *__restrict__ tile_list, int cap,
                                                   const int *__restrict__ bound, int lds_wave,
                                                   unsigned long long *__restrict__ counters,
-                                                  double dt0, uint8_t *__restrict__ state) {
+                                                  double dt0, uint8_t *__restrict__ state,
+                                                  int groups, walls::WallPass wp) {
 #pragma clang fp contract(fast)
   extern __shared__ __align__(16) unsigned char smem[];
+  if (WALLS && (int)blockIdx.x >= groups) {
+    constexpr int kWalls = VAR == TSPH_FORCES_BT ? TSPH_WALL_BT : TSPH_WALL_MDBC;
+    const int b = blockIdx.x - groups;  // (one wavefront per workgroup)
+    if (b < wp.walls + wp.sweep)
+      walls::wall_wave<kWalls>(b, wp, k0, cases, scal, reinterpret_cast<double *>(smem));
+    return;
+  }
   unsigned char *wl = wave_lds<DYN>(smem, lds_wave);
   int *tab = reinterpret_cast<int *>(wl);
   float2 *s_pos = reinterpret_cast<float2 *>(wl + kTabBytes);  // tile frame
@@ -679,7 +692,7 @@ __global__ __launch_bounds__(kWave * kPoolWaves) void k_tile32(Soa d, Mixed mx, 
   int pend_i = -1;  // particle whose results are still to be stored
   double2 pend_a = make_double2(0., 0.);
   double pend_dr = 0.;
-  TileQueue tq = tq_begin<DYN>(scal, bound, tile_list, smem, CORR ? 1 : 0);
+  TileQueue tq = tq_begin<DYN>(scal, bound, tile_list, smem, CORR ? 1 : 0, WALLS ? groups : 0);
   for (int it = tq_take<DYN>(tq, tq_ticket<DYN>(tq)); it >= 0;) {
   wave_sync();  // the previous tile's LDS is no longer read
   // the next tile's ticket: its atomic is in flight with this tile's loads,
@@ -1034,25 +1047,32 @@ int pass_groups(tsph_ctx *c, int variant) {
 
 namespace {
 
+// one mixed pair pass; walls: with the wall densities beside it
+template <int VAR, bool DYN, bool CORR, bool WALLS>
+void mixed_launch(tsph_ctx *c, const TileGrid &tg, int rows, int cap, double corr_dt) {
+  const walls::WallPass wp = WALLS ? walls::wall_pass(c, true) : walls::WallPass{};
+  const int groups = tg.grid.x, lds = std::max<int>(tg.lds, WALLS ? walls::kTerms * 8 : 0);
+  hipLaunchKernelGGL((k_tile32<VAR, DYN, CORR, WALLS>), dim3(groups + wp.walls + wp.sweep), tg.block,
+                     lds, c->stream, CORR ? old_state(c) : c->cur, c->mx, c->cell_start, c->cellof,
+                     c->k, c->cases, c->tile_base, c->ncases, rows, c->scal, c->tile_list, cap,
+                     c->tile_bound, tg.lds_wave, c->counters, corr_dt, c->seqstate, groups, wp);
+}
+
 // one pair pass: the kernel for the variant, the precision and the tile walk
 // (pooled or static)
 template <int VAR, bool DYN>
-void pair_launch(tsph_ctx *c, const TileGrid &tg, int rows, int cap, bool corr, double corr_dt) {
-  int *sc = c->scal;
-  if (c->prm.precision == TSPH_PREC_MIXED && corr)
-    hipLaunchKernelGGL((k_tile32<VAR, DYN, true>), tg.grid, tg.block, tg.lds, c->stream, old_state(c),
-                       c->mx, c->cell_start, c->cellof, c->k, c->cases, c->tile_base, c->ncases,
-                       rows, sc, c->tile_list, cap, c->tile_bound, tg.lds_wave, c->counters,
-                       corr_dt, c->seqstate);
-  else if (c->prm.precision == TSPH_PREC_MIXED)
-    hipLaunchKernelGGL((k_tile32<VAR, DYN, false>), tg.grid, tg.block, tg.lds, c->stream, c->cur,
-                       c->mx, c->cell_start, c->cellof, c->k, c->cases, c->tile_base, c->ncases,
-                       rows, sc, c->tile_list, cap, c->tile_bound, tg.lds_wave, c->counters, 0.,
-                       nullptr);
-  else
+void pair_launch(tsph_ctx *c, const TileGrid &tg, int rows, int cap, bool corr, double corr_dt,
+                 bool walls) {
+  if (c->prm.precision != TSPH_PREC_MIXED)
     hipLaunchKernelGGL((k_tile64<VAR, DYN>), tg.grid, tg.block, tg.lds, c->stream, c->cur,
-                       c->cell_start, c->cellof, c->k, c->cases, c->tile_base, c->ncases, rows, sc,
-                       c->tile_list, cap, c->tile_bound, tg.lds_wave, c->counters);
+                       c->cell_start, c->cellof, c->k, c->cases, c->tile_base, c->ncases, rows,
+                       c->scal, c->tile_list, cap, c->tile_bound, tg.lds_wave, c->counters);
+  else if (corr)
+    mixed_launch<VAR, DYN, true, false>(c, tg, rows, cap, corr_dt);
+  else if (!DYN && VAR != TSPH_FORCES_DBC && walls)
+    mixed_launch<VAR, DYN, false, !DYN && VAR != TSPH_FORCES_DBC>(c, tg, rows, cap, 0.);
+  else
+    mixed_launch<VAR, DYN, false, false>(c, tg, rows, cap, 0.);
 }
 
 template <int VAR>
@@ -1068,14 +1088,15 @@ void cell_launch(tsph_ctx *c) {
 }
 
 template <int VAR>
-void pair_launch(tsph_ctx *c, const TileGrid &tg, int rows, int cap, bool corr, double corr_dt) {
-  if (tg.pooled) pair_launch<VAR, true>(c, tg, rows, cap, corr, corr_dt);
-  else pair_launch<VAR, false>(c, tg, rows, cap, corr, corr_dt);
+void pair_launch(tsph_ctx *c, const TileGrid &tg, int rows, int cap, bool corr, double corr_dt,
+                 bool walls) {
+  if (tg.pooled) pair_launch<VAR, true>(c, tg, rows, cap, corr, corr_dt, false);
+  else pair_launch<VAR, false>(c, tg, rows, cap, corr, corr_dt, walls);
 }
 
 }  // namespace
 
-int launch_forces(tsph_ctx *c, int variant, bool corr, double corr_dt) {
+int launch_forces(tsph_ctx *c, int variant, bool corr, double corr_dt, bool walls) {
   const int rows = c->tile_rows;
   const int cap = 3 * (rows + 2) * kCellCap;
   const bool mixed = c->prm.precision == TSPH_PREC_MIXED;
@@ -1098,11 +1119,12 @@ int launch_forces(tsph_ctx *c, int variant, bool corr, double corr_dt) {
   if (int e = ensure_tile_list(c, tg.pooled ? tg.groups : 0, mixed && corr ? 1 : 0)) return e;
   const int e = launch_timed(c, [&] {
     switch (variant) {
-      case TSPH_FORCES_WCSPH: pair_launch<TSPH_FORCES_WCSPH>(c, tg, rows, cap, corr, corr_dt); break;
-      case TSPH_FORCES_DBC: pair_launch<TSPH_FORCES_DBC>(c, tg, rows, cap, corr, corr_dt); break;
-      default: pair_launch<TSPH_FORCES_BT>(c, tg, rows, cap, corr, corr_dt);
+      case TSPH_FORCES_WCSPH: pair_launch<TSPH_FORCES_WCSPH>(c, tg, rows, cap, corr, corr_dt, walls); break;
+      case TSPH_FORCES_DBC: pair_launch<TSPH_FORCES_DBC>(c, tg, rows, cap, corr, corr_dt, walls); break;
+      default: pair_launch<TSPH_FORCES_BT>(c, tg, rows, cap, corr, corr_dt, walls);
     }
   });
+  if (walls) c->records_valid = false;  // (of the wall particles)
   if (!e && mixed && corr) {  // as launch_corrector leaves them
     c->records_valid = false;
     c->marks_valid = true;

@@ -125,11 +125,12 @@ __device__ __forceinline__ int band_lo(int ntl, int b) { return (int)(((long lon
 template <bool DYN>
 __device__ __forceinline__ TileQueue tq_begin(int *__restrict__ scal, const int *__restrict__ bound,
                                               const int *__restrict__ tile_list,
-                                              unsigned char *smem, int table = 0) {
+                                              unsigned char *smem, int table = 0,
+                                              int groups = 0) {  // 0: the whole launch
   TileQueue tq;
   tq.ntl = 0;
   tq.band = blockIdx.x & 7;
-  tq.nwb = gridDim.x >> 3;
+  tq.nwb = (groups ? groups : (int)gridDim.x) >> 3;
   tq.wb = blockIdx.x >> 3;
   tq.j = -1;
   tq.lo = tq.hi = 0;

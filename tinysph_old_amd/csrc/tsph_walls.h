@@ -354,5 +354,31 @@ __device__ __forceinline__ void bt_wave(int b, int wall_blocks, int nsweep, cons
 // workgroups of a wall pass: wall workgroups, then sweep workgroups
 inline int wall_blocks(const tsph_ctx *c) { return grid_for(c->n_wall, kWallsPerWave); }
 
+// the pass beside another launch: its wavefronts' share
+struct WallPass {
+  Soa d;
+  const int *cell_start, *nwall;
+  const int2 *wall_list;
+  int walls, sweep;  // wall and sweep wavefronts
+  unsigned long long *counters;  // the density count (or nullptr)
+};
+inline WallPass wall_pass(const tsph_ctx *c, bool count_density) {
+  return {c->cur, c->cell_start, c->scal + c->nwall_idx, c->wall_list, wall_blocks(c),
+          count_density ? sweep_blocks(c->n_ub) : 0, count_density ? c->counters : nullptr};
+}
+
+// wavefront b of the wall pass; terms: walls::kTerms doubles of LDS
+template <int WALLS>
+__device__ __forceinline__ void wall_wave(int b, const WallPass &wp, const Consts &k0,
+                                          const Consts *__restrict__ cases,
+                                          const int *__restrict__ scal, double *terms) {
+  if (WALLS == TSPH_WALL_MDBC)
+    mdbc_wave(b, wp.walls, wp.sweep, wp.d, wp.cell_start, wp.nwall, wp.wall_list, k0, cases,
+              wp.counters, scal, terms);
+  else
+    bt_wave(b, wp.walls, wp.sweep, wp.d, wp.cell_start, wp.nwall, wp.wall_list, k0, cases,
+            wp.counters, scal, terms);
+}
+
 }  // namespace walls
 }  // namespace tsph
