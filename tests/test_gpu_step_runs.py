@@ -72,3 +72,38 @@ def test_batch_run_equals_single_steps(precision):
             assert np.array_equal(a[q][k], b[q][k]), (q, k)
     for k in COUNTS:
         assert ca[k] == cb[k], k
+
+
+@pytest.mark.parametrize("precision", [T.PREC_FP64, T.PREC_MIXED], ids=["fp64", "mixed"])
+@pytest.mark.parametrize("kind", ["rale", "ale", "leapfrog"])
+def test_other_steps_in_runs(kind, precision):
+    """Riemann-ALE, ALE-SPH MUSCL and leap-frog steps, the first one included."""
+    preset = T.CASE_DAM_BREAK_MDBC if kind == "leapfrog" else T.CASE_ALE_DAM_BREAK
+    case = T.build_case(preset, dx=0.02, jitter=0.05, seed=5)
+    print(f"[case] {kind} np={case.np} precision {precision}", flush=True)
+    out = []
+    for run in (False, True):
+        with T.system_for_case(case, precision=precision) as ps:
+            if kind == "leapfrog":
+                ps.history_enable()
+            else:
+                ps.ale_enable()
+            ps.particle_to_cell()
+            first = 1
+            for n in ([STEPS] if run else [1] * STEPS):
+                if kind == "rale":
+                    ps.step_rale(case.dt, first, n)
+                elif kind == "ale":
+                    ps.step_ale(case.dt, first, n, T.MUSCL_MINMOD)
+                else:
+                    ps.step_leapfrog(case.wall, case.dt, first, n)
+                first += n
+            more = {} if kind == "leapfrog" else ps.ale_download()
+            out.append((ps.download(FIELDS), more, ps.counters()))
+    (a, ea, ca), (b, eb, cb) = out
+    for k in FIELDS:
+        assert np.array_equal(a[k], b[k], equal_nan=True), k
+    for k in ea:
+        assert np.array_equal(ea[k], eb[k], equal_nan=True), k
+    for k in COUNTS:
+        assert ca[k] == cb[k], k

@@ -71,14 +71,19 @@ static void free_soa(Soa &s) {
 }
 
 static void drop_graph(tsph_ctx *c) {
-  for (Graph *g : {&c->graph[0], &c->graph[1], &c->graph[2], &c->graph[3], &c->rale_graph[0],
-                   &c->rale_graph[1],
-                   &c->ale_graph[0], &c->ale_graph[1], &c->inflow_graph[0], &c->inflow_graph[1],
-                   &c->verlet_graph[0], &c->verlet_graph[1], &c->euler_graph[0],
-                   &c->euler_graph[1], &c->lf_graph[0], &c->lf_graph[1]}) {
-    if (g->exec) (void)hipGraphExecDestroy(g->exec);
-    *g = Graph{};
-  }
+  auto drop = [](auto &slots) {
+    for (Graph &g : slots) {
+      if (g.exec) (void)hipGraphExecDestroy(g.exec);
+      g = Graph{};
+    }
+  };
+  drop(c->graph);
+  drop(c->rale_graph);
+  drop(c->ale_graph);
+  drop(c->inflow_graph);
+  drop(c->verlet_graph);
+  drop(c->euler_graph);
+  drop(c->lf_graph);
 }
 
 // default pair-loop launch: 7-cell tiles in the pooled walk (chunks cut by
@@ -95,7 +100,7 @@ static void set_walk_defaults(tsph_ctx *c) {
 
 static HostState host_state(const tsph_ctx *c) {
   return {c->cells_valid, c->tiles_valid, c->records_valid, c->marks_valid, c->olds_stale,
-          c->list_groups, c->list_table, c->list_cost_table};
+          c->list_split, c->list_groups, c->list_table, c->list_cost_table};
 }
 
 static void set_host_state(tsph_ctx *c, const HostState &h) {
@@ -107,6 +112,7 @@ static void set_host_state(tsph_ctx *c, const HostState &h) {
   c->records_valid = h.records_valid;
   c->marks_valid = h.marks_valid;
   c->olds_stale = h.olds_stale;
+  c->list_split = h.list_split;
 }
 
 // Runs nsteps steps from graphs: the graph of the current buffer parity is
@@ -1035,7 +1041,8 @@ int tsph_step_rale(tsph_ctx *c, double dt, int step, int nsteps) {
   for (; s < last && (s == 1 || c->time_pairs); ++s)
     if (int e = record_rale_step(c, dt, s)) return e;
   if (s >= last) return 0;
-  return replay_step(c, c->rale_graph, 100, dt, last - s, [&] { return record_rale_step(c, dt, 2); });
+  return replay_step(c, c->rale_graph, 100, dt, last - s, [&] { return record_rale_step(c, dt, 2); },
+                     kGraphSteps);
 }
 
 int tsph_ale_compute_density(tsph_ctx *c, int limited) {
@@ -1082,7 +1089,7 @@ int tsph_step_ale(tsph_ctx *c, double dt, int step, int nsteps, int muscl) {
     if (int e = record_ale_step(c, dt, s, muscl)) return e;
   if (s >= last) return 0;
   return replay_step(c, c->ale_graph, 200 + muscl, dt, last - s,
-                     [&] { return record_ale_step(c, dt, 2, muscl); });
+                     [&] { return record_ale_step(c, dt, 2, muscl); }, kGraphSteps);
 }
 
 int tsph_bz_add_zone(tsph_ctx *c, const tsph_zone *z, int *index) {
@@ -1453,7 +1460,7 @@ int tsph_step_leapfrog(tsph_ctx *c, int wall, double dt, int step, int nsteps) {
     if (int e = record_leapfrog_step(c, wall, dt, s)) return e;
   if (s >= last) return 0;
   return replay_step(c, c->lf_graph, 520 + wall, dt, last - s,
-                     [&] { return record_leapfrog_step(c, wall, dt, 2); });
+                     [&] { return record_leapfrog_step(c, wall, dt, 2); }, kGraphSteps);
 }
 
 int tsph_step_symplectic_reinit(tsph_ctx *c, int wall, double dt, int step, int nsteps,

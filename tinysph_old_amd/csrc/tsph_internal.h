@@ -132,7 +132,7 @@ __device__ __forceinline__ Consts case_consts(const Consts &k0, const Consts *__
 
 // host-side flags that describe what the device buffers hold
 struct HostState {
-  bool cells_valid, tiles_valid, records_valid, marks_valid, olds_stale;
+  bool cells_valid, tiles_valid, records_valid, marks_valid, olds_stale, list_split;
   int list_groups, list_table, list_cost_table;
 };
 
@@ -265,17 +265,20 @@ struct tsph_ctx {
   float last_pair_ms = 0.f;
   bool olds_in_alt = false;   // the old state is alt's r, v, rho, through perm
   int parity = 0;             // flips whenever cur and alt are swapped
-  // symplectic step, by parity at the step's start: one step ([0], [1]) or
-  // kGraphSteps steps ([2], [3])
-  tsph::Graph graph[4];
+  // the steps' graphs, by parity at the step's start: one step ([0], [1]) or a
+  // run of kGraphSteps ([2], [3]; each graph launch leaves some us idle before
+  // the next: Riemann-ALE steps of 47k particles 68.6 us one by one, 64.8 in
+  // runs, ALE ones of 183k 240 and 236, of 12k 109 and 105; 1M particles with
+  // buffer zones 447 and 446, so those stay single)
+  tsph::Graph graph[4];       // symplectic
+  tsph::Graph rale_graph[4];  // Riemann-ALE
+  tsph::Graph ale_graph[4];   // ALE-SPH MUSCL
+  tsph::Graph lf_graph[4];    // leap-frog driver (after the first step)
+  tsph::Graph inflow_graph[2];  // symplectic with buffer zones
+  tsph::Graph verlet_graph[2];  // Verlet driver (Verlet integrator)
+  tsph::Graph euler_graph[2];   // Verlet driver on its Euler steps
   // the step being recorded of the run that one graph holds
   int rec_step = 0, rec_steps = 1;
-  tsph::Graph rale_graph[2];  // Riemann-ALE step, by parity at the step's start
-  tsph::Graph ale_graph[2];   // ALE-SPH MUSCL step, by parity at the step's start
-  tsph::Graph inflow_graph[2];  // symplectic step with buffer zones
-  tsph::Graph verlet_graph[2];  // Verlet-driver step (Verlet integrator)
-  tsph::Graph euler_graph[2];   // Verlet-driver step on its Euler steps
-  tsph::Graph lf_graph[2];      // leap-frog-driver step (after the first)
   bool has_history = false;     // v_oo, rho_oo, rhoTemp allocated
   // asynchronous output (tsph_write_vtk): writer threads and their first error
   std::vector<std::thread> writers;
