@@ -251,8 +251,8 @@ static int record_step(tsph_ctx *c, int wall, double dt, int inlet = -1, int out
   // Without buffer zones nothing reads the pressures (or the mixed records)
   // this EOS writes before the cell build rewrites them all, so only its
   // out-of-range density count is taken, by the wall-density pass.  Without
-  // buffer zones the pass runs in workgroups of the first build's hash launch,
-  // beside the hash (on a second stream the fork and the join in the step
+  // buffer zones the pass runs in workgroups of the first build's hash or scan
+  // launch, or of the pair pass before it (below; on a second stream the fork and the join in the step
   // graph left about 25 us of idle time per step, more than the pass takes).
   // With buffer zones the pass runs in a launch of its own, before the
   // predictor (the zone passes act on predicted positions, so the build cannot

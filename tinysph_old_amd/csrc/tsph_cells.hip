@@ -58,8 +58,8 @@ __device__ __forceinline__ unsigned long long lanemask_lt() {
 // predictor itself is applied by the reorder that follows).  DECIDE: the
 // removal decision of RemoveParticlesOutOfDomain (k_rm_decide's) is taken here,
 // from the removal states of the corrector that precedes the build.  The
-// reference positions of removed particles are marked absent by k_scatter, so
-// no decision in this pass reads a state that this pass changes.
+// reference positions of removed particles are marked absent by the reorder
+// (or k_scatter), so no decision in this pass reads a state that this pass changes.
 // The wall-density pass that precedes a build in the symplectic step (WALLS:
 // TSPH_WALL_MDBC or TSPH_WALL_BT; 0: none) runs in the first wb.walls +
 // wb.sweep wavefronts of the hash launch, or of the scan launch where the
@@ -1183,7 +1183,7 @@ int launch_cell_list(tsph_ctx *c, bool eos, bool predict, double dt, unsigned ad
 #undef TSPH_HASH_W
 #undef TSPH_HASH
   // the pooled pair pass that follows (if any) has its chunks cut in the
-  // first workgroups of the scatter, from the costs the scan lists beside the
+  // first workgroups of the reorder (or the scatter), from the costs the scan lists beside the
   // tiles and its per-block sums of them
   const int cut = c->cut_groups;
   c->cut_groups = 0;

@@ -1,10 +1,11 @@
 // Internal declarations shared by the translation units of libtinysph_hip.so.
 // Device data layout (HBM), one SoA generation per field:
-//   r, v, a, r_o, v_o, gnr, n : double2   (16 B per particle each)
+//   r, v, a, r_o, v_o, n      : double2   (16 B per particle each)
 //   rho, drho, p, rho_o       : double    ( 8 B)
 //   type                      : uint8     (reference part_type; 255 = removed)
 //   seq                       : uint32    (position in reference order; gaps allowed)
-//   index                     : int32     (reference data.index)
+//   gnr, index                : double2, int32 (ghost node, reference data.index), by
+//                               reference position: one generation, never moved
 // After every Particle_To_Cell the arrays are permuted into (cell, seq) order,
 // so a cell's particles are contiguous and ordered exactly as the reference
 // iterates them; `cellof[k]` holds the cell of slot k and `cell_start` the CSR
@@ -26,7 +27,7 @@ namespace tsph {
 constexpr uint8_t kRemoved = 255;
 
 constexpr int kMaxTileRows = 24;  // upper bound of tile_rows
-// Pooled walk's cost model.  Every tile pass records the time each tile took
+// Pooled walk's cost model.  Every pooled pass records the time each tile took
 // its wavefront (tq_mark, tsph_tiles.h; 10 ns ticks of the device's constant
 // clock, averaged with the tile's previous record) in one of kCostTables
 // tables, at scal[S_NSCAL + kCostTables t + table] for global tile t; the
@@ -36,7 +37,7 @@ constexpr int kMaxTileRows = 24;  // upper bound of tile_rows
 // work would not: what else ran on its compute unit, so that the chunks of a
 // compute unit that ran slow shrink in the next pass.  Table 1 holds the mixed
 // pair passes that apply the symplectic corrector as well, table 0 every
-// other tile pass.  A tile without a record (the first pass after a change of
+// other pooled pass.  A tile without a record (the first pass after a change of
 // tile layout, or a tile newly occupied) is estimated from its own particles:
 // own particles x own + tile, the least-squares fit of the measured times of
 // the 740k-particle dam break's 13,147 tiles (near-empty tiles 4.4 us mixed,
@@ -344,30 +345,9 @@ struct TileGrid {
   bool pooled = false;
 };
 
-// tsph_cells.hip
-// hash, count, scan, scatter, order, reorder; eos: the reorder also runs
-// Density_to_pressure (and writes the mixed records) for the moved particles
-// predict: the symplectic predictor (step dt; per case in a batch) is applied
-// on the way, in place of a launch_predictor immediately before.  ad_skip: a
-// mask of particle types (bit t: type t) whose a, drho are left behind, for a
-// build that a pair pass overwriting exactly those follows (forces_active_types)
-// decide: RemoveParticlesOutOfDomain's decision is taken by the build, in
-// place of a launch_remove immediately before (the removal states must be
-// current: a corrector precedes)
-// skip_olds: r_o, v_o, rho_o are not moved (olds_stale afterwards), for a build
-// after which they are dead until the next predictor rewrites them; with
-// predict they are not written: a corrector that follows takes them from the
-// previous generation (old_state), and they are dead after it
-// skip_p: pressures are not written where an EOS will rewrite them before
-// anything reads them (the mixed path's pair passes read its records)
-// walls (TSPH_WALL_MDBC or TSPH_WALL_BT; 0: none): the wall densities of that
-// treatment are computed first, from the previous cell list, in the same
-// launch as the build's hash (as launch_mdbc / launch_bt_density with
-// count_density), or as its scan where it has none
-// hash_next (with eos, without predict): the build's reorder also takes the
-// hash of the predict build that follows it with nothing but a pair pass
-// between them (the next step's first, with time step dt); hashed: that build
+// doubles of probe results (tsph_stages.hip: {level, index} of 32 chunks, a height)
 constexpr int kProbeOut = 65;
+// tsph_cells.hip
 // heads of the chains that hold what the cells' rows do not (a power of two)
 constexpr int kRowHeads = 4096;
 // cells per bin, bins per round of a workgroup's scan of them, and the most
@@ -386,6 +366,28 @@ inline int bin_words(const tsph_ctx *c) {
 // the buffers that change places with every cell build: cur and alt, and this
 // build's cell-list buffers and the next one's
 void flip_build(tsph_ctx *c);
+// hash, scan, reorder; eos: the reorder also runs
+// Density_to_pressure (and writes the mixed records) for the moved particles
+// predict: the symplectic predictor (step dt; per case in a batch) is applied
+// on the way, in place of a launch_predictor immediately before.  ad_skip: a
+// mask of particle types (bit t: type t) whose a, drho are left behind, for a
+// build that a pair pass overwriting exactly those follows (forces_active_types)
+// decide: RemoveParticlesOutOfDomain's decision is taken by the build, in
+// place of a launch_remove immediately before (the removal states must be
+// current: a corrector precedes)
+// skip_olds: r_o, v_o, rho_o are not moved (olds_stale afterwards), for a build
+// after which they are dead until the next predictor rewrites them; with
+// predict they are not written: a corrector that follows takes them from the
+// previous generation (old_state), and they are dead after it
+// skip_p: pressures are not written where an EOS will rewrite them before
+// anything reads them (the mixed path's pair passes read its records)
+// walls (TSPH_WALL_MDBC or TSPH_WALL_BT; 0: none): the wall densities of that
+// treatment are computed first, from the previous cell list, in the same
+// launch as the build's hash, or as its scan where it has none (as launch_mdbc
+// / launch_bt_density with count_density)
+// hash_next (with eos, without predict): the build's reorder also takes the
+// hash of the predict build that follows it with nothing but a pair pass
+// between them (the next step's first, with time step dt); hashed: that build
 int launch_cell_list(tsph_ctx *c, bool eos = false, bool predict = false, double dt = 0.,
                      unsigned ad_skip = 0, bool decide = false, bool skip_olds = false,
                      int walls = 0, bool count_density = false, bool hashed = false,

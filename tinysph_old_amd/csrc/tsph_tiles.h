@@ -103,7 +103,7 @@ __device__ __forceinline__ void wave_sync() {
 //     unit thereby balance each other, and the compute units each other
 //     through the costs, without any device-wide atomic (those serialise
 //     across the XCDs).
-// Either walk records each tile's time (tq_mark) for the next pooled cut.
+// The pooled walk records each tile's time (tq_mark) for the next cut.
 struct TileQueue {
   int ntl;   // static: tiles in the list
   int band;  // static: band of the wave

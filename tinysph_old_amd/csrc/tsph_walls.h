@@ -1,6 +1,7 @@
 // Wall densities (mDBC, BT) by wavefronts, shared by their own launches
-// (tsph_stages.hip) and the first cell build of a symplectic step, whose hash
-// or scan launch runs them in wavefronts of its own (tsph_cells.hip):
+// (tsph_stages.hip), the first cell build of a symplectic step, whose hash or
+// scan launch runs them in wavefronts of its own (tsph_cells.hip), and static
+// mixed pair passes (tsph_pairs.hip):
 //   mDBC_compute_density_mdbcGeo   src/SPH_mDBC.h:9-50 with
 //                                  Kernel_density_approximation_MATRIX_mDBC,
 //                                  src/SPH_kernel_approx.h:1141-1342
