@@ -425,7 +425,7 @@ int tsph_autotune(tsph_ctx *ctx, int variant, int *tile_rows, int *waves_per_cu,
  * list of about equal cost, cut by the time each tile took in the previous
  * pass, whose tiles its wavefronts take from a counter in LDS, the costliest
  * first), 0 = static striding, one wavefront per workgroup.  Systems
- * with fewer than 80 (mixed) or 150 (FP64) particles per persistent wave, and
+ * with fewer than 95 (mixed) or 150 (FP64) particles per persistent wave, and
  * the ALE passes, always stride; FP64 passes over at most 70,000 particles go
  * by cells instead of tiles and do not depend on the setting.
  * Results do not depend on it.  No counterpart in the reference. */

@@ -317,11 +317,12 @@ inline int total_tiles(const tsph_ctx *c) {
 // whether a pair launch of `waves` persistent waves takes the pooled walk:
 // the precision's setting, for systems that give each wave enough particles to
 // balance.  Dam breaks, us per step pooled and static, on the first 400 steps
-// and after 1500: mixed (3072 waves) 210k particles 130 and 130, 143 and 131,
-// 333k 155 and 177, 167 and 182; FP64 (2048 waves; static with 6 rows) 233k 227
-// and 222, 266 and 225, 333k 294 and 291, 298 and 312, 517k 390 and 427, 392
-// and 428; 16 tanks of 879k particles in all, mixed, 354 and 432.
-constexpr int kPoolMixed = 80, kPoolFp64 = 150;  // particles per wave
+// and after 1500: mixed (3072 waves) 210k particles 130 and 124, 143 and 126,
+// 260k 137 and 130, 151 and 131, 333k 149 and 168, 161 and 174; FP64 (2048
+// waves; static with 6 rows) 233k 227 and 222, 266 and 225, 333k 294 and 291,
+// 298 and 312, 517k 390 and 427, 392 and 428; 16 tanks of 879k particles in
+// all, mixed, 354 and 432.
+constexpr int kPoolMixed = 95, kPoolFp64 = 150;  // particles per wave
 // Rows of a tile unless tsph_set_tile_rows chose them: 7, about a wavefront of
 // particles, or 6 in FP64 systems too small for the pooled walk.  There, with
 // about a tile per resident wavefront, the tiles of more than 64 particles set
