@@ -719,8 +719,9 @@ static int live_order(tsph_ctx *c, int n, std::vector<int> &order, std::vector<u
 // would run out of removal states (seq_cap); this relabels the live particles
 // 0..m-1 in order, carrying each one's removal state along, gives the removed
 // slots still in the range the positions after them (state 0: absent), and
-// resets S_MAXSEQ.  Cell order, tiles and records stay valid: the in-cell
-// order by seq is unchanged.
+// resets S_MAXSEQ.  The fields kept by position (gnr, index) and the positions
+// in the wall list move along.  Cell order, tiles and records stay valid: the
+// in-cell order by seq is unchanged.
 static int renumber_seq(tsph_ctx *c) {
   int n = 0, e = 0;
   TSPH_HIP(hipStreamSynchronize(c->stream));
@@ -750,6 +751,14 @@ static int renumber_seq(tsph_ctx *c) {
   for (int i = 0; i < n; ++i)
     if (type[i] == kRemoved) nseq[i] = next++;
   if (n > 0) TSPH_HIP(hipMemcpy(c->cur.seq, nseq.data(), 4 * (size_t)n, hipMemcpyHostToDevice));
+  int nwall = 0;  // walls of the last cell list (0: none since the upload)
+  TSPH_HIP(hipMemcpy(&nwall, &c->scal[c->nwall_idx], sizeof(int), hipMemcpyDeviceToHost));
+  std::vector<int2> walls((size_t)nwall);
+  if (nwall > 0) {
+    TSPH_HIP(hipMemcpy(walls.data(), c->wall_list, walls.size() * sizeof(int2), hipMemcpyDeviceToHost));
+    for (int2 &w : walls) w.y = (int)nseq[w.x];
+    TSPH_HIP(hipMemcpy(c->wall_list, walls.data(), walls.size() * sizeof(int2), hipMemcpyHostToDevice));
+  }
   TSPH_HIP(hipMemcpy(c->seqstate, nst.data(), (size_t)c->seq_cap, hipMemcpyHostToDevice));
   const int ms = (int)next;
   TSPH_HIP(hipMemcpy(&c->scal[S_MAXSEQ], &ms, sizeof(int), hipMemcpyHostToDevice));
