@@ -363,6 +363,21 @@ int tsph_abi_version(void) { return TSPH_ABI_VERSION; }
 
 namespace tsph {
 
+// Consts::r2max, by bisection over the non-negative doubles (ordered as their bits)
+static double support_r2(double h) {
+  auto value = [](uint64_t bits) {
+    double x;
+    std::memcpy(&x, &bits, sizeof x);
+    return x;
+  };
+  uint64_t in = 0, out = 0x7ff0000000000000ull;  // 0 and infinity
+  while (out - in > 1) {
+    const uint64_t mid = in + (out - in) / 2;
+    (std::sqrt(value(mid)) / h <= 2.0 ? in : out) = mid;
+  }
+  return value(in);
+}
+
 // Particle_system constructor + Divide_To_Cells for one case's constants
 static int make_consts(const tsph_params *prm, Consts &k) {
   if (!(prm->h > 0) || !(prm->kap > 0) || !(prm->dp > 0) || prm->capacity <= 0 ||
@@ -383,6 +398,7 @@ static int make_consts(const tsph_params *prm, Consts &k) {
   k.ih = 1. / prm->h;
   k.cb = prm->cs * prm->cs * prm->rho0 / 7.;
   k.icb = 1. / k.cb;
+  k.r2max = support_r2(prm->h);
   k.ncx = (int)((k.xm - k.x0 + k.of) / k.kh) + 1;  // src/SPH_find_pairs.h:19-20
   k.ncy = (int)((k.ym - k.y0 + k.of) / k.kh) + 1;
   const long long nc = (long long)k.ncx * k.ncy;

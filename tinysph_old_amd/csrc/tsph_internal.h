@@ -118,6 +118,9 @@ struct Consts {
   double kh, of;
   double awen, bwen;  // float-rounded Wendland constants, src/SPH_kernel.h:56-57
   double ih, cb, icb; // 1/h, cs^2 rho0 / 7, 1/cb
+  // the largest r^2 whose rounded sqrt(r^2) / h is at most 2: r^2 <= r2max is the
+  // reference's qq <= 2 without its root and division (both are monotonic)
+  double r2max;
   int ncx, ncy, ncells;
   // batched ensembles: the case's first global cell id and its time step
   // (single cases: 0 and unused)

@@ -77,7 +77,8 @@ __host__ __device__ __forceinline__ PairConsts pair_consts(const Consts &k) {
   return {k.h, k.ih, k.awen, k.bwen, k.cs, k.avisc, k.delta, k.m, k.gx, k.gy, k.rho0, k.cb, k.icb, k.dp};
 }
 
-// (airho, nirho = recip64 of the densities)
+// (airho, nirho = recip64 of the densities; the pair is inside the support,
+// Consts::r2max: beyond it a zero kernel times an infinite value would be NaN)
 template <int VAR, class K>
 __device__ __forceinline__ void pair64(const K &k, Acc64 &s, double2 ar, double2 av, double arho,
                                        double airho, double ap, double2 nr, double2 nv, double nrho,
@@ -86,7 +87,6 @@ __device__ __forceinline__ void pair64(const K &k, Acc64 &s, double2 ar, double2
   const double h = k.h;
   const double drx = ar.x - nr.x, dry = ar.y - nr.y;
   const Root64 rt = sqrt64((drx * drx) + (dry * dry));
-  // beyond the exact support (qq > 2) the kernel is 0 and so is every term
   const double drs = rt.s, qq = quot64(drs, h, k.ih);
   npair += qq < 2.0;
   const KW64 kw = wendland64(rt, qq, k.awen, k.bwen);
@@ -249,9 +249,12 @@ __device__ void particle64_global(const D &d, const int *__restrict__ cell_start
       const int nt = VAR != TSPH_FORCES_WCSPH ? d.type[j] : 0;
       if (VAR == TSPH_FORCES_DBC && at == TSPH_WALL && nt == TSPH_WALL) continue;
       ++ncand;
+      const double2 nr = d.r[j];
+      const double drx = ar.x - nr.x, dry = ar.y - nr.y;
+      if (drx * drx + dry * dry > g.c2) continue;
       const double2 nb = (VAR == TSPH_FORCES_BT) ? d.n[j] : make_double2(0., 0.);
       const double nrho = d.rho[j];
-      pair64<VAR>(k, s, ar, av, arho, airho, ap, d.r[j], d.v[j], nrho, recip64(nrho), d.p[j], nt, nb,
+      pair64<VAR>(k, s, ar, av, arho, airho, ap, nr, d.v[j], nrho, recip64(nrho), d.p[j], nt, nb,
                   npair);
     }
   }
@@ -467,12 +470,11 @@ __global__ __launch_bounds__(kWave * kPoolWaves) void k_tile64(Soa d, const int 
     // walk of the 9 stencil cells in reference order: cell q, LDS range [lj, lend).
     // A cell's candidates are tested kGroup at a time (their LDS loads in
     // flight together) and appended without branches: every slot of the group
-    // is written, the count advances by the test.  The test admits a superset
-    // of the support (r^2 <= 4h^2 (1 + 1e-12)); pair64 applies the reference's
-    // exact qq <= 2, and a candidate it drops adds nothing, as in the
-    // reference, so the list keeps every pair in the reference order.  Slots
-    // past the cell's end are masked (they lie inside the wave's LDS area).
-    const double c2 = 4.0 * k.h * k.h * (1.0 + 1e-12);
+    // is written, the count advances by the test, which is the reference's
+    // qq <= 2 (Consts::r2max), so the list holds the pairs in the reference
+    // order.  Slots past the cell's end are masked (they lie inside the wave's
+    // LDS area).
+    const double c2 = k.r2max;
     const bool dbc_wall = VAR == TSPH_FORCES_DBC && at == TSPH_WALL;
     int q = -1, lj = 0, lend = 0;
     bool more = act;

@@ -485,10 +485,9 @@ __device__ __forceinline__ int slice_of(const Tile &t, int l) {
 //   kWaves                        wavefronts of a workgroup
 //   kFlag                         sums() wants to know whether any of the
 //                                 particle's pairs has bit 1 set (below)
-//   terms(L, p, l, double (&t)[kSums])  the terms of pair (p, l), zeros
-//                                 beyond the exact support (the lists hold
-//                                 r^2 <= 4h^2 (1 + 1e-12)); bit 0 of the result:
-//                                 it counts as a pair interaction, bit 1: a flag
+//   terms(L, p, l, double (&t)[kSums])  the terms of pair (p, l), which is
+//                                 inside the support (Consts::r2max); bit 0 of the
+//                                 result: it counts as a pair interaction, bit 1: a flag
 //   sums(L, p, i, const double (&s)[kSums], flag)  writes particle i, slot p
 //   far(i, cs, g, c, counts...)   particle i of cell c from global memory
 constexpr int kCellSlots = 104;  // staged slots of a cell's neighbourhood
@@ -517,10 +516,10 @@ constexpr int cell_lds_bytes() {
 // what a cell walk knows of a case's grid
 struct CellGrid {
   int ncx, ncy, cell_base;
-  double c2;  // 4h^2 (1 + 1e-12)
+  double c2;  // Consts::r2max
 };
 __host__ __device__ __forceinline__ CellGrid cell_grid(const Consts &k) {
-  return {k.ncx, k.ncy, k.cell_base, 4.0 * k.h * k.h * (1.0 + 1e-12)};
+  return {k.ncx, k.ncy, k.cell_base, k.r2max};
 }
 
 // case whose cell range holds global cell c
@@ -708,9 +707,8 @@ __device__ __forceinline__ void cells64(P &pol, CellGrid g, const int *__restric
           unsigned long long m[2];
 #pragma unroll
           for (int h = 0; h < 2; ++h) {
-            // (fused: the superset's margin covers the rounding)
             const double drx = own.x - cp[h].x, dry = own.y - cp[h].y;
-            m[h] = __ballot(__builtin_fma(drx, drx, dry * dry) <= g.c2);
+            m[h] = __ballot(drx * drx + dry * dry <= g.c2);
             if (skips) m[h] &= ~skp[h];
           }
           m[0] &= ~(1ull << q);
