@@ -10,8 +10,15 @@ import numpy as np
 import pytest
 
 import tinysph_old_amd as T
+from oracle import pyoracle as po
+from tests.helpers import oracle_for, oracle_init, oracle_variant
 
 pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _oracle(oracle_built):
+    return oracle_built
 
 
 def state(preset, dx, crowd):
@@ -80,3 +87,21 @@ def test_spoilt_particle_reaches_its_support_only(preset, walk, crowd):
     for what, got in each:
         for k in got:
             assert np.array_equal(got[k][qq > 2], clean[k][qq > 2], equal_nan=True), (what, k)
+
+
+@pytest.mark.parametrize("preset,walk,crowd", WALKS)
+def test_sums_over_a_spoilt_particle_are_the_oracles(preset, walk, crowd):
+    """Within 2h: the same infinities, and NaN where the oracle's expressions give NaN.
+    (No other value is spoilt, so the oracle's sums over nine cells differ from sums
+    over the support by exact zeros.)"""
+    case, qq, _, each = spoilt(preset, walk, crowd)
+    inside = (qq <= 2) & (qq > 0)
+    for what, got in each:
+        O = oracle_for(case)
+        oracle_init(O)
+        O.call("compute_forces", oracle_variant(case.wall))
+        for k, ref in (("a", O.get(po.F_A)), ("drho", O.get(po.F_DRHO))):
+            x, y = got[k][inside], ref[inside]
+            assert np.array_equal(np.isnan(x), np.isnan(y)), (what, k)
+            inf = np.isinf(y)
+            assert np.array_equal(np.isinf(x), inf) and np.array_equal(x[inf], y[inf]), (what, k)
