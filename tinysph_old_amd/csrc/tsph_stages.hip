@@ -7,6 +7,7 @@
 //   Water_Elevation(_inverse)      src/SPH_water_level.h:6-150
 //   Kernel_velocity_approximation_TEST  src/testing.h:6-148
 // The streaming stages are HBM-bound (a few flops per 16-100 bytes).
+#include <climits>
 #include <cmath>
 #include <vector>
 
@@ -591,7 +592,9 @@ int launch_remove(tsph_ctx *c) {
 int run_water_elevation(tsph_ctx *c, double x, double y0, int inverse, double *out) {
   const Consts &k = c->k;
   const double dp_wl = k.dp * 0.00005;
-  const int nmax = int(k.ym / dp_wl);
+  // heights up to the top, as many as an int counts (a conversion beyond that is
+  // undefined on the host; on the device it saturates)
+  const int nmax = (int)std::clamp(k.ym / dp_wl, (double)INT_MIN, (double)INT_MAX);
   *out = NAN;
   // the march is out of the domain after sqrt(2 distance / dp_wl) heights; one
   // launch covers that, and the few calls that march on take more of them
