@@ -415,7 +415,9 @@ int tsph_batch_step(tsph_ctx *ctx, int wall, int nsteps);
  * wavefront take the particles of its tile in turn, so the depth sets the
  * particles per lane (thread): the depths above span about one to three at
  * the configured resolutions, and *particles_per_lane returns the chosen
- * tiling's mean (particles / (64 x non-empty tiles)).  Needs a cell list;
+ * tiling's mean (particles / (64 x non-empty tiles)).  FP64 passes over at most
+ * 70,000 particles go by cells and depend on none of this: there the settings
+ * stay as they are and the pass is timed with them.  Needs a cell list;
  * leaves a, drho as one pair pass with the chosen setting leaves them.
  * Outputs may be NULL.  No counterpart in the reference. */
 int tsph_autotune(tsph_ctx *ctx, int variant, int *tile_rows, int *waves_per_cu, int *balanced,

@@ -1865,53 +1865,65 @@ int tsph_autotune(tsph_ctx *c, int variant, int *tile_rows, int *waves_per_cu, i
     (void)hipEventDestroy(e0);
     return fail(TSPH_EHIP, "hipEventCreate failed");
   }
-  int best_r = c->tile_rows, best_w = c->waves_per_cu, best_b = 0, e = 0;
-  float best = 1e30f;
+  // a pass by cells depends on none of the settings: they stay as they are (and
+  // the rows, if by default, go on following the particle count)
+  const bool tiles = !cells_walk(c);
+  struct Setting {
+    int balanced, rows, waves;
+  } best{c->balanced[c->prm.precision == TSPH_PREC_MIXED], c->tile_rows, c->waves_per_cu};
+  std::vector<Setting> tried;
+  if (tiles) {
+    for (int b = 0; b < 2; ++b)
+      for (int r : kRows)
+        for (int w : kWaves) tried.push_back({b, r, w});
+  } else {
+    tried.push_back(best);
+  }
+  auto apply = [&](const Setting &t) -> int {
+    int e = 0;
+    if (tiles && ((e = tsph_set_balanced(c, t.balanced)) || (e = tsph_set_tile_rows(c, t.rows)) ||
+                  (e = tsph_set_waves_per_cu(c, t.waves))))
+      return e;
+    return launch_forces(c, variant);
+  };
+  float least = 1e30f;
+  int e = 0;
   // every candidate recomputes the same pair pass: its outputs a and drho are
   // overwritten from the unchanged state
-  for (int bal = 0; bal < 2 && !e; ++bal) {
-    if ((e = tsph_set_balanced(c, bal))) break;
-    for (int r : kRows) {
-      if ((e = tsph_set_tile_rows(c, r))) break;
-      for (int w : kWaves) {
-        if ((e = tsph_set_waves_per_cu(c, w)) || (e = launch_forces(c, variant))) break;  // warm-up
-        // a pooled walk is timed with chunks cut by the tile costs the
-        // warm-up recorded (its own chunks were cut by estimates)
-        c->list_groups = 0;
-        if ((e = launch_forces(c, variant))) break;
-        // Every timed pass follows a cell-list build, as in a step: the build
-        // re-sorts the sorted state (which leaves it as it is) and cuts a
-        // pooled pass's chunks.  Passes repeated on one build favoured the
-        // static walk, which then ran slower in whole steps (740k-particle dam
-        // break: 0.68 against 0.63 ms per FP64 step).
-        float ms = 0.f;
-        for (int k = 0; k < kReps && !e; ++k) {
-          c->cut_groups = pass_groups(c, variant);
-          c->cut_table = 0;
-          if ((e = launch_cell_list(c, false))) break;
-          if (c->prm.precision == TSPH_PREC_MIXED) {
-            if ((e = launch_mixed_records(c))) break;
-            c->records_valid = true;
-          }
-          float rep = 0.f;
-          if (hipEventRecord(e0, c->stream) != hipSuccess) { e = fail(TSPH_EHIP, "event record failed"); break; }
-          if ((e = launch_forces(c, variant))) break;
-          if (hipEventRecord(e1, c->stream) != hipSuccess || hipEventSynchronize(e1) != hipSuccess ||
-              hipEventElapsedTime(&rep, e0, e1) != hipSuccess) {
-            e = fail(TSPH_EHIP, "event timing failed");
-            break;
-          }
-          ms += rep;
-        }
-        if (e) break;
-        if (ms < best) {
-          best = ms;
-          best_r = r;
-          best_w = w;
-          best_b = bal;
-        }
+  for (const Setting &t : tried) {
+    if ((e = apply(t))) break;  // warm-up
+    // a pooled walk is timed with chunks cut by the tile costs the
+    // warm-up recorded (its own chunks were cut by estimates)
+    c->list_groups = 0;
+    if ((e = launch_forces(c, variant))) break;
+    // Every timed pass follows a cell-list build, as in a step: the build
+    // re-sorts the sorted state (which leaves it as it is) and cuts a
+    // pooled pass's chunks.  Passes repeated on one build favoured the
+    // static walk, which then ran slower in whole steps (740k-particle dam
+    // break: 0.68 against 0.63 ms per FP64 step).
+    float ms = 0.f;
+    for (int k = 0; k < kReps && !e; ++k) {
+      c->cut_groups = pass_groups(c, variant);
+      c->cut_table = 0;
+      if ((e = launch_cell_list(c, false))) break;
+      if (c->prm.precision == TSPH_PREC_MIXED) {
+        if ((e = launch_mixed_records(c))) break;
+        c->records_valid = true;
       }
-      if (e) break;
+      float rep = 0.f;
+      if (hipEventRecord(e0, c->stream) != hipSuccess) { e = fail(TSPH_EHIP, "event record failed"); break; }
+      if ((e = launch_forces(c, variant))) break;
+      if (hipEventRecord(e1, c->stream) != hipSuccess || hipEventSynchronize(e1) != hipSuccess ||
+          hipEventElapsedTime(&rep, e0, e1) != hipSuccess) {
+        e = fail(TSPH_EHIP, "event timing failed");
+        break;
+      }
+      ms += rep;
+    }
+    if (e) break;
+    if (ms < least) {
+      least = ms;
+      best = t;
     }
   }
   (void)hipEventDestroy(e0);
@@ -1919,13 +1931,11 @@ int tsph_autotune(tsph_ctx *c, int variant, int *tile_rows, int *waves_per_cu, i
   if (e) return e;
   // a last pass with the chosen setting, so that a and drho are what a pair
   // pass with it leaves (the mixed path rounds in a tile-relative frame)
-  if ((e = tsph_set_balanced(c, best_b)) || (e = tsph_set_tile_rows(c, best_r)) ||
-      (e = tsph_set_waves_per_cu(c, best_w)) || (e = launch_forces(c, variant)))
-    return e;
-  if (tile_rows) *tile_rows = best_r;
-  if (waves_per_cu) *waves_per_cu = best_w;
-  if (balanced) *balanced = best_b;
-  if (best_ms) *best_ms = best / kReps;
+  if ((e = apply(best))) return e;
+  if (tile_rows) *tile_rows = best.rows;
+  if (waves_per_cu) *waves_per_cu = best.waves;
+  if (balanced) *balanced = best.balanced;
+  if (best_ms) *best_ms = least / kReps;
   if (particles_per_lane) {
     // the chosen depth's particles per lane: every particle belongs to one
     // tile of the list, whose 64 lanes take its particles in turn

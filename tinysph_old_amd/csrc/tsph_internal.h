@@ -428,6 +428,8 @@ int clear_tile_costs(tsph_ctx *c);
 // cuts the current tile list into `groups` chunks by cost table `table` on
 // stream s (gathering the listed tiles' costs first unless the list build did)
 int launch_cut(tsph_ctx *c, hipStream_t s, int groups, int table);
+// whether the pair pass goes by cells instead of tiles
+bool cells_walk(const tsph_ctx *c);
 // workgroups of a pair pass of `variant` if it takes the pooled walk, else 0
 int pass_groups(tsph_ctx *c, int variant);
 // corr (mixed path only): the pass also applies the symplectic corrector to

@@ -1026,7 +1026,7 @@ TileGrid tile_grid(tsph_ctx *c, bool fp32, size_t lds_wave, bool may_pool) {
 // are walked whole (its tile list runs over all cases), so only up to
 // kCellsDirect cells.
 constexpr int kCellsMax = 70000;
-static bool cells_walk(const tsph_ctx *c) {
+bool cells_walk(const tsph_ctx *c) {
   return c->prm.precision == TSPH_PREC_FP64 && c->n_ub <= kCellsMax && (!c->cases || cells_direct(c));
 }
 
