@@ -432,6 +432,10 @@ int tsph_autotune(tsph_ctx *ctx, int variant, int *tile_rows, int *waves_per_cu,
  * by cells instead of tiles and do not depend on the setting.
  * Results do not depend on it.  No counterpart in the reference. */
 int tsph_set_balanced(tsph_ctx *ctx, int balanced);
+/* The walk that a pair pass of `variant` takes on the present state (0 by
+ * cells, 1 static tiles, 2 pooled tiles), and the entries of the present tile
+ * list.  Outputs may be NULL.  No counterpart in the reference. */
+int tsph_get_pair_walk(tsph_ctx *ctx, int variant, int *walk, int *entries);
 /* Per-cell order of the cell-list build (Particle_To_Cell's push_back in
  * ascending particle index, src/SPH_find_pairs.h:45-92): 1 = ranked by the
  * pass that moves the particles (each particle counts those of its cell with

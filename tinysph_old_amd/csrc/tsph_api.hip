@@ -407,18 +407,23 @@ static int make_consts(const tsph_params *prm, Consts &k) {
   return 0;
 }
 
-// entries of a cell's row: one and a half times the particles that a lattice of
-// spacing dp puts in a cell (the reference cases: 8 in a cell of 2.83 dp), as a
-// power of two, so that only cells packed well beyond the lattice are chained;
-// 0: cells too full for rows
-static int row_width_of(const tsph_ctx *c) {
+// particles that a lattice of spacing dp puts in a cell (the reference cases: 9 in
+// a cell of 2.97 dp), the most of the cases
+static double cell_lattice_of(const tsph_ctx *c) {
   double most = 0.;
   for (int q = 0; q < c->ncases; ++q) {
     const Consts &k = c->host_cases.empty() ? c->k : c->host_cases[q];
     most = std::max(most, k.kh / k.dp * (k.kh / k.dp));
   }
+  return most;
+}
+
+// entries of a cell's row: one and a half times the lattice's, as a power of two,
+// so that only cells packed well beyond the lattice are chained; 0: cells too
+// full for rows
+static int row_width_of(const tsph_ctx *c) {
   int w = 16;
-  while (w < 1.5 * most && w <= 128) w *= 2;
+  while (w < 1.5 * c->cell_lattice && w <= 128) w *= 2;
   return w <= 128 ? w : 0;
 }
 
@@ -429,6 +434,7 @@ static int alloc_context(tsph_ctx *c) {
   if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess)
     return fail(TSPH_EHIP, "hipStreamCreate failed");
   const int cap = c->capacity, nct = c->ncells_tot;
+  c->cell_lattice = cell_lattice_of(c);
   c->seq_cap = 2 * cap + kBzMax + c->ncases;
   const size_t slots = std::max<size_t>(cap, dl_words(c->seq_cap));
   if ((e = alloc_soa(c->cur, cap)) || (e = alloc_soa(c->alt, cap)) ||
@@ -1836,6 +1842,18 @@ int tsph_set_balanced(tsph_ctx *c, int on) {
   bool &b = c->balanced[c->prm.precision == TSPH_PREC_MIXED ? 1 : 0];
   if (b != (on != 0)) drop_graph(c);
   b = on != 0;
+  return 0;
+}
+
+int tsph_get_pair_walk(tsph_ctx *c, int variant, int *walk, int *entries) {
+  if (!c) return fail(TSPH_EINVAL, "null argument");
+  if (variant < TSPH_FORCES_WCSPH || variant > TSPH_FORCES_BT) return fail(TSPH_EINVAL, "unknown variant");
+  if (!c->cells_valid) return fail(TSPH_ESTATE, "no cell list: call tsph_particle_to_cell first");
+  if (walk) *walk = cells_walk(c) ? 0 : pass_groups(c, variant) > 0 ? 2 : 1;
+  if (entries) {
+    TSPH_HIP(hipStreamSynchronize(c->stream));
+    TSPH_HIP(hipMemcpy(entries, c->scal + S_NTILES, sizeof(int), hipMemcpyDeviceToHost));
+  }
   return 0;
 }
 

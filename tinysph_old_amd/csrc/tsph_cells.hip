@@ -1191,9 +1191,9 @@ int launch_cell_list(tsph_ctx *c, bool eos, bool predict, double dt, unsigned ad
     set_error("tile list: more pooled workgroups than allocated");
     return TSPH_ESTATE;
   }
-  // two entries for the fuller tiles where static tile walks follow (the FP64
-  // lists also serve the cell walks, and k_order_tiles takes each tile once)
-  const bool split = rank && cut == 0 && c->prm.precision == TSPH_PREC_MIXED;
+  // two entries for the fuller tiles (the FP64 lists also serve the cell walks,
+  // and k_order_tiles takes each tile once)
+  const bool split = rank && cut == 0 && c->prm.precision == TSPH_PREC_MIXED && split_pays(c);
   const ScanArgs sa = scan_args(c, cs, cut > 0 ? c->cut_table : -1, split);
   const bool own_scan = !(rank && binned) || cut > 0 || (hashed && walls);
   if (own_scan)

@@ -165,6 +165,7 @@ struct tsph_ctx {
   int capacity = 0;
   int n_ub = 0;  // host upper bound of the device particle count
   int ncells_tot = 0;            // cells of all cases (the single case: k.ncells)
+  double cell_lattice = 0.;      // particles that a lattice of spacing dp puts in a cell (the most of the cases)
   // batched ensembles: per-case constants on the device (nullptr for one case)
   int ncases = 1;
   tsph::Consts *cases = nullptr;
@@ -337,6 +338,19 @@ constexpr int kPoolMixed = 95, kPoolFp64 = 150;  // particles per wave
 constexpr int kTileRows = 7, kTileRowsFp64 = 6;
 inline bool walk_balanced(const tsph_ctx *c, bool fp32, int waves) {
   return c->balanced[fp32 ? 1 : 0] && c->n_ub >= (long long)(fp32 ? kPoolMixed : kPoolFp64) * waves;
+}
+// Whether a mixed system's tile list gives the fuller tiles two entries
+// (tiles::entry_part): where a wave has about a tile, that is up to the pooled
+// walk's limit.  Above it for the ALE passes alone, which always stride, and only
+// where a tile of the lattice is no fuller than a wavefront: if all tiles had two
+// entries, the waves, which stride by an even number, would meet only first or
+// only second ones.  us per step, one entry and two: ALE of 324k particles after
+// 1500 steps 431 and 377, of 727k 808 and 800; of 727k with 74 particles per tile
+// 1619 and 2160, Riemann-ALE 560 and 620.  (A pooled pass would list anew: 293k
+// particles stage by stage 85 and 91.)
+inline bool split_pays(const tsph_ctx *c) {
+  if (c->n_ub < (long long)kPoolMixed * c->num_cu * c->waves_per_cu) return true;
+  return c->has_ale && c->tile_rows * c->cell_lattice <= 64.;
 }
 
 // launch geometry of a tile kernel: `groups` workgroups (a multiple of 8) of

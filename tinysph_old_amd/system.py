@@ -449,6 +449,13 @@ class ParticleSystem:
     def set_balanced(self, on: bool):
         L.check(self.lib.tsph_set_balanced(self.ctx, int(bool(on))), "tsph_set_balanced")
 
+    def pair_walk(self, variant: int):
+        """(0 by cells, 1 static tiles, 2 pooled tiles; entries of the tile list)."""
+        w, n = C.c_int(), C.c_int()
+        L.check(self.lib.tsph_get_pair_walk(self.ctx, variant, C.byref(w), C.byref(n)),
+                "tsph_get_pair_walk")
+        return w.value, n.value
+
     def set_cell_order(self, mode: int):
         """0 (default), 1: ranked by the reorder, 2: placement and ordering passes."""
         L.check(self.lib.tsph_set_cell_order(self.ctx, mode), "tsph_set_cell_order")
