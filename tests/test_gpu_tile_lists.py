@@ -55,3 +55,36 @@ def test_entries_of_ale_systems(h_dp, split):
         ps.particle_to_cell()
         own = tiles(ps, ps.tile_rows)
         assert ps.pair_walk(T.FORCES_BT)[1] == len(own) + (int((own > 64).sum()) if split else 0)
+
+
+@pytest.mark.parametrize("precision,dx", [(T.PREC_FP64, 0.0033), (T.PREC_MIXED, 0.005)], ids=["fp64", "mixed"])
+def test_passes_stage_by_stage(precision, dx):
+    """A build cuts the chunks for a pass of the last variant; one of another variant, of
+    other settings or without a pass between gives the same bits as the static walk."""
+    case = crowded(T.CASE_DAM_BREAK_MDBC, dx, 0.8, 7)
+    print(f"[case] stage by stage np={case.np} precision {precision}", flush=True)
+    out = []
+    for pooled in (True, False):
+        got = []
+        with T.system_for_case(case, precision=precision) as ps:
+            ps.set_balanced(pooled)
+            ps.set_waves_per_cu(1)
+            for variant in (T.FORCES_WCSPH, T.FORCES_WCSPH, T.FORCES_DBC, T.FORCES_DBC, T.FORCES_WCSPH):
+                ps.particle_to_cell()
+                assert ps.pair_walk(variant)[0] == (2 if pooled else 1)
+                ps.density_to_pressure()
+                ps.compute_forces(variant)
+                got.append(ps.download(("a", "drho")))
+            ps.particle_to_cell()
+            ps.particle_to_cell()
+            ps.density_to_pressure()
+            if pooled:  # fewer chunks than the build has cut
+                ps.set_balanced(False)
+                ps.compute_forces(T.FORCES_WCSPH)
+                ps.set_balanced(True)
+            ps.compute_forces(T.FORCES_WCSPH)
+            got.append(ps.download(("a", "drho")))
+            out.append(got)
+    for x, y in zip(*out):
+        for k in x:
+            assert np.array_equal(x[k], y[k], equal_nan=True), k

@@ -206,6 +206,7 @@ struct tsph_ctx {
   // a pooled pair pass of `cut_groups` workgroups and cost table `cut_table`
   // follows the next cell build (0: none): the build cuts its chunks
   int cut_groups = 0, cut_table = 0;
+  int last_variant = TSPH_FORCES_WCSPH;  // of the last pair pass
   // {slot, reference position} of the wall particles of the current cell list
   int2 *wall_list = nullptr;
   int n_wall = 0;            // wall particles (walls are never created or removed)

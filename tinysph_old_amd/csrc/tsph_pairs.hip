@@ -1102,6 +1102,7 @@ int launch_forces(tsph_ctx *c, int variant, bool corr, double corr_dt, bool wall
   const int rows = c->tile_rows;
   const int cap = 3 * (rows + 2) * kCellCap;
   const bool mixed = c->prm.precision == TSPH_PREC_MIXED;
+  c->last_variant = variant;
   if (mixed && !c->records_valid) {
     if (int e = launch_mixed_records(c)) return e;
     c->records_valid = true;
