@@ -1,0 +1,34 @@
+"""FP32 ALE passes under budgets of LDS records from the least to the most.
+
+The budget follows the waves per compute unit; a tile beyond it is taken in runs of
+rows of the same frame, and one row beyond it from global memory.  The bits do not
+depend on it.
+"""
+import numpy as np
+import pytest
+
+import tinysph_old_amd as T
+from tests.test_gpu_full_tiles import CROWDS, crowded
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("spacing,cells", CROWDS, ids=str)
+def test_bits_do_not_depend_on_the_waves(spacing, cells):
+    case = crowded(T.CASE_ALE_DAM_BREAK, 0.0042, spacing, cells)
+    print(f"[case] ale budget spacing {spacing} cells {cells} np={case.np}", flush=True)
+    out = []
+    for waves in (1, 5, 8, 11, 12, 13, 24):
+        with T.system_for_case(case, precision=T.PREC_MIXED) as ps:
+            ps.set_waves_per_cu(waves)
+            ps.ale_enable()
+            ps.particle_to_cell()
+            ps.ale_kernel_gradient()
+            ps.ale_compute_density(True)
+            ps.ale_compute_acceleration(True)
+            out.append((ps.ale_download(), ps.counters()))
+    for fields, counts in out[1:]:
+        for k, v in out[0][0].items():
+            assert np.array_equal(v, fields[k], equal_nan=True), k
+        for k in ("pairs", "candidates", "active"):
+            assert counts[k] == out[0][1][k], k

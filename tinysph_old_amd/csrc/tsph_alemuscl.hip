@@ -829,24 +829,24 @@ __global__ void k_ale_lf2(Soa d, const int *__restrict__ scal, double dt, int fi
 template <class P, int SLOT>
 int launch_pass32(tsph_ctx *c, const P &pol) {
   const int rows = c->tile_rows;
-  // Slots per tile.  The ALE records are large (57 B with the MUSCL
-  // gradients) and the waves that a compute unit holds pay, so systems that
-  // fill the chip are budgeted kAleCellCap records per cell, which the fullest
-  // tiles of a running dam break just need: us per step with 9 and 10 records,
-  // at the start and after some thousand steps, 727k particles 770 and 807, 841
-  // and 811; 183k 236 and 238, 284 and 247 (a tile beyond the budget is taken
-  // in two runs; gathered from global memory instead, 183k took 467).  What
-  // those waves leave over, and all that fewer waves leave over in a system
-  // without a tile for each of them, goes to the tiles, up to kCellCap records
-  // per cell (47k particles after 1300 steps: 135, 357 with 9 records).
-  constexpr int kAleCellCap = 10;
+  // Slots per tile.  The ALE records are large (57 B with the MUSCL gradients)
+  // and the waves that a compute unit holds pay, so the budget is at least
+  // kAleCellCap records per cell (the lattice's), and beyond that what the waves
+  // leave over that it holds at once: those that fit with kAleCellCap records, no
+  // more than the launch has, and no more than the system has tiles for; up to
+  // kCellCap records per cell.  (A tile beyond its budget is taken in runs of
+  // rows.)  us per step, at the start and after 1500 steps, against 10 records
+  // for every pass, of which a compute unit held 11 of the gradient pass's 12
+  // waves: 727k particles 767 and 800, now 729 and 760; 324k 362 and 379, 341 and
+  // 353; 183k 227 and 235, 224 and 234; 47k 118 and 129, 118 and 129.
+  constexpr int kAleCellCap = 9;
   constexpr int kFixed = kTabBytes + sizeof(uint16_t) * kList * kWave;
   const int most = std::min(3 * (rows + 2) * kCellCap, (65536 - kPoolHdr - kFixed) / SLOT);
   const int base = std::min(3 * (rows + 2) * kAleCellCap, most);
   const int lds = kStaticHdr + kFixed + 32;  // (with the rounding to allocation granules below)
   const int fit = std::max(1, c->lds_cu / (lds + base * SLOT));
   const int want = std::max(1, grid_for(c->n_ub, 48 * c->num_cu));
-  const int share = c->lds_cu / std::min(fit, want) / kLdsGranule * kLdsGranule;
+  const int share = c->lds_cu / std::min({fit, want, c->waves_per_cu}) / kLdsGranule * kLdsGranule;
   const int cap = std::max(base, std::min(most, (share - lds) / SLOT));
   // the static walk: a cell build serves several passes of different cost
   // profiles, and the dam breaks these passes run on give each wave about ten
