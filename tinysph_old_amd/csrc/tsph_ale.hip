@@ -516,7 +516,7 @@ int launch_rale_forces(tsph_ctx *c) {
   } else {
     constexpr int lds = cell_lds_bytes<RaleCell64>();
     const Soa &d = c->cur;
-    if (!cells_direct(c) && (e = ensure_tile_list(c, 0))) return e;
+    if ((e = ensure_cell_entries(c))) return e;
     const int groups = cell_groups(c, k_rale_cells64, RaleCell64::kWaves, lds, c->ale_fit[7]);
     e = launch_timed(c, [&] {
       hipLaunchKernelGGL(k_rale_cells64, dim3(groups), dim3(RaleCell64::kWaves * kWave), lds, s,

@@ -866,8 +866,7 @@ int launch_pass64(tsph_ctx *c, int slot) {
   using P = AleCell64<A>;
   constexpr int lds = cell_lds_bytes<P>();
   const Soa &d = c->cur;
-  if (!cells_direct(c))
-    if (int e = ensure_tile_list(c, 0)) return e;
+  if (int e = ensure_cell_entries(c)) return e;
   const int groups = cell_groups(c, k_ale_cells64<P>, P::kWaves, lds, c->ale_fit[slot]);
   return launch_timed(c, [&] {
     hipLaunchKernelGGL(k_ale_cells64<P>, dim3(groups), dim3(P::kWaves * kWave), lds, c->stream,

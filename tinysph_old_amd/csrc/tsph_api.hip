@@ -100,7 +100,7 @@ static void set_walk_defaults(tsph_ctx *c) {
 
 static HostState host_state(const tsph_ctx *c) {
   return {c->cells_valid, c->tiles_valid, c->records_valid, c->marks_valid, c->olds_stale,
-          c->list_split, c->list_groups, c->list_table, c->list_cost_table};
+          c->list_split, c->list_groups, c->list_table, c->list_cost_table, c->list_rows};
 }
 
 static void set_host_state(tsph_ctx *c, const HostState &h) {
@@ -113,6 +113,7 @@ static void set_host_state(tsph_ctx *c, const HostState &h) {
   c->marks_valid = h.marks_valid;
   c->olds_stale = h.olds_stale;
   c->list_split = h.list_split;
+  c->list_rows = h.list_rows;
 }
 
 // Runs nsteps steps from graphs: the graph of the current buffer parity is
@@ -480,7 +481,7 @@ static int alloc_context(tsph_ctx *c) {
   ar.add(c->perm, cap);
   ar.add(c->probe_out, kProbeOut);
   ar.add(c->bz_list, 2 * kBzMax);
-  ar.add(c->tile_list, 2 * ((size_t)nct + 8));
+  ar.add(c->tile_list, tile_list_room(c));
   ar.add(c->list_cost, nct + 8);
   ar.add(c->wall_list, cap);
   ar.add(c->scan_cost, words);

@@ -567,14 +567,15 @@ __device__ __forceinline__ void scan_block(const ScanArgs &sa, int blk, int nb,
 template <int IT, int WALLS>
 __global__ __launch_bounds__(kScanBlock, WALLS ? 4 : 1) void k_scan(ScanArgs sa, int *__restrict__ scal,
                                                      unsigned long long *__restrict__ counters,
-                                                     int wall_groups, WallPass wp, Consts k0) {
+                                                     int wall_groups, WallPass wp, Consts k0,
+                                                     const Consts *__restrict__ cases) {
   const int nb = gridDim.x - (WALLS ? wall_groups : 0), blk = blockIdx.x;
   if (WALLS && blk >= nb) {
     constexpr int kWaves = kScanBlock / 64;
     __shared__ __align__(16) double s_terms[kWaves * walls::kTerms];
     const int wid = threadIdx.x >> 6, b = (blk - nb) * kWaves + wid;
     if (b < wp.walls + wp.sweep)
-      wall_wave<WALLS ? WALLS : TSPH_WALL_MDBC>(b, wp, k0, sa.ts.cases, scal,
+      wall_wave<WALLS ? WALLS : TSPH_WALL_MDBC>(b, wp, k0, cases, scal,
                                                 s_terms + wid * walls::kTerms);
     return;
   }
@@ -1061,14 +1062,17 @@ bool cells_ranked(const tsph_ctx *c) { return c->row_width > 0 && c->cell_order 
 
 // the arguments of the scan of the cell counts into cs, with the tile list of
 // the current tile_rows (and, for cost_table >= 0, the listed tiles' costs)
-ScanArgs scan_args(tsph_ctx *c, int *cs, int cost_table, bool split) {
-  const TileScan ts{c->k.ncy, c->k.ncells, c->k.cell_base, c->cases, c->tile_base, c->ncases,
-                    c->tile_rows, c->tile_list,
+// or the list of non-empty cells
+ScanArgs scan_args(tsph_ctx *c, int *cs, int cost_table, bool split, bool cells) {
+  const TileScan ts{cells ? c->ncells_tot : c->k.ncy, cells ? c->ncells_tot : c->k.ncells,
+                    cells ? 0 : c->k.cell_base, cells ? nullptr : c->cases, c->tile_base, c->ncases,
+                    cells ? 1 : c->tile_rows, c->tile_list,
                     cost_table >= 0 ? c->scal + S_NSCAL + cost_table : nullptr,
                     cost_table >= 0 ? c->list_cost : nullptr,
                     cost_estimate(c->prm.precision == TSPH_PREC_MIXED), split, c->scan_cost,
                     c->scan_tile0};
   c->list_split = split;
+  c->list_rows = cells ? kListCells : c->tile_rows;
   c->list_groups = 0;  // a pooled pass cuts the new list
   c->list_cost_table = cost_table;
   return {c->cell_count, c->ncells_tot + 1, c->scan_state, c->scan_state_next, cs, ts, c->scan_wait};
@@ -1080,7 +1084,7 @@ int launch_scan(tsph_ctx *c, const ScanArgs &sa, int walls, const WallPass &wp) 
   const int wg = walls ? grid_for(wp.walls + wp.sweep, kScanBlock / 64) : 0;
 #define TSPH_SCAN(IT, W)                                                                        \
   hipLaunchKernelGGL((k_scan<IT, W>), dim3(scan_blocks(c) + wg), dim3(kScanBlock), 0, c->stream, \
-                     sa, c->scal, c->counters, wg, wp, c->k)
+                     sa, c->scal, c->counters, wg, wp, c->k, c->cases)
 #define TSPH_SCAN_W(IT)                                                                         \
   if (walls == TSPH_WALL_MDBC) TSPH_SCAN(IT, TSPH_WALL_MDBC);                                  \
   else if (walls == TSPH_WALL_BT) TSPH_SCAN(IT, TSPH_WALL_BT);                                 \
@@ -1194,7 +1198,9 @@ int launch_cell_list(tsph_ctx *c, bool eos, bool predict, double dt, unsigned ad
   // two entries for the fuller tiles (the FP64 lists also serve the cell walks,
   // and k_order_tiles takes each tile once)
   const bool split = rank && cut == 0 && c->prm.precision == TSPH_PREC_MIXED && split_pays(c);
-  const ScanArgs sa = scan_args(c, cs, cut > 0 ? c->cut_table : -1, split);
+  // the cells for the FP64 passes that go by cells
+  const bool cells = cut == 0 && c->prm.precision == TSPH_PREC_FP64 && (c->has_ale || cells_walk(c));
+  const ScanArgs sa = scan_args(c, cs, cut > 0 ? c->cut_table : -1, split, cells);
   const bool own_scan = !(rank && binned) || cut > 0 || (hashed && walls);
   if (own_scan)
     if (int e = launch_scan(c, sa, hashed ? walls : 0, wp)) return e;
@@ -1215,7 +1221,7 @@ int launch_cell_list(tsph_ctx *c, bool eos, bool predict, double dt, unsigned ad
                          c->perm, c->cell_count);
     else
       hipLaunchKernelGGL(k_order_tiles, dim3(kOrderWaves * std::max(1, c->num_cu)), dim3(nb), 0, s,
-                         cs, c->scal, c->tile_list, c->tile_rows, k.ncy, nct, c->cur.seq, c->perm,
+                         cs, c->scal, c->tile_list, cells ? 1 : c->tile_rows, k.ncy, nct, c->cur.seq, c->perm,
                          c->cell_count);
   }
   const Mixed mx = c->prm.precision == TSPH_PREC_MIXED ? c->mx : Mixed{};

@@ -137,7 +137,7 @@ __device__ __forceinline__ Consts case_consts(const Consts &k0, const Consts *__
 // host-side flags that describe what the device buffers hold
 struct HostState {
   bool cells_valid, tiles_valid, records_valid, marks_valid, olds_stale, list_split;
-  int list_groups, list_table, list_cost_table;
+  int list_groups, list_table, list_cost_table, list_rows;
 };
 
 // one captured step.  A step may rebuild the cell list an odd number of times
@@ -193,6 +193,7 @@ struct tsph_ctx {
   // tiles of the current cell list, in tile order (tiles::part of each)
   int *tile_list = nullptr;
   bool list_split = false;  // tiles of more than a wavefront of particles have two entries
+  int list_rows = 0;        // cells per listed tile (kListCells: the list is one of cells)
   bool tiles_valid = false;  // tile_list matches the cell list and tile_rows
   int *list_part = nullptr;  // per list-build block: tiles, work
   int list_part_cap = 0;     // list-build blocks list_part holds
@@ -435,6 +436,8 @@ inline unsigned forces_active_types(int variant) {
 // for a pooled walk of that many workgroups, cut by the tile costs recorded
 // in cost table `table`
 int ensure_tile_list(tsph_ctx *c, int groups, int table = 0);
+// list of the non-empty cells, for a cell walk
+int ensure_cell_entries(tsph_ctx *c);
 // geometry of a tile-kernel launch at the context's waves per CU (pooled when
 // may_pool and walk_balanced hold for the precision)
 TileGrid tile_grid(tsph_ctx *c, bool fp32, size_t lds_wave, bool may_pool = true);
@@ -445,6 +448,11 @@ int clear_tile_costs(tsph_ctx *c);
 int launch_cut(tsph_ctx *c, hipStream_t s, int groups, int table);
 // whether the pair pass goes by cells instead of tiles
 bool cells_walk(const tsph_ctx *c);
+// entries of the tile list's buffer
+inline size_t tile_list_room(const tsph_ctx *c) { return 2 * ((size_t)c->ncells_tot + 8); }
+// list_rows of a list of non-empty cells (global ids): what the cell walks go
+// through, listed like tiles of one cell of a grid with a single column
+constexpr int kListCells = 0;
 // workgroups of a pair pass of `variant` if it takes the pooled walk, else 0
 int pass_groups(tsph_ctx *c, int variant);
 // corr (mixed path only): the pass also applies the symplectic corrector to

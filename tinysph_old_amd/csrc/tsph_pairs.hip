@@ -958,30 +958,48 @@ int launch_cut(tsph_ctx *c, hipStream_t s, int groups, int table) {
   return 0;
 }
 
-int ensure_tile_list(tsph_ctx *c, int groups, int table) {
-  const Consts &k = c->k;
-  const int rows = c->tile_rows;
-  hipStream_t s = c->stream;
-  if (!c->tiles_valid || (groups > 0 && c->list_split)) {
-    const int ntiles = total_tiles(c);
-    const int nb = grid_for(ntiles, kListBlock);
-    if (nb > c->list_part_cap) {
-      set_error("tile list: more tiles than allocated");
-      return TSPH_ESTATE;
-    }
-    hipLaunchKernelGGL(k_tile_count, dim3(nb), dim3(kListBlock), 0, s, c->cell_start, k, c->cases,
-                       c->tile_base, c->ncases, rows, ntiles, c->list_part);
-    hipLaunchKernelGGL(k_tile_emit, dim3(nb), dim3(kListBlock), 0, s, c->cell_start, k, c->cases,
-                       c->tile_base, c->ncases, rows, ntiles, c->list_part, c->scal, c->tile_list);
-    TSPH_HIP(hipGetLastError());
-    c->tiles_valid = true;
-    c->list_split = false;
-    c->list_groups = 0;
-    c->list_cost_table = -1;
+// the list of the non-empty tiles of `rows` cells (kListCells: of the cells)
+static int relist(tsph_ctx *c, int rows) {
+  Consts k = c->k;
+  const Consts *cases = c->cases;
+  int ntiles = 0, per = rows;
+  if (rows == kListCells) {
+    k.ncx = 1;
+    k.ncy = ntiles = c->ncells_tot;
+    k.cell_base = 0;
+    cases = nullptr;
+    per = 1;
+  } else {
+    ntiles = total_tiles(c);
   }
-  if (groups > 0 && (groups != c->list_groups || table != c->list_table))
-    return launch_cut(c, s, groups, table);
+  const int nb = grid_for(ntiles, kListBlock);
+  if (nb > c->list_part_cap) {
+    set_error("tile list: more tiles than allocated");
+    return TSPH_ESTATE;
+  }
+  hipLaunchKernelGGL(k_tile_count, dim3(nb), dim3(kListBlock), 0, c->stream, c->cell_start, k, cases,
+                     c->tile_base, c->ncases, per, ntiles, c->list_part);
+  hipLaunchKernelGGL(k_tile_emit, dim3(nb), dim3(kListBlock), 0, c->stream, c->cell_start, k, cases,
+                     c->tile_base, c->ncases, per, ntiles, c->list_part, c->scal, c->tile_list);
+  TSPH_HIP(hipGetLastError());
+  c->tiles_valid = true;
+  c->list_rows = rows;
+  c->list_split = false;
+  c->list_groups = 0;
+  c->list_cost_table = -1;
   return 0;
+}
+
+int ensure_tile_list(tsph_ctx *c, int groups, int table) {
+  if (!c->tiles_valid || c->list_rows != c->tile_rows || (groups > 0 && c->list_split))
+    if (int e = relist(c, c->tile_rows)) return e;
+  if (groups > 0 && (groups != c->list_groups || table != c->list_table))
+    return launch_cut(c, c->stream, groups, table);
+  return 0;
+}
+
+int ensure_cell_entries(tsph_ctx *c) {
+  return c->tiles_valid && c->list_rows == kListCells ? 0 : relist(c, kListCells);
 }
 
 int clear_tile_costs(tsph_ctx *c) {
@@ -1022,12 +1040,10 @@ TileGrid tile_grid(tsph_ctx *c, bool fp32, size_t lds_wave, bool may_pool) {
 // kCellsMax particles.  A tile's wavefront takes about 25 us however small the
 // system is, a cell's 8 us, while a full chip does more pairs per second by
 // tiles (a dam break, us per pass, cells and tiles: 6k particles 9 / 41, 23k
-// 14 / 23, 50k 24 / 34, 92k 39 / 36, 740k 259 / 204).  A batch's grids
-// are walked whole (its tile list runs over all cases), so only up to
-// kCellsDirect cells.
+// 14 / 23, 50k 24 / 34, 92k 39 / 36, 740k 259 / 204).
 constexpr int kCellsMax = 70000;
 bool cells_walk(const tsph_ctx *c) {
-  return c->prm.precision == TSPH_PREC_FP64 && c->n_ub <= kCellsMax && (!c->cases || cells_direct(c));
+  return c->prm.precision == TSPH_PREC_FP64 && c->n_ub <= kCellsMax;
 }
 
 // LDS bytes per wavefront of the pair pass of `variant` at the current tile rows
@@ -1108,8 +1124,7 @@ int launch_forces(tsph_ctx *c, int variant, bool corr, double corr_dt, bool wall
     c->records_valid = true;
   }
   if (cells_walk(c)) {
-    if (!cells_direct(c))
-      if (int e = ensure_tile_list(c, 0)) return e;
+    if (int e = ensure_cell_entries(c)) return e;
     return launch_timed(c, [&] {
       switch (variant) {
         case TSPH_FORCES_WCSPH: cell_launch<TSPH_FORCES_WCSPH>(c); break;

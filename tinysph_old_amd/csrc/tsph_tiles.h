@@ -5,6 +5,7 @@
 #pragma once
 
 #include <algorithm>
+#include <climits>
 
 #include "tsph_internal.h"
 #include "tsph_physics.h"
@@ -595,13 +596,10 @@ __device__ __forceinline__ CellSlots cell_slots(int lo, int cnt, typename P::Rec
   return {dj[0], __builtin_amdgcn_readlane(cnt, 0), tot};
 }
 
-// where a cell walk finds its cells: among all cells of the grid, or (tiles
-// set; a single case) among those of the listed tiles
+// the list of non-empty cells (global ids, ascending) that a cell walk goes through
 struct CellSource {
-  int ncells;        // cells of all cases
-  const int *tiles;  // the list of non-empty tiles, of `rows` cells each
-  const int *ntiles;
-  int rows;
+  const int *list, *count;
+  int room;  // entries of the list's buffer
 };
 
 template <class P>
@@ -622,32 +620,35 @@ __device__ __forceinline__ void cells64(P &pol, CellGrid g, const int *__restric
   const int lane = tile_lane();
   if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&counters[C_PASSES], 1ull);
   unsigned npair = 0, ncand = 0, nact = 0, scand = 0, snact = 0;
-  // Runs of kCellRun cells are dealt to the 8 XCDs in turn, so that a run's
+  // Runs of kCellRun listed cells are dealt to the 8 XCDs in turn, so that a run's
   // cells share staged particles through one L2 while every XCD gets a share
   // of each part of the domain.  The workgroups of an XCD stride through its
-  // cells, a thread per cell to find the non-empty ones, which the workgroup's
-  // wavefronts take from a counter in LDS.
+  // cells, a cell per thread, and their wavefronts take them from a counter in
+  // LDS.  (Dealt by grid cell, empty ones included, every third column's water
+  // fell to the same XCD where 512 cells were about three columns, and to few of
+  // its workgroups where their stride was: 61k and 52k particles of the dam break
+  // 152 and 88 us per step, 99 and 86 now.)
   const int band = blockIdx.x & 7, nwb = gridDim.x >> 3, wb = blockIdx.x >> 3;
-  const int all = src.tiles ? *src.ntiles * src.rows : src.ncells;
-  const int mine = (all + 8 * kCellRun - 1) / (8 * kCellRun) * kCellRun;  // cells per XCD
+  const auto entry = [&](int j0) {  // list position of the thread's cell from j0 on
+    const int u = j0 + (int)threadIdx.x * nwb;
+    return ((u / kCellRun) * 8 + band) * kCellRun + u % kCellRun;
+  };
+  int at = entry(wb);
+  int next = at < src.room ? src.list[at] : 0;  // (beside the list's length)
+  const int all = *src.count;
+  const int mine = (all + 8 * kCellRun - 1) / (8 * kCellRun) * kCellRun;  // entries per XCD
   for (int j0 = wb; j0 < mine; j0 += nwb * kBlock) {
+    if (j0 != wb) {
+      at = entry(j0);
+      next = at < all ? src.list[at] : 0;
+    }
     __syncthreads();
     if (threadIdx.x == 0) cq.count = cq.next = 0;
     __syncthreads();
-    const int u = j0 + (int)threadIdx.x * nwb;
-    int gc = ((u / kCellRun) * 8 + band) * kCellRun + u % kCellRun;
-    bool take = u < mine && gc < all;
-    if (take && src.tiles) {
-      const int tl = gc / src.rows, r = gc - tl * src.rows;
-      const int tile = src.tiles[tl], nty = (g.ncy + src.rows - 1) / src.rows;
-      const int cx = tile / nty, cy = (tile - cx * nty) * src.rows + r;
-      take = cy < g.ncy;
-      gc = cx * g.ncy + cy;
-    }
-    if (take && cell_start[gc + 1] > cell_start[gc]) {
-      const int at = atomicAdd(&cq.count, 1);
-      cq.cell[at] = gc;
-      if (cases) cq.cse[at] = (uint8_t)case_of_cell(cases, ncases, gc);
+    if (at < all) {
+      const int q = atomicAdd(&cq.count, 1);
+      cq.cell[q] = next;
+      if (cases) cq.cse[q] = (uint8_t)case_of_cell(cases, ncases, next);
     }
     __syncthreads();
     const int todo = cq.count;
@@ -939,15 +940,8 @@ int cell_groups(const tsph_ctx *c, K kernel, int waves, int lds, int &fit) {
   return 8 * ((std::min(most, want) + 7) / 8);
 }
 
-// A cell walk looks at every cell of grids of up to kCellsDirect cells (a
-// tile list's length, its entry and the cell's offsets would be three
-// dependent loads before the first cell, 2 us more per pass on small grids);
-// on larger ones, which may be mostly empty, at those of the listed tiles.
-constexpr int kCellsDirect = 1 << 20;
-inline bool cells_direct(const tsph_ctx *c) { return c->ncells_tot <= kCellsDirect; }
 inline CellSource cell_source(const tsph_ctx *c) {
-  if (cells_direct(c)) return {c->ncells_tot, nullptr, nullptr, 1};
-  return {c->ncells_tot, c->tile_list, c->scal + S_NTILES, c->tile_rows};
+  return {c->tile_list, c->scal + S_NTILES, (int)std::min<size_t>(tile_list_room(c), INT_MAX)};
 }
 
 // a pair-loop launch, bracketed by HIP events while pair timing is enabled
