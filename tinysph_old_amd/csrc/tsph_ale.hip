@@ -124,10 +124,12 @@ struct RalePtr {
   uint8_t *gflag;
 };
 
+template <int H>
 struct RaleCell64 {
   RalePtr d;
   Rale64 k;
-  static constexpr int kSums = 4, kSlotBytes = 4 * 16 + 1, kWaves = 4;
+  static constexpr int kSums = 4, kSlotBytes = 4 * 16 + 1, kWaves = H == 2 ? 4 : 2;
+  static constexpr int kSlots = cell_slots_of<H>();
   static constexpr bool kFlag = true, kSkip = false;
   struct Lds {
     double2 *r, *v, *rw, *n;  // rw = {rho, omega}
@@ -194,8 +196,9 @@ struct RaleCell64 {
   }
 };
 
-__global__ __launch_bounds__(RaleCell64::kWaves * kWave, 3) void k_rale_cells64(
-    RaleCell64 pol, CellGrid g, const int *__restrict__ cell_start, CellSource src,
+template <class P>
+__global__ __launch_bounds__(P::kWaves * kWave, cell_halves<P>() == 2 ? 3 : 2) void k_rale_cells64(
+    P pol, CellGrid g, const int *__restrict__ cell_start, CellSource src,
     unsigned long long *__restrict__ counters) {
   cells64(pol, g, cell_start, nullptr, 1, src, counters);
 }
@@ -496,6 +499,20 @@ int launch_ale_init(tsph_ctx *c) {
   return 0;
 }
 
+template <int H>
+static int launch_rale_cells(tsph_ctx *c) {
+  using P = RaleCell64<H>;
+  constexpr int lds = cell_lds_bytes<P>();
+  const Soa &d = c->cur;
+  const int groups = cell_groups(c, k_rale_cells64<P>, P::kWaves, lds, c->ale_fit[7]);
+  return launch_timed(c, [&] {
+    hipLaunchKernelGGL(k_rale_cells64<P>, dim3(groups), dim3(P::kWaves * kWave), lds, c->stream,
+                       P{{d.r, d.v, d.n, d.rho, d.omega, d.type, d.domega, d.domegarho, d.domegav,
+                          c->ale_flag}, rale64(c->k)},
+                       cell_grid(c->k), c->cell_start, cell_source(c), c->counters);
+  });
+}
+
 int launch_rale_forces(tsph_ctx *c) {
   const Consts &k = c->k;
   const int rows = c->tile_rows;
@@ -514,16 +531,8 @@ int launch_rale_forces(tsph_ctx *c) {
                             c->ale_flag, c->counters);
     });
   } else {
-    constexpr int lds = cell_lds_bytes<RaleCell64>();
-    const Soa &d = c->cur;
     if ((e = ensure_cell_entries(c))) return e;
-    const int groups = cell_groups(c, k_rale_cells64, RaleCell64::kWaves, lds, c->ale_fit[7]);
-    e = launch_timed(c, [&] {
-      hipLaunchKernelGGL(k_rale_cells64, dim3(groups), dim3(RaleCell64::kWaves * kWave), lds, s,
-                         RaleCell64{{d.r, d.v, d.n, d.rho, d.omega, d.type, d.domega, d.domegarho,
-                                     d.domegav, c->ale_flag}, rale64(k)},
-                         cell_grid(k), c->cell_start, cell_source(c), c->counters);
-    });
+    e = cells_wide(c) ? launch_rale_cells<4>(c) : launch_rale_cells<2>(c);
   }
   if (e) return e;
   hipLaunchKernelGGL(k_rale_isolated, dim3(grid_for(c->n_ub, 256)), dim3(256), 0, s, c->cur,

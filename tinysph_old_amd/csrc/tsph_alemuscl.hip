@@ -294,14 +294,15 @@ struct Acc64P {
 };
 
 // the cell walk's policy of pass A
-template <class A>
+template <class A, int H>
 struct AleCell64 {
   AlePtr d;
   Ale64 k;
   static constexpr bool G = A::kG;
   static constexpr int kSums = A::kSums;
   static constexpr int kSlotBytes = (G ? 7 : 4) * 16 + (A::kSound ? 8 : 0) + 1;
-  static constexpr int kWaves = G ? 2 : 4;
+  static constexpr int kWaves = (G ? 2 : 4) / (H / 2);
+  static constexpr int kSlots = cell_slots_of<H>();
   static constexpr bool kFlag = true, kSkip = false;
   struct Lds {
     double2 *r, *v, *ro, *n, *gr, *gx, *gy;  // ro = {rho, omega}
@@ -861,9 +862,9 @@ int launch_pass32(tsph_ctx *c, const P &pol) {
 }
 
 // launch of one FP64 pair pass by cells
-template <class A>
+template <class A, int H>
 int launch_pass64(tsph_ctx *c, int slot) {
-  using P = AleCell64<A>;
+  using P = AleCell64<A, H>;
   constexpr int lds = cell_lds_bytes<P>();
   const Soa &d = c->cur;
   if (int e = ensure_cell_entries(c)) return e;
@@ -874,6 +875,11 @@ int launch_pass64(tsph_ctx *c, int slot) {
                           d.domega, d.domegarho, d.domegav}, ale64(c->k)},
                        cell_grid(c->k), c->cell_start, cell_source(c), c->counters);
   });
+}
+
+template <class A>
+int launch_pass64(tsph_ctx *c, int slot) {
+  return cells_wide(c) ? launch_pass64<A, 4>(c, slot) : launch_pass64<A, 2>(c, slot);
 }
 
 }  // namespace

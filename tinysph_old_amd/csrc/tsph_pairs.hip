@@ -555,11 +555,12 @@ struct Pair64 {
   double *drho;
 };
 
-template <int VAR>
+template <int VAR, int H>
 struct Cell64 {
   Pair64 d;
   PairConsts k;
-  static constexpr int kSums = VAR == TSPH_FORCES_BT ? 5 : 4, kWaves = 4;
+  static constexpr int kSums = VAR == TSPH_FORCES_BT ? 5 : 4, kWaves = H == 2 ? 4 : 2;
+  static constexpr int kSlots = cell_slots_of<H>();
   static constexpr bool kFlag = false;
   static constexpr int kSlotBytes = (VAR == TSPH_FORCES_BT ? 4 : 3) * 16 + 9;
   struct Lds {
@@ -638,7 +639,7 @@ struct Cell64 {
 };
 
 template <class P>
-__global__ __launch_bounds__(P::kWaves * kWave, 3) void k_cells64(P pol, CellGrid g, const int *__restrict__ cell_start,
+__global__ __launch_bounds__(P::kWaves * kWave, cell_halves<P>() == 2 ? 3 : 2) void k_cells64(P pol, CellGrid g, const int *__restrict__ cell_start,
                                                         const Consts *__restrict__ cases,
                                                         int ncases, CellSource src,
                                                         unsigned long long *__restrict__ counters) {
@@ -1093,9 +1094,9 @@ void pair_launch(tsph_ctx *c, const TileGrid &tg, int rows, int cap, bool corr, 
     mixed_launch<VAR, DYN, false, false>(c, tg, rows, cap, 0.);
 }
 
-template <int VAR>
+template <int VAR, int H>
 void cell_launch(tsph_ctx *c) {
-  using P = Cell64<VAR>;
+  using P = Cell64<VAR, H>;
   constexpr int lds = cell_lds_bytes<P>();
   const Soa &d = c->cur;
   const int groups = cell_groups(c, k_cells64<P>, P::kWaves, lds, c->cells_fit[VAR]);
@@ -1103,6 +1104,11 @@ void cell_launch(tsph_ctx *c) {
                      P{{d.r, d.v, d.n, d.rho, d.p, d.type, d.a, d.drho}, pair_consts(c->k)},
                      cell_grid(c->k), c->cell_start, c->cases, c->ncases,
                      cell_source(c), c->counters);
+}
+template <int VAR>
+void cell_launch(tsph_ctx *c) {
+  if (cells_wide(c)) cell_launch<VAR, 4>(c);
+  else cell_launch<VAR, 2>(c);
 }
 
 template <int VAR>

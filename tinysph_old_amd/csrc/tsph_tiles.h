@@ -468,8 +468,8 @@ __device__ __forceinline__ int slice_of(const Tile &t, int l) {
 //      order (cell order, ascending index), so slot order is candidate order
 //      and the cell's own particles are the first slots;
 //   2. for each own particle the lanes test all candidate slots at once (two
-//      per lane) and append the pairs, in order, to one flat list (ballots and
-//      prefix counts; the bookkeeping is scalar);
+//      per lane, four in the wide form) and append the pairs, in order, to one
+//      flat list (ballots and prefix counts; the bookkeeping is scalar);
 //   3. the lanes evaluate 64 pairs of that list at a time, whichever particles
 //      they belong to, and leave each pair's kSums terms in LDS;
 //   4. lane (particle, term) adds its particle's terms in list order.
@@ -484,6 +484,8 @@ __device__ __forceinline__ int slice_of(const Tile &t, int l) {
 //   kSkip, skip_lds(L, l)         pairs of two slots with skip_lds are no
 //                                 candidates (DBC walls)
 //   kWaves                        wavefronts of a workgroup
+//   kSlots                        staged slots: cell_slots_of<H>(), H slots per
+//                                 lane (2, or 4: the wide form)
 //   kFlag                         sums() wants to know whether any of the
 //                                 particle's pairs has bit 1 set (below)
 //   terms(L, p, l, double (&t)[kSums])  the terms of pair (p, l), which is
@@ -491,8 +493,14 @@ __device__ __forceinline__ int slice_of(const Tile &t, int l) {
 //                                 result: it counts as a pair interaction, bit 1: a flag
 //   sums(L, p, i, const double (&s)[kSums], flag)  writes particle i, slot p
 //   far(i, cs, g, c, counts...)   particle i of cell c from global memory
-constexpr int kCellSlots = 104;  // staged slots of a cell's neighbourhood
-constexpr int kCellFlat = 640;   // flat list entries (own particles listed together x candidates)
+// staged slots of a cell's neighbourhood, and flat list entries (own particles
+// listed together x candidates), for H slots per lane
+template <int H>
+constexpr int cell_slots_of() { return H == 2 ? 104 : 232; }
+template <class P>
+constexpr int cell_halves() { return (P::kSlots + kWave - 1) / kWave; }
+template <class P>
+constexpr int cell_flat() { return cell_halves<P>() == 2 ? 640 : 2048; }
 constexpr double kFar64 = 1e150;  // coordinate of slots past the last (its square is finite)
 constexpr int kCellBlock = 4 * kWave;  // most threads of a workgroup
 constexpr int kCellRun = 64;     // consecutive cells of one XCD
@@ -507,7 +515,7 @@ struct CellQueue {
 // LDS bytes of a wavefront of a cell walk
 template <class P>
 constexpr int cell_wave_bytes() {
-  return (cell_terms<P>() * P::kSums * 8 + kCellFlat * 2 + kCellSlots * P::kSlotBytes + 15) / 16 * 16;
+  return (cell_terms<P>() * P::kSums * 8 + cell_flat<P>() * 2 + P::kSlots * P::kSlotBytes + 15) / 16 * 16;
 }
 template <class P>
 constexpr int cell_lds_bytes() {
@@ -566,13 +574,13 @@ __device__ __forceinline__ void cell_ranges(const CellGrid &g, const int *__rest
 }
 
 // the slots of those cells (lo, cnt: cell_ranges), and the loads of the
-// lane's two slots, in flight together
+// lane's slots, in flight together
 struct CellSlots {
   int own0, nown, tot;
 };
-template <class P>
-__device__ __forceinline__ CellSlots cell_slots(int lo, int cnt, typename P::Rec &r0,
-                                                typename P::Rec &r1, const P &pol) {
+template <class P, int H>
+__device__ __forceinline__ CellSlots cell_slots(int lo, int cnt, typename P::Rec (&rec)[H],
+                                                const P &pol) {
   const int lane = tile_lane();
   // slot l of cell q holds particle l + dj[q], for l in [pre[q], pre[q + 1])
   int pre[9], dj[9], tot = 0;
@@ -582,17 +590,17 @@ __device__ __forceinline__ CellSlots cell_slots(int lo, int cnt, typename P::Rec
     dj[q] = __builtin_amdgcn_readlane(lo, q) - tot;
     tot += __builtin_amdgcn_readlane(cnt, q);
   }
-  int j[2];
+  int j[H];
 #pragma unroll
-  for (int h = 0; h < 2; ++h) {
+  for (int h = 0; h < H; ++h) {
     const int l = h * kWave + lane;
     j[h] = l + dj[0];
 #pragma unroll
     for (int q = 1; q < 9; ++q) j[h] = l >= pre[q] ? l + dj[q] : j[h];
     if (l >= tot) j[h] = dj[0];
   }
-  r0 = pol.load(j[0]);
-  r1 = pol.load(j[1]);
+#pragma unroll
+  for (int h = 0; h < H; ++h) rec[h] = pol.load(j[h]);
   return {dj[0], __builtin_amdgcn_readlane(cnt, 0), tot};
 }
 
@@ -610,13 +618,15 @@ __device__ __forceinline__ void cells64(P &pol, CellGrid g, const int *__restric
   extern __shared__ __align__(16) unsigned char smem[];
   constexpr int NS = P::kSums;
   constexpr int NT = cell_terms<P>();
+  constexpr int H = cell_halves<P>();
+  static_assert(H <= 4 && P::kSlots < 256, "a list entry holds the slot in 8 bits");
   constexpr int kBlock = P::kWaves * kWave;
   constexpr int kOwn = NS < 4 ? 16 : 64 / NS;  // particles whose sums are formed together
   CellQueue &cq = *reinterpret_cast<CellQueue *>(smem);
   unsigned char *wl = smem + sizeof(CellQueue) + (threadIdx.x >> 6) * cell_wave_bytes<P>();
   double *terms = reinterpret_cast<double *>(wl);
   uint16_t *flat = reinterpret_cast<uint16_t *>(terms + NT * NS);
-  const typename P::Lds L = P::lds(reinterpret_cast<unsigned char *>(flat + kCellFlat), kCellSlots);
+  const typename P::Lds L = P::lds(reinterpret_cast<unsigned char *>(flat + cell_flat<P>()), P::kSlots);
   const int lane = tile_lane();
   if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&counters[C_PASSES], 1ull);
   unsigned npair = 0, ncand = 0, nact = 0, scand = 0, snact = 0;
@@ -661,39 +671,42 @@ __device__ __forceinline__ void cells64(P &pol, CellGrid g, const int *__restric
       }
       int lo, cnt;
       cell_ranges(g, cell_start, it.c, lo, cnt);
-      typename P::Rec r0, r1;
-      const CellSlots sl = cell_slots(lo, cnt, r0, r1, pol);
+      typename P::Rec rec[H];
+      const CellSlots sl = cell_slots(lo, cnt, rec, pol);
       const int own0 = sl.own0, nown = sl.nown, tot = sl.tot;
-      if (tot > kCellSlots || nown > kWave) {
+      if (tot > P::kSlots || nown > kWave) {
         // neighbourhood beyond the LDS budget: gather from global memory
         for (int p = lane; p < nown; p += kWave)
           pol.far(own0 + p, cell_start + g.cell_base, g, it.c - g.cell_base, npair, ncand, nact);
         continue;
       }
       wave_sync();  // the previous cell's LDS is no longer read
-      if (lane < tot) pol.store(L, lane, r0);
-      if (kWave + lane < tot) pol.store(L, kWave + lane, r1);
+#pragma unroll
+      for (int h = 0; h < H; ++h)
+        if (h * kWave + lane < tot) pol.store(L, h * kWave + lane, rec[h]);
       wave_sync();
-      // candidate slots lane and 64 + lane in registers (slots past the last:
+      // candidate slots lane, 64 + lane ... in registers (slots past the last:
       // far away); the active own particles, and the slots that skip each
       // other, as bit masks
-      double2 cp[2];
-      unsigned long long skp[2];
+      double2 cp[H];
+      unsigned long long skp[H];
+      int skips_tot = 0;
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
+      for (int h = 0; h < H; ++h) {
         const int l = h * kWave + lane;
         const bool real = l < tot;
         const double2 r = pol.pos_lds(L, real ? l : 0);
         cp[h] = real ? r : make_double2(kFar64, kFar64);
         skp[h] = P::kSkip ? __ballot(real && pol.skip_lds(L, real ? l : 0)) : 0ull;
+        skips_tot += __popcll(skp[h]);
       }
       const unsigned long long act =
           __ballot(lane < nown && pol.act_lds(L, lane < nown ? lane : 0));
       snact += __popcll(act);
       scand += __popcll(act & ~skp[0]) * (tot - 1);
-      if (P::kSkip) scand += __popcll(act & skp[0]) * (tot - __popcll(skp[0]) - __popcll(skp[1]));
+      if (P::kSkip) scand += __popcll(act & skp[0]) * (tot - skips_tot);
       if (!act) continue;
-      const int most = min(kOwn, kCellFlat / tot);  // own particles listed together
+      const int most = min(kOwn, cell_flat<P>() / tot);  // own particles listed together
       for (int p0 = 0; p0 < nown; p0 += most) {
         const int np = min(most, nown - p0);
         int e = 0, st = 0;  // st: lane p's first list position (lane np: the list's length)
@@ -705,16 +718,16 @@ __device__ __forceinline__ void cells64(P &pol, CellGrid g, const int *__restric
           st = lane == p ? e : st;
           if (!((act >> q) & 1ull)) continue;
           const bool skips = P::kSkip && ((skp[0] >> q) & 1ull);
-          unsigned long long m[2];
+          unsigned long long m[H];
 #pragma unroll
-          for (int h = 0; h < 2; ++h) {
+          for (int h = 0; h < H; ++h) {
             const double drx = own.x - cp[h].x, dry = own.y - cp[h].y;
             m[h] = __ballot(drx * drx + dry * dry <= g.c2);
             if (skips) m[h] &= ~skp[h];
           }
           m[0] &= ~(1ull << q);
 #pragma unroll
-          for (int h = 0; h < 2; ++h) {
+          for (int h = 0; h < H; ++h) {
             if (__builtin_amdgcn_inverse_ballot_w64(m[h]))
               flat[__builtin_amdgcn_mbcnt_hi((unsigned)(m[h] >> 32),
                                              __builtin_amdgcn_mbcnt_lo((unsigned)m[h], e))] =
@@ -924,6 +937,21 @@ __device__ __forceinline__ void walk32(const P &pol, const Consts &k, const int 
     }  // runs of rows
   }
   wave_count(npair, ncand, nact, counters);
+}
+
+// Whether a context's cell walks take the wide form: where the lattice puts more
+// into a neighbourhood than the narrow one's slots hold at most places, and no more
+// than the wide one's hold.  What is not staged is gathered from global memory,
+// which takes 3 to 5 times as long; the wide form's LDS leaves fewer wavefronts.
+// us per step, narrow and wide, at h = 1.5, 1.6, 1.7, 2, 2.2 and 2.5 dp (89, 102,
+// 115, 159, 192 and 248 in a neighbourhood): dam break of 61k particles 102 and
+// 127, 236 and 137, 390 and 141, 376 and 158, 377 and 192, 481 and 509; ALE of 183k
+// 397 and 600, 1132 and 700, 2379 and 686, 2390 and 805, 2536 and 969, 2607 and 3827.
+// (By tiles before, which staged 99 per neighbourhood: dam break at 1.7 dp 377, ALE
+// 1900.)
+constexpr double kWideFrom = 97., kWideTo = 215.;
+inline bool cells_wide(const tsph_ctx *c) {
+  return 9. * c->cell_lattice > kWideFrom && 9. * c->cell_lattice <= kWideTo;
 }
 
 // workgroups of a cell-walk launch: those that are resident at once (the walk
