@@ -832,8 +832,13 @@ static int download_impl(tsph_ctx *c, tsph_particles *h, int icase) {
   const int m = n[0] > 0 ? n[1] : 0;
   h->np = m;
   if (m == 0) return 0;
+  // The stream is idle, so the copies may take either call: a synchronous one to
+  // pageable memory costs 6 us less, after 25 us for the first (2.7k particles:
+  // two fields 89 us by asynchronous copies and 97, all thirteen 252 and 218).
+  const bool many = __builtin_popcount(mask) > 4;
   auto get = [&](void *to, const void *from, size_t bytes) {
-    return hipMemcpyAsync(to, from, bytes, hipMemcpyDeviceToHost, c->stream);
+    return many ? hipMemcpy(to, from, bytes, hipMemcpyDeviceToHost)
+                : hipMemcpyAsync(to, from, bytes, hipMemcpyDeviceToHost, c->stream);
   };
   for (const Field &f : fields) {
     if (!f.to) continue;
@@ -843,7 +848,7 @@ static int download_impl(tsph_ctx *c, tsph_particles *h, int icase) {
   std::vector<uint8_t> type(h->type ? m : 0);
   if (h->type) TSPH_HIP(get(type.data(), d.type, (size_t)m));
   if (h->index) TSPH_HIP(get(h->index, c->pos_index, 4 * (size_t)m));
-  TSPH_HIP(hipStreamSynchronize(c->stream));
+  if (!many) TSPH_HIP(hipStreamSynchronize(c->stream));
   for (size_t k = 0; k < type.size(); ++k) h->type[k] = type[k];
   return 0;
 }
