@@ -80,3 +80,40 @@ def test_inflow_steps_after_a_relabel(precision):
             assert c["removed"] > 0 and c["zone_rejected"] == 0
             out.append(ps.download(FIELDS))
     same(*out)
+
+
+@pytest.mark.parametrize("n", [1, 33, 8193, 131073, 300001])
+def test_relabel_with_removed_particles_still_in_their_slots(n):
+    """A relabel between the removal decision and the build that drops the particles:
+    every field stays with its particle, and the next decisions (every other one of a
+    run of candidates) are those without the relabel."""
+    g = np.random.RandomState(n)
+    arrays = {k: g.rand(n, 2) for k in ("r", "v", "gnr", "n")}
+    arrays["rho"] = 1000.0 + g.rand(n)
+    arrays["type"] = np.where(g.rand(n) < 0.2, T.WALL, T.FLUID).astype(np.int32)
+    arrays["index"] = g.permutation(n).astype(np.int32)
+    out = g.rand(n) < 0.3  # runs of candidates among them
+    arrays["r"][out, 0] = 1.1 + 0.015
+    prm = {"h": 0.01, "kap": 2.0, "cs": 20.0, "rho0": 1000.0, "avisc": 0.01, "delta": 0.1, "dp": 0.01,
+           "x_0": -0.1, "x_m": 1.1, "y_0": -0.1, "y_m": 1.1}
+    print(f"[case] relabel of {n} particles, {int(out.sum())} of them leaving", flush=True)
+    fields = ("type", "index", "r", "v", "rho", "gnr", "n")
+    got = []
+    for relabel in (False, True):
+        some = []
+        with T.ParticleSystem(prm, capacity=n) as ps:
+            ps.upload(arrays)
+            ps.particle_to_cell()
+            for _ in range(3):
+                ps.remove_out_of_domain()
+                if relabel:
+                    ps.renumber()
+                some.append(ps.download(fields))
+                ps.particle_to_cell()
+                if relabel:
+                    ps.renumber()
+                some.append(ps.download(fields))
+            got.append((some, ps.counters()["removed"]))
+    assert got[0][1] == got[1][1] and (n == 1 or got[0][1] > 0)
+    for x, y in zip(got[0][0], got[1][0]):
+        same(x, y)

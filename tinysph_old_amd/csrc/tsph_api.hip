@@ -746,45 +746,10 @@ static int live_order(tsph_ctx *c, int n, std::vector<int> &order, std::vector<u
 // in the wall list move along.  Cell order, tiles and records stay valid: the
 // in-cell order by seq is unchanged.
 static int renumber_seq(tsph_ctx *c) {
-  int n = 0, e = 0;
+  if (int e = launch_renumber(c)) return e;
+  int ms = 0;
+  TSPH_HIP(hipMemcpyAsync(&ms, &c->scal[S_MAXSEQ], sizeof(int), hipMemcpyDeviceToHost, c->stream));
   TSPH_HIP(hipStreamSynchronize(c->stream));
-  TSPH_HIP(hipMemcpy(&n, &c->scal[S_NP], sizeof(int), hipMemcpyDeviceToHost));
-  std::vector<int> order;
-  std::vector<uint32_t> seq;
-  std::vector<uint8_t> type;
-  if ((e = live_order(c, n, order, seq, type))) return e;
-  std::vector<uint8_t> st((size_t)c->seq_cap), nst((size_t)c->seq_cap, 0);
-  TSPH_HIP(hipMemcpy(st.data(), c->seqstate, (size_t)c->seq_cap, hipMemcpyDeviceToHost));
-  std::vector<uint32_t> nseq((size_t)std::max(n, 1));
-  std::vector<int32_t> index((size_t)c->seq_cap);
-  std::vector<double2> gnr(c->has_gnr ? (size_t)c->seq_cap : 0);
-  TSPH_HIP(hipMemcpy(index.data(), c->cur.index, index.size() * sizeof(int32_t), hipMemcpyDeviceToHost));
-  if (c->has_gnr)
-    TSPH_HIP(hipMemcpy(gnr.data(), c->cur.gnr, gnr.size() * sizeof(double2), hipMemcpyDeviceToHost));
-  uint32_t next = 0;
-  for (int i : order) {  // (positions ascending, so none is read after it was written)
-    nst[next] = st[seq[i]];
-    index[next] = index[seq[i]];
-    if (c->has_gnr) gnr[next] = gnr[seq[i]];
-    nseq[i] = next++;
-  }
-  TSPH_HIP(hipMemcpy(c->cur.index, index.data(), index.size() * sizeof(int32_t), hipMemcpyHostToDevice));
-  if (c->has_gnr)
-    TSPH_HIP(hipMemcpy(c->cur.gnr, gnr.data(), gnr.size() * sizeof(double2), hipMemcpyHostToDevice));
-  for (int i = 0; i < n; ++i)
-    if (type[i] == kRemoved) nseq[i] = next++;
-  if (n > 0) TSPH_HIP(hipMemcpy(c->cur.seq, nseq.data(), 4 * (size_t)n, hipMemcpyHostToDevice));
-  int nwall = 0;  // walls of the last cell list (0: none since the upload)
-  TSPH_HIP(hipMemcpy(&nwall, &c->scal[c->nwall_idx], sizeof(int), hipMemcpyDeviceToHost));
-  std::vector<int2> walls((size_t)nwall);
-  if (nwall > 0) {
-    TSPH_HIP(hipMemcpy(walls.data(), c->wall_list, walls.size() * sizeof(int2), hipMemcpyDeviceToHost));
-    for (int2 &w : walls) w.y = (int)nseq[w.x];
-    TSPH_HIP(hipMemcpy(c->wall_list, walls.data(), walls.size() * sizeof(int2), hipMemcpyHostToDevice));
-  }
-  TSPH_HIP(hipMemcpy(c->seqstate, nst.data(), (size_t)c->seq_cap, hipMemcpyHostToDevice));
-  const int ms = (int)next;
-  TSPH_HIP(hipMemcpy(&c->scal[S_MAXSEQ], &ms, sizeof(int), hipMemcpyHostToDevice));
   c->seq_ub = ms;
   return 0;
 }

@@ -54,7 +54,7 @@ inline CostEstimate cost_estimate(bool mixed) { return mixed ? kCostMixed : kCos
 // buffers: a build fills the other one, see cell_start_next); the per-tile
 // costs follow them (kCostTables (ncells_tot + 8) slots)
 enum { S_NP = 0, S_MAXSEQ = 1, S_NTILES = 2, S_NWALL = 3, S_BZCNT = 4, S_NWALL_B = 5,
-       S_DLNP = 6, S_NSCAL = 32 };
+       S_DLNP = 6, S_NEWSEQ = 7, S_NSCAL = 32 };
 // device counter slots (uint64)
 enum {
   C_PAIRS = 0, C_CAND = 1, C_ACTIVE = 2, C_PASSES = 3, C_BADRHO = 4, C_OUTGRID = 5,
@@ -484,6 +484,10 @@ enum {
   DL_RHO = 256, DL_DRHO = 512, DL_RHO_O = 1024, DL_TYPE = 2048, DL_INDEX = 4096
 };
 int launch_download_gather(tsph_ctx *c, int icase, unsigned fields);
+// The live particles' reference positions relabelled 0..m-1 in order, the removed
+// slots' m..; the removal states, gnr, index and the wall list's positions move
+// along, S_MAXSEQ follows (alt's seq and type, pos_gnr and pos_index are scratch).
+int launch_renumber(tsph_ctx *c);
 // p[i] = i for i < n
 int launch_iota(tsph_ctx *c, int *p, int n);
 // live particles of every case of a batch into counts[ncases] (device memory)
