@@ -90,7 +90,7 @@ __device__ __forceinline__ double diff_fourtakas64(double h, double d, double yd
                                                    double inrho, double rho0, double cb, double icb,
                                                    double c0, double delta, double m,
                                                    double gravity) {
-  const double dpH = 1. + quot64_any(dr_z * rho0 * gravity, cb, icb);
+  const double dpH = 1. + quot64(dr_z * rho0 * gravity, cb, icb);
   const double drhoH = rho0 * root7(dpH) - rho0;  // pow(dpH, 1/7), tsph_root7.h
   const double psi = quot64_any(2. * c0 * h * delta * ((nrho - arho) - drhoH), d, yd);
   return quot64_any(psi * drdW * m, nrho, inrho);

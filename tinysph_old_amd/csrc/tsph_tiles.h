@@ -503,7 +503,7 @@ template <class P>
 constexpr int cell_flat() { return cell_halves<P>() == 2 ? 640 : 2048; }
 constexpr double kFar64 = 1e150;  // coordinate of slots past the last (its square is finite)
 constexpr int kCellBlock = 4 * kWave;  // most threads of a workgroup
-constexpr int kCellRun = 64;     // consecutive cells of one XCD
+constexpr int kCellRun = 6;      // log2 of the most consecutive listed cells of one XCD
 template <class P>
 constexpr int cell_terms() { return P::kSums <= 4 ? 184 : 128; }  // pairs whose terms are in LDS together
 // a workgroup's non-empty cells (and their cases), and the next to take
@@ -542,15 +542,10 @@ __device__ __forceinline__ int case_of_cell(const Consts *__restrict__ cases, in
   return lo;
 }
 
-struct CellItem {
-  int c, cse;  // global cell (-1: none left), its case
-};
-__device__ __forceinline__ CellItem cell_take(CellQueue &cq, int todo) {
+__device__ __forceinline__ int cell_take(CellQueue &cq) {
   int at = 0;
   if (tile_lane() == 0) at = atomicAdd(&cq.next, 1);
-  at = __builtin_amdgcn_readfirstlane(at);
-  if (at >= todo) return {-1, 0};
-  return {__builtin_amdgcn_readfirstlane(cq.cell[at]), __builtin_amdgcn_readfirstlane((int)cq.cse[at])};
+  return __builtin_amdgcn_readfirstlane(at);
 }
 
 // the 9 stencil cells of global cell gc, one per lane: first particle and
@@ -608,6 +603,7 @@ __device__ __forceinline__ CellSlots cell_slots(int lo, int cnt, typename P::Rec
 struct CellSource {
   const int *list, *count;
   int room;  // entries of the list's buffer
+  int run;   // log2 of the consecutive entries of one XCD
 };
 
 template <class P>
@@ -630,7 +626,7 @@ __device__ __forceinline__ void cells64(P &pol, CellGrid g, const int *__restric
   const int lane = tile_lane();
   if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&counters[C_PASSES], 1ull);
   unsigned npair = 0, ncand = 0, nact = 0, scand = 0, snact = 0;
-  // Runs of kCellRun listed cells are dealt to the 8 XCDs in turn, so that a run's
+  // Runs of 2^run listed cells are dealt to the 8 XCDs in turn, so that a run's
   // cells share staged particles through one L2 while every XCD gets a share
   // of each part of the domain.  The workgroups of an XCD stride through its
   // cells, a cell per thread, and their wavefronts take them from a counter in
@@ -641,19 +637,29 @@ __device__ __forceinline__ void cells64(P &pol, CellGrid g, const int *__restric
   const int band = blockIdx.x & 7, nwb = gridDim.x >> 3, wb = blockIdx.x >> 3;
   const auto entry = [&](int j0) {  // list position of the thread's cell from j0 on
     const int u = j0 + (int)threadIdx.x * nwb;
-    return ((u / kCellRun) * 8 + band) * kCellRun + u % kCellRun;
+    return (((u >> src.run) * 8 + band) << src.run) + (u & ((1 << src.run) - 1));
   };
+  // A wavefront's first cell is the one at its own position, turned by two for
+  // every second round of the workgroups over the XCD's 32 CUs: where a
+  // workgroup has but one or two cells, those of a CU's workgroups would meet on
+  // the same SIMDs (a pass of 9k particles 12.9 us not turned, 13.8 with all cells
+  // taken from the counter, 11.4 now; of 7k 11.4, 12.7 and 10.1).
+  const int first =
+      __builtin_amdgcn_readfirstlane(((threadIdx.x >> 6) + (wb >> 5) * 2) & (P::kWaves - 1));
   int at = entry(wb);
   int next = at < src.room ? src.list[at] : 0;  // (beside the list's length)
   const int all = *src.count;
-  const int mine = (all + 8 * kCellRun - 1) / (8 * kCellRun) * kCellRun;  // entries per XCD
+  const int mine = ((all + (8 << src.run) - 1) >> (3 + src.run)) << src.run;  // entries per XCD
   for (int j0 = wb; j0 < mine; j0 += nwb * kBlock) {
     if (j0 != wb) {
       at = entry(j0);
       next = at < all ? src.list[at] : 0;
     }
     __syncthreads();
-    if (threadIdx.x == 0) cq.count = cq.next = 0;
+    if (threadIdx.x == 0) {
+      cq.count = 0;
+      cq.next = P::kWaves;
+    }
     __syncthreads();
     if (at < all) {
       const int q = atomicAdd(&cq.count, 1);
@@ -662,22 +668,22 @@ __device__ __forceinline__ void cells64(P &pol, CellGrid g, const int *__restric
     }
     __syncthreads();
     const int todo = cq.count;
-    for (;;) {
-      const CellItem it = cell_take(cq, todo);
-      if (it.c < 0) break;
+    for (int q = first; q < todo; q = cell_take(cq)) {
+      const int c = __builtin_amdgcn_readfirstlane(cq.cell[q]);
       if (cases) {
-        g = cell_grid(cases[it.cse]);
-        pol.set(cases[it.cse]);
+        const Consts &k = cases[__builtin_amdgcn_readfirstlane((int)cq.cse[q])];
+        g = cell_grid(k);
+        pol.set(k);
       }
       int lo, cnt;
-      cell_ranges(g, cell_start, it.c, lo, cnt);
+      cell_ranges(g, cell_start, c, lo, cnt);
       typename P::Rec rec[H];
       const CellSlots sl = cell_slots(lo, cnt, rec, pol);
       const int own0 = sl.own0, nown = sl.nown, tot = sl.tot;
       if (tot > P::kSlots || nown > kWave) {
         // neighbourhood beyond the LDS budget: gather from global memory
         for (int p = lane; p < nown; p += kWave)
-          pol.far(own0 + p, cell_start + g.cell_base, g, it.c - g.cell_base, npair, ncand, nact);
+          pol.far(own0 + p, cell_start + g.cell_base, g, c - g.cell_base, npair, ncand, nact);
         continue;
       }
       wave_sync();  // the previous cell's LDS is no longer read
@@ -968,8 +974,14 @@ int cell_groups(const tsph_ctx *c, K kernel, int waves, int lds, int &fit) {
   return 8 * ((std::min(most, want) + 7) / 8);
 }
 
+// Runs of up to 64 cells, shorter ones where an XCD would get fewer than about 8
+// runs: some XCDs then have one run more than others (runs of 64 against the
+// shorter ones: a pass of 6k particles 12.3 and 11.2 us, of 7k 11.1 and 10.1; from
+// 18k particles on no difference).
 inline CellSource cell_source(const tsph_ctx *c) {
-  return {c->tile_list, c->scal + S_NTILES, (int)std::min<size_t>(tile_list_room(c), INT_MAX)};
+  int run = kCellRun;
+  while (run > 2 && c->n_ub / 8 < 64 << run) --run;
+  return {c->tile_list, c->scal + S_NTILES, (int)std::min<size_t>(tile_list_room(c), INT_MAX), run};
 }
 
 // a pair-loop launch, bracketed by HIP events while pair timing is enabled
