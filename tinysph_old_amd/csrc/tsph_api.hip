@@ -89,8 +89,8 @@ static void drop_graph(tsph_ctx *c) {
 // default pair-loop launch: 7-cell tiles in the pooled walk (chunks cut by
 // the recorded tile costs); the mixed path's shorter records hide more
 // latency with 12 waves per CU, the FP64 path's larger LDS records allow 8
-// (740k-particle dam break, pair pass: mixed 0.070 ms pooled against 0.088
-// ms static, FP64 0.248 ms against 0.277 ms)
+// (740k-particle dam break, pair pass: mixed 0.073 ms pooled against 0.102
+// ms static, FP64 0.197 ms against 0.224 ms)
 static void set_walk_defaults(tsph_ctx *c) {
   const bool mixed = c->prm.precision == TSPH_PREC_MIXED;
   c->waves_per_cu = mixed ? 12 : 8;

@@ -1164,17 +1164,18 @@ int launch_cell_list(tsph_ctx *c, bool eos, bool predict, double dt, unsigned ad
   }
   const CellRows rw_next{c->row_seq_next, c->row_head_next, rank ? c->hrank_next : nullptr,
                          rank ? c->row_width : 0};
-  if (!hashed) {
 #define TSPH_HASH(P, D, W)                                                                     \
-  hipLaunchKernelGGL((k_hash<P, D, W>), dim3(hg), dim3(hbs), 0, s, c->cur.r, c->cur.v,            \
-                     c->cur.type, c->cur.seq, c->scal, k, c->cases, c->cur.cid, dt, nct,          \
-                     c->cell_count, c->hcell, c->hrank, rw, c->bin_count, clear, c->seqstate,   \
+  hipLaunchKernelGGL((k_hash<P, D, W>), dim3(hg), dim3(hbs), 0, s, c->cur.r, c->cur.v,         \
+                     c->cur.type, c->cur.seq, c->scal, k, c->cases, c->cur.cid, dt, nct,       \
+                     c->cell_count, c->hcell, c->hrank, rw, c->bin_count, clear, c->seqstate,  \
                      c->counters, wp)
 #define TSPH_HASH_W(P, D)                                                                      \
-  if (walls == TSPH_WALL_MDBC) TSPH_HASH(P, D, TSPH_WALL_MDBC);                               \
-  else if (walls == TSPH_WALL_BT) TSPH_HASH(P, D, TSPH_WALL_BT);                              \
+  if (walls == TSPH_WALL_MDBC) TSPH_HASH(P, D, TSPH_WALL_MDBC);                                \
+  else if (walls == TSPH_WALL_BT) TSPH_HASH(P, D, TSPH_WALL_BT);                               \
   else TSPH_HASH(P, D, 0)
-  if (predict && decide) {
+  if (hashed) {
+    // the build before took it
+  } else if (predict && decide) {
     TSPH_HASH_W(true, true);
   } else if (predict) {
     TSPH_HASH_W(true, false);
@@ -1183,12 +1184,11 @@ int launch_cell_list(tsph_ctx *c, bool eos, bool predict, double dt, unsigned ad
   } else {
     TSPH_HASH_W(false, false);
   }
-  }
 #undef TSPH_HASH_W
 #undef TSPH_HASH
-  // the pooled pair pass that follows (if any) has its chunks cut in the
-  // first workgroups of the reorder (or the scatter), from the costs the scan lists beside the
-  // tiles and its per-block sums of them
+  // the pooled pair pass that follows (if any) has its chunks cut in the first
+  // workgroups of the reorder (or the scatter), from the costs the scan lists
+  // beside the tiles and its per-block sums of them
   const int cut = c->cut_groups;
   c->cut_groups = 0;
   if (cut > c->bound_cap) {

@@ -14,8 +14,10 @@
 // a particle's density, or the pair's r^2 + eps h^2, which two terms divide
 // by.  quot64_any adds the special values (zero, infinite or NaN operands) as
 // the operator gives them, for whatever holds a velocity, a density or a
-// pressure; lengths alone (finite, and not 0 below) go without (with it three
-// more quotients per pair: 740k particles 498 us per step and 501).
+// pressure.  Quotients of a pair's distances and the case's constants go without:
+// both are finite, and the denominators positive (with it three more quotients
+// per pair: 740k particles 498 us per step and 501).  Denormal operands are not
+// provided for: a density of 1e-310 may give NaN where the operator overflows.
 //
 // sqrt64 runs the coupled iteration for sqrt(x) and 1/(2 sqrt(x)) (Goldschmidt
 // 1964) from the reciprocal square root estimate and corrects the root with

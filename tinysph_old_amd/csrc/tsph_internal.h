@@ -189,12 +189,12 @@ struct tsph_ctx {
   // waves) or the plain static walk; defaults set at creation
   bool balanced[2] = {false, false};
   int cell_order = 0;  // tsph_set_cell_order: 0 and 1 ranked, 2 separate passes
-  // the entries of the static walks and the tiles of the pooled ones: non-empty
-  // tiles of the current cell list, in tile order (tiles::part of each)
+  // the entries of the pair walks: non-empty tiles of the current cell list, in
+  // tile order (tiles::part of each), or non-empty cells (list_rows kListCells)
   int *tile_list = nullptr;
   bool list_split = false;  // tiles of more than a wavefront of particles have two entries
   int list_rows = 0;        // cells per listed tile (kListCells: the list is one of cells)
-  bool tiles_valid = false;  // tile_list matches the cell list and tile_rows
+  bool tiles_valid = false;  // tile_list is of the current cell list, list_rows deep
   int *list_part = nullptr;  // per list-build block: tiles, work
   int list_part_cap = 0;     // list-build blocks list_part holds
   int *tile_bound = nullptr; // pooled walk: first list entry of each workgroup's chunk
@@ -490,10 +490,10 @@ int launch_download_gather(tsph_ctx *c, int icase, unsigned fields);
 int launch_renumber(tsph_ctx *c);
 // p[i] = i for i < n
 int launch_iota(tsph_ctx *c, int *p, int n);
-// live particles of every case of a batch into counts[ncases] (device memory)
 // gnr (if gnr) and index of n uploaded particles from pos_gnr, pos_index to their
 // reference positions (cur.seq)
 int launch_place(tsph_ctx *c, int n, bool gnr);
+// live particles of every case of a batch into counts[ncases] (device memory)
 int launch_case_counts(tsph_ctx *c, int *counts);
 // words of the bitmap over reference positions that launch_download_gather
 // keeps in hcell (and its prefix in hrank)

@@ -850,97 +850,97 @@ __device__ __forceinline__ void walk32(const P &pol, const Consts &k, const int 
       if (fit > 0) sub = max(1, min(fit, sub / ((t.lq[3] + cap - 1) / cap)));
     }
     for (int cy = cy0; cy < cy1; cy += sub) {
-    if (sub < cy1 - cy0) {
-      wave_sync();  // the previous run's LDS is no longer read
-      tile_begin(k, cell_start, t.cx, cy, min(cy + sub, cy1), tab, t);
-      t.own0 = max(t.own0, own0);
-      t.own1 = min(t.own1, own1);
-    }
-    const bool staged = t.lq[3] <= cap;
-    if (staged)
-      for (int l = lane; l < t.lq[3]; l += kWave)
-        pol.stage(L, l, l - sel3(t.base, slice_of(t, l)), ox, oy);
-    wave_sync();
-    uint16_t *my_list = s_list + lane;
-    for (int i0 = t.own0; i0 < t.own1; i0 += kWave) {
-      const int i = i0 + lane;
-      int li = 0, ri = 0;
-      bool act = false;
-      if (i < t.own1) {
-        li = i + t.base[1];
-        act = pol.active(i);
-        ri = cellof[i] - t.cx * k.ncy - t.row_lo;
+      if (sub < cy1 - cy0) {
+        wave_sync();  // the previous run's LDS is no longer read
+        tile_begin(k, cell_start, t.cx, cy, min(cy + sub, cy1), tab, t);
+        t.own0 = max(t.own0, own0);
+        t.own1 = min(t.own1, own1);
       }
-      nact += act;
-      const typename P::Own o = pol.own(act ? i : -1, ox, oy);
-      typename P::Acc acc{};
-      if (!staged) {
-        if (act) {
-          const int cc = cellof[i];
-          const int cy = cc - t.cx * k.ncy;
-          for (int dx = -1; dx <= 1; ++dx) {
-            if (t.cx + dx < 0 || t.cx + dx >= k.ncx) continue;
-            for (int dy = -1; dy <= 1; ++dy) {
-              if (cy + dy < 0 || cy + dy >= k.ncy) continue;
-              const int cl = cc + dy + dx * k.ncy;
-              for (int j = cell_start[cl]; j < cell_start[cl + 1]; ++j) {
-                if (j == i) continue;
-                ++ncand;
-                const float2 pj = pol.pos_glob(j, ox, oy);
-                const float drx = o.p.x - pj.x, dry = o.p.y - pj.y;
-                const float r2 = drx * drx + dry * dry;
-                if (!(r2 < r2cut)) continue;
-                ++npair;
-                pol.pair_glob(acc, o, j, drx, dry, r2);
+      const bool staged = t.lq[3] <= cap;
+      if (staged)
+        for (int l = lane; l < t.lq[3]; l += kWave)
+          pol.stage(L, l, l - sel3(t.base, slice_of(t, l)), ox, oy);
+      wave_sync();
+      uint16_t *my_list = s_list + lane;
+      for (int i0 = t.own0; i0 < t.own1; i0 += kWave) {
+        const int i = i0 + lane;
+        int li = 0, ri = 0;
+        bool act = false;
+        if (i < t.own1) {
+          li = i + t.base[1];
+          act = pol.active(i);
+          ri = cellof[i] - t.cx * k.ncy - t.row_lo;
+        }
+        nact += act;
+        const typename P::Own o = pol.own(act ? i : -1, ox, oy);
+        typename P::Acc acc{};
+        if (!staged) {
+          if (act) {
+            const int cc = cellof[i];
+            const int cy = cc - t.cx * k.ncy;
+            for (int dx = -1; dx <= 1; ++dx) {
+              if (t.cx + dx < 0 || t.cx + dx >= k.ncx) continue;
+              for (int dy = -1; dy <= 1; ++dy) {
+                if (cy + dy < 0 || cy + dy >= k.ncy) continue;
+                const int cl = cc + dy + dx * k.ncy;
+                for (int j = cell_start[cl]; j < cell_start[cl + 1]; ++j) {
+                  if (j == i) continue;
+                  ++ncand;
+                  const float2 pj = pol.pos_glob(j, ox, oy);
+                  const float drx = o.p.x - pj.x, dry = o.p.y - pj.y;
+                  const float r2 = drx * drx + dry * dry;
+                  if (!(r2 < r2cut)) continue;
+                  ++npair;
+                  pol.pair_glob(acc, o, j, drx, dry, r2);
+                }
               }
             }
           }
-        }
-      } else {
-        const int rlo = max(ri - 1, 0), rhi = min(ri + 2, t.nrows);
-        const int a0 = tab[rlo] + t.base[0], n0 = tab[rhi] + t.base[0] - a0;
-        const int a1 = tab[t.w + rlo] + t.base[1], n1 = tab[t.w + rhi] + t.base[1] - a1;
-        const int a2 = tab[2 * t.w + rlo] + t.base[2], n2 = tab[2 * t.w + rhi] + t.base[2] - a2;
-        const int tot = act ? n0 + n1 + n2 : 0;
-        // candidates kGroup at a time from one column slice, their LDS loads
-        // in flight together, appended without branches; slots past the
-        // slice's range are masked (they lie in the staged area or the next
-        // array of the wave's slots, positions coming first)
-        const int n01 = n0 + n1;
-        int cur = 0;
-        while (__any(cur < tot)) {
-          int cnt = 0;
-          while (cur < tot && cnt <= kList - kGroup) {
-            const bool in0 = cur < n0, in01 = cur < n01;
-            const int end = in0 ? n0 : (in01 ? n01 : tot);
-            const int j0 = cur + (in0 ? a0 : (in01 ? a1 - n0 : a2 - n01));
-            const int m = min(kGroup, end - cur);
-            float2 pp[kGroup];
+        } else {
+          const int rlo = max(ri - 1, 0), rhi = min(ri + 2, t.nrows);
+          const int a0 = tab[rlo] + t.base[0], n0 = tab[rhi] + t.base[0] - a0;
+          const int a1 = tab[t.w + rlo] + t.base[1], n1 = tab[t.w + rhi] + t.base[1] - a1;
+          const int a2 = tab[2 * t.w + rlo] + t.base[2], n2 = tab[2 * t.w + rhi] + t.base[2] - a2;
+          const int tot = act ? n0 + n1 + n2 : 0;
+          // candidates kGroup at a time from one column slice, their LDS loads
+          // in flight together, appended without branches; slots past the
+          // slice's range are masked (they lie in the staged area or the next
+          // array of the wave's slots, positions coming first)
+          const int n01 = n0 + n1;
+          int cur = 0;
+          while (__any(cur < tot)) {
+            int cnt = 0;
+            while (cur < tot && cnt <= kList - kGroup) {
+              const bool in0 = cur < n0, in01 = cur < n01;
+              const int end = in0 ? n0 : (in01 ? n01 : tot);
+              const int j0 = cur + (in0 ? a0 : (in01 ? a1 - n0 : a2 - n01));
+              const int m = min(kGroup, end - cur);
+              float2 pp[kGroup];
 #pragma unroll
-            for (int u = 0; u < kGroup; ++u) pp[u] = pol.pos_lds(L, j0 + u);
+              for (int u = 0; u < kGroup; ++u) pp[u] = pol.pos_lds(L, j0 + u);
 #pragma unroll
-            for (int u = 0; u < kGroup; ++u) {
-              const int j = j0 + u;
-              const bool cand = u < m && j != li;
-              ncand += cand;
-              const float drx = o.p.x - pp[u].x, dry = o.p.y - pp[u].y;
-              my_list[cnt * kWave] = (uint16_t)j;
-              cnt += cand && drx * drx + dry * dry < r2cut;
+              for (int u = 0; u < kGroup; ++u) {
+                const int j = j0 + u;
+                const bool cand = u < m && j != li;
+                ncand += cand;
+                const float drx = o.p.x - pp[u].x, dry = o.p.y - pp[u].y;
+                my_list[cnt * kWave] = (uint16_t)j;
+                cnt += cand && drx * drx + dry * dry < r2cut;
+              }
+              cur += m;
             }
-            cur += m;
-          }
-          npair += cnt;
-          for (int e = 0; e < cnt; ++e) {
-            const int j = my_list[e * kWave];
-            const float2 pj = pol.pos_lds(L, j);
-            const float drx = o.p.x - pj.x, dry = o.p.y - pj.y;
-            pol.pair_lds(acc, o, L, j, drx, dry, drx * drx + dry * dry);
+            npair += cnt;
+            for (int e = 0; e < cnt; ++e) {
+              const int j = my_list[e * kWave];
+              const float2 pj = pol.pos_lds(L, j);
+              const float drx = o.p.x - pj.x, dry = o.p.y - pj.y;
+              pol.pair_lds(acc, o, L, j, drx, dry, drx * drx + dry * dry);
+            }
           }
         }
+        if (act) pol.finish(acc, o, i);
       }
-      if (act) pol.finish(acc, o, i);
     }
-    }  // runs of rows
   }
   wave_count(npair, ncand, nact, counters);
 }
